@@ -99,6 +99,8 @@ struct cnd_ctx {
     // or cnd_step), 1..4 cnd_rk_stage(nk), 5 cnd_end_step
     int next_call = 0;
     bool any_gcbc = false, any_wall = false, any_avg = false, any_sponge = false, any_visc = false;
+    bool gcbc_dir[3] = {}, wall_dir[3] = {};   // directions with such faces
+    bool any_frame = false;   // some instance's frame accelerates (nsmf = 0)
     bool use_graph = false;
     hipGraphExec_t gexec = nullptr;
     // section timers

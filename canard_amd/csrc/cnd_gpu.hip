@@ -94,17 +94,22 @@ __device__ __forceinline__ double wave_max(double v)
 
 // Spectral-radius maxima of calc_time_step (src/mo_physics.f90:185-207);
 // runs only on steps where mod(n,10) == 1.  Each workgroup (one point tile)
-// folds its two maxima into its instance's (I.red, cleared at stage 1) with
+// folds its two maxima into its instance's (I.red, cleared by k_sched) with
 // an atomic max of their bit patterns, which order like the values for
 // non-negative doubles: the result does not depend on the order of the
 // workgroups.  A workgroup whose maximum does not exceed what it reads
 // there already skips the atomic.
-__global__ __launch_bounds__(kPts) void k_tstep(const BlkDev *__restrict__ blks, InstDev *__restrict__ inst,
-                                               const Tile *__restrict__ tiles, const double *__restrict__ q,
-                                               const double *__restrict__ met, int64_t NT)
+//
+// Nine launches of ten find no instance due, so the grid is at most
+// kTstepBlocks workgroups that walk the tiles, and they leave after one look
+// at the instances: one workgroup per tile spent 40 us of a 257^3 step on
+// 66 k workgroups that only returned.
+constexpr unsigned kTstepBlocks = 2048;   // 8 workgroups of 4 waves on each of 256 CUs
+
+__device__ __forceinline__ void tstep_tile(const Tile t, const BlkDev *__restrict__ blks, InstDev *__restrict__ inst,
+                                           const double *__restrict__ q, const double *__restrict__ met, int64_t NT,
+                                           double (&red)[2][kPts / 64])
 {
-    __shared__ double red[2][kPts / 64];
-    const Tile t = tiles[blockIdx.x];
     const BlkDev &B = blks[t.b];
     InstDev &I = inst[B.inst];
     if (I.n % 10 != 1) return;
@@ -143,6 +148,18 @@ __global__ __launch_bounds__(kPts) void k_tstep(const BlkDev *__restrict__ blks,
         if (a >= 0.0 && ab > seen[0]) atomicMax(&I.red[0], ab);
         if (c >= 0.0 && cb > seen[1]) atomicMax(&I.red[1], cb);
     }
+    __syncthreads();   // red is read
+}
+
+__global__ __launch_bounds__(kPts) void k_tstep(const BlkDev *__restrict__ blks, InstDev *__restrict__ inst, int ninst,
+                                               const Tile *__restrict__ tiles, int ntiles,
+                                               const double *__restrict__ q, const double *__restrict__ met, int64_t NT)
+{
+    __shared__ double red[2][kPts / 64];
+    int due = 0;
+    for (int i = threadIdx.x; i < ninst; i += kPts) due |= inst[i].n % 10 == 1;
+    if (!__syncthreads_or(due)) return;
+    for (int i = blockIdx.x; i < ntiles; i += gridDim.x) tstep_tile(tiles[i], blks, inst, q, met, NT, red);
 }
 
 // moving-frame velocity (src/mo_physics.f90:144-169)
@@ -162,8 +179,9 @@ __device__ void movef(InstDev &I, double dtko, double dtk)
     }
 }
 
-// Start of stage nk: frame velocity for fluxes (mo_canard_driver.f90:261-263)
-// and, in stage 1, clearing of the time-step maxima.
+// Start of stage nk: frame velocity for fluxes (mo_canard_driver.f90:261-263).
+// Launched only where some instance's frame accelerates (nsmf = 0); the others
+// keep the velocity upload_inst gave them.
 __global__ void k_stage_begin(InstDev *inst, int ninst, int nk)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -171,7 +189,6 @@ __global__ void k_stage_begin(InstDev *inst, int ninst, int nk)
     InstDev &I = inst[i];
     const int a = nk - 2 > 0 ? (nk - 2 < 1 ? nk - 2 : 1) : 0, c = nk - 1 < 1 ? nk - 1 : 1;
     movef(I, (I.dt * double(a)) / double(4 - nk + 3), (I.dt * double(c)) / double(4 - nk + 2));
-    if (nk == 1) { I.red[0] = 0ull; I.red[1] = 0ull; }
 }
 
 // dt schedule (mo_canard_driver.f90:278-285).
@@ -187,6 +204,8 @@ __global__ void k_sched(InstDev *inst, const TabDev *tabs, int ninst)
         double ra1 = ra0;
         if (I.viscous) ra1 = 0.5 / __longlong_as_double((long long)I.red[1]);
         I.dte = fmin(ra0, ra1);
+        I.red[0] = 0ull;   // for the next time they are due
+        I.red[1] = 0ull;
     }
     const int k = I.n - I.ndt;
     double r;
@@ -344,19 +363,39 @@ __device__ __forceinline__ double pressure(const double *q, int64_t NT, int64_t 
     return kGm1 * (q[4 * NT + g] - 0.5 * ((q2 * (q2 * ri) + q3 * (q3 * ri)) + q4 * (q4 * ri)));
 }
 
+// The face tiles of all three directions in one launch: blockIdx.x runs over
+// the tiles of direction 0, then 1, then 2.
+struct FaceSet {
+    const Tile *tiles[3];
+    int n0, n01;
+    double *sv[3];
+    int64_t FT[3];
+    __device__ Tile tile(int bx, int &d) const
+    {
+        d = bx < n0 ? 0 : (bx < n01 ? 1 : 2);
+        return tiles[d][bx - (d == 0 ? 0 : (d == 1 ? n0 : n01))];
+    }
+};
+
+struct Faces3 { const double *p[3]; };   // a face array per direction
+
 // gcbc_setup: characteristic transform of the face derivative (BC 10) or of
-// the full right-hand side (walls, curvilinear interfaces).  grid (tiles, side).
+// the full right-hand side (walls, curvilinear interfaces), the faces of all
+// directions in one launch.  grid (tiles, side).
 __global__ __launch_bounds__(kLine) void k_gcbc_setup(const BlkDev *__restrict__ blks,
-                                                     const InstDev *__restrict__ inst,
-                                                     const Tile *__restrict__ tiles, int d, const double *q,
-                                                     const double *de, const double *met, const double *cmf,
-                                                     double *drva, int64_t NT, int64_t FT)
+                                                     const InstDev *__restrict__ inst, const FaceSet fs,
+                                                     const Faces3 cmf3, const double *q, const double *de,
+                                                     const double *met, int64_t NT)
 {
-    const Tile t = tiles[blockIdx.x];
+    int d;
+    const Tile t = fs.tile(blockIdx.x, d);
     const BlkDev &B = blks[t.b];
     const int side = blockIdx.y, qq = t.q0 + threadIdx.x;
     const int code = B.bc[d][side];
     if (qq >= npencils(B, d) || !is_gcbc(code)) return;
+    double *drva = fs.sv[d];
+    const double *cmf = cmf3.p[d];
+    const int64_t FT = fs.FT[d];
     int64_t g, st;
     face_point(B, d, qq, side, g, st);
     const int64_t fi = B.foff[d] + qq;
@@ -376,28 +415,42 @@ __global__ __launch_bounds__(kLine) void k_gcbc_setup(const BlkDev *__restrict__
     }
 }
 
-// gcbc_update of face (d, side); faces are applied in the reference's order.
-__global__ __launch_bounds__(kLine) void k_gcbc_update(const BlkDev *__restrict__ blks,
-                                                      const InstDev *__restrict__ inst,
-                                                      const TabDev *__restrict__ tabs,
-                                                      const Tile *__restrict__ tiles, int d, int side,
-                                                      const double *q, double *de, const double *met,
-                                                      const double *cmf, const double *drva, int64_t NT, int64_t FT)
+// gcbc_update of both faces of direction d (blockIdx.y; their bands of
+// kGcbcBand points never meet, a block having 13 points or more); the
+// directions follow each other in the reference's order.  Bound by latency:
+// a face has few points, each a long chain of loads and divisions, so every
+// point of the band has its own lane (threadIdx.y, one wave each) that forms
+// the face's correction itself, instead of one lane walking the band (13 us
+// a launch on faces of 80 x 70 points, at six launches a stage).
+constexpr int kGcbcBand = 5;
+__global__ __launch_bounds__(kLine * kGcbcBand) void k_gcbc_update(const BlkDev *__restrict__ blks,
+                                                                  const InstDev *__restrict__ inst,
+                                                                  const TabDev *__restrict__ tabs,
+                                                                  const Tile *__restrict__ tiles, int d,
+                                                                  const double *q, double *de, const double *met,
+                                                                  const double *cmf, const double *drva, int64_t NT,
+                                                                  int64_t FT)
 {
     const Tile t = tiles[blockIdx.x];
     const BlkDev &B = blks[t.b];
-    const int qq = t.q0 + threadIdx.x;
+    const int side = blockIdx.y, qq = t.q0 + threadIdx.x, ii = threadIdx.y;
     const int code = B.bc[d][side];
     if (qq >= npencils(B, d) || !is_gcbc(code)) return;
     const InstDev &I = inst[B.inst];
-    int64_t g, st;
-    face_point(B, d, qq, side, g, st);
+    int64_t base, st;
+    pencil_of(B, d, qq, base, st);
+    const int i0 = side == 0 ? 0 : B.n[d] - 1, ip = side == 0 ? ii : i0 - ii;
+    const int64_t g = base + int64_t(i0) * st, gl = base + int64_t(ip) * st;
+    // the right-hand side of the lane's own point, loaded with the face's data
+    double tot[5];
+    for (int c = 0; c < 5; ++c) tot[c] = (de[c * NT + gl] + de[(5 + c) * NT + gl]) + de[(10 + c) * NT + gl];
     const int64_t fi = B.foff[d] + qq;
     const double ra0 = side == 0 ? 1.0 : -1.0;
     double cm[3], q24[3], cha[5], dha[5], dif[5], xt[5][5];
     for (int c = 0; c < 3; ++c) { cm[c] = cmf[(side * 3 + c) * FT + fi]; q24[c] = q[(c + 1) * NT + g]; }
     const Elem e = eleme(cm, q[g], q24, pressure(q, NT, g), I.umf);
     for (int c = 0; c < 5; ++c) cha[c] = drva[(side * 5 + c) * FT + fi];
+    for (int c = 0; c < 5; ++c) dif[c] = cha[c];
     if (code == 10) {
         if (ra0 * ((e.vn + e.vs) + e.ao) > 0.0) cha[3] = 0.0;
         if (ra0 * ((e.vn + e.vs) - e.ao) > 0.0) cha[4] = 0.0;
@@ -415,7 +468,7 @@ __global__ __launch_bounds__(kLine) void k_gcbc_update(const BlkDev *__restrict_
         if (ra0 * ((e.vn + e.vs) - e.ao) > 0.0) cha[4] = dha[4];
     }
     xtr2q(e, cm, xt);
-    for (int c = 0; c < 5; ++c) dif[c] = cha[c] - drva[(side * 5 + c) * FT + fi];
+    for (int c = 0; c < 5; ++c) dif[c] = cha[c] - dif[c];
     for (int r = 0; r < 5; ++r) {
         double s = 0.0;
         for (int c = 0; c < 5; ++c) s = s + xt[r][c] * dif[c];
@@ -425,45 +478,34 @@ __global__ __launch_bounds__(kLine) void k_gcbc_update(const BlkDev *__restrict_
     // point, scaled by sbci for inward points, divided by the number of
     // characteristic faces whose 5-point band covers the point.
     const double res = 1.0 / met[9 * NT + g];
-    const int sgn = side == 0 ? 1 : -1;
-    int64_t base; int64_t st2;
-    pencil_of(B, d, qq, base, st2);
-    const int i0 = side == 0 ? 0 : B.n[d] - 1;
-    for (int ii = 0; ii <= 4; ++ii) {
-        const int ip = i0 + sgn * ii;
-        const int64_t gl = base + int64_t(ip) * st2;
-        const int64_t lloc = gl - B.off;
-        int idx[3];
-        idx[0] = int(lloc % B.n[0]);
-        idx[1] = int((lloc / B.n[0]) % B.n[1]);
-        idx[2] = int(lloc / (int64_t(B.n[0]) * B.n[1]));
-        int cnt = 0;
-        for (int dd = 0; dd < 3; ++dd)
-            for (int s = 0; s < 2; ++s)
-                if (is_gcbc(B.bc[dd][s])) {
-                    const int dist = s == 0 ? idx[dd] : B.n[dd] - 1 - idx[dd];
-                    if (dist <= 4) ++cnt;
-                }
-        const double wv = ii == 0 ? res : res * tabs[B.inst].gcbc_w[ii - 1];
-        const double sbcc = wv / double(cnt);
-        // the right-hand side is the sum of the three direction buffers: the
-        // corrected sum goes to the first, the others are cleared
-        for (int c = 0; c < 5; ++c) {
-            const double tot = (de[c * NT + gl] + de[(5 + c) * NT + gl]) + de[(10 + c) * NT + gl];
-            de[c * NT + gl] = tot + sbcc * dha[c];
-            de[(5 + c) * NT + gl] = 0.0;
-            de[(10 + c) * NT + gl] = 0.0;
-        }
+    const int w = d == 0 ? B.n[1] : B.n[0], qa = qq % w, qb = qq / w;   // pencil_of's transverse indices
+    const int idx[3] = {d == 0 ? ip : qa, d == 1 ? ip : (d == 0 ? qa : qb), d == 2 ? ip : qb};
+    int cnt = 0;
+    for (int dd = 0; dd < 3; ++dd)
+        for (int s = 0; s < 2; ++s)
+            if (is_gcbc(B.bc[dd][s])) {
+                const int dist = s == 0 ? idx[dd] : B.n[dd] - 1 - idx[dd];
+                if (dist < kGcbcBand) ++cnt;
+            }
+    const double wv = ii == 0 ? res : res * tabs[B.inst].gcbc_w[ii - 1];
+    const double sbcc = wv / double(cnt);
+    // the right-hand side is the sum of the three direction buffers: the
+    // corrected sum goes to the first, the others are cleared
+    for (int c = 0; c < 5; ++c) {
+        de[c * NT + gl] = tot[c] + sbcc * dha[c];
+        de[(5 + c) * NT + gl] = 0.0;
+        de[(10 + c) * NT + gl] = 0.0;
     }
 }
 
-// wall_condition_update (mo_gcbc.f90:424-459) on face (d, side)
+// wall_condition_update (mo_gcbc.f90:424-459) on both faces of direction d
+// (blockIdx.y)
 __global__ __launch_bounds__(kLine) void k_wall(const BlkDev *__restrict__ blks, const InstDev *__restrict__ inst,
-                                               const Tile *__restrict__ tiles, int d, int side, double *q, int64_t NT)
+                                               const Tile *__restrict__ tiles, int d, double *q, int64_t NT)
 {
     const Tile t = tiles[blockIdx.x];
     const BlkDev &B = blks[t.b];
-    const int qq = t.q0 + threadIdx.x;
+    const int side = blockIdx.y, qq = t.q0 + threadIdx.x;
     const int code = B.bc[d][side];
     if (qq >= npencils(B, d) || (code != 20 && code != 25)) return;
     int64_t g, st;
@@ -529,20 +571,6 @@ __global__ void k_junc_scatter(const JuncDev J, double *q, int64_t NT)
     if (i >= J.n || !J.write[i]) return;
     q[m * NT + J.tgt[i]] = J.tmp[m * int64_t(J.n) + i];
 }
-
-// The face tiles of all three directions in one launch: blockIdx.x runs over
-// the tiles of direction 0, then 1, then 2.
-struct FaceSet {
-    const Tile *tiles[3];
-    int n0, n01;
-    double *sv[3];
-    int64_t FT[3];
-    __device__ Tile tile(int bx, int &d) const
-    {
-        d = bx < n0 ? 0 : (bx < n01 ? 1 : 2);
-        return tiles[d][bx - (d == 0 ? 0 : (d == 1 ? n0 : n01))];
-    }
-};
 
 // pencil of direction d through point (i, j, k) (the inverse of pencil_of)
 __device__ __forceinline__ int pencil_at(const BlkDev &B, int d, const int idx[3])
@@ -717,6 +745,7 @@ int upload_inst(cnd_ctx *c)
         I.srefoo = 111 / p.tempoo;
         I.srefp1dre = (I.srefoo + 1.0) / I.reoo;
         I.uoo[0] = p.amach1; I.uoo[1] = p.amach2; I.uoo[2] = p.amach3;
+        if (p.nsmf != 0) std::memcpy(I.umf, I.uoo, sizeof I.umf);   // a steady frame: movef's values, dudtmf = 0
         I.timf = p.timf; I.cfl = p.cfl; I.nsmf = p.nsmf; I.viscous = p.viscous; I.sponge = p.sponge;
         I.ndata = 0;
         I.ndati = -1;
@@ -822,11 +851,22 @@ int join_side(cnd_ctx *c)
     return CND_OK;
 }
 
+// The faces of all three directions with an array per direction.
+FaceSet face_set(cnd_ctx *c, double *const (&arr)[3])
+{
+    FaceSet fs;
+    for (int d = 0; d < 3; ++d) { fs.tiles[d] = c->dtiles[d]; fs.sv[d] = arr[d]; fs.FT[d] = c->FT[d]; }
+    fs.n0 = ntiles(c, 0);
+    fs.n01 = ntiles(c, 0) + ntiles(c, 1);
+    return fs;
+}
+dim3 faces_grid(cnd_ctx *c) { return dim3(unsigned(ntiles(c, 0) + ntiles(c, 1) + ntiles(c, 2)), 2); }
+
 int enqueue_stage(cnd_ctx *c, int nk)
 {
     const double *cur = nk == 1 ? c->qo : c->qa;
     const unsigned ib = unsigned((c->ninst + 63) / 64);
-    hipLaunchKernelGGL(k_stage_begin, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst, nk);
+    if (c->any_frame) hipLaunchKernelGGL(k_stage_begin, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst, nk);
     int r;
     // the time step of stage 1 runs beside the xi gradient sweep of viscous
     // stages, which reads neither dt nor the maxima (its time then counts in
@@ -834,8 +874,9 @@ int enqueue_stage(cnd_ctx *c, int nk)
     const bool tstep_side = nk == 1 && c->any_visc && c->overlap;
     if (nk == 1) {
         auto tstep = [&] {
-            hipLaunchKernelGGL(k_tstep, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dinst, c->dpt, cur, c->met,
-                               c->NT);
+            const int npt = int(c->hpt.size());
+            hipLaunchKernelGGL(k_tstep, dim3(std::min(unsigned(npt), kTstepBlocks)), dim3(kPts), 0, c->st, c->dblk,
+                               c->dinst, c->ninst, c->dpt, npt, cur, c->met, c->NT);
             hipLaunchKernelGGL(k_sched, dim3(ib), dim3(64), 0, c->st, c->dinst, c->dtab, c->ninst);
             return check_launch(c);
         };
@@ -881,15 +922,15 @@ int enqueue_stage(cnd_ctx *c, int nk)
     }
     }
     if (c->any_gcbc) {
-        Section sec(c, CND_SEC_GCBC, 9);
+        const FaceSet fs = face_set(c, c->drva);
+        Section sec(c, CND_SEC_GCBC, 1 + c->gcbc_dir[0] + c->gcbc_dir[1] + c->gcbc_dir[2]);
+        hipLaunchKernelGGL(k_gcbc_setup, faces_grid(c), dim3(kLine), 0, c->st, c->dblk, c->dinst, fs,
+                           Faces3{{c->cmf[0], c->cmf[1], c->cmf[2]}}, cur, c->de, c->met, c->NT);
         for (int d = 0; d < 3; ++d)
-            hipLaunchKernelGGL(k_gcbc_setup, tiles_grid(c, d, 2), dim3(kLine), 0, c->st, c->dblk, c->dinst,
-                               c->dtiles[d], d, cur, c->de, c->met, c->cmf[d], c->drva[d], c->NT, c->FT[d]);
-        for (int d = 0; d < 3; ++d)
-            for (int s = 0; s < 2; ++s)
-                hipLaunchKernelGGL(k_gcbc_update, tiles_grid(c, d, 1), dim3(kLine), 0, c->st, c->dblk, c->dinst,
-                                   c->dtab, c->dtiles[d], d, s, cur, c->de, c->met, c->cmf[d], c->drva[d], c->NT,
-                                   c->FT[d]);
+            if (c->gcbc_dir[d])
+                hipLaunchKernelGGL(k_gcbc_update, tiles_grid(c, d, 2), dim3(kLine, kGcbcBand), 0, c->st, c->dblk,
+                                   c->dinst, c->dtab, c->dtiles[d], d, cur, c->de, c->met, c->cmf[d], c->drva[d],
+                                   c->NT, c->FT[d]);
     }
     if (fused) {
         Section sec(c, CND_SEC_UPDATE, 1);
@@ -903,24 +944,20 @@ int enqueue_stage(cnd_ctx *c, int nk)
     // (and, after the step, by the output); without walls the next stage's
     // frame velocity replaces it unread, and stage 4's is set at the end of
     // the step.
-    if (c->any_wall) hipLaunchKernelGGL(k_stage_mid, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst, nk);
+    if (c->any_wall && c->any_frame) hipLaunchKernelGGL(k_stage_mid, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst, nk);
     Section avg(c, CND_SEC_AVG, 1);
-    if (c->any_wall)
-        for (int d = 0; d < 3; ++d)
-            for (int s = 0; s < 2; ++s)
-                hipLaunchKernelGGL(k_wall, tiles_grid(c, d, 1), dim3(kLine), 0, c->st, c->dblk, c->dinst,
-                                   c->dtiles[d], d, s, c->qa, c->NT);
+    for (int d = 0; d < 3; ++d)
+        if (c->wall_dir[d])
+            hipLaunchKernelGGL(k_wall, tiles_grid(c, d, 2), dim3(kLine), 0, c->st, c->dblk, c->dinst, c->dtiles[d], d,
+                               c->qa, c->NT);
     if (c->jn.n > 0) {
         const unsigned nb = unsigned((c->jn.n + 127) / 128);
         hipLaunchKernelGGL(k_junc_gather, dim3(nb, 5), dim3(128), 0, c->st, c->jn, c->qa, c->NT);
         hipLaunchKernelGGL(k_junc_scatter, dim3(nb, 5), dim3(128), 0, c->st, c->jn, c->qa, c->NT);
     }
     if (c->any_avg) {
-        FaceSet fs;
-        for (int d = 0; d < 3; ++d) { fs.tiles[d] = c->dtiles[d]; fs.sv[d] = c->surf[d]; fs.FT[d] = c->FT[d]; }
-        fs.n0 = ntiles(c, 0);
-        fs.n01 = ntiles(c, 0) + ntiles(c, 1);
-        const dim3 grid(unsigned(fs.n01 + ntiles(c, 2)), 2);
+        const FaceSet fs = face_set(c, c->surf);
+        const dim3 grid = faces_grid(c);
         hipLaunchKernelGGL(k_surf_snap, grid, dim3(kLine), 0, c->st, c->dblk, fs, c->qa, c->NT);
         hipLaunchKernelGGL(k_surf_avg, grid, dim3(kLine), 0, c->st, c->dblk, fs, c->qa, c->NT);
     }
@@ -930,7 +967,8 @@ int enqueue_stage(cnd_ctx *c, int nk)
 int enqueue_end(cnd_ctx *c)
 {
     const unsigned ib = unsigned((c->ninst + 63) / 64);
-    hipLaunchKernelGGL(k_end_step, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst, c->any_wall ? 0 : 1);
+    hipLaunchKernelGGL(k_end_step, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst,
+                       c->any_frame && !c->any_wall ? 1 : 0);
     if (c->recording) {
         hipLaunchKernelGGL(k_record, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dinst, c->dpt, c->qo, c->qa,
                            c->qb, c->NT);
@@ -988,6 +1026,7 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
             delete c;
             return fail(nullptr, CND_EINVAL, "sponge needs szth0 > 0 and szth1 > 0");
         }
+        c->any_frame |= p.nsmf == 0;
         if (p.nsmf == 0 && !(p.timf > 0.0)) { delete c; return fail(nullptr, CND_EINVAL, "nsmf = 0 needs timf > 0"); }
     }
     for (int b = 0; b < nblocks; ++b) {
@@ -1021,9 +1060,9 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
                 B.qd[d][e] = (cd == kInterStraight || cd == kInterSub || cd == kPeriodic) ? 1 : 0;
                 if (B.qd[d][e] && B.part[d][e] != b) c->part_other[d] = true;
                 if (cd == kNonReflective || cd == kWallInviscid || cd == kWallViscous || cd == kInterCurv) {
-                    c->any_gcbc = true; B.gcbc_any = 1;
+                    c->any_gcbc = c->gcbc_dir[d] = true; B.gcbc_any = 1;
                 }
-                if (cd == kWallInviscid || cd == kWallViscous) c->any_wall = true;
+                if (cd == kWallInviscid || cd == kWallViscous) c->any_wall = c->wall_dir[d] = true;
                 if (cd == kInterCurv || cd == kInterStraight || cd == kPeriodic) c->any_avg = true;
             }
         }
@@ -1206,9 +1245,9 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
     if (!r) {
         JunctionPlan pc, pe;
         junction_plans(c->spec, c->off, pc, pe);
-        const JunctionProgram p = junction_program(pc, pe);
+        JunctionProgram p = junction_program(pc, pe);
         JuncDev &j = c->jn;
-        j.n = int(p.target.size());
+        j.n = drop_self_averages(p) > 0 ? int(p.target.size()) : 0;
         if (j.n > 0 &&
             !((r = dalloc(c, &j.tgt, p.target.size())) || (r = dalloc(c, &j.src, p.src.size())) ||
               (r = dalloc(c, &j.first, p.first.size())) || (r = dalloc(c, &j.tc, p.tc.size())) ||

@@ -520,4 +520,20 @@ JunctionProgram junction_program(const JunctionPlan &corners, const JunctionPlan
     return p;
 }
 
+int drop_self_averages(JunctionProgram &p)
+{
+    const int n = int(p.target.size());
+    std::vector<char> self(n, 0);   // corners come first, so an edge finds its corners' marks set
+    int left = 0;
+    for (int i = 0; i < n; ++i) {
+        bool own = p.tc[i] < 0 || self[p.tc[i]];
+        for (int k = p.first[i]; k < p.first[i + 1] && own; ++k)
+            own = p.src[k] == p.target[i] && (p.sc[k] < 0 || self[p.sc[k]]);
+        self[i] = own;
+        if (own) p.write[i] = 0;
+        left += p.write[i] != 0;
+    }
+    return left;
+}
+
 }  // namespace cnd

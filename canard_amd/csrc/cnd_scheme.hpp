@@ -122,4 +122,11 @@ struct JunctionProgram {
 };
 JunctionProgram junction_program(const JunctionPlan &corners, const JunctionPlan &edges);
 
+// Clears write for every entry that averages a point with copies of itself
+// only (all corners and edges of a block that is its own periodic partner:
+// its messages come back to the item that sent them), which leaves the point
+// as it is up to the rounding of the sum.  Returns the entries that still
+// write; with none the averaging needs no launch.
+int drop_self_averages(JunctionProgram &p);
+
 }  // namespace cnd
