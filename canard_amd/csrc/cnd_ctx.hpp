@@ -87,10 +87,7 @@ struct cnd_ctx {
     bool part_other[3] = {};   // some block has another block as interface partner along d
     int64_t ys_len = 0;        // doubles in the forward-value scratch
     double *drva[3] = {}, *cmf[3] = {}, *surf[3] = {};
-    // mixed precision: FP32 gradients and stresses; FP32 LU / homogeneous
-    // tables and the FP64 banded LHS for the refinement
-    float *gradf = nullptr, *dlu32 = nullptr, *dseg32[kNumL] = {};
-    double *dlhs = nullptr;
+    float *gradf = nullptr;   // mixed precision: the gradients in FP32
     JuncDev jn;
     std::vector<char> grid_set;
     bool metrics_ready = false, state_in_qo = false;
@@ -159,51 +156,55 @@ inline dim3 pts_grid(cnd_ctx *c) { return dim3(unsigned(c->hpt.size())); }
 
 
 inline int ntiles(cnd_ctx *c, int d) { return int(c->htiles[d].size()); }
-// Launch the segmented sweep K<G, MIX> (NV variables) for kind along d with
-// the shape chosen for them; the arguments after the common ones follow.
-#define SEG_CASE(i, K, MIX, NV, c, kind, d, xm, y, ...)                                                    \
+// Launch the segmented sweep K (a template-id of the shape G, in parentheses;
+// NV variables) for kind along d with the shape chosen for them; the arguments after the common ones follow.
+#define SEG_CASE(i, K, NV, c, kind, d, xm, y, ...)                                                    \
     case i: {                                                                                              \
         using G = Sh##i;                                                                                   \
         const int sp_ = (c)->seg_sp[kind][d];                                                              \
         const int pi_ = p_index(G::P);                                                                     \
         const int nt_ = int((c)->hstiles[pi_][d].size());                                                  \
-        hipLaunchKernelGGL((K<G, MIX>), dim3(unsigned(xcd_width((xm) * nt_)), unsigned(y)),                \
+        hipLaunchKernelGGL(K, dim3(unsigned(xcd_width((xm) * nt_)), unsigned(y)),                \
                            dim3(unsigned((NV) * G::P * sp_)),                                              \
                            (SegShape<NV, 0, G::L, G::P, G::C, G::XI>::lds_bytes(sp_, G::SPMAX, (c)->nmax[d],     \
                                                                                 (c)->part_other[d])),              \
                            (c)->st, (c)->dblk,                                                             \
                            (c)->dtab, seg_tabs(c, G::L), (c)->dstiles[pi_][d], nt_, sp_, d, __VA_ARGS__);   \
     } break;
-#define LAUNCH_SEG_XM(K, MIX, NV, c, kind, d, xm, y, ...)                                                       \
+#define LAUNCH_SEG_XM(K, NV, c, kind, d, xm, y, ...)                                                       \
     do {                                                                                                   \
         switch ((c)->shape[kind][d]) {                                                                     \
-            SEG_CASE(0, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(1, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(2, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(3, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(4, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(5, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(6, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(7, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(8, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(9, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(10, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(11, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(12, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(13, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(14, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(15, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(16, K, MIX, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
+            SEG_CASE(0, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
+            SEG_CASE(1, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
+            SEG_CASE(2, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
+            SEG_CASE(3, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
+            SEG_CASE(4, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
+            SEG_CASE(5, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
+            SEG_CASE(6, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
+            SEG_CASE(7, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
+            SEG_CASE(8, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
+            SEG_CASE(9, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
+            SEG_CASE(10, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
+            SEG_CASE(11, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
+            SEG_CASE(12, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
+            SEG_CASE(13, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
+            SEG_CASE(14, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
+            SEG_CASE(15, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
+            SEG_CASE(16, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
+            SEG_CASE(17, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
+            SEG_CASE(18, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
+            SEG_CASE(19, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
+            SEG_CASE(20, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
             default: break;                                                                                \
         }                                                                                                  \
     } while (0)
 // grid x covers xm * tiles workgroups (kernels that split a tile's work
 // over xm workgroups themselves); LAUNCH_SEG: one workgroup per tile and y
-#define LAUNCH_SEG(K, MIX, NV, c, kind, d, y, ...) LAUNCH_SEG_XM(K, MIX, NV, c, kind, d, 1, y, __VA_ARGS__)
+#define LAUNCH_SEG(K, NV, c, kind, d, y, ...) LAUNCH_SEG_XM(K, NV, c, kind, d, 1, y, __VA_ARGS__)
 
 inline SegTabs seg_tabs(cnd_ctx *c, int L)
 {
-    return SegTabs{c->dlu, c->dseg[l_index(L)], c->dlhs, c->dlu32, c->dseg32[l_index(L)]};
+    return SegTabs{c->dlu, c->dseg[l_index(L)]};
 }
 inline bool seg_on(cnd_ctx *c, int kind, int d) { return c->shape[kind][d] != kTiled; }
 
@@ -230,10 +231,9 @@ inline bool fuse_possible(const cnd_ctx *c)
 
 // Sweep launches, one translation unit per sweep kind (cnd_run_*.hip).
 // Filter (kind CND_KIND_FILTER) and plain derivative (CND_KIND_FIELD) sweeps
-// of nvar fields; mix: FP32 solves with FP64 refinement (segmented only).
-int run_filter_field(cnd_ctx *c, int d, const double *in, double *out, int nvar, bool mix = false);
-int run_fd_field(cnd_ctx *c, int d, int n45, const double *in, int64_t ivs, double *out, int64_t ovs, int nvar,
-                 bool mix = false);
+// of nvar fields.
+int run_filter_field(cnd_ctx *c, int d, const double *in, double *out, int nvar);
+int run_fd_field(cnd_ctx *c, int d, int n45, const double *in, int64_t ivs, double *out, int64_t ovs, int nvar);
 // Gradient sweep along d of the state cur (kind CND_KIND_GRAD).  The xi
 // sweep (d = 0) also stores the primitives u, v, w, T in the flux scratch
 // fl, and the eta and zeta sweeps (segmented) differentiate those: the

@@ -803,7 +803,7 @@ int shape_sp(cnd_ctx *c, int sh, int d, int nv)
     int sp = 1;
     for (const BlockSpec &B : c->spec) {
         const int S = seg_count(B.n[d], G.L);
-        if (S == 0) return 0;
+        if (S == 0 || B.n[d] > kSegMaxPoints) return 0;
         sp = std::max(sp, S);
     }
     if (sp > G.SPMAX) return 0;
@@ -822,10 +822,9 @@ int enqueue_filter(cnd_ctx *c)
 {
     Section sec(c, CND_SEC_FILTER, 3);
     int r;
-    const bool mix = c->precision == CND_MIXED;
-    if ((r = run_filter_field(c, 1, c->qa, c->qo, 5, mix))) return r;
-    if ((r = run_filter_field(c, 2, c->qo, c->qa, 5, mix))) return r;
-    if ((r = run_filter_field(c, 0, c->qa, c->qo, 5, mix))) return r;
+    if ((r = run_filter_field(c, 1, c->qa, c->qo, 5))) return r;
+    if ((r = run_filter_field(c, 2, c->qo, c->qa, 5))) return r;
+    if ((r = run_filter_field(c, 0, c->qa, c->qo, 5))) return r;
     return CND_OK;
 }
 
@@ -888,7 +887,7 @@ int enqueue_stage(cnd_ctx *c, int nk)
         Section sec(c, CND_SEC_GRAD, 3);
         if ((r = run_grad(c, 0, cur))) return r;
         if (tstep_side && (r = join_side(c))) return r;
-        if (c->overlap && (c->precision == CND_MIXED || seg_on(c, CND_KIND_GRAD, 1))) {
+        if (c->overlap && seg_on(c, CND_KIND_GRAD, 1)) {
             if ((r = on_side(c, [&] { return run_grad(c, 1, cur); })) || (r = run_grad(c, 2, cur)) ||
                 (r = join_side(c)))
                 return r;
@@ -906,13 +905,13 @@ int enqueue_stage(cnd_ctx *c, int nk)
             hipLaunchKernelGGL(k_visc_flux<double>, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dinst, c->dpt,
                                cur, c->grad, c->met, c->fl, c->NT);
     }
-    const bool fused = fuse_possible(c) && (c->precision == CND_MIXED || seg_on(c, CND_KIND_FLUX, c->fuse_dir));
+    const bool fused = fuse_possible(c) && seg_on(c, CND_KIND_FLUX, c->fuse_dir);
     {
     // the flux sweeps the update does not take in, the eta one beside the
     // others when it is a segmented one
     Section sec(c, CND_SEC_FLUX, fused ? 2 : 3);
     const int other = fused && c->fuse_dir == 0 ? 2 : 0;
-    if (c->overlap && (c->precision == CND_MIXED || seg_on(c, CND_KIND_FLUX, 1))) {
+    if (c->overlap && seg_on(c, CND_KIND_FLUX, 1)) {
         if ((r = on_side(c, [&] { return run_flux(c, 1, cur); })) || (r = run_flux(c, other, cur)) ||
             (!fused && (r = run_flux(c, 2, cur))) || (r = join_side(c)))
             return r;
@@ -1044,7 +1043,7 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
     for (int i = 0; i < ninst; ++i) build_tables(params[i].fltk, params[i].fltrbc, c->htab[i]);
 
     // layout
-    std::vector<double> lu, segtab[kNumL], lhs;
+    std::vector<double> lu, segtab[kNumL];
     c->hblk.resize(nblocks);
     int64_t off = 0, foff[3] = {0, 0, 0};
     for (int b = 0; b < nblocks; ++b) {
@@ -1085,8 +1084,6 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
                 const size_t at = lu.size();
                 lu.resize(at + 5 * size_t(s.n[d]));
                 lu_factors(c->htab[s.inst], sch, s.n[d], B.qd[d][0] != 0, B.qd[d][1] != 0, lu.data() + at);
-                lhs.resize(lu.size());
-                lhs_rows(c->htab[s.inst], sch, s.n[d], B.qd[d][0] != 0, B.qd[d][1] != 0, lhs.data() + at);
                 const int nd = s.n[d];
                 for (int li = 0; li < kNumL; ++li) {
                     const int SL = kLs[li], S = seg_count(nd, SL);
@@ -1181,11 +1178,7 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
                 ok(dalloc(c, &c->sp_par, 5 * ninst));
     for (int li = 0; good && li < kNumL; ++li) good = ok(dalloc(c, &c->dseg[li], segtab[li].size()));
     if (good && c->any_sponge) good = ok(dalloc(c, &c->sponge, 2 * NT));
-    if (good && precision == CND_MIXED)
-        good = ok(dalloc(c, &c->gradf, 12 * NT)) &&
-               ok(dalloc(c, &c->dlu32, lu.size())) && ok(dalloc(c, &c->dlhs, lhs.size()));
-    for (int li = 0; good && precision == CND_MIXED && li < kNumL; ++li)
-        good = ok(dalloc(c, &c->dseg32[li], segtab[li].size()));
+    if (good && precision == CND_MIXED) good = ok(dalloc(c, &c->gradf, 12 * NT));
     for (int d = 0; good && d < 3; ++d)
         good = ok(dalloc(c, &c->dtiles[d], c->htiles[d].size())) && ok(dalloc(c, &c->drva[d], 10 * c->FT[d])) &&
                ok(dalloc(c, &c->cmf[d], 6 * c->FT[d])) && ok(dalloc(c, &c->surf[d], 10 * c->FT[d]));
@@ -1225,15 +1218,6 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
         for (int d = 0; d < 3; ++d)
             up(c->dstiles[pi][d], c->hstiles[pi][d].data(), sizeof(Tile) * c->hstiles[pi][d].size());
     for (int li = 0; li < kNumL; ++li) up(c->dseg[li], segtab[li].data(), sizeof(double) * segtab[li].size());
-    if (precision == CND_MIXED) {
-        const std::vector<float> lu32(lu.begin(), lu.end());
-        up(c->dlu32, lu32.data(), sizeof(float) * lu32.size());
-        for (int li = 0; li < kNumL; ++li) {
-            const std::vector<float> seg32(segtab[li].begin(), segtab[li].end());
-            up(c->dseg32[li], seg32.data(), sizeof(float) * seg32.size());
-        }
-        up(c->dlhs, lhs.data(), sizeof(double) * lhs.size());
-    }
     up(c->dpt, c->hpt.data(), sizeof(Tile) * c->hpt.size());
     if (!r) r = upload_inst(c);
     if (!r) {
@@ -1278,13 +1262,11 @@ void cnd_destroy(cnd_ctx *c)
     for (auto &m : c->marks) { hipEventDestroy(m.a); hipEventDestroy(m.b); }
     for (hipEvent_t e : c->pool) hipEventDestroy(e);
     void *ptrs[] = {c->dblk, c->dtab, c->dinst, c->dlu, c->qa, c->qo, c->de, c->grad, c->fl, c->met, c->ys,
-                    c->xyz, c->sponge, c->sp_par, c->dpt, c->gradf, c->dlu32, c->dlhs, c->jn.tgt, c->jn.src,
+                    c->xyz, c->sponge, c->sp_par, c->dpt, c->gradf, c->jn.tgt, c->jn.src,
                     c->jn.first, c->jn.tc, c->jn.sc, c->jn.write, c->jn.scale, c->jn.tmp, c->qb};
     for (void *p : ptrs) if (p) hipFree(p);
-    for (int li = 0; li < kNumL; ++li) {
+    for (int li = 0; li < kNumL; ++li)
         if (c->dseg[li]) hipFree(c->dseg[li]);
-        if (c->dseg32[li]) hipFree(c->dseg32[li]);
-    }
     for (int d = 0; d < 3; ++d) {
         if (c->dtiles[d]) hipFree(c->dtiles[d]);
         for (int pi = 0; pi < kNumP; ++pi)
@@ -1432,7 +1414,7 @@ static int tune(cnd_ctx *c)
     // fused with the update (into the gradient scratch) where fusion applies
     const bool fz = fuse_possible(c);
     auto run = [&](int kind, int d) {
-        if (kind == CND_KIND_FILTER) return run_filter_field(c, d, c->qa, c->fl, 5, mix);
+        if (kind == CND_KIND_FILTER) return run_filter_field(c, d, c->qa, c->fl, 5);
         if (kind == CND_KIND_GRAD) return run_grad(c, d, c->qa);
         if (d == c->fuse_dir && fz) return run_flux_update(c, 1, c->grad);
         return run_flux(c, d, c->qa);
@@ -1670,7 +1652,7 @@ int cnd_deriv_sweep(cnd_ctx *c, int dir, const double *const *in, double *const 
     int r;
     double *a = c->fl, *o = c->fl + c->NT;   // scratch fields
     if ((r = sweep_io(c, in, a))) return r;
-    if ((r = run_fd_field(c, dir, 0, a, 0, o, 0, 1, c->precision == CND_MIXED))) return r;
+    if ((r = run_fd_field(c, dir, 0, a, 0, o, 0, 1))) return r;
     return sweep_out(c, o, out);
 }
 
@@ -1680,7 +1662,7 @@ int cnd_filter_sweep(cnd_ctx *c, int dir, double *const *f)
     int r;
     double *a = c->fl, *o = c->fl + c->NT;   // scratch fields
     if ((r = sweep_io(c, (const double *const *)f, a))) return r;
-    if ((r = run_filter_field(c, dir, a, o, 1, c->precision == CND_MIXED))) return r;
+    if ((r = run_filter_field(c, dir, a, o, 1))) return r;
     return sweep_out(c, o, f);
 }
 

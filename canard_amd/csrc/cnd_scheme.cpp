@@ -241,23 +241,6 @@ static void end_rows(const Tables &t, int scheme, bool qd, double (*r)[5])
     }
 }
 
-void lhs_rows(const Tables &t, int scheme, int n, bool qd_lo, bool qd_hi, double *o)
-{
-    double lo[3][5], hi[3][5];
-    end_rows(t, scheme, qd_lo, lo);
-    end_rows(t, scheme, qd_hi, hi);
-    const double al = scheme == 0 ? kAl : t.alf, be = scheme == 0 ? kBe : t.bef;
-    for (int i = 0; i < n; ++i) {
-        double *r = o + 5 * i;
-        r[0] = be; r[1] = al; r[2] = 1.0; r[3] = al; r[4] = be;
-    }
-    for (int i = 0; i < 3; ++i)
-        for (int c = 0; c < 5; ++c) {
-            o[5 * i + c] = lo[i][c];
-            o[5 * (n - 1 - i) + c] = hi[i][4 - c];   // the far end mirrors the near-end rows
-        }
-}
-
 void lu_factors(const Tables &t, int scheme, int n, bool qd_lo, bool qd_hi, double *o)
 {
     // LHS rows 0..2 for the end family (offsets -2..2)

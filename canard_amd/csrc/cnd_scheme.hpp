@@ -43,8 +43,6 @@ void build_tables(double fltk_over_pi, double fltrbc, Tables &t);
 // 1 = filter; qd_lo/qd_hi select the quasi-disjoint rows at each end.
 // Output rows: (xl1, xl2, xu1, xu2, xu3) per point.
 void lu_factors(const Tables &t, int scheme, int n, bool qd_lo, bool qd_hi, double *rows5);
-// The banded LHS itself, 5 entries per row at offsets -2..2 (diagonal 1).
-void lhs_rows(const Tables &t, int scheme, int n, bool qd_lo, bool qd_hi, double *rows5);
 
 // Homogeneous solutions of the LU recurrences of one line (rows5 as from
 // lu_factors) restarted at every segment of an S-segment partition: per row

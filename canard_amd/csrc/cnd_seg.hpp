@@ -137,7 +137,7 @@ struct SegLane {
 __host__ __device__ constexpr double seg_pass_row(int c) { return c == 0 || c == 4 ? -1.0 : 0.0; }
 
 // Solve the line for the lane's segment held in Y (right-hand side in,
-// solution out; Y[0 .. kb - 1] must be zero) in arithmetic T.  LUs: the
+// solution out; Y[0 .. kb - 1] must be zero).  LUs: the
 // LU rows of every segment as the lanes hold them, [SP][L][5] in LDS
 // (pass-through rows in front); SM: per-segment transfer values in LDS
 // (phi1, phi2 at the segment's last two rows, psi1, psi2 at its first two);
@@ -151,8 +151,8 @@ __host__ __device__ constexpr double seg_pass_row(int c) { return c == 0 || c ==
 // is always register L - 1, and the kb pass-through registers carry the
 // state across the front of the segment (swapped kb times, which the start
 // or end values undo).
-template <class T, int L, int SPM>
-__device__ __forceinline__ void seg_solve(T (&Y)[L], const SegLane &ln, const double *LUs, const double *SM,
+template <int L, int SPM>
+__device__ __forceinline__ void seg_solve(double (&Y)[L], const SegLane &ln, const double *LUs, const double *SM,
                                           double *ex)
 {
     const int s = ln.s;
@@ -160,36 +160,36 @@ __device__ __forceinline__ void seg_solve(T (&Y)[L], const SegLane &ln, const do
     const double *lu = LUs + 5 * L * s;
     // forward, pass 1: zero incoming values, outgoing values only
     {
-        T ya = T(0), yb = T(0);
+        double ya = 0.0, yb = 0.0;
 #pragma unroll
         for (int k = 0; k < L; ++k) {
-            const T y = (Y[k] - T(lu[5 * k]) * ya) - T(lu[5 * k + 1]) * yb;
+            const double y = (Y[k] - lu[5 * k] * ya) - lu[5 * k + 1] * yb;
             ya = yb;
             yb = y;
         }
         __syncthreads();
-        ex[ln.exi] = double(ya);
-        ex[ln.exs + ln.exi] = double(yb);
+        ex[ln.exi] = ya;
+        ex[ln.exs + ln.exi] = yb;
         __syncthreads();
     }
     // incoming values y(a-2), y(a-1): scan over the segments before this one
-    T t0 = T(0), t1 = T(0);
+    double t0 = 0.0, t1 = 0.0;
     if (ln.ok) {
         for (int sp = 0; sp < s; ++sp) {
             const double *m = SM + 8 * sp;
             const int xi = ln.exi + (sp - s) * ln.P;
-            const T n0 = (T(m[0]) * t0 + T(m[1]) * t1) + T(ex[xi]);
-            const T n1 = (T(m[2]) * t0 + T(m[3]) * t1) + T(ex[ln.exs + xi]);
+            const double n0 = (m[0] * t0 + m[1] * t1) + ex[xi];
+            const double n1 = (m[2] * t0 + m[3] * t1) + ex[ln.exs + xi];
             t0 = n0;
             t1 = n1;
         }
     }
     // forward, pass 2: from the true incoming values
     {
-        T ya = odd ? t1 : t0, yb = odd ? t0 : t1;
+        double ya = odd ? t1 : t0, yb = odd ? t0 : t1;
 #pragma unroll
         for (int k = 0; k < L; ++k) {
-            const T y = (Y[k] - T(lu[5 * k]) * ya) - T(lu[5 * k + 1]) * yb;
+            const double y = (Y[k] - lu[5 * k] * ya) - lu[5 * k + 1] * yb;
             Y[k] = y;
             ya = yb;
             yb = y;
@@ -197,36 +197,36 @@ __device__ __forceinline__ void seg_solve(T (&Y)[L], const SegLane &ln, const do
     }
     // backward, pass 1: zero incoming values, outgoing values only
     {
-        T xa = T(0), xb = T(0);
+        double xa = 0.0, xb = 0.0;
 #pragma unroll
         for (int k = L - 1; k >= 0; --k) {
-            const T x = (T(lu[5 * k + 2]) * Y[k] - T(lu[5 * k + 3]) * xa) - T(lu[5 * k + 4]) * xb;
+            const double x = (lu[5 * k + 2] * Y[k] - lu[5 * k + 3] * xa) - lu[5 * k + 4] * xb;
             xb = xa;
             xa = x;
         }
         __syncthreads();
-        ex[ln.exi] = double(odd ? xb : xa);
-        ex[ln.exs + ln.exi] = double(odd ? xa : xb);
+        ex[ln.exi] = odd ? xb : xa;
+        ex[ln.exs + ln.exi] = odd ? xa : xb;
         __syncthreads();
     }
     // incoming values x(b), x(b+1): scan over the segments after this one
-    T h0 = T(0), h1 = T(0);
+    double h0 = 0.0, h1 = 0.0;
     if (ln.ok) {
         for (int sp = ln.S - 1; sp > s; --sp) {
             const double *m = SM + 8 * sp + 4;
             const int xi = ln.exi + (sp - s) * ln.P;
-            const T n0 = (T(m[0]) * h0 + T(m[1]) * h1) + T(ex[xi]);
-            const T n1 = (T(m[2]) * h0 + T(m[3]) * h1) + T(ex[ln.exs + xi]);
+            const double n0 = (m[0] * h0 + m[1] * h1) + ex[xi];
+            const double n1 = (m[2] * h0 + m[3] * h1) + ex[ln.exs + xi];
             h0 = n0;
             h1 = n1;
         }
     }
     // backward, pass 2
     {
-        T xa = h0, xb = h1;
+        double xa = h0, xb = h1;
 #pragma unroll
         for (int k = L - 1; k >= 0; --k) {
-            const T x = (T(lu[5 * k + 2]) * Y[k] - T(lu[5 * k + 3]) * xa) - T(lu[5 * k + 4]) * xb;
+            const double x = (lu[5 * k + 2] * Y[k] - lu[5 * k + 3] * xa) - lu[5 * k + 4] * xb;
             Y[k] = x;
             xb = xa;
             xa = x;
@@ -239,11 +239,9 @@ __device__ __forceinline__ void seg_solve(T (&Y)[L], const SegLane &ln, const do
 }
 
 // Coefficient tables of the segmented sweeps, indexed like the LU rows:
-// LU factors and homogeneous solutions in FP64 and FP32, and the banded LHS
-// (for the FP64 residual of the mixed-precision solve).
+// LU factors and homogeneous solutions.
 struct SegTabs {
-    const double *lu, *seg, *lhs;
-    const float *lu32, *seg32;
+    const double *lu, *seg;
 };
 
 // Sinks that read operands of their own at each point (type Pre, filled by
@@ -259,9 +257,7 @@ template <class S> struct sink_pre<S, std::void_t<typename S::Pre>> : std::true_
 //        put_raw: write such a value (eta/zeta sweeps of plain fields, which
 //        still hold the source in registers, use these instead of put);
 //        optionally Pre, pre and put_pre (sink_pre)
-// MIX: solve in FP32 and refine once with the FP64 residual r = b - A x
-// (A the banded LHS), x += A^-1 r solved in FP32.
-template <int NV, int SCH, int L, int P, int C, bool XI, bool MIX, int SPM, class Src, class Sink>
+template <int NV, int SCH, int L, int P, int C, bool XI, int SPM, class Src, class Sink>
 __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs,
                                          const SegTabs &tb, Tile tile, int d, int n45, int SP, const Src &src,
                                          Sink &sink, double *lds)
@@ -732,65 +728,9 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
         __syncthreads();
     }
 
-    // ---- 4. solve: FP64, or FP32 with one FP64 residual refinement ----------
+    // ---- 4. solve ---------------------------------------------------------------
     const SegLane ln{a, len, kb, s, S, n, L, lane_ok, (v * SP + s) * P + p, NV * SP * P, v, p, P, SP};
-    if constexpr (!MIX) {
-        seg_solve<double, L, SPM>(Y, ln, LUs, SM, ex);
-    } else {
-        float X[L];
-#pragma unroll
-        for (int k = 0; k < L; ++k) X[k] = float(Y[k]);
-        seg_solve<float, L, SPM>(X, ln, LUs, SM, ex);
-        // edge values of the neighbouring segments: x(a-2), x(a-1), x(b), x(b+1)
-        double l2 = 0.0, l1 = 0.0, r1 = 0.0, r2 = 0.0;
-        {
-            double f0 = 0.0, f1 = 0.0, e0 = 0.0, e1 = 0.0;
-#pragma unroll
-            for (int k = 0; k < L; ++k) {
-                if (k == kb) f0 = X[k];
-                if (k == kb + 1) f1 = X[k];
-                if (k == L - 2) e0 = X[k];
-                if (k == L - 1) e1 = X[k];
-            }
-            __syncthreads();
-            ex[ln.exi] = f0;
-            ex[ln.exs + ln.exi] = f1;
-            ex[2 * ln.exs + ln.exi] = e0;
-            ex[3 * ln.exs + ln.exi] = e1;
-            __syncthreads();
-            if (lane_ok && s > 0) {
-                const int xi = ln.exi - P;
-                l2 = ex[2 * ln.exs + xi];
-                l1 = ex[3 * ln.exs + xi];
-            }
-            if (lane_ok && s < S - 1) {
-                const int xi = ln.exi + P;
-                r1 = ex[xi];
-                r2 = ex[ln.exs + xi];
-            }
-        }
-        // r = b - A x in FP64 with the banded rows of the line
-        const double *AR = tb.lhs + 5 * int64_t(B.lu[SCH][d]);
-#pragma unroll
-        for (int k = 0; k < L; ++k) {
-            if (have(k)) {
-                const int e = L;
-                const double *ar = AR + 5 * (a - kb + k);
-                const double xm2 = k - 2 >= kb ? double(X[k >= 2 ? k - 2 : 0]) : (k - 1 >= kb ? l1 : l2);
-                const double xm1 = k - 1 >= kb ? double(X[k >= 1 ? k - 1 : 0]) : l1;
-                const double xp1 = k + 1 < e ? double(X[k + 1 < L ? k + 1 : L - 1]) : r1;
-                const double xp2 = k + 2 < e ? double(X[k + 2 < L ? k + 2 : L - 1]) : (k + 1 < e ? r1 : r2);
-                const double ax = (((ar[0] * xm2 + ar[1] * xm1) + double(X[k])) + ar[3] * xp1) + ar[4] * xp2;
-                Y[k] = Y[k] - ax;
-            }
-        }
-        float D[L];
-#pragma unroll
-        for (int k = 0; k < L; ++k) D[k] = float(Y[k]);
-        seg_solve<float, L, SPM>(D, ln, LUs, SM, ex);
-#pragma unroll
-        for (int k = 0; k < L; ++k) Y[k] = double(X[k]) + double(D[k]);
-    }
+    seg_solve<L, SPM>(Y, ln, LUs, SM, ex);
     if (lane_ok && s == 0) {
         double x0 = 0.0;
 #pragma unroll
@@ -800,7 +740,7 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     }
     if (lane_ok && s == S - 1) sink.ends(1, p, v, Y[L - 1]);
 
-    // ---- 6. results ------------------------------------------------------------
+    // ---- 5. results ------------------------------------------------------------
     if constexpr (!XI) {
         // eta/zeta: lanes of a wave hold P neighbouring pencils, stores coalesce
         if (lane_ok) {

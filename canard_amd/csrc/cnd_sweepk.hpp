@@ -319,7 +319,7 @@ __global__ __launch_bounds__(kTile) void k_fd_flux_field(const BlkDev *__restric
 template <int L_, int P_, int C_, int SPMAX_, bool XI_>
 struct SegG { static constexpr int L = L_, P = P_, C = C_, SPMAX = SPMAX_; static constexpr bool XI = XI_; };
 struct ShapeInfo { int L, P, C, SPMAX; bool XI; };
-constexpr int kNumShapes = 17;
+constexpr int kNumShapes = 21;
 constexpr ShapeInfo kShapes[kNumShapes] = {
     {17, 4, 16, 16, true},    // 0: xi default (pencils up to 272 points)
     {33, 4, 16, 8, true},     // 1
@@ -337,7 +337,15 @@ constexpr ShapeInfo kShapes[kNumShapes] = {
     {17, 64, 8, 16, false},   // 13
     {17, 32, 16, 16, true},   // 14: xi, 32-pencil tiles (single-field sweeps)
     {17, 20, 16, 16, true},   // 15: xi, tiles sized for three workgroups per CU
-    {17, 24, 16, 16, true}};  // 16
+    {17, 24, 16, 16, true},   // 16
+    // 17-point segments on pencils of up to 528 points: with 33-point ones a
+    // workgroup has 4 pencils and half the waves (513-point xi pencils of
+    // the four sheared blocks: flux 1.26 -> 0.89 ms beside the eta sweep,
+    // filter 1.28 -> 0.64, gradients 0.63 -> 0.59)
+    {17, 16, 16, 32, true},   // 17
+    {17, 8, 16, 32, true},    // 18
+    {17, 4, 16, 32, true},    // 19
+    {17, 16, 8, 32, false}};  // 20
 using Sh0 = SegG<17, 4, 16, 16, true>;
 using Sh1 = SegG<33, 4, 16, 8, true>;
 using Sh2 = SegG<33, 16, 8, 8, false>;
@@ -355,15 +363,20 @@ using Sh13 = SegG<17, 64, 8, 16, false>;
 using Sh14 = SegG<17, 32, 16, 16, true>;
 using Sh15 = SegG<17, 20, 16, 16, true>;
 using Sh16 = SegG<17, 24, 16, 16, true>;
+using Sh17 = SegG<17, 16, 16, 32, true>;
+using Sh18 = SegG<17, 8, 16, 32, true>;
+using Sh19 = SegG<17, 4, 16, 32, true>;
+using Sh20 = SegG<17, 16, 8, 32, false>;
 // workgroup size bound of a kernel (shapes whose NV * P * SPMAX exceeds the
 // 1024-thread limit are rejected at launch time by shape_sp)
 __host__ __device__ constexpr int wg_bound(int x) { return x > 1024 ? 1024 : x; }
 // waves per SIMD a segmented sweep is compiled for: shapes of 17-point
 // segments are held to 128 VGPRs (4 waves, so two 512-thread workgroups
-// share a CU), which their LDS also allows -- eta/zeta ones in FP64 only,
-// where it costs no spills; the others are left to the compiler
-template <class G, bool MIX>
-__host__ __device__ constexpr int seg_waves() { return G::L <= 17 && (G::XI || !MIX) ? 4 : 1; }
+// share a CU), which their LDS also allows and which costs no spills; the
+// others are left to the compiler
+template <class G>
+__host__ __device__ constexpr int seg_waves() { return G::L <= 17 ? 4 : 1; }
+constexpr int kSegMaxPoints = 528;   // longest pencil of a segmented sweep
 constexpr int kTiled = -1;   // shape index of the tiled sweep
 // pencils-per-workgroup values (tile lists) and segment lengths (tables)
 constexpr int kNumP = 7, kPs[kNumP] = {4, 8, 16, 32, 64, 20, 24};
@@ -379,8 +392,8 @@ __host__ __device__ constexpr int l_index(int L) { return L == 17 ? 0 : 1; }
     if (tix >= (ntiles)) return;           \
     extern __shared__ double lds[];
 
-template <class G, bool MIX>
-__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G, MIX>())) void k_seg_fd_field(
+template <class G>
+__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_fd_field(
     const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
     int ntiles, int SP, int d, int n45, const double *in, int64_t in_vstride, double *out, int64_t out_vstride)
 {
@@ -388,11 +401,11 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G, MIX>())) v
     const int v = blockIdx.y;
     SrcField<1> src{in + v * in_vstride, 0};
     SinkOut<1> sink{out + v * out_vstride, 0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI, MIX, G::SPMAX>(blks, tabs, tb, tiles[tix], d, n45, SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles[tix], d, n45, SP, src, sink, lds);
 }
 
-template <class G, bool MIX>
-__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G, MIX>())) void k_seg_filter_field(
+template <class G>
+__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_filter_field(
     const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
     int ntiles, int SP, int d, const double *in, double *out, int64_t vstride)
 {
@@ -400,44 +413,41 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G, MIX>())) v
     const int v = blockIdx.y;
     SrcField<1> src{in + v * vstride, 0};
     SinkFilt<1> sink{out + v * vstride, in + v * vstride, 0};
-    seg_tile<1, 1, G::L, G::P, G::C, G::XI, MIX, G::SPMAX>(blks, tabs, tb, tiles[tix], d, 0, SP, src, sink, lds);
+    seg_tile<1, 1, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles[tix], d, 0, SP, src, sink, lds);
 }
 
-// Velocity and temperature gradients along d; in mixed mode they are stored
-// in FP32.  prim (xi sweeps, or null): the primitives u, v, w, T are also
+// Velocity and temperature gradients along d, stored as TG (float in mixed
+// precision).  prim (xi sweeps, or null): the primitives u, v, w, T are also
 // written there.
-template <class G, bool MIX>
-__global__ __launch_bounds__(wg_bound(4 * G::P * G::SPMAX), (seg_waves<G, MIX>())) void k_seg_grad(
+template <class G, class TG>
+__global__ __launch_bounds__(wg_bound(4 * G::P * G::SPMAX), (seg_waves<G>())) void k_seg_grad(
     const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
-    int ntiles, int SP, int d, const double *q, typename std::conditional<MIX, float, double>::type *grad,
+    int ntiles, int SP, int d, const double *q, TG *grad,
     int64_t NT, double *prim)
 {
     SEG_PROLOGUE(ntiles)
-    using TG = typename std::conditional<MIX, float, double>::type;
     SrcPrim src{q, NT, prim};
     SinkOut<4, TG> sink{grad + 4 * d * NT, NT};
-    seg_tile<4, 0, G::L, G::P, G::C, G::XI, MIX, G::SPMAX>(blks, tabs, tb, tiles[tix], d, 0, SP, src, sink, lds);
+    seg_tile<4, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles[tix], d, 0, SP, src, sink, lds);
 }
 
 // Gradients along d (eta, zeta) of the primitive v = blockIdx.y that the xi
-// gradient sweep stored (prim, four fields NT apart), into grad; in mixed
-// mode FP32.
-template <class G, bool MIX>
-__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G, MIX>())) void k_seg_grad_prim(
+// gradient sweep stored (prim, four fields NT apart), into grad as TG.
+template <class G, class TG>
+__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_grad_prim(
     const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
-    int ntiles, int SP, int d, const double *prim, typename std::conditional<MIX, float, double>::type *grad,
+    int ntiles, int SP, int d, const double *prim, TG *grad,
     int64_t NT)
 {
     SEG_PROLOGUE(ntiles)
-    using TG = typename std::conditional<MIX, float, double>::type;
     const int v = blockIdx.y;
     SrcField<1> src{prim + v * NT, 0};
     SinkOut<1, TG> sink{grad + (4 * d + v) * NT, 0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI, MIX, G::SPMAX>(blks, tabs, tb, tiles[tix], d, 0, SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles[tix], d, 0, SP, src, sink, lds);
 }
 
-template <class G, bool MIX>
-__global__ __launch_bounds__(wg_bound(5 * G::P * G::SPMAX), (seg_waves<G, MIX>())) void k_seg_flux(
+template <class G>
+__global__ __launch_bounds__(wg_bound(5 * G::P * G::SPMAX), (seg_waves<G>())) void k_seg_flux(
     const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
     int ntiles, int SP, int d, const InstDev *__restrict__ inst, const double *q, const double *met, double *de,
     double *drva, int64_t NT, int64_t FT)
@@ -446,11 +456,11 @@ __global__ __launch_bounds__(wg_bound(5 * G::P * G::SPMAX), (seg_waves<G, MIX>()
     const Tile t = tiles[tix];
     SrcFlux src{q, met, blks, inst, NT, d};
     SinkFlux sink{de, drva, NT, FT, blks[t.b].foff[d] + t.q0};
-    seg_tile<5, 0, G::L, G::P, G::C, G::XI, MIX, G::SPMAX>(blks, tabs, tb, t, d, 0, SP, src, sink, lds);
+    seg_tile<5, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, SP, src, sink, lds);
 }
 
-template <class G, bool MIX>
-__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G, MIX>())) void k_seg_flux_field(
+template <class G>
+__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_flux_field(
     const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
     int ntiles, int SP, int d, const double *F, double *de, double *drva, int64_t NT, int64_t FT)
 {
@@ -459,14 +469,14 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G, MIX>())) v
     const Tile t = tiles[tix];
     SrcField<1> src{F + v * NT, 0};
     SinkFluxV sink{de + v * NT, drva, v, FT, blks[t.b].foff[d] + t.q0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI, MIX, G::SPMAX>(blks, tabs, tb, t, d, 0, SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, SP, src, sink, lds);
 }
 
 // Last flux sweep of a stage fused with the RK update: sweep of the stored
 // flux component v along d (xi or zeta), written as the updated state qa.
 // Grid x: five workgroups (components) per tile.
-template <class G, bool MIX>
-__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G, MIX>())) void k_seg_flux_update(
+template <class G>
+__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_flux_update(
     const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
     int ntiles, int SP, int d, const InstDev *__restrict__ inst, const double *F, const double *de,
     const double *__restrict__ qo, const double *__restrict__ met, double *qa, double *drva, int64_t NT, int64_t FT,
@@ -484,7 +494,7 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G, MIX>())) v
     // the two other directions' right-hand sides
     const double *da = de + ((G::XI ? 5 : 0) + v) * NT, *db = de + ((G::XI ? 10 : 5) + v) * NT;
     SinkUpdateV<G::XI> sink{qa + v * NT, drva, qo + v * NT, da, db, met, dtk, v, NT, FT, blks[t.b].foff[d] + t.q0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI, MIX, G::SPMAX>(blks, tabs, tb, t, d, 0, SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, SP, src, sink, lds);
 }
 
 }  // namespace cnd

@@ -39,10 +39,11 @@ enum {
     CND_ENOMEM = -4
 };
 
-/* Precision of the step: CND_FP64; CND_MIXED, FP32 line solves with one
- * FP64 residual refinement and the stage's velocity and temperature
- * gradients stored in FP32 (state, metrics, fluxes, right-hand sides, RK
- * update and characteristic boundaries stay FP64).                         */
+/* Precision of the step: CND_FP64; CND_MIXED, the stage's velocity and
+ * temperature gradients stored in FP32 (line solves, state, metrics, fluxes,
+ * right-hand sides, RK update and characteristic boundaries are FP64: an FP32
+ * line solve needs an FP64 refinement to stay within 1e-6 of FP64 over a
+ * run, and the two together cost more than the FP64 solve).                */
 enum { CND_FP64 = 0, CND_MIXED = 1 };
 
 typedef struct cnd_ctx cnd_ctx;
@@ -75,7 +76,7 @@ typedef struct {
 /* Replaces the set-up half of canard_driver (mo_canard_driver.f90:103-148):
  * domain tables, numerics coefficients (init_extracoeff_bounds, init_penta,
  * mo_numerics.f90:114-249) and device allocation.  precision = CND_FP64 or
- * CND_MIXED (FP32 sweeps with one FP64 refinement pass).                   */
+ * CND_MIXED.                                                                */
 int  cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks,
                 int nblocks, int precision, cnd_ctx **ctx);
 void cnd_destroy(cnd_ctx *ctx);
