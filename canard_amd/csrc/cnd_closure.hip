@@ -4,18 +4,18 @@
 // runs.  It has no counterpart in the reference; the compact filter stays in
 // every step, so a context without a network is the plain scheme.
 //
-// Every convolution is an implicit GEMM on the gfx950 BF16 matrix cores: one
-// wave computes a 32 (voxels) x 32 (channels) tile with
-// v_mfma_f32_32x32x16_bf16 (FP32 accumulate), stepping K over the 27 taps x
-// input channels, its workgroup's input halo and weights staged in LDS;
-// activations are BF16 channel-last [voxel][channel].
+// Every convolution is an implicit GEMM on the gfx950 BF16 matrix cores
+// (v_mfma_f32_32x32x16_bf16, FP32 accumulate), its input halo staged in LDS
+// and its weights held in registers; activations are BF16 channel-last
+// [voxel][channel].
 //   forward        out[v][o]  = sum_{t,c} a[nb(v,t)][c] W[o][t][c] (+ b[o])
 //   data gradient  g[v][c]    = sum_{t,o} go[nb(v,t)][o] W[o][26-t][c]
 //   weight grad.   gW[o][t][c] = sum_v go[v][o] a[nb(v,t)][c]   (partial sums
 //                  per workgroup of voxel tiles, then summed in a fixed order)
-// Parameters are FP32 (Adam); BF16 copies in both layouts are rebuilt after
-// every update.  The grid is periodic, n^3 voxels (the context's stored
-// duplicate planes are filled from their originals).
+// Parameters are FP32 (Adam); the update writes their BF16 copies in the
+// order in which the kernels' lanes hold them.  The grid is periodic, n^3
+// voxels (the context's stored duplicate planes are filled from their
+// originals).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -43,8 +43,13 @@ constexpr int kC0 = 5, kC0P = 8, kC1 = 32, kC2 = 32, kC3 = 5, kCP = 32, kTaps = 
 // W3 [5][27][32], b3 [5]
 constexpr int kOW1 = 0, kOB1 = kOW1 + kC1 * kTaps * kC0, kOW2 = kOB1 + kC1, kOB2 = kOW2 + kC2 * kTaps * kC1,
               kOW3 = kOB2 + kC2, kOB3 = kOW3 + kC3 * kTaps * kC2, kNParam = kOB3 + kC3;
-constexpr int kM1 = kTaps * kC0P, kM2 = kTaps * kCP;   // weight-gradient row lengths
-constexpr int kWgSlices = 8;                           // slices of the first weight-gradient reduction level
+// one workgroup's weight gradients: layer 2 [tap][4][64 lanes][4], layer 3
+// [tap][64][4] (8 output channels), layer 1 [column tile][4][64][4]
+constexpr int kP2 = kTaps * 1024, kP3 = kTaps * 256, kP1 = 7 * 1024;
+// a slice of the summed gradients: layers 2, 1, 3, then their biases
+constexpr int kS2 = 0, kS1 = kP2, kS3 = kS1 + kP1, kSB1 = kS3 + kP3, kSB2 = kSB1 + kCP, kSB3 = kSB2 + kCP,
+              kSlice = kSB3 + kCP;
+constexpr int kWgSlices = 8;            // slices of the first reduction level
 
 __host__ __device__ inline uint32_t f2u(float f)
 {
@@ -68,41 +73,18 @@ __host__ __device__ inline bf16 to_bf16(float f)
 }
 __host__ __device__ inline float from_bf16(bf16 h) { return u2f(uint32_t(h) << 16); }
 
-__device__ inline int wrap(int a, int n) { return a < 0 ? a + n : (a >= n ? a - n : a); }
-// neighbour of voxel (x, y, z) at tap t = (dx+1) + 3 (dy+1) + 9 (dz+1)
-__device__ inline int nbr(int x, int y, int z, int t, int n)
+// a modulo n for -n <= a < 2 n: of a, a + n and a - n the one in range is the
+// smallest as an unsigned number
+__device__ __forceinline__ int wrap(int a, int n)
 {
-    const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-    return wrap(x + dx, n) + n * (wrap(y + dy, n) + n * wrap(z + dz, n));
+    const unsigned b = min(unsigned(a), unsigned(a + n));
+    return int(min(b, b - unsigned(n)));
 }
-
-// Convolution as an implicit GEMM on v_mfma_f32_32x32x16_bf16 (gfx950: 16
-// K values per instruction, 8 per lane).  A workgroup of 8 waves owns a
-// tile of X (x) by 2R (y) by 4 (z) voxels, X = 32, 16 or 8 dividing n and
-// R = 32 / X; wave (wy, wz) computes the 32 voxels of its R rows of X at
-// plane wz against all 32 output channels.  The tile's input halo (one voxel
-// each side, periodic) and the layer's weights are staged in LDS first, so
-// the 27 taps read LDS only; voxel and weight rows are padded by 8 BF16
-// values, which spreads a wave's 16-byte reads over distinct banks.
-//   K order: for CIP = 32, tap t and channel block cb of 16 (lanes kh = 0, 1
-//   take its halves); for CIP = 8, one instruction covers the 8 channels of
-//   taps 2 tt (lanes kh = 0) and 2 tt + 1 (kh = 1), the 28th tap being zero.
-// EPI 0: + bias, ReLU, BF16 [V][32]; EPI 1: (+ bias) FP32 [V][ostride] for
-// o < cout; EPI 2: times (mask[v][o] > 0), BF16 [V][32].
-constexpr int kConvWaves = 8;
-
-__host__ __device__ constexpr int conv_vs(int cip) { return cip + 8; }           // LDS BF16 per halo voxel
-__host__ __device__ constexpr int conv_ws(int cip) { return kTaps * cip + 8; }   // LDS BF16 per weight row
-// x extent of a wave's voxel tile for an n^3 grid (n a multiple of 8)
-__host__ __device__ inline int conv_x(int n) { return n % 32 == 0 ? 32 : (n % 16 == 0 ? 16 : 8); }
-__host__ inline size_t conv_lds_bytes(int cip, int n)
-{
-    const int X = conv_x(n), R = 32 / X;
-    return sizeof(bf16) * (size_t(32) * conv_ws(cip) + size_t(X + 2) * (2 * R + 2) * 6 * conv_vs(cip));
-}
-
 typedef short s8v __attribute__((ext_vector_type(8)));
+typedef short s4v __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s4v *lds_s4;
 
 __device__ __forceinline__ f16v mfma16(const s8v &a, const s8v &b, const f16v &c)
 {
@@ -110,292 +92,619 @@ __device__ __forceinline__ f16v mfma16(const s8v &a, const s8v &b, const f16v &c
                                                   0);
 }
 
-template <int CIP, int EPI>
-__global__ __launch_bounds__(64 * kConvWaves) void k_conv(const bf16 *__restrict__ in, const bf16 *__restrict__ w,
-                                                         const float *__restrict__ bias,
-                                                         const bf16 *__restrict__ mask, void *__restrict__ out, int n,
-                                                         int cout, int ostride)
+// four values rounded to BF16 (nearest even, as to_bf16; v_cvt_pk_bf16_f32)
+__device__ __forceinline__ s4v pack4(const float (&x)[4])
 {
-    constexpr int VS = conv_vs(CIP), WS = conv_ws(CIP), KT = kTaps * CIP;
-    extern __shared__ unsigned short conv_lds[];
-    bf16 *sw = conv_lds;             // weights [32][WS]
-    bf16 *sa = conv_lds + 32 * WS;   // halo [HZ][HY][HX][VS]
-    const int X = conv_x(n), R = 32 / X;
-    const int TY = 2 * R, HX = X + 2, HY = TY + 2, HZ = 6;
-    int wg = blockIdx.x;
-    const int ntx = n / X, nty = n / TY;
-    const int x0 = (wg % ntx) * X;
-    wg /= ntx;
-    const int y0 = (wg % nty) * TY, z0 = (wg / nty) * 4;
-    const int tid = threadIdx.x, nthr = blockDim.x;
-    for (int e = tid; e < 32 * (KT / 8); e += nthr) {
-        const int o = e / (KT / 8), k8 = e - o * (KT / 8);
-        *reinterpret_cast<s8v *>(sw + o * WS + 8 * k8) = *reinterpret_cast<const s8v *>(w + o * KT + 8 * k8);
+    typedef __bf16 b4v __attribute__((ext_vector_type(4)));
+    b4v b;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) b[k] = __bf16(x[k]);
+    return __builtin_bit_cast(s4v, b);
+}
+
+// x extent of a wave's 32 voxels for an n^3 grid (n a multiple of 8)
+__host__ inline int conv_x(int n) { return n % 32 == 0 ? 32 : (n % 16 == 0 ? 16 : 8); }
+
+// Tiles of a workgroup: each XCD (blockIdx.x % 8) takes a contiguous eighth of
+// the tiles, a slab of the grid whose halos its L2 then holds (64^3, 32
+// channels: 2 MB of 4), and its workgroups, `rank` of `ranks`, walk it together.
+struct Walk {
+    int first, end, step;
+    __device__ Walk(int ntiles, int rank, int ranks)
+    {
+        const int per = (ntiles + 7) / 8, a = int(blockIdx.x % 8) * per;
+        first = a + rank;
+        end = min(a + per, ntiles);
+        step = ranks;
     }
-    const int HV = HX * HY * HZ;
-    for (int e = tid; e < HV * (CIP / 8); e += nthr) {
-        const int hv = e / (CIP / 8), c8 = e - hv * (CIP / 8);
-        const int hx = hv % HX, hy = (hv / HX) % HY, hz = hv / (HX * HY);
-        const int64_t gv = wrap(x0 + hx - 1, n) + int64_t(n) * (wrap(y0 + hy - 1, n) + int64_t(n) * wrap(z0 + hz - 1, n));
-        *reinterpret_cast<s8v *>(sa + hv * VS + 8 * c8) = *reinterpret_cast<const s8v *>(in + gv * CIP + 8 * c8);
+};
+
+// What a convolution reads and writes besides its input: FWD, BF16 [V][32]
+// out = ReLU(acc + bias); OUT, FP32 [V][5] out = acc (+ bias); MASK, BF16
+// [V][32] out = acc where mask > 0, else 0; LOSS, the mean-square loss of
+// y = acc + bias against the FP32 [V][5] target tg: each workgroup's sum of
+// (y - tg)^2 to lpart and, with out, its gradient 2 (y - tg) / (5 V) as BF16
+// [V][8] (channels 5.. zero).
+enum Epi { FWD, OUT, MASK, LOSS };
+// How K = 16 of an instruction is filled: C32, half the 32 channels of one
+// tap; PAIR, the 8 channels of two taps (lanes kh = 0 and 1; the 28th tap is
+// zero); SINGLE, the 8 channels of one tap (lanes kh = 1 hold zeros: the sums
+// are those of 32 zero-padded channels, term by term).
+enum Fill { C32, PAIR, SINGLE };
+
+struct ConvArgs {
+    const bf16 *in, *w;
+    const float *bias;
+    const bf16 *mask;
+    void *out;
+    const float *tg;
+    double *lpart;
+    int n, ntiles;
+};
+
+// Convolution on v_mfma_f32_32x32x16_bf16: rows are the 32 output channels,
+// columns 32 voxels (so a lane holds four runs of four channels of one voxel
+// and stores them whole).  A workgroup of 4 waves walks the tiles of X (x) by
+// 2R (y) by 2 ZT (z) voxels, X = 32, 16 or 8 dividing n and R = 32 / X; a
+// wave owns the X x R voxels of ZT planes.
+//
+// Bound by the matrix cores if they are fed: the layer's weights stay in the
+// wave's registers (216 of 512 with 32 channels, so one wave per SIMD), and a
+// voxel row read from LDS serves the taps of all ZT planes it touches, 0.67
+// KB of LDS per instruction and wave instead of 2 KB with the weights in LDS
+// as well (4 waves at 32 cycles an instruction: 85 of 128 B/cycle).  The next
+// tile's halo is loaded into registers while this one is computed.  Every
+// accumulator adds its taps in the order t = 0 .. 26.
+// 64^3, 32 -> 32 channels: 36.8 -> 21.2 us; 5 -> 32: 17.2 -> 12.5 us; the
+// 32 -> 5 layer with its loss: 41.1 + 10.8 -> 18.4 us; data gradients 52 ->
+// 19.2 (5 -> 32 channels) and 21.2 us.
+constexpr int kConvThreads = 256;
+__host__ __device__ constexpr int fill_ch(Fill f) { return f == C32 ? 32 : 8; }
+__host__ __device__ constexpr int fill_vs(Fill f) { return f == C32 ? 40 : 8; }   // LDS BF16 per voxel: 32 channels padded against bank conflicts
+__host__ __device__ constexpr int fill_frags(Fill f) { return f == C32 ? 2 * kTaps : (f == PAIR ? (kTaps + 1) / 2 : kTaps); }
+
+// Scheduling of a group of N matrix instructions: behind each one R LDS reads
+// and V vector instructions, which issue while it executes.
+template <int N, int R, int V> __device__ __forceinline__ void interleave()
+{
+    if constexpr (N > 0) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // matrix
+        __builtin_amdgcn_sched_group_barrier(0x100, R, 0);   // LDS read
+        __builtin_amdgcn_sched_group_barrier(0x002, V, 0);   // vector
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);   // global read
+        interleave<N - 1, R, V>();
     }
-    __syncthreads();
-    const int wave = tid >> 6, lane = tid & 63;
-    const int wy = wave & 1, wz = wave >> 1;
-    const int i = lane & 31, kh = lane >> 5;
-    const int lx = i % X, ly = wy * R + i / X;   // voxel i of the wave in the tile (plane wz)
+}
+
+template <Fill F, Epi E, int X, int ZT>
+__global__ __launch_bounds__(kConvThreads, (F == C32 ? 1 : 2)) void k_conv(const ConvArgs A)
+{
+    constexpr int R = 32 / X, TY = 2 * R, TZ = 2 * ZT, HX = X + 2, HY = TY + 2, HZ = TZ + 2, HV = HX * HY * HZ;
+    constexpr int CI = fill_ch(F), VS = fill_vs(F), NF = fill_frags(F), NC = CI / 8;
+    constexpr int NJ = (HV * NC + kConvThreads - 1) / kConvThreads;   // halo chunks of 16 bytes per thread
+    __shared__ __align__(16) bf16 sa[HV * VS];
+    const int n = A.n, ntx = n / X, nty = n / TY;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int wy = wave & 1, wz = wave >> 1, i = lane & 31, kh = lane >> 5;
+    float bv[16];
+    if constexpr (E == FWD) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) bv[r] = A.bias[8 * (r >> 2) + 4 * kh + (r & 3)];
+    } else if constexpr (E == OUT || E == LOSS) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bv[r] = A.bias && 4 * kh + r < kC3 ? A.bias[4 * kh + r] : 0.f;
+    }
+    double lsum = 0.0;
+    int x0, y0, z0;
+    auto origin = [&](int tile) {
+        x0 = (tile % ntx) * X;
+        tile /= ntx;
+        y0 = (tile % nty) * TY;
+        z0 = (tile / nty) * TZ;
+    };
+    // halo coordinates of the thread's chunks, the same for every tile
+    int hc[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int hv = min((tid + j * kConvThreads) / NC, HV - 1);
+        hc[j] = hv % HX | (hv / HX % HY) << 8 | (hv / (HX * HY)) << 16;
+        asm volatile("" : "+v"(hc[j]));   // keep it: the compiler would divide again for every tile
+    }
+    s8v pre[NJ];
+    auto fetch1 = [&](int j) {   // (a thread without a last chunk loads another's again)
+        const int gx = wrap(x0 - 1 + (hc[j] & 255), n), gy = wrap(y0 - 1 + (hc[j] >> 8 & 255), n),
+                  gz = wrap(z0 - 1 + (hc[j] >> 16), n);
+        pre[j] = *reinterpret_cast<const s8v *>(A.in + int64_t(gx + n * (gy + n * gz)) * CI + 8 * (tid % NC));
+    };
+    // halo voxel of the lane's voxel at tap (-1, -1, -1), plane 0 of the wave
+    const bf16 *ap = sa + ((wz * ZT * HY + wy * R + i / X) * HX + i % X) * VS + (F == C32 ? 8 * kh : 0);
+    constexpr auto off = [](int t) { return ((t / 9) * HY + (t / 3) % 3) * HX + t % 3; };
+    const Walk walk(A.ntiles, blockIdx.x / 8, gridDim.x / 8);
+    int tile = walk.first;
+    origin(min(tile, A.ntiles - 1));
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) fetch1(j);
+    s8v wr[NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) wr[f] = reinterpret_cast<const s8v *>(A.w)[f * 64 + lane];
+    for (; tile < walk.end; tile += walk.step) {
+        __syncthreads();   // the previous tile is read
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int e = tid + j * kConvThreads;
+            if ((j + 1) * kConvThreads > HV * NC && e >= HV * NC) continue;
+            *reinterpret_cast<s8v *>(sa + (e / NC) * VS + 8 * (e % NC)) = pre[j];
+        }
+        __syncthreads();
+        const int gx = x0 + i % X, gy = y0 + wy * R + i / X, gz = z0 + wz * ZT;
+        // the next tile's loads go between the matrix instructions (after the
+        // last tile, its own again)
+        origin(tile + walk.step < walk.end ? tile + walk.step : tile);
+        f16v acc[ZT];
+        s4v m4[ZT][4];     // MASK: the lane's mask values, LOSS: its targets, in flight meanwhile
+        float tv[ZT][4];
+#pragma unroll
+        for (int z = 0; z < ZT; ++z) {
+            const int64_t v = gx + n * (gy + n * (gz + z));   // n <= 512: 2^27 voxels
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if constexpr (E == MASK) m4[z][q] = *reinterpret_cast<const s4v *>(A.mask + v * kCP + 8 * q + 4 * kh);
+                if constexpr (E == LOSS) tv[z][q] = 4 * kh + q < kC3 ? A.tg[v * kC3 + 4 * kh + q] : 0.f;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[z][r] = 0.f;
+        }
+        // operands are read a group ahead of the instructions that use them
+        // (the compiler alone reads each just before, and a wave waits out the
+        // LDS latency on every instruction)
+        if constexpr (F == C32) {
+            constexpr int NG = 3 * (ZT + 2);   // groups: plane p and dy, 3 dx x 2 halves of the channels
+            s8v fr[2][6];
+            auto read = [&](int g, s8v (&f)[6]) {
+#pragma unroll
+                for (int k = 0; k < 6; ++k)
+                    f[k] = *reinterpret_cast<const s8v *>(ap + (g / 3 * HY * HX + g % 3 * HX + k / 2) * VS + 16 * (k % 2));
+            };
+            read(0, fr[0]);
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (g + 1 < NG) read(g + 1, fr[(g + 1) & 1]);
+#pragma unroll
+                for (int j = g * NJ / NG; j < (g + 1) * NJ / NG; ++j) fetch1(j);
+                const int p = g / 3;
+                int nm = 0;
+#pragma unroll
+                for (int k = 0; k < 6; ++k)
+#pragma unroll
+                    for (int z = 0; z < ZT; ++z)
+                        if (p - z >= 0 && p - z < 3) {
+                            acc[z] = mfma16(wr[((p - z) * 9 + g % 3 * 3) * 2 + k], fr[g & 1][k], acc[z]);
+                            ++nm;
+                        }
+                // one LDS read and a few address instructions behind each matrix instruction
+                if (nm == 12) interleave<12, 1, 4>();
+                else interleave<6, 1, 7>();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        } else {
+            constexpr int GF = 4, NG = (NF + GF - 1) / GF;   // groups of 4 instructions x ZT planes
+            s8v fr[2][GF * ZT];
+            auto read = [&](int g, s8v (&r)[GF * ZT]) {
+#pragma unroll
+                for (int k = 0; k < GF; ++k) {
+                    const int f = g * GF + k;
+                    if (f >= NF) continue;
+                    const int t0 = F == PAIR ? 2 * f : f, t1 = F == PAIR ? (2 * f + 1 < kTaps ? 2 * f + 1 : 2 * f) : f;
+#pragma unroll
+                    for (int z = 0; z < ZT; ++z)
+                        r[k * ZT + z] = *reinterpret_cast<const s8v *>(
+                            ap + ((kh ? off(t1) : off(t0)) + z * HY * HX) * VS);
+                }
+            };
+            read(0, fr[0]);
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (g + 1 < NG) read(g + 1, fr[(g + 1) & 1]);
+#pragma unroll
+                for (int j = g * NJ / NG; j < (g + 1) * NJ / NG; ++j) fetch1(j);
+#pragma unroll
+                for (int k = 0; k < GF; ++k) {
+                    const int f = g * GF + k;
+                    if (f >= NF) continue;
+                    const bool zero = kh && (F == SINGLE || 2 * f + 1 >= kTaps);
+#pragma unroll
+                    for (int z = 0; z < ZT; ++z) {
+                        s8v b = fr[g & 1][k * ZT + z];
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) b[e] = zero ? short(0) : b[e];
+                        acc[z] = mfma16(wr[f], b, acc[z]);
+                    }
+                }
+                interleave<GF * ZT, 1, 7>();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int z = 0; z < ZT; ++z) {
+            const int64_t v = gx + n * (gy + n * (gz + z));
+            if constexpr (E == FWD || E == MASK) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    float x[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        float val = acc[z][4 * q + k];
+                        if constexpr (E == FWD) {
+                            val += bv[4 * q + k];
+                            x[k] = val > 0.f ? val : 0.f;
+                        } else {
+                            x[k] = from_bf16(bf16(m4[z][q][k])) > 0.f ? val : 0.f;
+                        }
+                    }
+                    *reinterpret_cast<s4v *>(static_cast<bf16 *>(A.out) + v * kCP + 8 * q + 4 * kh) = pack4(x);
+                }
+            } else if constexpr (E == OUT) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (4 * kh + k < kC3) {
+                        float val = acc[z][k];
+                        if (A.bias) val += bv[k];
+                        static_cast<float *>(A.out)[v * kC3 + 4 * kh + k] = val;
+                    }
+            } else {
+                const float sc = 2.0f / (5.0f * (float(n) * float(n) * float(n)));
+                float x[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    float gv = 0.f;
+                    if (4 * kh + k < kC3) {
+                        float val = acc[z][k];
+                        val += bv[k];
+                        const float d = val - tv[z][k];
+                        lsum += double(d) * double(d);
+                        gv = sc * d;
+                    }
+                    x[k] = gv;
+                }
+                if (A.out) *reinterpret_cast<s4v *>(static_cast<bf16 *>(A.out) + v * kC0P + 4 * kh) = pack4(x);
+            }
+        }
+    }
+    if constexpr (E == LOSS) {
+        __shared__ double wl[4];
+        for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
+        if (lane == 0) wl[wave] = lsum;
+        __syncthreads();
+        if (tid == 0) A.lpart[blockIdx.x] = ((wl[0] + wl[1]) + wl[2]) + wl[3];
+    }
+}
+
+// Tiles of a convolution: 256 voxels, or 128 where 256-voxel ones would be
+// fewer than two per CU (32^3 has 128 of them for 256 CUs).
+struct ConvGrid { int zt, ntiles, blocks; };
+constexpr int kConvBlocks = 256;   // persistent workgroups (CUs) of a convolution, at most
+__host__ inline ConvGrid conv_grid(int n)
+{
+    const int64_t v = int64_t(n) * n * n;
+    ConvGrid g;
+    g.zt = v / 256 >= 2 * kConvBlocks ? 2 : 1;
+    g.ntiles = int(v / (128 * g.zt));
+    g.blocks = 8 * std::min((g.ntiles + 7) / 8, kConvBlocks / 8);
+    return g;
+}
+
+// Weight and bias gradients of a layer as a GEMM over voxels:
+// gW[o][t][c] = sum_v go[v][o] act[nb(v, t)][c] and gb[o] = sum_v go[v][o].
+// Slot b of G = min(V / 256, 256) takes the 256-voxel tiles b, b + G, ... (X
+// by 2R by 4 voxels, as the convolutions') and one workgroup; each gradient
+// entry of a slot is one chain of matrix instructions over its tiles' 16-voxel
+// runs in order, and k_grad_slices and k_grad_adam add the slots in order (no
+// atomics).  Training amplifies a last-bit change of a gradient to 1e-4 of the
+// parameters within 40 iterations, so this order is part of the result.
+//
+// Both operands come from channel-last rows: the gfx950 transposing LDS read
+// gives lane l of 16 the l-th of the 16 channels its group reads for four
+// voxels, so two of them make an operand's eight voxels per lane (before:
+// eight 2-byte reads per operand).  The next tile's loads go between the
+// matrix instructions.
+constexpr int kWgThreads = 512, kWgSlots = 256;
+__host__ inline int wg_slots(int n)
+{
+    const int64_t tiles = int64_t(n) * n * n / 256;
+    return tiles < kWgSlots ? int(tiles) : kWgSlots;
+}
+// the slot of a workgroup: neighbouring slots on one XCD where they divide evenly
+__device__ __forceinline__ int wg_slot()
+{
+    const int G = gridDim.x;
+    return G % 8 == 0 ? int(blockIdx.x % 8) * (G / 8) + int(blockIdx.x / 8) : int(blockIdx.x);
+}
+
+__device__ __forceinline__ s8v tr_read(const bf16 *lo, const bf16 *hi)
+{
+    const s4v a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(lo)),
+              b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(hi));
+    s8v r;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) { r[k] = a[k]; r[4 + k] = b[k]; }
+    return r;
+}
+
+// A tile's halo of CA-channel activations and its GC-channel output gradient,
+// staged through registers: NJ 16-byte chunks per thread.
+template <int X, int CA, int GC> struct WgTile {
+    static constexpr int R = 32 / X, TY = 2 * R, HX = X + 2, HY = TY + 2, HV = HX * HY * 6;
+    static constexpr int NCA = CA / 8, NCG = GC / 8, NA = HV * NCA, NG = 256 * NCG;
+    static constexpr int JA = (NA + kWgThreads - 1) / kWgThreads, JG = (NG + kWgThreads - 1) / kWgThreads, NJ = JA + JG;
+    // a lane's first voxel of run q = 4 lz + qq sits at its base + row(qq) + lz planes
+    static constexpr int row(int qq) { return X == 32 ? (qq >> 1) * HX + 16 * (qq & 1) : (X == 16 ? qq * HX : 2 * qq * HX); }
+    static constexpr int half_step() { return X == 8 ? HX : 8; }   // to the second eight voxels of a run
+    int x0, y0, z0, n;
+    const bf16 *act, *go;
+    __device__ void origin(int tile)
+    {
+        const int ntx = n / X, nty = n / TY;
+        x0 = (tile % ntx) * X;
+        y0 = (tile / ntx % nty) * TY;
+        z0 = tile / (ntx * nty) * 4;
+    }
+    __device__ __forceinline__ s8v fetch(int j) const   // (a thread without a last chunk loads another's again)
+    {
+        const int tid = threadIdx.x;
+        if (j < JA) {
+            const int hv = min((tid + j * kWgThreads) / NCA, HV - 1);
+            const int gx = wrap(x0 - 1 + hv % HX, n), gy = wrap(y0 - 1 + hv / HX % HY, n),
+                      gz = wrap(z0 - 1 + hv / (HX * HY), n);
+            return *reinterpret_cast<const s8v *>(act + int64_t(gx + n * (gy + n * gz)) * CA + 8 * (tid % NCA));
+        }
+        const int vl = min((tid + (j - JA) * kWgThreads) / NCG, 255);
+        const int v = x0 + vl % X + n * (y0 + vl / X % TY + n * (z0 + vl / (X * TY)));
+        return *reinterpret_cast<const s8v *>(go + int64_t(v) * GC + 8 * (tid % NCG));
+    }
+    __device__ __forceinline__ void put(int j, const s8v &x, bf16 *sa, bf16 *sg) const
+    {
+        const int e = threadIdx.x + (j < JA ? j : j - JA) * kWgThreads;
+        if (j < JA) {
+            if ((j + 1) * kWgThreads <= NA || e < NA) *reinterpret_cast<s8v *>(sa + 8 * e) = x;
+        } else if ((j - JA + 1) * kWgThreads <= NG || e < NG) {
+            *reinterpret_cast<s8v *>(sg + 8 * e) = x;
+        }
+    }
+};
+
+// LDS of the kernels below (BF16 values): halo, output gradient and, for 8 of
+// them, as many zeros for the absent channels
+template <int X, int CA, int GC> constexpr size_t wg_lds()
+{
+    return sizeof(bf16) * (size_t(WgTile<X, CA, GC>::HV) * CA + 256 * GC * (GC == 8 ? 2 : 1));
+}
+
+// Against 32-channel activations (layers 2 and 3; the latter with the 8-channel
+// output gradient).  Wave w < 8 owns the taps of (dy, dx) = (w / 3, w % 3) for
+// the three dz, so a row of activations read once serves three instructions;
+// the three taps left, (dy, dx) = (2, 2), go to waves 0 to 2: 13 or 14 taps on
+// each SIMD.  64^3: 55 -> 20.5 (layer 2) and 16.4 us (layer 3).
+template <int X, int GC>
+__global__ __launch_bounds__(kWgThreads, 2) void k_wgrad32(const bf16 *__restrict__ go, const bf16 *__restrict__ act,
+                                                           float *__restrict__ part, float *__restrict__ bpart, int n,
+                                                           int ntiles)
+{
+    using T = WgTile<X, kCP, GC>;
+    constexpr int P = T::HY * T::HX;
+    extern __shared__ __align__(16) unsigned short wg_mem[];
+    bf16 *sa = wg_mem, *sg = wg_mem + T::HV * kCP;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, kh = lane >> 5;
+    const int lv = (lane & 15) >> 2, lc = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);   // voxel and channel the lane loads
+    if constexpr (GC == 8)
+        for (int e = tid; e < 256 * GC; e += kWgThreads) sg[256 * GC + e] = 0;
+    const bf16 *gp = sg + (GC == 8 && lc >= GC ? 256 * GC : (8 * kh + lv) * GC + lc);
+    const int lane_at = (lv + kh * T::half_step()) * kCP + lc;
+    const bf16 *bp = sa + ((wave / 3) * T::HX + wave % 3) * kCP + lane_at;
+    const bf16 *bx = sa + ((min(wave, 2)) * P + 2 * T::HX + 2) * kCP + lane_at;
+    f16v acc[3], accx;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = acc[2][r] = accx[r] = 0.f;
+    float bsum = 0.f;
+    T t;
+    t.n = n;
+    t.act = act;
+    t.go = go;
+    const int slot = wg_slot();
+    t.origin(slot);
+    s8v pre[T::NJ];
+#pragma unroll
+    for (int j = 0; j < T::NJ; ++j) pre[j] = t.fetch(j);
+    for (int tile = slot; tile < ntiles; tile += gridDim.x) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < T::NJ; ++j) t.put(j, pre[j], sa, sg);
+        __syncthreads();
+        t.origin(tile + int(gridDim.x) < ntiles ? tile + int(gridDim.x) : tile);
+        s8v g[16], br[2][4];
+        auto read_g = [&](int lz) {
+#pragma unroll
+            for (int qq = 0; qq < 4; ++qq) {
+                const bf16 *q = gp + 16 * (4 * lz + qq) * GC;
+                g[4 * lz + qq] = tr_read(q, q + 4 * GC);
+            }
+        };
+        auto read_b = [&](int p, const bf16 *base, s8v (&b)[4]) {
+#pragma unroll
+            for (int qq = 0; qq < 4; ++qq) {
+                const bf16 *q = base + (p * P + T::row(qq)) * kCP;
+                b[qq] = tr_read(q, q + 4 * kCP);
+            }
+        };
+        read_g(0);
+        read_b(0, bp, br[0]);
+#pragma unroll
+        for (int p = 0; p < 6; ++p) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (p + 1 < 4) read_g(p + 1);
+            if (p + 1 < 6) read_b(p + 1, bp, br[(p + 1) & 1]);
+#pragma unroll
+            for (int j = p * T::NJ / 6; j < (p + 1) * T::NJ / 6; ++j) pre[j] = t.fetch(j);
+#pragma unroll
+            for (int dz = 0; dz < 3; ++dz)
+                if (p - dz >= 0 && p - dz < 4) {
+#pragma unroll
+                    for (int qq = 0; qq < 4; ++qq) acc[dz] = mfma16(g[4 * (p - dz) + qq], br[p & 1][qq], acc[dz]);
+                }
+            if (p == 0 || p == 5) interleave<4, 4, 10>();
+            else if (p == 1 || p == 4) interleave<8, 2, 6>();
+            else interleave<12, 2, 4>();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (wave < 3) {
+            read_b(0, bx, br[0]);
+#pragma unroll
+            for (int lz = 0; lz < 4; ++lz) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (lz < 3) read_b(lz + 1, bx, br[(lz + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int qq = 0; qq < 4; ++qq) accx = mfma16(g[4 * lz + qq], br[lz & 1][qq], accx);
+            }
+        } else if (wave == 7) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) bsum += from_bf16(bf16(g[q][e]));
+        }
+    }
+    auto store = [&](int tap, const f16v &a) {
+#pragma unroll
+        for (int q = 0; q < GC / 8; ++q) {
+            f4v x;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) x[k] = a[4 * q + k];
+            *reinterpret_cast<f4v *>(part + ((int64_t(slot) * kTaps + tap) * (GC / 8) + q) * 256 + 4 * lane) = x;
+        }
+    };
+#pragma unroll
+    for (int dz = 0; dz < 3; ++dz) store(9 * dz + wave, acc[dz]);
+    if (wave < 3) store(9 * wave + 8, accx);
+    if (wave == 7) {
+        bsum += __shfl_xor(bsum, 32);
+        if (lane < kCP) bpart[slot * kCP + lane] = bsum;
+    }
+}
+
+// Against the 8-channel input (layer 1): the 27 x 8 columns in seven tiles of
+// four taps, one per wave; wave 7 sums the bias.  64^3: 26.7 -> 10.3 us.
+template <int X>
+__global__ __launch_bounds__(kWgThreads, 2) void k_wgrad8(const bf16 *__restrict__ go, const bf16 *__restrict__ act,
+                                                          float *__restrict__ part, float *__restrict__ bpart, int n,
+                                                          int ntiles)
+{
+    using T = WgTile<X, kC0P, kCP>;
+    constexpr int P = T::HY * T::HX;
+    extern __shared__ __align__(16) unsigned short wg_mem[];
+    bf16 *sa = wg_mem, *sg = wg_mem + T::HV * kC0P;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, kh = lane >> 5;
+    const int lv = (lane & 15) >> 2, half = (lane >> 4) & 1;
+    const bf16 *gp = sg + (8 * kh + lv) * kCP + 16 * half + 4 * (lane & 3);
+    // the lane loads 4 channels of tap 4 wave + 2 half + ((lane & 3) >> 1);
+    // the columns of a 28th tap (and wave 7's) are never read
+    const int tap = min(4 * wave + 2 * half + ((lane & 3) >> 1), kTaps - 1);
+    const bf16 *bp = sa + (tap / 9 * P + tap / 3 % 3 * T::HX + tap % 3 + lv + kh * T::half_step()) * kC0P + 4 * (lane & 1);
     f16v acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    const bf16 *wrow = sw + i * WS;   // B column: output channel i
-    auto halo = [&](int t) { return ((wz + t / 9) * HY + (ly + (t / 3) % 3)) * HX + (lx + t % 3); };
-    if constexpr (CIP == 8) {
-#pragma unroll 2
-        for (int tt = 0; tt < (kTaps + 1) / 2; ++tt) {
-            const int t = 2 * tt + kh;
-            s8v a, b;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) { a[e] = 0; b[e] = 0; }
-            if (t < kTaps) {
-                a = *reinterpret_cast<const s8v *>(sa + halo(t) * VS);
-                b = *reinterpret_cast<const s8v *>(wrow + t * CIP);
-            }
-            acc = mfma16(a, b, acc);
-        }
-    } else {
-        for (int t = 0; t < kTaps; ++t) {
-            const bf16 *arow = sa + halo(t) * VS + 8 * kh;
-            const bf16 *brow = wrow + t * CIP + 8 * kh;
-#pragma unroll
-            for (int cb = 0; cb < CIP / 16; ++cb)
-                acc = mfma16(*reinterpret_cast<const s8v *>(arow + 16 * cb), *reinterpret_cast<const s8v *>(brow + 16 * cb),
-                             acc);
-        }
-    }
-    const int o = i;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int vl = 8 * (r >> 2) + 4 * kh + (r & 3);   // row of the result: voxel vl of the wave
-        const int gx = x0 + vl % X, gy = y0 + wy * R + vl / X, gz = z0 + wz;
-        const int64_t v = gx + int64_t(n) * (gy + int64_t(n) * gz);
-        float val = acc[r];
-        if constexpr (EPI == 0) {
-            val += bias[o];
-            static_cast<bf16 *>(out)[v * kCP + o] = to_bf16(val > 0.f ? val : 0.f);
-        } else if constexpr (EPI == 1) {
-            if (o < cout) {
-                if (bias) val += bias[o];
-                static_cast<float *>(out)[v * ostride + o] = val;
-            }
-        } else {
-            const float m = from_bf16(mask[v * kCP + o]);
-            static_cast<bf16 *>(out)[v * kCP + o] = to_bf16(m > 0.f ? val : 0.f);
-        }
-    }
-}
-
-// Weight and bias gradients of one layer as a GEMM over voxels on
-// v_mfma_f32_32x32x16_bf16: dW[o][m] = sum_v go[v][o] a[nb(v, m / CIP)][m % CIP]
-// (M = 27 CIP columns, in 32-column tiles) and db[o] = sum_v go[v][o].
-// Workgroups of 8 waves walk the 256-voxel tiles of k_conv (tile =
-// blockIdx.x, blockIdx.x + gridDim.x, ...).  Per tile they stage the
-// activation halo (VS BF16 per voxel: the two lane halves, 8 voxels apart,
-// then read different LDS banks) and the output gradient transposed,
-// goT[o][vl] with vl = lx + X (ly + TY lz), in LDS.  Wave w accumulates the
-// column tiles w, w + 8, ... over all voxels of its workgroup, 16 per
-// instruction: the A operand (lane: o = lane % 32, 8 consecutive voxels
-// along x) is one 16-byte LDS read shared by all of the wave's columns, the
-// B operand the 8 neighbour values of the lane's (tap, channel).  Wave 7
-// also sums the A operands for the bias gradient.  The workgroup's sums go
-// to part[block][o][m] and bpart[block][o]; k_grad_part and k_grad_reduce
-// add the blocks in a fixed order (no atomics: the gradient is the same on
-// every run).
-constexpr int kWgGS = 256 + 8;   // goT row stride (voxels)
-constexpr int kWgBlocks = 256;   // workgroups of a weight-gradient launch (at most)
-__host__ __device__ constexpr int wg_vs(int cip) { return cip + 4; }
-__host__ inline size_t wgrad_lds_bytes(int cip, int n)
-{
-    const int X = conv_x(n), R = 32 / X;
-    return sizeof(bf16) * (size_t(32) * kWgGS + size_t(X + 2) * (2 * R + 2) * 6 * wg_vs(cip));
-}
-__host__ inline int wgrad_blocks(int n)
-{
-    const int tiles = n * n * n / 256;
-    return tiles < kWgBlocks ? tiles : kWgBlocks;
-}
-typedef short s4v __attribute__((ext_vector_type(4)));
-
-template <int CIP>
-__global__ __launch_bounds__(512) void k_wgrad(const bf16 *__restrict__ go, const bf16 *__restrict__ act,
-                                               float *__restrict__ part, float *__restrict__ bpart, int n)
-{
-    constexpr int VS = wg_vs(CIP), M = kTaps * CIP, NT = (M + 31) / 32, TPW = (NT + 7) / 8;
-    extern __shared__ unsigned short wg_lds[];
-    bf16 *goT = wg_lds;               // [32][kWgGS]
-    bf16 *sa = wg_lds + 32 * kWgGS;   // halo [HZ][HY][HX][VS]
-    const int X = conv_x(n), R = 32 / X;
-    const int TY = 2 * R, HX = X + 2, HY = TY + 2, HZ = 6, HV = HX * HY * HZ;
-    const int ntx = n / X, nty = n / TY;
-    const int ntiles = ntx * nty * (n / 4);
-    const int tid = threadIdx.x, nthr = blockDim.x;
-    const int wave = tid >> 6, lane = tid & 63, i = lane & 31, kh = lane >> 5;
-    // the wave's column tiles j = wave + 8 u: the lane's column m = 32 j + i,
-    // its tap's halo offset and its channel
-    int toff[TPW], coff[TPW];
-    bool jok[TPW], mok[TPW];
-#pragma unroll
-    for (int u = 0; u < TPW; ++u) {
-        const int j = wave + 8 * u, m = 32 * j + i;
-        jok[u] = j < NT;
-        mok[u] = jok[u] && m < M;
-        const int t = mok[u] ? m / CIP : 0;
-        toff[u] = ((t / 9) * HY + (t / 3) % 3) * HX + t % 3;
-        coff[u] = mok[u] ? m % CIP : 0;
-    }
-    f16v acc[TPW];
-#pragma unroll
-    for (int u = 0; u < TPW; ++u)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[u][r] = 0.f;
     float bsum = 0.f;
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        int w = tile;
-        const int x0 = (w % ntx) * X;
-        w /= ntx;
-        const int y0 = (w % nty) * TY, z0 = (w / nty) * 4;
-        __syncthreads();   // the previous tile's operands are read
-        for (int e = tid; e < HV * (CIP / 4); e += nthr) {
-            const int hv = e / (CIP / 4), c4 = e - hv * (CIP / 4);
-            const int hx = hv % HX, hy = (hv / HX) % HY, hz = hv / (HX * HY);
-            const int64_t gv = wrap(x0 + hx - 1, n) + int64_t(n) * (wrap(y0 + hy - 1, n) + int64_t(n) * wrap(z0 + hz - 1, n));
-            *reinterpret_cast<s4v *>(sa + hv * VS + 4 * c4) = *reinterpret_cast<const s4v *>(act + gv * CIP + 4 * c4);
-        }
-        for (int e = tid; e < 256 * (kCP / 8); e += nthr) {
-            const int vl = e / (kCP / 8), c8 = e - vl * (kCP / 8);
-            const int lx = vl % X, ly = (vl / X) % TY, lz = vl / (X * TY);
-            const int64_t v = (x0 + lx) + int64_t(n) * ((y0 + ly) + int64_t(n) * (z0 + lz));
-            const s8v g = *reinterpret_cast<const s8v *>(go + v * kCP + 8 * c8);
+    T t;
+    t.n = n;
+    t.act = act;
+    t.go = go;
+    const int slot = wg_slot();
+    t.origin(slot);
+    s8v pre[T::NJ];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) goT[(8 * c8 + k) * kWgGS + vl] = bf16(g[k]);
-        }
+    for (int j = 0; j < T::NJ; ++j) pre[j] = t.fetch(j);
+    for (int tile = slot; tile < ntiles; tile += gridDim.x) {
         __syncthreads();
-        for (int q = 0; q < 16; ++q) {
-            const int vl0 = 16 * q + 8 * kh;   // the lane's 8 voxels: vl0 .. vl0 + 7, along x
-            const s8v a = *reinterpret_cast<const s8v *>(goT + i * kWgGS + vl0);
+#pragma unroll
+        for (int j = 0; j < T::NJ; ++j) t.put(j, pre[j], sa, sg);
+        __syncthreads();
+        t.origin(tile + int(gridDim.x) < ntiles ? tile + int(gridDim.x) : tile);
+        s8v g[2][4], br[2][4];
+        auto read = [&](int lz) {
+#pragma unroll
+            for (int qq = 0; qq < 4; ++qq) {
+                const bf16 *q = gp + 16 * (4 * lz + qq) * kCP, *b = bp + (lz * P + T::row(qq)) * kC0P;
+                g[lz & 1][qq] = tr_read(q, q + 4 * kCP);
+                br[lz & 1][qq] = tr_read(b, b + 4 * kC0P);
+            }
+        };
+        read(0);
+#pragma unroll
+        for (int lz = 0; lz < 4; ++lz) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (lz < 3) read(lz + 1);
+#pragma unroll
+            for (int j = lz * T::NJ / 4; j < (lz + 1) * T::NJ / 4; ++j) pre[j] = t.fetch(j);
             if (wave == 7) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) bsum += from_bf16(bf16(a[e]));
-            }
-            const int lx = vl0 % X, ly = (vl0 / X) % TY, lz = vl0 / (X * TY);
-            const int hb = (lz * HY + ly) * HX + lx;
+                for (int qq = 0; qq < 4; ++qq)
 #pragma unroll
-            for (int u = 0; u < TPW; ++u) {
-                if (!jok[u]) continue;
-                const bf16 *bp = sa + (hb + toff[u]) * VS + coff[u];
-                s8v bv;
+                    for (int e = 0; e < 8; ++e) bsum += from_bf16(bf16(g[lz & 1][qq][e]));
+            } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) bv[e] = mok[u] ? short(bp[e * VS]) : short(0);
-                acc[u] = mfma16(a, bv, acc[u]);
+                for (int qq = 0; qq < 4; ++qq) acc = mfma16(g[lz & 1][qq], br[lz & 1][qq], acc);
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
     }
+    if (wave < 7) {
 #pragma unroll
-    for (int u = 0; u < TPW; ++u) {
-        if (!mok[u]) continue;
-        const int m = 32 * (wave + 8 * u) + i;
+        for (int q = 0; q < 4; ++q) {
+            f4v x;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int o = 8 * (r >> 2) + 4 * kh + (r & 3);
-            part[(int64_t(blockIdx.x) * kCP + o) * M + m] = acc[u][r];
+            for (int k = 0; k < 4; ++k) x[k] = acc[4 * q + k];
+            *reinterpret_cast<f4v *>(part + ((int64_t(slot) * 7 + wave) * 4 + q) * 256 + 4 * lane) = x;
         }
-    }
-    if (wave == 7) {
+    } else {
         bsum += __shfl_xor(bsum, 32);
-        if (kh == 0) bpart[blockIdx.x * kCP + i] = bsum;
+        if (lane < kCP) bpart[slot * kCP + lane] = bsum;
     }
 }
 
-// Bias gradient: gb[o] = sum of part[c][o] over the nch blocks c; one
-// workgroup, eight slices of blocks summed in order.
-__global__ __launch_bounds__(256) void k_bias_reduce(const float *__restrict__ part, float *__restrict__ gb, int nch)
+// First level of the gradient reductions, all layers in one launch: out[s][k]
+// = sum over slice s of the G slots of element k of a slice (kS2, kS1, ...):
+// slots s per .. in order for the weights, s, s + 8, ... for the biases.
+struct GradParts { const float *p2, *p1, *p3, *b1, *b2, *b3; };
+__global__ __launch_bounds__(256) void k_grad_slices(const GradParts P, float *__restrict__ out, int G)
 {
-    __shared__ float sl[8][kCP];
-    const int o = threadIdx.x & (kCP - 1), k = threadIdx.x / kCP;
-    float s = 0.f;
-    for (int c = k; c < nch; c += 8) s += part[c * kCP + o];
-    sl[k][o] = s;
-    __syncthreads();
-    if (threadIdx.x < kCP) {
-        float t = 0.f;
-        for (int j = 0; j < 8; ++j) t += sl[j][o];
-        gb[o] = t;
+    const int k = blockIdx.x * 256 + threadIdx.x, sl = blockIdx.y;
+    if (k >= kSlice) return;
+    const float *src;
+    int stride, c0, c1, step;
+    if (k < kSB1) {
+        if (k < kS1) { src = P.p2 + k; stride = kP2; }
+        else if (k < kS3) { src = P.p1 + (k - kS1); stride = kP1; }
+        else { src = P.p3 + (k - kS3); stride = kP3; }
+        const int per = (G + kWgSlices - 1) / kWgSlices;
+        c0 = sl * per;
+        c1 = min(G, c0 + per);
+        step = 1;
+    } else {
+        src = k < kSB2 ? P.b1 + (k - kSB1) : (k < kSB3 ? P.b2 + (k - kSB2) : P.b3 + (k - kSB3));
+        stride = kCP;
+        c0 = sl;
+        c1 = G;
+        step = kWgSlices;
     }
-}
-
-// First level of the block reductions: out[s][k] = sum of part[c][k] over
-// blocks c = s per .. (s + 1) per - 1 (below nch), k < len; grid (len / 256,
-// slices).
-__global__ __launch_bounds__(256) void k_grad_part(const float *__restrict__ part, float *__restrict__ out, int len,
-                                                   int nch, int per)
-{
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= len) return;
-    const int c0 = blockIdx.y * per, c1 = min(nch, c0 + per);
     float s = 0.f;
-    for (int c = c0; c < c1; ++c) s += part[int64_t(c) * len + k];
-    out[int64_t(blockIdx.y) * len + k] = s;
+#pragma unroll 8
+    for (int c = c0; c < c1; c += step) s += src[int64_t(c) * stride];
+    out[int64_t(sl) * kSlice + k] = s;
 }
 
-// g[k] = sum over nch chunks of part[chunk][k], k < len (second level of the
-// gradient reductions).
-__global__ __launch_bounds__(256) void k_grad_reduce(const float *__restrict__ part, float *__restrict__ g, int len,
-                                                     int nch)
-{
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= len) return;
-    float s = 0.f;
-    for (int ch = 0; ch < nch; ++ch) s += part[int64_t(ch) * len + k];
-    g[k] = s;
-}
-
-// Mean-square loss over V x 5 values: g = 2 (y - t) / (5 V) as BF16 [V][32]
-// (channels 5.. zero), and each workgroup's sum of (y - t)^2 in
-// lpart[block] (k_loss_add adds them to the running loss in order).
-__global__ __launch_bounds__(256) void k_mse(const float *__restrict__ y, const float *__restrict__ tg,
-                                             bf16 *__restrict__ g, double *__restrict__ lpart, int V)
-{
-    __shared__ double ws[4];
-    const int v = blockIdx.x * 256 + threadIdx.x;
-    double s = 0.0;
-    if (v < V) {
-        const float sc = 2.0f / (5.0f * float(V));
-        s8v g0;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            float gv = 0.f;
-            if (c < kC3) {
-                const float d = y[int64_t(v) * kC3 + c] - tg[int64_t(v) * kC3 + c];
-                s += double(d) * double(d);
-                gv = sc * d;
-            }
-            g0[c] = short(to_bf16(gv));
-        }
-        s8v z;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) z[c] = 0;
-        s8v *gp = reinterpret_cast<s8v *>(g + int64_t(v) * kCP);
-        gp[0] = g0;
-#pragma unroll
-        for (int k = 1; k < kCP / 8; ++k) gp[k] = z;
-    }
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) lpart[blockIdx.x] = ((ws[0] + ws[1]) + ws[2]) + ws[3];
-}
-
-// loss += the sum of lpart[0 .. nb - 1] (one workgroup, slices summed in order).
-__global__ __launch_bounds__(256) void k_loss_add(const double *__restrict__ lpart, double *__restrict__ loss, int nb)
+// loss += the sum of lpart[0 .. nb - 1] (one workgroup of 256, slices summed
+// in order).
+__device__ __forceinline__ void loss_add(const double *__restrict__ lpart, double *__restrict__ loss, int nb)
 {
     __shared__ double sl[256];
     double s = 0.0;
@@ -408,16 +717,12 @@ __global__ __launch_bounds__(256) void k_loss_add(const double *__restrict__ lpa
     }
     if (threadIdx.x == 0) *loss += sl[0];
 }
-
-// BF16 [V][32] from an FP32 [V][5] gradient (test hook).
-__global__ void k_pad_grad(const float *__restrict__ gy, bf16 *__restrict__ g, int V)
+__global__ __launch_bounds__(256) void k_loss_add(const double *__restrict__ lpart, double *__restrict__ loss, int nb)
 {
-    const int v = blockIdx.x * 256 + threadIdx.x;
-    if (v >= V) return;
-    for (int c = 0; c < kCP; ++c) g[int64_t(v) * kCP + c] = to_bf16(c < kC3 ? gy[int64_t(v) * kC3 + c] : 0.f);
+    loss_add(lpart, loss, nb);
 }
 
-// BF16 [V][8] input from FP32 [V][5] (test hook).
+// BF16 [V][8] from FP32 [V][5] (inputs and output gradients of the test hooks).
 __global__ void k_pack_host_in(const float *__restrict__ x, bf16 *__restrict__ a, int V)
 {
     const int v = blockIdx.x * 256 + threadIdx.x;
@@ -505,68 +810,97 @@ __global__ void k_target(const double *__restrict__ qc, int64_t NTc, int64_t off
             float((qt[c * NTt + offt + l] - qc[c * NTc + offc + l]) / double(nm.out_scale[c]));
 }
 
-// BF16 weight layouts from the FP32 parameters.
-//  wf1 [32][27][8], wf2 [32][27][32], wf3 [32][27][32] (o < 5 used): forward
-//  wd2 [32][27][32] = W2[o][26-t][c] transposed (c, t, o): data gradient
-//  through layer 2; wd3 (o < 5) through layer 3; wd1 (c < 5) to the input
-//  bb1..3 [32] FP32 biases (zero padded)
+// BF16 weights as the convolutions' lanes hold them: [instruction][lane][8],
+// lane = 32 (K half) + row.  wf1 (PAIR), wf2, wf3 (C32): forward, rows are
+// output channels; wd3 (SINGLE), wd2, wd1 (C32): data gradients, rows are
+// input channels and the tap is the opposite one.  Rows and channels without
+// a parameter stay zero.
 struct Wts {
     bf16 *wf1, *wf2, *wf3, *wd1, *wd2, *wd3;
-    float *bb1, *bb2, *bb3;
 };
-__global__ void k_prep(const float *__restrict__ p, Wts W)
+constexpr int64_t frag_size(Fill f) { return int64_t(fill_frags(f)) * 64 * 8; }
+
+__device__ __forceinline__ int frag_c32(int t, int ch, int row)
 {
-    const int e = blockIdx.x * 256 + threadIdx.x;
-    constexpr int S8 = kCP * kTaps * kC0P, S32 = kCP * kTaps * kCP;
-    if (e < S8) {   // wf1
-        const int o = e / (kTaps * kC0P), t = (e / kC0P) % kTaps, c = e % kC0P;
-        W.wf1[e] = to_bf16(c < kC0 ? p[kOW1 + (o * kTaps + t) * kC0 + c] : 0.f);
-    }
-    if (e < S32) {
-        const int a = e / (kTaps * kCP), t = (e / kCP) % kTaps, b = e % kCP;   // [a][t][b]
-        W.wf2[e] = to_bf16(p[kOW2 + (a * kTaps + t) * kC1 + b]);
-        W.wf3[e] = to_bf16(a < kC3 ? p[kOW3 + (a * kTaps + t) * kC2 + b] : 0.f);
-        // data gradient layouts: row a = input channel c, column b = output channel o
-        const int tf = kTaps - 1 - t;
-        W.wd2[e] = to_bf16(p[kOW2 + (b * kTaps + tf) * kC1 + a]);
-        W.wd3[e] = to_bf16(b < kC3 ? p[kOW3 + (b * kTaps + tf) * kC2 + a] : 0.f);
-        W.wd1[e] = to_bf16(a < kC0 ? p[kOW1 + (b * kTaps + tf) * kC0 + a] : 0.f);
-    }
-    if (e < kCP) {
-        W.bb1[e] = p[kOB1 + e];
-        W.bb2[e] = p[kOB2 + e];
-        W.bb3[e] = e < kC3 ? p[kOB3 + e] : 0.f;
+    return (((2 * t + (ch >> 4)) * 64) + ((ch >> 3) & 1) * 32 + row) * 8 + (ch & 7);
+}
+// Parameter k (value x) into the layouts it appears in.
+__device__ __forceinline__ void put_weight(const Wts &W, int k, float x)
+{
+    const bf16 h = to_bf16(x);
+    if (k < kOB1) {
+        const int o = k / (kTaps * kC0), t = k / kC0 % kTaps, c = k % kC0;
+        W.wf1[((t >> 1) * 64 + (t & 1) * 32 + o) * 8 + c] = h;
+        W.wd1[frag_c32(kTaps - 1 - t, o, c)] = h;
+    } else if (k >= kOW2 && k < kOB2) {
+        const int e = k - kOW2, o = e / (kTaps * kC1), t = e / kC1 % kTaps, c = e % kC1;
+        W.wf2[frag_c32(t, c, o)] = h;
+        W.wd2[frag_c32(kTaps - 1 - t, o, c)] = h;
+    } else if (k >= kOW3 && k < kOB3) {
+        const int e = k - kOW3, o = e / (kTaps * kC2), t = e / kC2 % kTaps, c = e % kC2;
+        W.wf3[frag_c32(t, c, o)] = h;
+        W.wd3[((kTaps - 1 - t) * 64 + c) * 8 + o] = h;
     }
 }
-
-// Flat parameter gradient from the accumulation buffers.
-__device__ inline float param_grad(int k, const float *gw1, const float *gw2, const float *gw3, const float *gb)
-{
-    if (k < kOB1) { const int o = k / (kTaps * kC0), r = k % (kTaps * kC0); return gw1[o * kM1 + (r / kC0) * kC0P + r % kC0]; }
-    if (k < kOW2) return gb[k - kOB1];
-    if (k < kOB2) { const int o = (k - kOW2) / kM2, r = (k - kOW2) % kM2; return gw2[o * kM2 + r]; }
-    if (k < kOW3) return gb[kCP + k - kOB2];
-    if (k < kOB3) { const int o = (k - kOW3) / kM2, r = (k - kOW3) % kM2; return gw3[o * kM2 + r]; }
-    return gb[2 * kCP + k - kOB3];
-}
-
-__global__ void k_gather_grad(const float *gw1, const float *gw2, const float *gw3, const float *gb, float *g)
+__global__ __launch_bounds__(256) void k_prep(const float *__restrict__ p, Wts W)
 {
     const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k < kNParam) g[k] = param_grad(k, gw1, gw2, gw3, gb);
+    if (k < kNParam) put_weight(W, k, p[k]);
 }
 
-__global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m1,
-                       float *__restrict__ m2, float lr, float c1, float c2)
+// Place of parameter k in a slice: row r and column m of an accumulator tile
+// sit at lane 32 ((r >> 2) & 1) + m, value 4 (r >> 3) + r % 4.
+__device__ __forceinline__ int slice_at(int r, int m)
 {
+    return ((r >> 3) * 64 + ((r >> 2) & 1) * 32 + m) * 4 + (r & 3);
+}
+__device__ __forceinline__ int slice_index(int k)
+{
+    if (k < kOB1) {
+        const int o = k / (kTaps * kC0), m = (k / kC0 % kTaps) * kC0P + k % kC0;
+        return kS1 + (m >> 5) * 1024 + slice_at(o, m & 31);
+    }
+    if (k < kOW2) return kSB1 + k - kOB1;
+    if (k < kOB2) {
+        const int e = k - kOW2;
+        return kS2 + e / kC1 % kTaps * 1024 + slice_at(e / (kTaps * kC1), e % kC1);
+    }
+    if (k < kOW3) return kSB2 + k - kOB2;
+    if (k < kOB3) {
+        const int e = k - kOW3;
+        return kS3 + e / kC2 % kTaps * 256 + slice_at(e / (kTaps * kC2), e % kC2);
+    }
+    return kSB3 + k - kOB3;
+}
+
+// Second level: the flat gradient g from the slices and, with update, the
+// Adam update of the parameters and their BF16 copies; the last workgroup
+// adds the nl partial losses to the running loss (lpart null: no loss).
+__global__ __launch_bounds__(256) void k_grad_adam(const float *__restrict__ slices, float *__restrict__ g,
+                                                   float *__restrict__ p, float *__restrict__ m1,
+                                                   float *__restrict__ m2, Wts W, int update, float lr, float c1,
+                                                   float c2,
+                                                   const double *__restrict__ lpart, double *__restrict__ loss, int nl)
+{
+    if (blockIdx.x == gridDim.x - 1) {
+        if (lpart) loss_add(lpart, loss, nl);
+        return;
+    }
     const int k = blockIdx.x * 256 + threadIdx.x;
     if (k >= kNParam) return;
+    const int at = slice_index(k);
+    float gk = 0.f;
+#pragma unroll
+    for (int s = 0; s < kWgSlices; ++s) gk += slices[s * kSlice + at];
+    g[k] = gk;
+    if (!update) return;
     constexpr float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float gk = g[k];
     const float a = b1 * m1[k] + (1.f - b1) * gk, b = b2 * m2[k] + (1.f - b2) * gk * gk;
     m1[k] = a;
     m2[k] = b;
-    p[k] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
+    const float x = p[k] - lr * (a / c1) / (sqrtf(b / c2) + eps);
+    p[k] = x;
+    put_weight(W, k, x);
 }
 
 __global__ void k_fill(float *a, float v, int64_t n)
@@ -599,9 +933,10 @@ struct cnd_net {
     hipEvent_t done = nullptr;
     Norm nm{};
     float *p = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr;   // parameters, gradient, Adam moments
-    float *gacc = nullptr;                                            // gw1 | gw2 | gw3 | gb (3 x 32)
-    // weight and bias gradients per workgroup, and per slice of workgroups
-    float *gpart = nullptr, *gpart2 = nullptr, *bpart = nullptr;
+    // weight and bias gradients per workgroup (layers 2, 1 and 3), and per
+    // slice of workgroups
+    float *gp2 = nullptr, *gp1 = nullptr, *gp3 = nullptr, *b1 = nullptr, *b2 = nullptr, *b3 = nullptr;
+    float *slices = nullptr;
     Wts W{};
     bf16 *x0 = nullptr, *a1 = nullptr, *a2 = nullptr, *g3 = nullptr, *g2 = nullptr, *g1 = nullptr;
     float *y = nullptr, *gx = nullptr, *hx = nullptr;
@@ -630,31 +965,46 @@ int nfail(cnd_net *net, int code, const std::string &m)
 
 inline unsigned blocks_for(int64_t n, int per) { return unsigned((n + per - 1) / per); }
 
-float *gw1(cnd_net *t) { return t->gacc; }
-float *gw2(cnd_net *t) { return t->gacc + kCP * kM1; }
-float *gw3(cnd_net *t) { return t->gacc + kCP * kM1 + kCP * kM2; }
-float *gbias(cnd_net *t) { return t->gacc + kCP * kM1 + 2 * kCP * kM2; }
-constexpr int64_t kGacc = int64_t(kCP) * kM1 + 2 * int64_t(kCP) * kM2 + 3 * kCP;
-
 int net_begin(cnd_net *t, hipStream_t st);
 int net_end(cnd_net *t, hipStream_t st);
 
 int prep(cnd_net *t, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_prep, dim3(blocks_for(kCP * kTaps * kCP, 256)), dim3(256), 0, st, t->p, t->W);
+    hipLaunchKernelGGL(k_prep, dim3(blocks_for(kNParam, 256)), dim3(256), 0, st, t->p, t->W);
     NHIP(t, hipGetLastError());
     return CND_OK;
 }
 
-// forward of the input in x0 into y (normalised correction, FP32 [V][5]),
-// with the hidden activations in a1, a2 (BF16 [V][32])
+template <Fill F, Epi E>
+void conv(cnd_net *t, hipStream_t st, const bf16 *in, const bf16 *w, const float *bias, const bf16 *mask, void *out,
+          const float *tg = nullptr)
+{
+    const ConvGrid g = conv_grid(t->n);
+    const ConvArgs A{in, w, bias, mask, out, tg, t->lpart, t->n, g.ntiles};
+    const dim3 gr(unsigned(g.blocks)), b(kConvThreads);
+    auto go = [&](auto x) {
+        constexpr int X = decltype(x)::value;
+        if (g.zt == 2) hipLaunchKernelGGL((k_conv<F, E, X, 2>), gr, b, 0, st, A);
+        else hipLaunchKernelGGL((k_conv<F, E, X, 1>), gr, b, 0, st, A);
+    };
+    const int x = conv_x(t->n);
+    if (x == 32) go(std::integral_constant<int, 32>{});
+    else if (x == 16) go(std::integral_constant<int, 16>{});
+    else go(std::integral_constant<int, 8>{});
+}
+
+// the hidden activations a1, a2 (BF16 [V][32]) of the input x0
+void hidden(cnd_net *t, const bf16 *x0, bf16 *a1, bf16 *a2, hipStream_t st)
+{
+    conv<PAIR, FWD>(t, st, x0, t->W.wf1, t->p + kOB1, nullptr, a1);
+    conv<C32, FWD>(t, st, a1, t->W.wf2, t->p + kOB2, nullptr, a2);
+}
+
+// forward of the input in x0 into y (normalised correction, FP32 [V][5])
 int forward_into(cnd_net *t, const bf16 *x0, bf16 *a1, bf16 *a2, float *y, hipStream_t st)
 {
-    const dim3 gv(unsigned(t->V / (32 * kConvWaves))), b(64 * kConvWaves);
-    const size_t l8 = conv_lds_bytes(kC0P, t->n), l32 = conv_lds_bytes(kCP, t->n);
-    hipLaunchKernelGGL((k_conv<kC0P, 0>), gv, b, l8, st, x0, t->W.wf1, t->W.bb1, nullptr, a1, t->n, kCP, kCP);
-    hipLaunchKernelGGL((k_conv<kCP, 0>), gv, b, l32, st, a1, t->W.wf2, t->W.bb2, nullptr, a2, t->n, kCP, kCP);
-    hipLaunchKernelGGL((k_conv<kCP, 1>), gv, b, l32, st, a2, t->W.wf3, t->W.bb3, nullptr, y, t->n, kC3, kC3);
+    hidden(t, x0, a1, a2, st);
+    conv<C32, OUT>(t, st, a2, t->W.wf3, t->p + kOB3, nullptr, y);
     NHIP(t, hipGetLastError());
     return CND_OK;
 }
@@ -677,44 +1027,59 @@ int apply_into(cnd_net *t, const CtxView &C, bf16 *x0, bf16 *a1, bf16 *a2, float
     return net_end(t, C.st);
 }
 
-// backward from g3 (dL/dy, BF16 [V][32]) with the activations of the last
-// forward: parameter gradient into t->g; with gx, dL/dx0 into gx (FP32 [V][5]).
+// Sums of the squared errors of the pair (x0, tg) into lpart and, with g3,
+// the loss gradient.
+void forward_loss(cnd_net *t, const bf16 *x0, const float *tg, bf16 *g3, hipStream_t st)
+{
+    hidden(t, x0, t->a1, t->a2, st);
+    conv<C32, LOSS>(t, st, t->a2, t->W.wf3, t->p + kOB3, nullptr, g3, tg);
+}
+
+// Weight and bias gradients of layer 1, 2 or 3 from its output gradient go and
+// its input act.
+void wgrad(cnd_net *t, hipStream_t st, int layer, const bf16 *go, const bf16 *act, float *part, float *bpart)
+{
+    const int tiles = t->V / 256;
+    const dim3 g(unsigned(wg_slots(t->n))), b(kWgThreads);
+    auto run = [&](auto x) {
+        constexpr int X = decltype(x)::value;
+        if (layer == 1)
+            hipLaunchKernelGGL(k_wgrad8<X>, g, b, (wg_lds<X, kC0P, kCP>()), st, go, act, part, bpart, t->n, tiles);
+        else if (layer == 2)
+            hipLaunchKernelGGL((k_wgrad32<X, kCP>), g, b, (wg_lds<X, kCP, kCP>()), st, go, act, part, bpart, t->n, tiles);
+        else
+            hipLaunchKernelGGL((k_wgrad32<X, kC0P>), g, b, (wg_lds<X, kCP, kC0P>()), st, go, act, part, bpart, t->n,
+                               tiles);
+    };
+    const int x = conv_x(t->n);
+    if (x == 32) run(std::integral_constant<int, 32>{});
+    else if (x == 16) run(std::integral_constant<int, 16>{});
+    else run(std::integral_constant<int, 8>{});
+}
+
+// backward from g3 (dL/dy, BF16 [V][8]) with the activations of the last
+// forward: slices of the parameter gradient; with gx, dL/dx0 into gx (FP32
+// [V][5]).
 int backward(cnd_net *t, const bf16 *x0, float *gx, hipStream_t st)
 {
-    const int V = t->V;
-    const dim3 b(256), gv(unsigned(V / (32 * kConvWaves))), bc(64 * kConvWaves);
-    const size_t l32 = conv_lds_bytes(kCP, t->n);
-    const int G = wgrad_blocks(t->n);
-    // weight and bias gradients of a layer from its output gradient go and
-    // input activations act (CIP channels): G block partials, then
-    // kWgSlices slice sums, then the total
-    auto wgrad = [&](auto cip, const bf16 *go, const bf16 *act, float *gw, float *gb) {
-        constexpr int CIP = decltype(cip)::value, M = kTaps * CIP;
-        hipLaunchKernelGGL(k_wgrad<CIP>, dim3(unsigned(G)), dim3(512), wgrad_lds_bytes(CIP, t->n), st, go, act,
-                           t->gpart, t->bpart, t->n);
-        const int per = (G + kWgSlices - 1) / kWgSlices;
-        hipLaunchKernelGGL(k_grad_part, dim3(blocks_for(int64_t(kCP) * M, 256), kWgSlices), b, 0, st, t->gpart,
-                           t->gpart2, kCP * M, G, per);
-        hipLaunchKernelGGL(k_grad_reduce, dim3(blocks_for(int64_t(kCP) * M, 256)), b, 0, st, t->gpart2, gw, kCP * M,
-                           kWgSlices);
-        hipLaunchKernelGGL(k_bias_reduce, dim3(1), b, 0, st, t->bpart, gb, G);
-    };
-    using C32 = std::integral_constant<int, kCP>;
-    using C8 = std::integral_constant<int, kC0P>;
-    // layer 3
-    wgrad(C32{}, t->g3, t->a2, gw3(t), gbias(t) + 2 * kCP);
-    hipLaunchKernelGGL((k_conv<kCP, 2>), gv, bc, l32, st, t->g3, t->W.wd3, nullptr, t->a2, t->g2, t->n, kCP, kCP);
-    // layer 2
-    wgrad(C32{}, t->g2, t->a1, gw2(t), gbias(t) + kCP);
-    hipLaunchKernelGGL((k_conv<kCP, 2>), gv, bc, l32, st, t->g2, t->W.wd2, nullptr, t->a1, t->g1, t->n, kCP, kCP);
-    // layer 1
-    wgrad(C8{}, t->g1, x0, gw1(t), gbias(t));
-    if (gx)
-        hipLaunchKernelGGL((k_conv<kCP, 1>), gv, bc, l32, st, t->g1, t->W.wd1, nullptr, nullptr, gx, t->n, kC0, kC0);
-    hipLaunchKernelGGL(k_gather_grad, dim3(blocks_for(kNParam, 256)), b, 0, st, gw1(t), gw2(t), gw3(t), gbias(t),
-                       t->g);
+    wgrad(t, st, 3, t->g3, t->a2, t->gp3, t->b3);
+    conv<SINGLE, MASK>(t, st, t->g3, t->W.wd3, nullptr, t->a2, t->g2);
+    wgrad(t, st, 2, t->g2, t->a1, t->gp2, t->b2);
+    conv<C32, MASK>(t, st, t->g2, t->W.wd2, nullptr, t->a1, t->g1);
+    wgrad(t, st, 1, t->g1, x0, t->gp1, t->b1);
+    if (gx) conv<C32, OUT>(t, st, t->g1, t->W.wd1, nullptr, nullptr, gx);
+    hipLaunchKernelGGL(k_grad_slices, dim3(blocks_for(kSlice, 256), kWgSlices), dim3(256), 0, st,
+                       GradParts{t->gp2, t->gp1, t->gp3, t->b1, t->b2, t->b3}, t->slices, wg_slots(t->n));
     NHIP(t, hipGetLastError());
     return CND_OK;
+}
+
+// The flat gradient from the slices and, with update, the Adam step; with nl,
+// the partial losses of the pair to the running loss.
+void finish(cnd_net *t, bool update, float lr, float c1, float c2, int nl, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_grad_adam, dim3(blocks_for(kNParam, 256) + 1), dim3(256), 0, st, t->slices, t->g, t->p, t->m1,
+                       t->m2, t->W, update ? 1 : 0, lr, c1, c2, nl ? t->lpart : nullptr, t->loss, nl);
 }
 
 template <class T>
@@ -785,9 +1150,9 @@ int cnd_net_create(int n, int capacity, unsigned long long seed, cnd_net **out)
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
             return nfail(nullptr, CND_EDEVICE, "cnd_net_create: device attributes");
-        const size_t need = std::max(conv_lds_bytes(kCP, n), wgrad_lds_bytes(kCP, n));
+        const size_t need = wg_lds<32, kCP, kCP>();   // the largest of the kernels
         if (need > size_t(lds))
-            return nfail(nullptr, CND_EDEVICE, "cnd_net_create: the convolution tiles need " + std::to_string(need) +
+            return nfail(nullptr, CND_EDEVICE, "cnd_net_create: the weight gradients need " + std::to_string(need) +
                                                    " bytes of LDS, the device has " + std::to_string(lds));
     }
     cnd_net *t = new cnd_net;
@@ -797,22 +1162,23 @@ int cnd_net_create(int n, int capacity, unsigned long long seed, cnd_net **out)
     const int64_t V = t->V;
     int r = CND_OK;
     auto ok = [&](int rc) { if (rc) r = rc; return rc == CND_OK; };
-    const int64_t S8 = int64_t(kCP) * kTaps * kC0P, S32 = int64_t(kCP) * kTaps * kCP;
+    const int64_t S32 = frag_size(C32);
+    const int64_t G = wg_slots(n);
     bool good = hipStreamCreateWithFlags(&t->st, hipStreamNonBlocking) == hipSuccess &&
                 hipEventCreateWithFlags(&t->done, hipEventDisableTiming) == hipSuccess;
     if (!good) r = nfail(t, CND_EDEVICE, "stream or event creation failed");
     good = good && ok(nalloc(t, &t->p, kNParam)) && ok(nalloc(t, &t->g, kNParam)) && ok(nalloc(t, &t->m1, kNParam)) &&
-           ok(nalloc(t, &t->m2, kNParam)) && ok(nalloc(t, &t->gacc, kGacc)) && ok(nalloc(t, &t->W.wf1, S8)) &&
-           ok(nalloc(t, &t->gpart, int64_t(wgrad_blocks(n)) * kCP * kM2)) &&
-           ok(nalloc(t, &t->gpart2, int64_t(kWgSlices) * kCP * kM2)) &&
-           ok(nalloc(t, &t->bpart, int64_t(wgrad_blocks(n)) * kCP)) &&
-           ok(nalloc(t, &t->W.wf2, S32)) && ok(nalloc(t, &t->W.wf3, S32)) && ok(nalloc(t, &t->W.wd1, S32)) &&
-           ok(nalloc(t, &t->W.wd2, S32)) && ok(nalloc(t, &t->W.wd3, S32)) && ok(nalloc(t, &t->W.bb1, kCP)) &&
-           ok(nalloc(t, &t->W.bb2, kCP)) && ok(nalloc(t, &t->W.bb3, kCP)) && ok(nalloc(t, &t->x0, V * kC0P)) &&
-           ok(nalloc(t, &t->a1, V * kCP)) && ok(nalloc(t, &t->a2, V * kCP)) && ok(nalloc(t, &t->g3, V * kCP)) &&
+           ok(nalloc(t, &t->m2, kNParam)) && ok(nalloc(t, &t->gp2, G * kP2)) &&
+           ok(nalloc(t, &t->gp1, G * kP1)) && ok(nalloc(t, &t->gp3, G * kP3)) && ok(nalloc(t, &t->b1, G * kCP)) &&
+           ok(nalloc(t, &t->b2, G * kCP)) && ok(nalloc(t, &t->b3, G * kCP)) &&
+           ok(nalloc(t, &t->slices, kWgSlices * kSlice)) &&
+           ok(nalloc(t, &t->W.wf1, frag_size(PAIR))) && ok(nalloc(t, &t->W.wf2, S32)) &&
+           ok(nalloc(t, &t->W.wf3, S32)) && ok(nalloc(t, &t->W.wd1, S32)) && ok(nalloc(t, &t->W.wd2, S32)) &&
+           ok(nalloc(t, &t->W.wd3, frag_size(SINGLE))) && ok(nalloc(t, &t->x0, V * kC0P)) &&
+           ok(nalloc(t, &t->a1, V * kCP)) && ok(nalloc(t, &t->a2, V * kCP)) && ok(nalloc(t, &t->g3, V * kC0P)) &&
            ok(nalloc(t, &t->g2, V * kCP)) && ok(nalloc(t, &t->g1, V * kCP)) && ok(nalloc(t, &t->y, V * kC3)) &&
            ok(nalloc(t, &t->gx, V * kC0)) && ok(nalloc(t, &t->hx, V * kC0)) && ok(nalloc(t, &t->loss, 1)) &&
-           ok(nalloc(t, &t->lpart, (V + 255) / 256)) &&
+           ok(nalloc(t, &t->lpart, kConvBlocks)) &&
            ok(nalloc(t, &t->din, int64_t(capacity) * V * kC0P)) && ok(nalloc(t, &t->dtg, int64_t(capacity) * V * kC3));
     if (!good) {
         std::string m = t->err;
@@ -834,7 +1200,14 @@ int cnd_net_create(int n, int capacity, unsigned long long seed, cnd_net **out)
     for (int c = 0; c < 5; ++c) { t->nm.in_mean[c] = 0.f; t->nm.in_scale[c] = 1.f; t->nm.out_scale[c] = 1.f; }
     if (hipMemcpy(t->p, h.data(), sizeof(float) * kNParam, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(t->m1, 0, sizeof(float) * kNParam) != hipSuccess ||
-        hipMemset(t->m2, 0, sizeof(float) * kNParam) != hipSuccess || prep(t, t->st) != CND_OK ||
+        hipMemset(t->m2, 0, sizeof(float) * kNParam) != hipSuccess ||
+        hipMemset(t->W.wf1, 0, sizeof(bf16) * frag_size(PAIR)) != hipSuccess ||
+        hipMemset(t->W.wf2, 0, sizeof(bf16) * S32) != hipSuccess ||
+        hipMemset(t->W.wf3, 0, sizeof(bf16) * S32) != hipSuccess ||
+        hipMemset(t->W.wd1, 0, sizeof(bf16) * S32) != hipSuccess ||
+        hipMemset(t->W.wd2, 0, sizeof(bf16) * S32) != hipSuccess ||
+        hipMemset(t->W.wd3, 0, sizeof(bf16) * frag_size(SINGLE)) != hipSuccess ||
+        hipDeviceSynchronize() != hipSuccess || prep(t, t->st) != CND_OK ||
         hipEventRecord(t->done, t->st) != hipSuccess || hipStreamSynchronize(t->st) != hipSuccess) {
         cnd_net_destroy(t);
         return nfail(nullptr, CND_EDEVICE, "initial upload failed");
@@ -848,9 +1221,9 @@ void cnd_net_destroy(cnd_net *t)
     if (!t) return;
     if (t->done) (void)hipEventSynchronize(t->done);
     if (t->st) (void)hipStreamSynchronize(t->st);
-    void *ptrs[] = {t->p, t->g, t->m1, t->m2, t->gacc, t->gpart, t->gpart2, t->bpart, t->W.wf1, t->W.wf2, t->W.wf3, t->W.wd1, t->W.wd2, t->W.wd3,
-                    t->W.bb1, t->W.bb2, t->W.bb3, t->x0, t->a1, t->a2, t->g3, t->g2, t->g1, t->y, t->gx, t->hx,
-                    t->loss, t->lpart, t->din, t->dtg};
+    void *ptrs[] = {t->p, t->g, t->m1, t->m2, t->gp2, t->gp1, t->gp3, t->b1, t->b2, t->b3, t->slices, t->W.wf1,
+                    t->W.wf2, t->W.wf3, t->W.wd1, t->W.wd2, t->W.wd3, t->x0, t->a1, t->a2, t->g3, t->g2, t->g1, t->y,
+                    t->gx, t->hx, t->loss, t->lpart, t->din, t->dtg};
     for (void *p : ptrs) if (p) (void)hipFree(p);
     if (t->done) (void)hipEventDestroy(t->done);
     if (t->st) (void)hipStreamDestroy(t->st);
@@ -966,16 +1339,12 @@ int cnd_net_train(cnd_net *t, int iters, double lr, unsigned long long seed, dou
     for (int it = 0; it < iters; ++it) {
         const int k = pick(rng);
         const bf16 *x0 = t->din + int64_t(k) * V * kC0P;
-        if ((r = forward(t, x0, st))) return r;
-        hipLaunchKernelGGL(k_mse, dim3(blocks_for(V, 256)), dim3(256), 0, st, t->y, t->dtg + int64_t(k) * V * kC3,
-                           t->g3, t->lpart, int(V));
-        hipLaunchKernelGGL(k_loss_add, dim3(1), dim3(256), 0, st, t->lpart, t->loss, int(blocks_for(V, 256)));
+        forward_loss(t, x0, t->dtg + int64_t(k) * V * kC3, t->g3, st);
+        const int nl = conv_grid(t->n).blocks;
         if ((r = backward(t, x0, nullptr, st))) return r;
         ++t->adam_t;
         const float c1 = 1.f - std::pow(0.9f, float(t->adam_t)), c2 = 1.f - std::pow(0.999f, float(t->adam_t));
-        hipLaunchKernelGGL(k_adam, dim3(blocks_for(kNParam, 256)), dim3(256), 0, st, t->p, t->g, t->m1, t->m2,
-                           float(lr), c1, c2);
-        if ((r = prep(t, st))) return r;
+        finish(t, true, float(lr), c1, c2, nl, st);
     }
     double s = 0.0;
     NHIP(t, hipMemcpyAsync(&s, t->loss, sizeof(double), hipMemcpyDeviceToHost, st));
@@ -995,10 +1364,8 @@ int cnd_net_eval(cnd_net *t, int first, int count, double *mean_loss)
     if ((r = net_begin(t, st))) return r;
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, st, reinterpret_cast<float *>(t->loss), 0.f, 2);
     for (int k = first; k < first + count; ++k) {
-        if ((r = forward(t, t->din + int64_t(k) * V * kC0P, st))) return r;
-        hipLaunchKernelGGL(k_mse, dim3(blocks_for(V, 256)), dim3(256), 0, st, t->y, t->dtg + int64_t(k) * V * kC3,
-                           t->g3, t->lpart, int(V));
-        hipLaunchKernelGGL(k_loss_add, dim3(1), dim3(256), 0, st, t->lpart, t->loss, int(blocks_for(V, 256)));
+        forward_loss(t, t->din + int64_t(k) * V * kC0P, t->dtg + int64_t(k) * V * kC3, nullptr, st);
+        hipLaunchKernelGGL(k_loss_add, dim3(1), dim3(256), 0, st, t->lpart, t->loss, conv_grid(t->n).blocks);
     }
     double s = 0.0;
     NHIP(t, hipMemcpyAsync(&s, t->loss, sizeof(double), hipMemcpyDeviceToHost, st));
@@ -1064,8 +1431,9 @@ int cnd_net_grad_host(cnd_net *t, const float *x, const float *gy, float *gx, fl
     hipLaunchKernelGGL(k_pack_host_in, dim3(blocks_for(V, 256)), dim3(256), 0, st, t->hx, t->x0, int(V));
     if ((r = forward(t, t->x0, st))) return r;
     NHIP(t, hipMemcpyAsync(t->gx, gy, sizeof(float) * V * kC3, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_pad_grad, dim3(blocks_for(V, 256)), dim3(256), 0, st, t->gx, t->g3, int(V));
+    hipLaunchKernelGGL(k_pack_host_in, dim3(blocks_for(V, 256)), dim3(256), 0, st, t->gx, t->g3, int(V));
     if ((r = backward(t, t->x0, t->hx, st))) return r;
+    finish(t, false, 0.f, 1.f, 1.f, 0, st);
     NHIP(t, hipMemcpyAsync(gx, t->hx, sizeof(float) * V * kC0, hipMemcpyDeviceToHost, st));
     NHIP(t, hipMemcpyAsync(gp, t->g, sizeof(float) * kNParam, hipMemcpyDeviceToHost, st));
     if ((r = net_end(t, st))) return r;
