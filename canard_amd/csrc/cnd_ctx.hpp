@@ -156,51 +156,101 @@ inline dim3 pts_grid(cnd_ctx *c) { return dim3(unsigned(c->hpt.size())); }
 
 
 inline int ntiles(cnd_ctx *c, int d) { return int(c->htiles[d].size()); }
-// Launch the segmented sweep K (a template-id of the shape G, in parentheses;
-// NV variables) for kind along d with the shape chosen for them; the arguments after the common ones follow.
-#define SEG_CASE(i, K, NV, c, kind, d, xm, y, ...)                                                    \
+// LDS bytes of a segmented launch (cnd_seg.hpp SegShape::lds_bytes).
+inline size_t seg_lds_bytes(const ShapeInfo &G, int nv, int sp, int nmax, bool has_part)
+{
+    const size_t chunk = size_t(G.C) * nv * sp * G.P, part = size_t(2) * kSegEndRows * nv * G.P,
+                 ex = size_t(4) * nv * sp * G.P, lu = size_t(5) * G.L * sp;
+    const size_t tile = size_t(nv) * G.P * size_t(nmax | 1);   // pencils n | 1 apart (SegShape::pencil_stride)
+    if (G.XI) return sizeof(double) * (std::max(tile, lu + ex) + size_t(8) * G.SPMAX + (has_part ? part : 0));
+    return sizeof(double) * (std::max(std::max(chunk, part), ex) + lu + part + size_t(8) * G.SPMAX);
+}
+
+// One segmented launch: shape, tiles, workgroup size and LDS.
+struct SegLaunch {
+    int shape;
+    SegTiles tiles;
+    unsigned threads;
+    size_t lds;
+};
+
+// Eta and zeta sweeps of a kind go in one launch where both have the same
+// shape and the lanes the direction with fewer segments leaves idle are at
+// most a quarter: a launch of a small block is a chain of latencies (10-15 us
+// from 17^3 to 65^3 points), so one launch takes half the time of two, and
+// on large blocks it fills the GPU as two streams did.
+inline bool eta_zeta_joint(const cnd_ctx *c, int kind)
+{
+    const int sh = c->shape[kind][1];
+    if (sh == kTiled || sh != c->shape[kind][2]) return false;
+    const int pi = p_index(kShapes[sh].P), a = c->seg_sp[kind][1], b = c->seg_sp[kind][2], m = std::max(a, b);
+    const int64_t na = int64_t(c->hstiles[pi][1].size()), nb = int64_t(c->hstiles[pi][2].size());
+    return 4 * ((m - a) * na + (m - b) * nb) <= m * (na + nb);
+}
+
+// Launch of nv variables per workgroup for kind along d; joint: of eta (d = 1)
+// and zeta together.
+inline SegLaunch seg_launch(const cnd_ctx *c, int kind, int d, int nv, bool joint = false)
+{
+    const int sh = c->shape[kind][d], pi = p_index(kShapes[sh].P);
+    const int n = int(c->hstiles[pi][d].size()), n2 = joint ? int(c->hstiles[pi][2].size()) : 0;
+    const int sp = joint ? std::max(c->seg_sp[kind][1], c->seg_sp[kind][2]) : c->seg_sp[kind][d];
+    const int nmax = joint ? std::max(c->nmax[1], c->nmax[2]) : c->nmax[d];
+    const bool part = c->part_other[d] || (joint && c->part_other[2]);
+    return SegLaunch{sh, SegTiles{c->dstiles[pi][d], n + n2, sp, d, n}, unsigned(nv * kShapes[sh].P * sp),
+                     seg_lds_bytes(kShapes[sh], nv, sp, nmax, part)};
+}
+
+// Launch the segmented sweep K (a template-id of the shape G, in parentheses)
+// as SL (a SegLaunch) says, over xm x its tiles x y workgroups (kernels with xm > 1 split a
+// tile's work themselves); the arguments after the common ones follow.
+#define SEG_CASE(i, K, c, SL, y, ...)                                                                       \
     case i: {                                                                                              \
         using G = Sh##i;                                                                                   \
-        const int sp_ = (c)->seg_sp[kind][d];                                                              \
-        const int pi_ = p_index(G::P);                                                                     \
-        const int nt_ = int((c)->hstiles[pi_][d].size());                                                  \
-        hipLaunchKernelGGL(K, dim3(unsigned(xcd_width((xm) * nt_)), unsigned(y)),                \
-                           dim3(unsigned((NV) * G::P * sp_)),                                              \
-                           (SegShape<NV, 0, G::L, G::P, G::C, G::XI>::lds_bytes(sp_, G::SPMAX, (c)->nmax[d],     \
-                                                                                (c)->part_other[d])),              \
-                           (c)->st, (c)->dblk,                                                             \
-                           (c)->dtab, seg_tabs(c, G::L), (c)->dstiles[pi_][d], nt_, sp_, d, __VA_ARGS__);   \
+        hipLaunchKernelGGL(K, dim3(unsigned(xcd_width(seg_xm * (SL).tiles.n)), unsigned(y)), dim3((SL).threads), \
+                           (SL).lds, (c)->st, (c)->dblk, (c)->dtab, seg_tabs(c, G::L), (SL).tiles, __VA_ARGS__); \
     } break;
-#define LAUNCH_SEG_XM(K, NV, c, kind, d, xm, y, ...)                                                       \
+// xi shapes, eta / zeta shapes
+#define LAUNCH_SEG_XI(K, c, SL, xm, y, ...)                                                                 \
     do {                                                                                                   \
-        switch ((c)->shape[kind][d]) {                                                                     \
-            SEG_CASE(0, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(1, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(2, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(3, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(4, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(5, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(6, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(7, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(8, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(9, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                       \
-            SEG_CASE(10, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(11, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(12, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(13, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(14, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(15, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(16, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(17, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(18, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(19, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
-            SEG_CASE(20, K, NV, c, kind, d, xm, y, __VA_ARGS__)                                      \
+        constexpr int seg_xm = xm;                                                                         \
+        switch ((SL).shape) {                                                                               \
+            SEG_CASE(0, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(1, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(5, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(7, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(8, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(14, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(15, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(16, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(17, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(18, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(19, K, c, SL, y, __VA_ARGS__) \
             default: break;                                                                                \
         }                                                                                                  \
     } while (0)
-// grid x covers xm * tiles workgroups (kernels that split a tile's work
-// over xm workgroups themselves); LAUNCH_SEG: one workgroup per tile and y
-#define LAUNCH_SEG(K, NV, c, kind, d, y, ...) LAUNCH_SEG_XM(K, NV, c, kind, d, 1, y, __VA_ARGS__)
+#define LAUNCH_SEG_EZ(K, c, SL, xm, y, ...)                                                                 \
+    do {                                                                                                   \
+        constexpr int seg_xm = xm;                                                                         \
+        switch ((SL).shape) {                                                                               \
+            SEG_CASE(2, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(3, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(4, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(6, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(9, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(10, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(11, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(12, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(13, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(20, K, c, SL, y, __VA_ARGS__) \
+            default: break;                                                                                \
+        }                                                                                                  \
+    } while (0)
+#define LAUNCH_SEG(K, c, SL, xm, y, ...)                                                                    \
+    do {                                                                                                   \
+        if ((SL).tiles.d == 0) LAUNCH_SEG_XI(K, c, SL, xm, y, __VA_ARGS__);                                  \
+        else LAUNCH_SEG_EZ(K, c, SL, xm, y, __VA_ARGS__);                                                   \
+    } while (0)
 
 inline SegTabs seg_tabs(cnd_ctx *c, int L)
 {
@@ -234,14 +284,21 @@ inline bool fuse_possible(const cnd_ctx *c)
 // of nvar fields.
 int run_filter_field(cnd_ctx *c, int d, const double *in, double *out, int nvar);
 int run_fd_field(cnd_ctx *c, int d, int n45, const double *in, int64_t ivs, double *out, int64_t ovs, int nvar);
+// Pencil-end arrays of the flux sweeps.
+inline Ends3 ends3(const cnd_ctx *c)
+{
+    return Ends3{{c->drva[0], c->drva[1], c->drva[2]}, {c->FT[0], c->FT[1], c->FT[2]}};
+}
+
 // Gradient sweep along d of the state cur (kind CND_KIND_GRAD).  The xi
 // sweep (d = 0) also stores the primitives u, v, w, T in the flux scratch
 // fl, and the eta and zeta sweeps (segmented) differentiate those: the
-// three must run in order, d = 0 first.
-int run_grad(cnd_ctx *c, int d, const double *cur);
+// three must run in order, d = 0 first.  joint (d = 1): eta and zeta in one
+// launch (eta_zeta_joint).
+int run_grad(cnd_ctx *c, int d, const double *cur, bool joint = false);
 // Flux sweep along d into the d-th right-hand-side buffer (kind
-// CND_KIND_FLUX).
-int run_flux(cnd_ctx *c, int d, const double *cur);
+// CND_KIND_FLUX); joint as for run_grad.
+int run_flux(cnd_ctx *c, int d, const double *cur, bool joint = false);
 // Flux sweep of the stored fluxes along fuse_dir (xi, or zeta) fused with the
 // RK update of stage nk, written to qa; the other two directions' buffers
 // must be complete.

@@ -786,16 +786,6 @@ struct Section {
 // Segments per pencil a launch of shape sh along d needs (the largest over
 // blocks, rounded up to whole waves per variable where that fits), or 0 when
 // some block's pencils do not fit the shape.
-// LDS bytes of a segmented launch (cnd_seg.hpp SegShape::lds_bytes).
-size_t seg_lds_bytes(const ShapeInfo &G, int nv, int sp, int nmax, bool has_part)
-{
-    const size_t chunk = size_t(G.C) * nv * sp * G.P, part = size_t(2) * kSegEndRows * nv * G.P,
-                 ex = size_t(4) * nv * sp * G.P, lu = size_t(5) * G.L * sp;
-    const size_t tile = size_t(nv) * G.P * size_t(nmax | 1);   // pencils n | 1 apart (SegShape::pencil_stride)
-    if (G.XI) return sizeof(double) * (std::max(tile, lu + ex) + size_t(8) * G.SPMAX + (has_part ? part : 0));
-    return sizeof(double) * (std::max(std::max(chunk, part), ex) + lu + part + size_t(8) * G.SPMAX);
-}
-
 int shape_sp(cnd_ctx *c, int sh, int d, int nv)
 {
     const ShapeInfo &G = kShapes[sh];
@@ -883,11 +873,15 @@ int enqueue_stage(cnd_ctx *c, int nk)
         if ((r = tstep_side ? on_side(c, tstep) : tstep())) return r;
     }
     if (c->any_visc) {
-        // the eta sweep beside the zeta sweep when it is a segmented one
-        Section sec(c, CND_SEC_GRAD, 3);
+        // eta and zeta in one launch, or the eta sweep beside the zeta sweep
+        // when it is a segmented one
+        const bool joint = eta_zeta_joint(c, CND_KIND_GRAD);
+        Section sec(c, CND_SEC_GRAD, joint ? 2 : 3);
         if ((r = run_grad(c, 0, cur))) return r;
         if (tstep_side && (r = join_side(c))) return r;
-        if (c->overlap && seg_on(c, CND_KIND_GRAD, 1)) {
+        if (joint) {
+            if ((r = run_grad(c, 1, cur, true))) return r;
+        } else if (c->overlap && seg_on(c, CND_KIND_GRAD, 1)) {
             if ((r = on_side(c, [&] { return run_grad(c, 1, cur); })) || (r = run_grad(c, 2, cur)) ||
                 (r = join_side(c)))
                 return r;
@@ -907,11 +901,22 @@ int enqueue_stage(cnd_ctx *c, int nk)
     }
     const bool fused = fuse_possible(c) && seg_on(c, CND_KIND_FLUX, c->fuse_dir);
     {
-    // the flux sweeps the update does not take in, the eta one beside the
-    // others when it is a segmented one
-    Section sec(c, CND_SEC_FLUX, fused ? 2 : 3);
+    // the flux sweeps the update does not take in: eta and zeta in one launch,
+    // or the eta one beside the others when it is a segmented one
+    const bool joint = !(fused && c->fuse_dir == 2) && eta_zeta_joint(c, CND_KIND_FLUX);
+    Section sec(c, CND_SEC_FLUX, (fused ? 2 : 3) - (joint ? 1 : 0));
     const int other = fused && c->fuse_dir == 0 ? 2 : 0;
-    if (c->overlap && seg_on(c, CND_KIND_FLUX, 1)) {
+    if (joint) {
+        if (fused) {
+            if ((r = run_flux(c, 1, cur, true))) return r;
+        } else if (c->overlap) {
+            if ((r = on_side(c, [&] { return run_flux(c, 1, cur, true); })) || (r = run_flux(c, 0, cur)) ||
+                (r = join_side(c)))
+                return r;
+        } else if ((r = run_flux(c, 0, cur)) || (r = run_flux(c, 1, cur, true))) {
+            return r;
+        }
+    } else if (c->overlap && seg_on(c, CND_KIND_FLUX, 1)) {
         if ((r = on_side(c, [&] { return run_flux(c, 1, cur); })) || (r = run_flux(c, other, cur)) ||
             (!fused && (r = run_flux(c, 2, cur))) || (r = join_side(c)))
             return r;
@@ -1183,7 +1188,11 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
         good = ok(dalloc(c, &c->dtiles[d], c->htiles[d].size())) && ok(dalloc(c, &c->drva[d], 10 * c->FT[d])) &&
                ok(dalloc(c, &c->cmf[d], 6 * c->FT[d])) && ok(dalloc(c, &c->surf[d], 10 * c->FT[d]));
     for (int d = 0; good && d < 3; ++d)
-        for (int pi = 0; good && pi < kNumP; ++pi) good = ok(dalloc(c, &c->dstiles[pi][d], c->hstiles[pi][d].size()));
+        for (int pi = 0; good && pi < kNumP && d != 2; ++pi) {
+            // zeta's list follows eta's, so one launch can cover both
+            good = ok(dalloc(c, &c->dstiles[pi][d], c->hstiles[pi][d].size() + (d == 1 ? c->hstiles[pi][2].size() : 0)));
+            if (good && d == 1) c->dstiles[pi][2] = c->dstiles[pi][1] + c->hstiles[pi][1].size();
+        }
     if (good)
         good = ok(dalloc(c, &c->dpt, c->hpt.size()));
     if (!good) { std::string m = c->err; cnd_destroy(c); return fail(nullptr, r ? r : CND_ENOMEM, m); }
@@ -1269,7 +1278,7 @@ void cnd_destroy(cnd_ctx *c)
         if (c->dseg[li]) hipFree(c->dseg[li]);
     for (int d = 0; d < 3; ++d) {
         if (c->dtiles[d]) hipFree(c->dtiles[d]);
-        for (int pi = 0; pi < kNumP; ++pi)
+        for (int pi = 0; pi < kNumP && d != 2; ++pi)   // zeta's lists are part of eta's
             if (c->dstiles[pi][d]) hipFree(c->dstiles[pi][d]);
         if (c->drva[d]) hipFree(c->drva[d]);
         if (c->cmf[d]) hipFree(c->cmf[d]);
@@ -1398,8 +1407,10 @@ static int ready(cnd_ctx *c)
 
 // Autotuner: for each sweep kind of the step and each direction, times every
 // compiled segmented shape that fits the blocks (and, in FP64, the tiled
-// sweep) on the context's own arrays and keeps the fastest.  All candidates
-// compute the same values up to rounding.  Runs once, before the first step.
+// sweep) on the context's own arrays and keeps the fastest; where eta and zeta
+// can share a launch (eta_zeta_joint), the shapes of that launch.  All
+// candidates compute the same values up to rounding.  Runs once, before the
+// first step.
 static int tune(cnd_ctx *c)
 {
     if (c->tuned) return CND_OK;
@@ -1413,29 +1424,65 @@ static int tune(cnd_ctx *c)
     // the flux sweep that carries the update is timed as the step runs it:
     // fused with the update (into the gradient scratch) where fusion applies
     const bool fz = fuse_possible(c);
-    auto run = [&](int kind, int d) {
+    auto run = [&](int kind, int d, bool joint) {
         if (kind == CND_KIND_FILTER) return run_filter_field(c, d, c->qa, c->fl, 5);
-        if (kind == CND_KIND_GRAD) return run_grad(c, d, c->qa);
+        if (kind == CND_KIND_GRAD) return run_grad(c, d, c->qa, joint);
         if (d == c->fuse_dir && fz) return run_flux_update(c, 1, c->grad);
-        return run_flux(c, d, c->qa);
+        return run_flux(c, d, c->qa, joint);
     };
+    auto set = [&](int kind, int d, int sh) {
+        c->shape[kind][d] = sh;
+        c->seg_sp[kind][d] = sh == kTiled ? 0 : shape_sp(c, sh, d, kind_nv(c, kind, d));
+    };
+    // a compiled shape worth timing: it fits, no shape with the same segments
+    // and pencils but fewer segments per pencil does, and, for sweeps that
+    // stage nothing in runs, none that differs in the run length only
+    auto worth = [&](int kind, int d, int sh) {
+        const int nv = kind_nv(c, kind, d);
+        if (shape_sp(c, sh, d, nv) == 0) return false;
+        const ShapeInfo &A = kShapes[sh];
+        for (int o = 0; o < kNumShapes; ++o) {
+            const ShapeInfo &B = kShapes[o];
+            if (o == sh || B.L != A.L || B.P != A.P || B.XI != A.XI || shape_sp(c, o, d, nv) == 0) continue;
+            if (B.SPMAX < A.SPMAX) return false;
+            if (B.SPMAX == A.SPMAX && (A.XI || nv == 1) && o < sh) return false;
+        }
+        return true;
+    };
+    constexpr int reps = 3;
     for (int kind : {int(CND_KIND_FILTER), int(CND_KIND_GRAD), int(CND_KIND_FLUX)}) {
         if (kind == CND_KIND_GRAD && !c->any_visc) continue;
+        // eta and zeta as one launch, if any shape lets them (no tiled form)
+        bool joint = false;
         for (int d = 0; d < 3 && !r; ++d) {
+            if (joint) break;   // zeta went with eta
             std::vector<int> cands;
-            if (!mix && !(kind == CND_KIND_FLUX && d == c->fuse_dir && fz)) cands.push_back(kTiled);   // no fused tiled form
-            for (int sh = 0; sh < kNumShapes; ++sh)
-                if (shape_sp(c, sh, d, kind_nv(c, kind, d)) > 0) cands.push_back(sh);
-            if (cands.size() < 2) continue;
+            if (d == 1 && kind != CND_KIND_FILTER && !(kind == CND_KIND_FLUX && fz && c->fuse_dir == 2)) {
+                const int s1 = c->shape[kind][1], s2 = c->shape[kind][2];
+                for (int sh = 0; sh < kNumShapes; ++sh) {
+                    if (!worth(kind, 1, sh) || !worth(kind, 2, sh)) continue;
+                    set(kind, 1, sh);
+                    set(kind, 2, sh);
+                    if (eta_zeta_joint(c, kind)) cands.push_back(sh);
+                }
+                set(kind, 1, s1);
+                set(kind, 2, s2);
+                joint = !cands.empty();
+            }
+            if (!joint) {
+                if (!mix && !(kind == CND_KIND_FLUX && d == c->fuse_dir && fz)) cands.push_back(kTiled);   // no fused tiled form
+                for (int sh = 0; sh < kNumShapes; ++sh)
+                    if (worth(kind, d, sh)) cands.push_back(sh);
+                if (cands.size() < 2) continue;
+            }
             int best = c->shape[kind][d];
             double best_ms = 1e300;
             for (int cand : cands) {
-                c->shape[kind][d] = cand;
-                c->seg_sp[kind][d] = cand == kTiled ? 0 : shape_sp(c, cand, d, kind_nv(c, kind, d));
-                constexpr int reps = 3;
-                if ((r = run(kind, d))) break;
+                set(kind, d, cand);
+                if (joint) set(kind, 2, cand);
+                if ((r = run(kind, d, joint))) break;
                 (void)hipEventRecord(e0, c->st);
-                for (int i = 0; i < reps && !r; ++i) r = run(kind, d);
+                for (int i = 0; i < reps && !r; ++i) r = run(kind, d, joint);
                 (void)hipEventRecord(e1, c->st);
                 if (r) break;
                 float ms = 0.f;
@@ -1445,9 +1492,12 @@ static int tune(cnd_ctx *c)
                 }
                 if (ms / reps < best_ms) { best_ms = ms / reps; best = cand; }
             }
-            c->shape[kind][d] = best;
-            c->seg_sp[kind][d] = best == kTiled ? 0 : shape_sp(c, best, d, kind_nv(c, kind, d));
+            set(kind, d, best);
             c->tune_ms[kind][d] = best_ms;
+            if (joint) {   // a direction's share of the common launch
+                set(kind, 2, best);
+                c->tune_ms[kind][1] = c->tune_ms[kind][2] = best_ms / 2;
+            }
         }
     }
     (void)hipEventDestroy(e0);

@@ -28,16 +28,16 @@ __global__ __launch_bounds__(kPts) void k_prims(const BlkDev *__restrict__ blks,
 
 }  // namespace
 
-int run_grad(cnd_ctx *c, int d, const double *cur)
+int run_grad(cnd_ctx *c, int d, const double *cur, bool joint)
 {
     const int K = CND_KIND_GRAD;
     const bool mix = c->precision == CND_MIXED;   // FP32 gradients (segmented only)
     double *prim = c->fl;   // the fluxes of the previous stage are consumed by now
     if (d == 0) {
         if (mix) {
-            LAUNCH_SEG((k_seg_grad<G, float>), 4, c, K, 0, 1, cur, c->gradf, c->NT, prim);
+            LAUNCH_SEG_XI((k_seg_grad<G, float>), c, seg_launch(c, K, 0, 4), 1, 1, cur, c->gradf, c->NT, prim);
         } else if (seg_on(c, K, 0)) {
-            LAUNCH_SEG((k_seg_grad<G, double>), 4, c, K, 0, 1, cur, c->grad, c->NT, prim);
+            LAUNCH_SEG_XI((k_seg_grad<G, double>), c, seg_launch(c, K, 0, 4), 1, 1, cur, c->grad, c->NT, prim);
         } else {
             LAUNCH_SWEEP(k_fd_grad, 4, c, 0, 1, 4 * kTile, c->dblk, c->dtab, c->dlu, c->dtiles[0], ntiles(c, 0), 0,
                          c->nmax[0], c->ys, cur, c->grad, c->NT);
@@ -45,9 +45,9 @@ int run_grad(cnd_ctx *c, int d, const double *cur)
                 hipLaunchKernelGGL(k_prims, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dpt, cur, prim, c->NT);
         }
     } else if (mix) {
-        LAUNCH_SEG((k_seg_grad_prim<G, float>), 1, c, K, d, 4, prim, c->gradf, c->NT);
+        LAUNCH_SEG_EZ((k_seg_grad_prim<G, float>), c, seg_launch(c, K, d, 1, joint), 1, 4, prim, c->gradf, c->NT);
     } else if (seg_on(c, K, d)) {
-        LAUNCH_SEG((k_seg_grad_prim<G, double>), 1, c, K, d, 4, prim, c->grad, c->NT);
+        LAUNCH_SEG_EZ((k_seg_grad_prim<G, double>), c, seg_launch(c, K, d, 1, joint), 1, 4, prim, c->grad, c->NT);
     } else {
         LAUNCH_SWEEP(k_fd_grad, 4, c, d, 1, 4 * kTile, c->dblk, c->dtab, c->dlu, c->dtiles[d], ntiles(c, d), d,
                      c->nmax[d], c->ys, cur, c->grad, c->NT);

@@ -6,10 +6,8 @@ namespace cnd {
 
 int run_flux_update(cnd_ctx *c, int nk, double *qa)
 {
-    const int K = CND_KIND_FLUX, d = c->fuse_dir;
-    const double *F = c->fl + 5 * d * c->NT;
-    LAUNCH_SEG_XM((k_seg_flux_update<G>), 1, c, K, d, 5, 1, c->dinst, F, c->de, c->qo, c->met, qa, c->drva[d], c->NT,
-                  c->FT[d], nk);
+    const SegLaunch L = seg_launch(c, CND_KIND_FLUX, c->fuse_dir, 1);
+    LAUNCH_SEG((k_seg_flux_update<G>), c, L, 5, 1, c->dinst, c->fl, c->de, c->qo, c->met, qa, ends3(c), c->NT, nk);
     return check_launch(c);
 }
 

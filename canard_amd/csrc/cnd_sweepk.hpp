@@ -387,33 +387,39 @@ __host__ __device__ constexpr int p_index(int P)
 }
 __host__ __device__ constexpr int l_index(int L) { return L == 17 ? 0 : 1; }
 
-#define SEG_PROLOGUE(ntiles)               \
-    const int tix = xcd_tile(ntiles);      \
-    if (tix >= (ntiles)) return;           \
+// Tiles of one direction d (split = ntiles), or of eta and zeta in one launch
+// (d = 1; tiles from split on are zeta's).
+struct SegTiles {
+    const Tile *list;
+    int n, SP, d, split;
+    __device__ int dir(int tix) const { return d + (tix >= split ? 1 : 0); }
+};
+#define SEG_PROLOGUE                       \
+    const int tix = xcd_tile(tiles.n);     \
+    if (tix >= tiles.n) return;            \
+    const int d = tiles.dir(tix);          \
     extern __shared__ double lds[];
 
 template <class G>
 __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_fd_field(
-    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
-    int ntiles, int SP, int d, int n45, const double *in, int64_t in_vstride, double *out, int64_t out_vstride)
+    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles, int n45, const double *in, int64_t in_vstride, double *out, int64_t out_vstride)
 {
-    SEG_PROLOGUE(ntiles)
+    SEG_PROLOGUE
     const int v = blockIdx.y;
     SrcField<1> src{in + v * in_vstride, 0};
     SinkOut<1> sink{out + v * out_vstride, 0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles[tix], d, n45, SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles.list[tix], d, n45, tiles.SP, src, sink, lds);
 }
 
 template <class G>
 __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_filter_field(
-    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
-    int ntiles, int SP, int d, const double *in, double *out, int64_t vstride)
+    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles, const double *in, double *out, int64_t vstride)
 {
-    SEG_PROLOGUE(ntiles)
+    SEG_PROLOGUE
     const int v = blockIdx.y;
     SrcField<1> src{in + v * vstride, 0};
     SinkFilt<1> sink{out + v * vstride, in + v * vstride, 0};
-    seg_tile<1, 1, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles[tix], d, 0, SP, src, sink, lds);
+    seg_tile<1, 1, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles.list[tix], d, 0, tiles.SP, src, sink, lds);
 }
 
 // Velocity and temperature gradients along d, stored as TG (float in mixed
@@ -421,55 +427,58 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
 // written there.
 template <class G, class TG>
 __global__ __launch_bounds__(wg_bound(4 * G::P * G::SPMAX), (seg_waves<G>())) void k_seg_grad(
-    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
-    int ntiles, int SP, int d, const double *q, TG *grad,
+    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles, const double *q, TG *grad,
     int64_t NT, double *prim)
 {
-    SEG_PROLOGUE(ntiles)
+    SEG_PROLOGUE
     SrcPrim src{q, NT, prim};
     SinkOut<4, TG> sink{grad + 4 * d * NT, NT};
-    seg_tile<4, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles[tix], d, 0, SP, src, sink, lds);
+    seg_tile<4, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles.list[tix], d, 0, tiles.SP, src, sink, lds);
 }
 
 // Gradients along d (eta, zeta) of the primitive v = blockIdx.y that the xi
 // gradient sweep stored (prim, four fields NT apart), into grad as TG.
 template <class G, class TG>
 __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_grad_prim(
-    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
-    int ntiles, int SP, int d, const double *prim, TG *grad,
+    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles, const double *prim, TG *grad,
     int64_t NT)
 {
-    SEG_PROLOGUE(ntiles)
+    SEG_PROLOGUE
     const int v = blockIdx.y;
     SrcField<1> src{prim + v * NT, 0};
     SinkOut<1, TG> sink{grad + (4 * d + v) * NT, 0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles[tix], d, 0, SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles.list[tix], d, 0, tiles.SP, src, sink, lds);
 }
 
+// Pencil-end derivatives of the three directions, and their face strides.
+struct Ends3 { double *drva[3]; int64_t FT[3]; };
+
+// Flux derivatives along d into the d-th right-hand-side buffer of de:
+// inviscid fluxes evaluated in the sweep ...
 template <class G>
 __global__ __launch_bounds__(wg_bound(5 * G::P * G::SPMAX), (seg_waves<G>())) void k_seg_flux(
-    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
-    int ntiles, int SP, int d, const InstDev *__restrict__ inst, const double *q, const double *met, double *de,
-    double *drva, int64_t NT, int64_t FT)
+    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles,
+    const InstDev *__restrict__ inst, const double *q, const double *met, double *de, const Ends3 ends, int64_t NT)
 {
-    SEG_PROLOGUE(ntiles)
-    const Tile t = tiles[tix];
+    SEG_PROLOGUE
+    const Tile t = tiles.list[tix];
     SrcFlux src{q, met, blks, inst, NT, d};
-    SinkFlux sink{de, drva, NT, FT, blks[t.b].foff[d] + t.q0};
-    seg_tile<5, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, SP, src, sink, lds);
+    SinkFlux sink{de + 5 * d * NT, ends.drva[d], NT, ends.FT[d], blks[t.b].foff[d] + t.q0};
+    seg_tile<5, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
 }
 
+// ... or component v = blockIdx.y of the stored ones.
 template <class G>
 __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_flux_field(
-    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
-    int ntiles, int SP, int d, const double *F, double *de, double *drva, int64_t NT, int64_t FT)
+    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles,
+    const double *F, double *de, const Ends3 ends, int64_t NT)
 {
-    SEG_PROLOGUE(ntiles)
+    SEG_PROLOGUE
     const int v = blockIdx.y;
-    const Tile t = tiles[tix];
-    SrcField<1> src{F + v * NT, 0};
-    SinkFluxV sink{de + v * NT, drva, v, FT, blks[t.b].foff[d] + t.q0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, SP, src, sink, lds);
+    const Tile t = tiles.list[tix];
+    SrcField<1> src{F + (5 * d + v) * NT, 0};
+    SinkFluxV sink{de + (5 * d + v) * NT, ends.drva[d], v, ends.FT[d], blks[t.b].foff[d] + t.q0};
+    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
 }
 
 // Last flux sweep of a stage fused with the RK update: sweep of the stored
@@ -477,24 +486,24 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
 // Grid x: five workgroups (components) per tile.
 template <class G>
 __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_flux_update(
-    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const Tile *__restrict__ tiles,
-    int ntiles, int SP, int d, const InstDev *__restrict__ inst, const double *F, const double *de,
-    const double *__restrict__ qo, const double *__restrict__ met, double *qa, double *drva, int64_t NT, int64_t FT,
-    int nk)
+    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles,
+    const InstDev *__restrict__ inst, const double *F, const double *de, const double *__restrict__ qo,
+    const double *__restrict__ met, double *qa, const Ends3 ends, int64_t NT, int nk)
 {
     // the five component workgroups of a tile follow each other on one XCD,
     // so the Jacobian they all read is fetched once into that XCD's L2
-    const int w = xcd_tile(5 * ntiles);
-    if (w >= 5 * ntiles) return;
+    const int w = xcd_tile(5 * tiles.n);
+    if (w >= 5 * tiles.n) return;
     extern __shared__ double lds[];
-    const int tix = w / 5, v = w % 5;
-    const Tile t = tiles[tix];
-    SrcField<1> src{F + v * NT, 0};
+    const int tix = w / 5, v = w % 5, d = tiles.d;
+    const Tile t = tiles.list[tix];
+    SrcField<1> src{F + (5 * d + v) * NT, 0};
     const double dtk = inst[blks[t.b].inst].dt / double(4 - nk + 1);
     // the two other directions' right-hand sides
     const double *da = de + ((G::XI ? 5 : 0) + v) * NT, *db = de + ((G::XI ? 10 : 5) + v) * NT;
-    SinkUpdateV<G::XI> sink{qa + v * NT, drva, qo + v * NT, da, db, met, dtk, v, NT, FT, blks[t.b].foff[d] + t.q0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, SP, src, sink, lds);
+    SinkUpdateV<G::XI> sink{qa + v * NT, ends.drva[d], qo + v * NT, da, db, met, dtk, v, NT, ends.FT[d],
+                            blks[t.b].foff[d] + t.q0};
+    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
 }
 
 }  // namespace cnd
