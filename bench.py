@@ -33,20 +33,22 @@ STEP_BYTES_MODEL = 5048.0  # compulsory FP64 bytes per stored point per viscous 
 # Algorithmic HBM bytes per stored point of one launch of each kernel group
 # (reads + writes of FP64 fields the kernel must touch):
 #   filter sweep (5 variables, one direction): read 5 + write 5 fields
-#   gradient sweeps (u,v,w,T, three directions): the xi sweep reads q (5)
-#                   and writes the 4 gradients and the 4 primitives, the
-#                   eta and zeta sweeps read the primitives (4) and write
-#                   4 gradients: 232 B over three launches, 77.33 per launch
-#   stress + flux assembly: read q 5, 12 gradients, 9 metrics + Jacobian;
-#                           write the fluxes of all three directions (15)
-#   flux sweep (one direction): read the 5 fluxes of d, write its own
-#                               right-hand-side buffer (5)
+#   gradients: the primitives (read q 5, write u,v,w,T; stages 2 to 4 write
+#              them with the averaging of the stage before, in the "avg"
+#              section) and one launch of the eta and zeta sweeps (read the
+#              primitives 4, write 4 gradients, each): 72 / 4 + 128 over
+#              1.25 launches a stage, 116.8 per launch
+#   stress: the xi gradients, stresses and fluxes in one kernel: read q 5,
+#           8 gradients, 9 metrics + Jacobian; write the fluxes of all three
+#           directions (15)
+#   flux sweeps (eta and zeta in one launch): read the 10 fluxes, write the
+#              two right-hand-side buffers (10)
 #   update: read qo 5, the three right-hand-side buffers (15), Jacobian;
 #           write qa 5.  Viscous stages without characteristic faces run it
 #           in the xi flux sweep (the "flux" group then has the eta and zeta
-#           launches): read the 5 xi fluxes, the eta and zeta buffers (10),
+#           launch): read the 5 xi fluxes, the eta and zeta buffers (10),
 #           qo 5, Jacobian; write qa 5 -- the same 208 B
-SECTION_BYTES = {"filter": 80.0, "grad": 232.0 / 3.0, "stress": 336.0, "flux": 80.0, "update": 208.0}
+SECTION_BYTES = {"filter": 80.0, "grad": (72.0 / 4.0 + 128.0) / 1.25, "stress": 304.0, "flux": 160.0, "update": 208.0}
 
 
 def parse():

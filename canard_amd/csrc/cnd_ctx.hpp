@@ -84,6 +84,7 @@ struct cnd_ctx {
     double *qa = nullptr, *qo = nullptr, *de = nullptr, *grad = nullptr, *fl = nullptr, *met = nullptr;
     double *ys = nullptr, *xyz = nullptr, *sponge = nullptr, *sp_par = nullptr;
     int nmax[3] = {0, 0, 0};   // longest pencil per direction
+    int segs[kNumL][3] = {};   // its segments of L points
     bool part_other[3] = {};   // some block has another block as interface partner along d
     int64_t ys_len = 0;        // doubles in the forward-value scratch
     double *drva[3] = {}, *cmf[3] = {}, *surf[3] = {};
@@ -96,6 +97,9 @@ struct cnd_ctx {
     // or cnd_step), 1..4 cnd_rk_stage(nk), 5 cnd_end_step
     int next_call = 0;
     bool any_gcbc = false, any_wall = false, any_avg = false, any_sponge = false, any_visc = false;
+    bool avg_self = false;    // averaged faces, each between a block and itself
+    bool ended = false;       // the step's last averaging has ended the step
+    unsigned *tstep_done = nullptr;   // workgroups of k_tstep that are through
     bool gcbc_dir[3] = {}, wall_dir[3] = {};   // directions with such faces
     bool any_frame = false;   // some instance's frame accelerates (nsmf = 0)
     bool use_graph = false;
@@ -183,7 +187,8 @@ inline bool eta_zeta_joint(const cnd_ctx *c, int kind)
 {
     const int sh = c->shape[kind][1];
     if (sh == kTiled || sh != c->shape[kind][2]) return false;
-    const int pi = p_index(kShapes[sh].P), a = c->seg_sp[kind][1], b = c->seg_sp[kind][2], m = std::max(a, b);
+    const int pi = p_index(kShapes[sh].P), li = l_index(kShapes[sh].L);
+    const int a = c->segs[li][1], b = c->segs[li][2], m = std::max(a, b);
     const int64_t na = int64_t(c->hstiles[pi][1].size()), nb = int64_t(c->hstiles[pi][2].size());
     return 4 * ((m - a) * na + (m - b) * nb) <= m * (na + nb);
 }
@@ -256,7 +261,7 @@ inline SegTabs seg_tabs(cnd_ctx *c, int L)
 {
     return SegTabs{c->dlu, c->dseg[l_index(L)]};
 }
-inline bool seg_on(cnd_ctx *c, int kind, int d) { return c->shape[kind][d] != kTiled; }
+inline bool seg_on(const cnd_ctx *c, int kind, int d) { return c->shape[kind][d] != kTiled; }
 
 
 // Variables per workgroup of a sweep kind along d (viscous flux sweeps run
@@ -290,12 +295,18 @@ inline Ends3 ends3(const cnd_ctx *c)
     return Ends3{{c->drva[0], c->drva[1], c->drva[2]}, {c->FT[0], c->FT[1], c->FT[2]}};
 }
 
-// Gradient sweep along d of the state cur (kind CND_KIND_GRAD).  The xi
-// sweep (d = 0) also stores the primitives u, v, w, T in the flux scratch
-// fl, and the eta and zeta sweeps (segmented) differentiate those: the
-// three must run in order, d = 0 first.  joint (d = 1): eta and zeta in one
-// launch (eta_zeta_joint).
+// Viscous stages, in this order.  run_prims: u, v, w, T of the state cur in
+// the flux scratch fl, for segmented eta and zeta sweeps.  run_grad: gradient
+// sweep along d (kind CND_KIND_GRAD; eta and zeta, xi only where it is the
+// tiled one); joint (d = 1): eta and zeta in one launch (eta_zeta_joint).
+// run_grad_flux: the xi gradients with the stresses and all fluxes into fl.
+inline bool prims_wanted(const cnd_ctx *c)
+{
+    return c->any_visc && (seg_on(c, CND_KIND_GRAD, 1) || seg_on(c, CND_KIND_GRAD, 2));
+}
+int run_prims(cnd_ctx *c, const double *cur);
 int run_grad(cnd_ctx *c, int d, const double *cur, bool joint = false);
+int run_grad_flux(cnd_ctx *c, const double *cur);
 // Flux sweep along d into the d-th right-hand-side buffer (kind
 // CND_KIND_FLUX); joint as for run_grad.
 int run_flux(cnd_ctx *c, int d, const double *cur, bool joint = false);

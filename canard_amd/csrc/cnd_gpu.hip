@@ -38,52 +38,18 @@ namespace {
     if (lp >= npt) return;                                               \
     const int64_t g = B.off + lp;
 
-// Viscous stresses and heat flux (src/mo_physics.f90:245-299) and, from
-// them, the fluxes of all three directions (src/mo_physics.f90:319-382),
-// stored as F[5 d + m] for the flux sweeps.  TG: storage type of the
-// gradients (float in mixed mode); stresses and fluxes are FP64.
-template <class TG>
+// Viscous stresses, heat flux and fluxes (visc_point) from stored gradients of
+// all three directions, where the xi gradient sweep is the tiled one.
 __global__ __launch_bounds__(kPts) void k_visc_flux(const BlkDev *__restrict__ blks, const InstDev *__restrict__ inst,
                                                    const Tile *__restrict__ tiles, const double *__restrict__ q,
-                                                   const TG *__restrict__ grad, const double *__restrict__ met,
+                                                   const double *__restrict__ grad, const double *__restrict__ met,
                                                    double *__restrict__ F, int64_t NT)
 {
     POINT_PROLOGUE
-    const InstDev &I = inst[B.inst];
-    const double q1 = q[g], q5 = q[4 * NT + g];
-    const double ri = 1.0 / q1;
-    const double q2 = q[NT + g], q3 = q[2 * NT + g], q4 = q[3 * NT + g];
-    const double u = q2 * ri, v = q3 * ri, w = q4 * ri;
-    const double p = kGm1 * (q5 - 0.5 * ((q2 * u + q3 * v) + q4 * w));
-    const double T = (kGam * p) * ri;
-    const double mu = (I.srefp1dre * pow(T, 1.5)) / (T + I.srefoo);
-    double mt[9];
+    double gx[4];
 #pragma unroll
-    for (int c = 0; c < 9; ++c) mt[c] = met[c * NT + g];
-    auto G = [&](int d, int var) { return double(grad[(4 * d + var) * NT + g]); };
-    auto CT = [&](int c, int var) { return (mt[c] * G(0, var) + mt[3 + c] * G(1, var)) + mt[6 + c] * G(2, var); };
-    const double vtxx = CT(0, 0), vhzz = CT(1, 0), vtzx = CT(2, 0);
-    const double vtxy = CT(0, 1), vtyy = CT(1, 1), vhxx = CT(2, 1);
-    const double vhyy = CT(0, 2), vtyz = CT(1, 2), vtzz = CT(2, 2);
-    const double s1 = CT(0, 3), s2 = CT(1, 3), s3 = CT(2, 3);
-    const double r1 = mu * met[9 * NT + g];
-    const double r2 = kGm1PrI * r1;
-    const double d5 = kTwoThirds * ((vtxx + vtyy) + vtzz);
-    double ts[9];
-    const double txx = r1 * ((vtxx + vtxx) - d5), tyy = r1 * ((vtyy + vtyy) - d5), tzz = r1 * ((vtzz + vtzz) - d5);
-    const double txy = r1 * (vtxy + vhzz), tyz = r1 * (vtyz + vhxx), tzx = r1 * (vtzx + vhyy);
-    ts[0] = txx; ts[1] = tyy; ts[2] = tzz; ts[3] = txy; ts[4] = tyz; ts[5] = tzx;
-    ts[6] = ((r2 * s1 + u * txx) + v * txy) + w * tzx;
-    ts[7] = ((r2 * s2 + u * txy) + v * tyy) + w * tyz;
-    ts[8] = ((r2 * s3 + u * tzx) + v * tyz) + w * tzz;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const double m[3] = {mt[3 * d], mt[3 * d + 1], mt[3 * d + 2]};
-        double o[5];
-        dir_flux<true>(q1, q2, q3, q4, q5, u, v, w, p, m, I.umf, ts, o);
-#pragma unroll
-        for (int c = 0; c < 5; ++c) F[(5 * d + c) * NT + g] = o[c];
-    }
+    for (int k = 0; k < 4; ++k) gx[k] = grad[k * NT + g];
+    visc_point(inst[B.inst], g, gx, q, grad, met, F, NT);
 }
 
 __device__ __forceinline__ double wave_max(double v)
@@ -94,7 +60,7 @@ __device__ __forceinline__ double wave_max(double v)
 
 // Spectral-radius maxima of calc_time_step (src/mo_physics.f90:185-207);
 // runs only on steps where mod(n,10) == 1.  Each workgroup (one point tile)
-// folds its two maxima into its instance's (I.red, cleared by k_sched) with
+// folds its two maxima into its instance's (I.red, cleared by sched) with
 // an atomic max of their bit patterns, which order like the values for
 // non-negative doubles: the result does not depend on the order of the
 // workgroups.  A workgroup whose maximum does not exceed what it reads
@@ -123,7 +89,7 @@ __device__ __forceinline__ void tstep_tile(const Tile t, const BlkDev *__restric
         const double u = q2 * ri, v = q3 * ri, w = q4 * ri;
         const double p = kGm1 * (q[4 * NT + g] - 0.5 * ((q2 * u + q3 * v) + q4 * w));
         const double T = (kGam * p) * ri;
-        const double mu = (I.srefp1dre * pow(T, 1.5)) / (T + I.srefoo);
+        const double mu = viscosity(I, T);
         double mt[9];
         for (int c = 0; c < 9; ++c) mt[c] = met[c * NT + g];
         double r1 = mt[0] * mt[0] + mt[1] * mt[1];
@@ -145,21 +111,74 @@ __device__ __forceinline__ void tstep_tile(const Tile t, const BlkDev *__restric
         const unsigned long long ab = (unsigned long long)__double_as_longlong(a),
                                  cb = (unsigned long long)__double_as_longlong(c);
         volatile unsigned long long *seen = I.red;
-        if (a >= 0.0 && ab > seen[0]) atomicMax(&I.red[0], ab);
-        if (c >= 0.0 && cb > seen[1]) atomicMax(&I.red[1], cb);
+        // (the old values are waited for, so both maxima stand before the lane
+        // counts its workgroup; a fence would write back the whole L2)
+        unsigned long long o0 = 0, o1 = 0;
+        if (a >= 0.0 && ab > seen[0]) o0 = atomicMax(&I.red[0], ab);
+        if (c >= 0.0 && cb > seen[1]) o1 = atomicMax(&I.red[1], cb);
+        asm volatile("" ::"v"(o0), "v"(o1) : "memory");
     }
     __syncthreads();   // red is read
 }
 
-__global__ __launch_bounds__(kPts) void k_tstep(const BlkDev *__restrict__ blks, InstDev *__restrict__ inst, int ninst,
+// dt schedule (mo_canard_driver.f90:278-285).
+__device__ __forceinline__ void sched(InstDev &I, const TabDev &T)
+{
+    if (I.n % 10 == 1) {
+        // the maxima as the other workgroups' atomics left them
+        auto red = [&](int k) {
+            return __longlong_as_double(
+                (long long)__hip_atomic_load(&I.red[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        };
+        I.ndt = I.n;
+        I.dts = I.dte;
+        const double ra0 = I.cfl / red(0);
+        double ra1 = ra0;
+        if (I.viscous) ra1 = 0.5 / red(1);
+        I.dte = fmin(ra0, ra1);
+        I.red[0] = 0ull;   // for the next time they are due
+        I.red[1] = 0ull;
+    }
+    const int k = I.n - I.ndt;
+    double r;
+    if (k >= 0 && k < 64) r = T.ramp[k];
+    else { const double s = sin((0.05 * 3.141592653589793) * double(k)); r = s * s; }
+    I.dt = I.dts + (I.dte - I.dts) * r;
+    // output time (mo_canard_driver.f90:286-291)
+    I.nout = 0;
+    if (I.ndata > 0) {
+        const double res = (double(I.ndati + 1) * I.tmax) / double(I.ndata);
+        if ((I.timo - res) * ((I.timo + I.dt) - res) <= 0.0) {
+            I.nout = 1;
+            I.ndati = I.ndati + 1;
+        }
+    }
+}
+
+// The last workgroup to finish (by the counter done, which it clears) also
+// runs the dt schedule, the first one where no instance is due.
+__global__ __launch_bounds__(kPts) void k_tstep(const BlkDev *__restrict__ blks, InstDev *__restrict__ inst,
+                                               const TabDev *__restrict__ tabs, int ninst,
                                                const Tile *__restrict__ tiles, int ntiles,
-                                               const double *__restrict__ q, const double *__restrict__ met, int64_t NT)
+                                               const double *__restrict__ q, const double *__restrict__ met,
+                                               unsigned *done, int64_t NT)
 {
     __shared__ double red[2][kPts / 64];
+    __shared__ int last;
     int due = 0;
     for (int i = threadIdx.x; i < ninst; i += kPts) due |= inst[i].n % 10 == 1;
-    if (!__syncthreads_or(due)) return;
-    for (int i = blockIdx.x; i < ntiles; i += gridDim.x) tstep_tile(tiles[i], blks, inst, q, met, NT, red);
+    if (__syncthreads_or(due)) {
+        for (int i = blockIdx.x; i < ntiles; i += gridDim.x) tstep_tile(tiles[i], blks, inst, q, met, NT, red);
+        if (threadIdx.x == 0) {
+            last = atomicAdd(done, 1u) == gridDim.x - 1;
+            if (last) *done = 0u;
+        }
+        __syncthreads();
+        if (!last) return;
+    } else if (blockIdx.x != 0) {
+        return;
+    }
+    for (int i = threadIdx.x; i < ninst; i += kPts) sched(inst[i], tabs[i]);
 }
 
 // moving-frame velocity (src/mo_physics.f90:144-169)
@@ -189,38 +208,6 @@ __global__ void k_stage_begin(InstDev *inst, int ninst, int nk)
     InstDev &I = inst[i];
     const int a = nk - 2 > 0 ? (nk - 2 < 1 ? nk - 2 : 1) : 0, c = nk - 1 < 1 ? nk - 1 : 1;
     movef(I, (I.dt * double(a)) / double(4 - nk + 3), (I.dt * double(c)) / double(4 - nk + 2));
-}
-
-// dt schedule (mo_canard_driver.f90:278-285).
-__global__ void k_sched(InstDev *inst, const TabDev *tabs, int ninst)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ninst) return;
-    InstDev &I = inst[i];
-    if (I.n % 10 == 1) {
-        I.ndt = I.n;
-        I.dts = I.dte;
-        const double ra0 = I.cfl / __longlong_as_double((long long)I.red[0]);
-        double ra1 = ra0;
-        if (I.viscous) ra1 = 0.5 / __longlong_as_double((long long)I.red[1]);
-        I.dte = fmin(ra0, ra1);
-        I.red[0] = 0ull;   // for the next time they are due
-        I.red[1] = 0ull;
-    }
-    const int k = I.n - I.ndt;
-    double r;
-    if (k >= 0 && k < 64) r = tabs[i].ramp[k];
-    else { const double s = sin((0.05 * 3.141592653589793) * double(k)); r = s * s; }
-    I.dt = I.dts + (I.dte - I.dts) * r;
-    // output time (mo_canard_driver.f90:286-291)
-    I.nout = 0;
-    if (I.ndata > 0) {
-        const double res = (double(I.ndati + 1) * I.tmax) / double(I.ndata);
-        if ((I.timo - res) * ((I.timo + I.dt) - res) <= 0.0) {
-            I.nout = 1;
-            I.ndati = I.ndati + 1;
-        }
-    }
 }
 
 // frame velocity for the update half of the stage (mo_canard_driver.f90:325-327)
@@ -637,6 +624,107 @@ __global__ __launch_bounds__(kLine) void k_surf_avg(const BlkDev *__restrict__ b
     for (int m = 0; m < 5; ++m) q[m * NT + g] = v[m];
 }
 
+// End of a stage where every averaged face's partner is its own block (each
+// instance one periodic block): a point on such faces and its copies across
+// them form a group of 2, 4 or 8 that no other group touches, so the lane of
+// the group's member on the low faces applies every copy's running means
+// (those of k_surf_avg) in place, with no snapshot.  In the same launch the
+// primitives u, v, w, T of the new state for the next stage's gradient sweeps
+// (prim, or null) and the end of the step (end_step): from 17^3 to 65^3 points
+// each of these was a launch of its own of 2-6 us.  Workgroups below nfb take
+// four face tiles (side 0) each, the others one point tile.
+template <int NS>
+__device__ __forceinline__ void avg_group(double *q, double *prim, int64_t NT, int64_t g, const int64_t (&off)[3])
+{
+    constexpr int NC = 1 << NS;
+    double o[NC][5];
+    int64_t at[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        at[c] = g;
+#pragma unroll
+        for (int k = 0; k < NS; ++k) at[c] += (c >> k & 1) ? off[k] : 0;
+#pragma unroll
+        for (int m = 0; m < 5; ++m) o[c][m] = q[m * NT + at[c]];
+    }
+    SrcPrim src{q, NT};
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        SrcPrim::Raw raw;
+#pragma unroll
+        for (int m = 0; m < 5; ++m) {
+            double v = o[c][m], cnt = 1.0;
+#pragma unroll
+            for (int k = 0; k < NS; ++k) {
+                cnt = cnt + 1.0;
+                const double r2 = 1.0 / cnt;
+                v = r2 * ((cnt - 1.0) * v + o[c ^ (1 << k)][m]) + 0.0 * v;
+            }
+            raw.q[m] = v;
+            q[m * NT + at[c]] = v;
+        }
+        if (prim) {
+            double f[4];
+            src.finish(raw, 0, f);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) prim[m * NT + at[c]] = f[m];
+        }
+    }
+}
+
+__global__ __launch_bounds__(kPts) void k_self_avg(const BlkDev *__restrict__ blks, InstDev *__restrict__ inst,
+                                                  int ninst, const FaceSet fs, int nft, int nfb,
+                                                  const Tile *__restrict__ tiles, double *q, double *prim, int64_t NT,
+                                                  int end_step)
+{
+    if (end_step && blockIdx.x == 0)
+        for (int i = threadIdx.x; i < ninst; i += kPts) {
+            inst[i].n = inst[i].n + 1;
+            inst[i].timo = inst[i].timo + inst[i].dt;
+        }
+    if (int(blockIdx.x) >= nfb) {
+        const Tile t = tiles[blockIdx.x - nfb];
+        const BlkDev &B = blks[t.b];
+        const unsigned nx = B.n[0], ny = B.n[1], nz = B.n[2], lp = unsigned(t.q0) + threadIdx.x;
+        if (lp >= nx * ny * nz) return;
+        const unsigned r = lp / nx, idx[3] = {lp - r * nx, r % ny, r / ny};
+        for (int d = 0; d < 3; ++d)
+            if (is_avg(B.bc[d][0]) && (idx[d] == 0 || int(idx[d]) == B.n[d] - 1)) return;
+        const int64_t g = B.off + lp;
+        SrcPrim src{q, NT};
+        SrcPrim::Raw raw;
+        src.load(g, t.b, raw);
+        double f[4];
+        src.finish(raw, t.b, f);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) prim[m * NT + g] = f[m];
+        return;
+    }
+    const int ft = int(blockIdx.x) * (kPts / kLine) + int(threadIdx.x) / kLine;
+    if (ft >= nft) return;
+    int d;
+    const Tile t = fs.tile(ft, d);
+    const BlkDev &B = blks[t.b];
+    const int qq = t.q0 + int(threadIdx.x) % kLine;
+    if (qq >= npencils(B, d) || !is_avg(B.bc[d][0])) return;
+    const int w = d == 0 ? B.n[1] : B.n[0], qa = qq % w, qb = qq / w;
+    const int idx[3] = {d == 0 ? 0 : qa, d == 1 ? 0 : (d == 0 ? qa : qb), d == 2 ? 0 : qb};
+    const int64_t stride[3] = {1, B.n[0], int64_t(B.n[0]) * B.n[1]};
+    // the averaged directions the point lies on, in order; another lane has
+    // the group if one of them is at its high face or comes before d
+    int64_t off[3] = {0, 0, 0};
+    int ns = 0;
+    for (int dd = 0; dd < 3; ++dd) {
+        if (!is_avg(B.bc[dd][0])) continue;
+        if (idx[dd] == B.n[dd] - 1 || (dd < d && idx[dd] == 0)) return;
+        if (idx[dd] == 0) off[ns++] = (B.n[dd] - 1) * stride[dd];
+    }
+    const int64_t g = B.off + idx[0] + idx[1] * stride[1] + idx[2] * stride[2];
+    if (ns == 1) avg_group<1>(q, prim, NT, g, off);
+    else if (ns == 2) avg_group<2>(q, prim, NT, g, off);
+    else avg_group<3>(q, prim, NT, g, off);
+}
+
 // ---- grid metrics (mo_grid.f90:107-186) ----------------------------------------
 // dx[(3c+d)] = d(coord c)/d(xi_d)
 __global__ __launch_bounds__(kPts) void k_cross(const BlkDev *__restrict__ blks, const Tile *__restrict__ tiles,
@@ -851,53 +939,66 @@ FaceSet face_set(cnd_ctx *c, double *const (&arr)[3])
 }
 dim3 faces_grid(cnd_ctx *c) { return dim3(unsigned(ntiles(c, 0) + ntiles(c, 1) + ntiles(c, 2)), 2); }
 
-int enqueue_stage(cnd_ctx *c, int nk)
+// The xi gradients and, with the stored eta and zeta ones, the stresses and
+// fluxes of all directions: one kernel, or the tiled sweep and a pointwise one.
+int run_xi_grad_flux(cnd_ctx *c, const double *cur)
+{
+    if (seg_on(c, CND_KIND_GRAD, 0)) return run_grad_flux(c, cur);
+    if (int r = run_grad(c, 0, cur)) return r;
+    hipLaunchKernelGGL(k_visc_flux, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dinst, c->dpt, cur, c->grad, c->met,
+                       c->fl, c->NT);
+    return check_launch(c);
+}
+
+// Stage nk.  whole: as part of a whole step, where stages follow each other
+// with nothing in between, so the end of a stage may prepare the next one's
+// primitives and end the step (c->ended then).
+int enqueue_stage(cnd_ctx *c, int nk, bool whole)
 {
     const double *cur = nk == 1 ? c->qo : c->qa;
     const unsigned ib = unsigned((c->ninst + 63) / 64);
     if (c->any_frame) hipLaunchKernelGGL(k_stage_begin, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst, nk);
     int r;
-    // the time step of stage 1 runs beside the xi gradient sweep of viscous
-    // stages, which reads neither dt nor the maxima (its time then counts in
+    // the time step of stage 1 runs beside the gradient sweeps of viscous
+    // stages, which read neither dt nor the maxima (its time then counts in
     // the gradient section)
     const bool tstep_side = nk == 1 && c->any_visc && c->overlap;
     if (nk == 1) {
         auto tstep = [&] {
             const int npt = int(c->hpt.size());
             hipLaunchKernelGGL(k_tstep, dim3(std::min(unsigned(npt), kTstepBlocks)), dim3(kPts), 0, c->st, c->dblk,
-                               c->dinst, c->ninst, c->dpt, npt, cur, c->met, c->NT);
-            hipLaunchKernelGGL(k_sched, dim3(ib), dim3(64), 0, c->st, c->dinst, c->dtab, c->ninst);
+                               c->dinst, c->dtab, c->ninst, c->dpt, npt, cur, c->met, c->tstep_done, c->NT);
             return check_launch(c);
         };
         Section sec(c, CND_SEC_TSTEP, 1);
         if ((r = tstep_side ? on_side(c, tstep) : tstep())) return r;
     }
     if (c->any_visc) {
-        // eta and zeta in one launch, or the eta sweep beside the zeta sweep
-        // when it is a segmented one
+        // the primitives, then eta and zeta in one launch, or the eta sweep
+        // beside the zeta sweep when it is a segmented one
         const bool joint = eta_zeta_joint(c, CND_KIND_GRAD);
-        Section sec(c, CND_SEC_GRAD, joint ? 2 : 3);
-        if ((r = run_grad(c, 0, cur))) return r;
-        if (tstep_side && (r = join_side(c))) return r;
-        if (joint) {
-            if ((r = run_grad(c, 1, cur, true))) return r;
-        } else if (c->overlap && seg_on(c, CND_KIND_GRAD, 1)) {
-            if ((r = on_side(c, [&] { return run_grad(c, 1, cur); })) || (r = run_grad(c, 2, cur)) ||
-                (r = join_side(c)))
-                return r;
-        } else {
-            for (int d = 1; d < 3; ++d)
-                if ((r = run_grad(c, d, cur))) return r;
+        const bool xi_tiled = !seg_on(c, CND_KIND_GRAD, 0);
+        {
+            const bool have = whole && nk > 1 && c->avg_self;   // primitives from the previous stage's end
+            Section sec(c, CND_SEC_GRAD, (joint ? 1 : 2) + (have ? 0 : 1));
+            if (!have && (r = run_prims(c, cur))) return r;
+            if (joint) {
+                if ((r = run_grad(c, 1, cur, true))) return r;
+                if (tstep_side && (r = join_side(c))) return r;
+            } else {
+                if (tstep_side && (r = join_side(c))) return r;
+                if (c->overlap && seg_on(c, CND_KIND_GRAD, 1)) {
+                    if ((r = on_side(c, [&] { return run_grad(c, 1, cur); })) || (r = run_grad(c, 2, cur)) ||
+                        (r = join_side(c)))
+                        return r;
+                } else {
+                    for (int d = 1; d < 3; ++d)
+                        if ((r = run_grad(c, d, cur))) return r;
+                }
+            }
         }
-    }
-    if (c->any_visc) {
-        Section sec(c, CND_SEC_STRESS, 1);
-        if (c->precision == CND_MIXED)
-            hipLaunchKernelGGL(k_visc_flux<float>, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dinst, c->dpt, cur,
-                               c->gradf, c->met, c->fl, c->NT);
-        else
-            hipLaunchKernelGGL(k_visc_flux<double>, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dinst, c->dpt,
-                               cur, c->grad, c->met, c->fl, c->NT);
+        Section sec(c, CND_SEC_STRESS, xi_tiled ? 2 : 1);
+        if ((r = run_xi_grad_flux(c, cur))) return r;
     }
     const bool fused = fuse_possible(c) && seg_on(c, CND_KIND_FLUX, c->fuse_dir);
     {
@@ -959,9 +1060,17 @@ int enqueue_stage(cnd_ctx *c, int nk)
         hipLaunchKernelGGL(k_junc_gather, dim3(nb, 5), dim3(128), 0, c->st, c->jn, c->qa, c->NT);
         hipLaunchKernelGGL(k_junc_scatter, dim3(nb, 5), dim3(128), 0, c->st, c->jn, c->qa, c->NT);
     }
-    if (c->any_avg) {
+    if (c->avg_self) {
         const FaceSet fs = face_set(c, c->surf);
-        const dim3 grid = faces_grid(c);
+        const int nft = fs.n01 + ntiles(c, 2), nfb = (nft + kPts / kLine - 1) / (kPts / kLine);
+        const bool prims = whole && nk < 4 && prims_wanted(c);
+        c->ended = whole && nk == 4 && !c->any_frame;
+        hipLaunchKernelGGL(k_self_avg, dim3(unsigned(nfb + (prims ? int(c->hpt.size()) : 0))), dim3(kPts), 0, c->st,
+                           c->dblk, c->dinst, c->ninst, fs, nft, nfb, c->dpt, c->qa, prims ? c->fl : nullptr, c->NT,
+                           c->ended ? 1 : 0);
+    } else if (c->any_avg) {
+        const FaceSet fs = face_set(c, c->surf);
+        const dim3 grid(unsigned(fs.n01 + ntiles(c, 2)), 2);
         hipLaunchKernelGGL(k_surf_snap, grid, dim3(kLine), 0, c->st, c->dblk, fs, c->qa, c->NT);
         hipLaunchKernelGGL(k_surf_avg, grid, dim3(kLine), 0, c->st, c->dblk, fs, c->qa, c->NT);
     }
@@ -971,8 +1080,10 @@ int enqueue_stage(cnd_ctx *c, int nk)
 int enqueue_end(cnd_ctx *c)
 {
     const unsigned ib = unsigned((c->ninst + 63) / 64);
-    hipLaunchKernelGGL(k_end_step, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst,
-                       c->any_frame && !c->any_wall ? 1 : 0);
+    if (!c->ended)
+        hipLaunchKernelGGL(k_end_step, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst,
+                           c->any_frame && !c->any_wall ? 1 : 0);
+    c->ended = false;
     if (c->recording) {
         hipLaunchKernelGGL(k_record, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dinst, c->dpt, c->qo, c->qa,
                            c->qb, c->NT);
@@ -986,7 +1097,7 @@ int enqueue_step(cnd_ctx *c)
     int r;
     if ((r = enqueue_filter(c))) return r;
     for (int nk = 1; nk <= 4; ++nk)
-        if ((r = enqueue_stage(c, nk))) return r;
+        if ((r = enqueue_stage(c, nk, true))) return r;
     return enqueue_end(c);
 }
 
@@ -1051,6 +1162,7 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
     std::vector<double> lu, segtab[kNumL];
     c->hblk.resize(nblocks);
     int64_t off = 0, foff[3] = {0, 0, 0};
+    bool avg_other = false;   // some averaged face belongs to two blocks
     for (int b = 0; b < nblocks; ++b) {
         const BlockSpec &s = c->spec[b];
         BlkDev &B = c->hblk[b];
@@ -1067,7 +1179,10 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
                     c->any_gcbc = c->gcbc_dir[d] = true; B.gcbc_any = 1;
                 }
                 if (cd == kWallInviscid || cd == kWallViscous) c->any_wall = c->wall_dir[d] = true;
-                if (cd == kInterCurv || cd == kInterStraight || cd == kPeriodic) c->any_avg = true;
+                if (cd == kInterCurv || cd == kInterStraight || cd == kPeriodic) {
+                    c->any_avg = true;
+                    if (B.part[d][e] != b) avg_other = true;
+                }
             }
         }
         B.inst = s.inst;
@@ -1103,10 +1218,14 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
         for (int64_t p0 = 0; p0 < npt; p0 += kPts) c->hpt.push_back(Tile{b, int(p0)});
         if (npt > int64_t(2000000000)) { delete c; return fail(nullptr, CND_EINVAL, "block too large"); }
     }
+    c->avg_self = c->any_avg && !avg_other;
     c->NT = off;
     for (int d = 0; d < 3; ++d) c->FT[d] = foff[d];
     for (int b = 0; b < nblocks; ++b)
-        for (int d = 0; d < 3; ++d) c->nmax[d] = std::max(c->nmax[d], c->spec[b].n[d]);
+        for (int d = 0; d < 3; ++d) {
+            c->nmax[d] = std::max(c->nmax[d], c->spec[b].n[d]);
+            for (int li = 0; li < kNumL; ++li) c->segs[li][d] = std::max(c->segs[li][d], seg_count(c->spec[b].n[d], kLs[li]));
+        }
     // sweep shapes: the default segmented shape of each direction where every
     // block's pencils fit it (else another compiled shape, else the tiled
     // sweep); CANARD_SWEEP=tiled keeps the tiled sweeps everywhere and
@@ -1180,7 +1299,7 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
                 ok(dalloc(c, &c->dlu, lu.size())) && ok(dalloc(c, &c->qa, 5 * NT)) && ok(dalloc(c, &c->qo, 5 * NT)) &&
                 ok(dalloc(c, &c->de, 15 * NT)) && ok(dalloc(c, &c->grad, 12 * NT)) && ok(dalloc(c, &c->fl, 15 * NT)) &&
                 ok(dalloc(c, &c->met, 10 * NT)) && ok(dalloc(c, &c->ys, c->ys_len)) && ok(dalloc(c, &c->xyz, 3 * NT)) &&
-                ok(dalloc(c, &c->sp_par, 5 * ninst));
+                ok(dalloc(c, &c->sp_par, 5 * ninst)) && ok(dalloc(c, &c->tstep_done, 1));
     for (int li = 0; good && li < kNumL; ++li) good = ok(dalloc(c, &c->dseg[li], segtab[li].size()));
     if (good && c->any_sponge) good = ok(dalloc(c, &c->sponge, 2 * NT));
     if (good && precision == CND_MIXED) good = ok(dalloc(c, &c->gradf, 12 * NT));
@@ -1232,6 +1351,7 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
     if (!r) {
         hipError_t e = hipMemset(c->de, 0, sizeof(double) * 15 * NT);
         if (e == hipSuccess) e = hipMemset(c->fl, 0, sizeof(double) * 15 * NT);
+        if (e == hipSuccess) e = hipMemset(c->tstep_done, 0, sizeof(unsigned));
         if (e != hipSuccess) r = fail(c, CND_EDEVICE, "memset");
     }
     // junction averaging (search_point / search_line, average_point / average_line)
@@ -1272,7 +1392,7 @@ void cnd_destroy(cnd_ctx *c)
     for (hipEvent_t e : c->pool) hipEventDestroy(e);
     void *ptrs[] = {c->dblk, c->dtab, c->dinst, c->dlu, c->qa, c->qo, c->de, c->grad, c->fl, c->met, c->ys,
                     c->xyz, c->sponge, c->sp_par, c->dpt, c->gradf, c->jn.tgt, c->jn.src,
-                    c->jn.first, c->jn.tc, c->jn.sc, c->jn.write, c->jn.scale, c->jn.tmp, c->qb};
+                    c->jn.first, c->jn.tc, c->jn.sc, c->jn.write, c->jn.scale, c->jn.tmp, c->qb, c->tstep_done};
     for (void *p : ptrs) if (p) hipFree(p);
     for (int li = 0; li < kNumL; ++li)
         if (c->dseg[li]) hipFree(c->dseg[li]);
@@ -1426,6 +1546,7 @@ static int tune(cnd_ctx *c)
     const bool fz = fuse_possible(c);
     auto run = [&](int kind, int d, bool joint) {
         if (kind == CND_KIND_FILTER) return run_filter_field(c, d, c->qa, c->fl, 5);
+        if (kind == CND_KIND_GRAD && d == 0) return run_xi_grad_flux(c, c->qa);
         if (kind == CND_KIND_GRAD) return run_grad(c, d, c->qa, joint);
         if (d == c->fuse_dir && fz) return run_flux_update(c, 1, c->grad);
         return run_flux(c, d, c->qa, joint);
@@ -1589,7 +1710,7 @@ int cnd_rk_stage(cnd_ctx *c, int nk)
         return fail(c, CND_ESTATE, "cnd_rk_stage: stage " + std::to_string(nk) + " out of order (expected " +
                                        expected_call(c) + ")");
     if ((r = tune(c))) return r;
-    if ((r = enqueue_stage(c, nk))) return r;
+    if ((r = enqueue_stage(c, nk, false))) return r;
     c->state_in_qo = false;
     c->next_call = nk + 1;
     return CND_OK;

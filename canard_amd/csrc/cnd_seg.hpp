@@ -409,16 +409,6 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
         }
         __syncthreads();
         lu_fetch();
-        if constexpr (Src::kEmit) {
-            // the staged values of the tile, written out point after point
-            if (src.po) {
-                for (int e = t; e < elim; e += nthr) {
-                    const int li = place(e);
-#pragma unroll
-                    for (int m = 0; m < NV; ++m) src.po[m * src.NT + g0 + e] = buf[li + m * FS];
-                }
-            }
-        }
 #pragma unroll
         for (int kr = 0; kr < Sh::KR; ++kr) {
             const int row = a - kb - H + kr;

@@ -21,7 +21,6 @@ struct SrcField {   // NV plain fields, vs apart
     int64_t vs;
     struct Raw { double v[NV]; };
     static constexpr bool kDirect = true;   // variable v reads field v only
-    static constexpr bool kEmit = false;    // writes no copy of its values
     __device__ double field(int64_t g, int v) const { return a[v * vs + g]; }
     __device__ void load(int64_t g, int, Raw &r) const
     {
@@ -36,16 +35,14 @@ struct SrcField {   // NV plain fields, vs apart
 };
 
 // u, v, w, T of a state, exactly as the reference's primitives step
-// (src/mo_canard_driver.f90:267-274).  With po set, xi sweeps also write the
+// (src/mo_canard_driver.f90:267-274).
 // values they stage to po (four fields NT apart), for the eta and zeta
 // sweeps to differentiate as plain fields.
 struct SrcPrim {
     const double *q;
     int64_t NT;
-    double *po = nullptr;
     struct Raw { double q[5]; };
     static constexpr bool kDirect = false;
-    static constexpr bool kEmit = true;
     __device__ double field(int64_t, int) const { return 0.0; }
     __device__ void load(int64_t g, int, Raw &r) const
     {
@@ -89,6 +86,62 @@ __device__ __forceinline__ void dir_flux(double q1, double q2, double q3, double
     }
 }
 
+// Sutherland's law in the reference's scaling (src/mo_physics.f90:245-247);
+// T^1.5 as T sqrt(T): two roundings instead of a general power's ~200
+// instructions.
+__device__ __forceinline__ double viscosity(const InstDev &I, double T)
+{
+    return (I.srefp1dre * (T * sqrt(T))) / (T + I.srefoo);
+}
+
+// Viscous stresses and heat flux (src/mo_physics.f90:249-299) at point g and,
+// from them, the fluxes of all three directions (src/mo_physics.f90:319-382)
+// into F[5 d + m]: gx the xi gradients of u, v, w, T, grad the stored ones
+// (fields 4 .. 11: eta and zeta).
+template <class TG>
+__device__ __forceinline__ void visc_point(const InstDev &I, int64_t g, const double (&gx)[4], const double *q,
+                                           const TG *grad, const double *met, double *F, int64_t NT)
+{
+    const double q1 = q[g], q5 = q[4 * NT + g];
+    const double q2 = q[NT + g], q3 = q[2 * NT + g], q4 = q[3 * NT + g];
+    double ge[4], gz[4], mt[9];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) ge[k] = double(grad[(4 + k) * NT + g]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) gz[k] = double(grad[(8 + k) * NT + g]);
+#pragma unroll
+    for (int c = 0; c < 9; ++c) mt[c] = met[c * NT + g];
+    const double J = met[9 * NT + g];
+    const double ri = 1.0 / q1;
+    const double u = q2 * ri, v = q3 * ri, w = q4 * ri;
+    const double p = kGm1 * (q5 - 0.5 * ((q2 * u + q3 * v) + q4 * w));
+    const double T = (kGam * p) * ri;
+    const double mu = viscosity(I, T);
+    auto CT = [&](int c, int var) { return (mt[c] * gx[var] + mt[3 + c] * ge[var]) + mt[6 + c] * gz[var]; };
+    const double vtxx = CT(0, 0), vhzz = CT(1, 0), vtzx = CT(2, 0);
+    const double vtxy = CT(0, 1), vtyy = CT(1, 1), vhxx = CT(2, 1);
+    const double vhyy = CT(0, 2), vtyz = CT(1, 2), vtzz = CT(2, 2);
+    const double s1 = CT(0, 3), s2 = CT(1, 3), s3 = CT(2, 3);
+    const double r1 = mu * J;
+    const double r2 = kGm1PrI * r1;
+    const double d5 = kTwoThirds * ((vtxx + vtyy) + vtzz);
+    double ts[9];
+    const double txx = r1 * ((vtxx + vtxx) - d5), tyy = r1 * ((vtyy + vtyy) - d5), tzz = r1 * ((vtzz + vtzz) - d5);
+    const double txy = r1 * (vtxy + vhzz), tyz = r1 * (vtyz + vhxx), tzx = r1 * (vtzx + vhyy);
+    ts[0] = txx; ts[1] = tyy; ts[2] = tzz; ts[3] = txy; ts[4] = tyz; ts[5] = tzx;
+    ts[6] = ((r2 * s1 + u * txx) + v * txy) + w * tzx;
+    ts[7] = ((r2 * s2 + u * txy) + v * tyy) + w * tyz;
+    ts[8] = ((r2 * s3 + u * tzx) + v * tyz) + w * tzz;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const double m[3] = {mt[3 * d], mt[3 * d + 1], mt[3 * d + 2]};
+        double o[5];
+        dir_flux<true>(q1, q2, q3, q4, q5, u, v, w, p, m, I.umf, ts, o);
+#pragma unroll
+        for (int c = 0; c < 5; ++c) F[(5 * d + c) * NT + g] = o[c];
+    }
+}
+
 // Inviscid fluxes of direction d evaluated in the sweep from q and the
 // metric row of d (viscous runs differentiate the stored fluxes instead).
 struct SrcFlux {
@@ -100,7 +153,6 @@ struct SrcFlux {
     int d;
     struct Raw { double q[5], m[3]; };
     static constexpr bool kDirect = false;
-    static constexpr bool kEmit = false;
     __device__ double field(int64_t, int) const { return 0.0; }
     __device__ void load(int64_t g, int, Raw &r) const
     {
@@ -137,6 +189,20 @@ struct SinkOut {   // out fields vs apart, stored as TO
     __device__ double src(int64_t, int) const { return 0.0; }
     __device__ double fold(double, double x) const { return x; }
     __device__ void put_raw(int64_t g, int b, int k, double x) { put(g, b, k, x); }
+    __device__ void ends(int, int, int, double) {}
+};
+
+// The xi gradients of u, v, w, T straight into the point's stresses and fluxes.
+template <class TG>
+struct SinkVisc {
+    const InstDev *I;
+    const double *q;
+    const TG *grad;
+    const double *met;
+    double *F;
+    int64_t NT;
+    __device__ void store(int64_t g, int, const double (&x)[4]) { visc_point(*I, g, x, q, grad, met, F, NT); }
+    static constexpr bool kReadBack = false;
     __device__ void ends(int, int, int, double) {}
 };
 
@@ -422,22 +488,28 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
     seg_tile<1, 1, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles.list[tix], d, 0, tiles.SP, src, sink, lds);
 }
 
-// Velocity and temperature gradients along d, stored as TG (float in mixed
-// precision).  prim (xi sweeps, or null): the primitives u, v, w, T are also
-// written there.
+// Xi gradients of u, v, w, T and, from them and the stored eta and zeta ones
+// (TG: float in mixed precision), the stresses and the fluxes of all three
+// directions: a tile is one contiguous run of points, so the sink streams the
+// point's other operands like a pointwise kernel.  The xi gradients are never
+// stored: 344 B per point (40 of them the state again, mostly from the
+// last-level cache) against 72 + 336 for a sweep and a pointwise kernel.
+// 257^3, a stage: 0.386 + 1.087 -> 1.222 ms, and 0.221 for the primitives the
+// separate sweep stored; 65^3: 16.3 + 15.3 -> 26.1 us.
 template <class G, class TG>
-__global__ __launch_bounds__(wg_bound(4 * G::P * G::SPMAX), (seg_waves<G>())) void k_seg_grad(
-    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles, const double *q, TG *grad,
-    int64_t NT, double *prim)
+__global__ __launch_bounds__(wg_bound(4 * G::P * G::SPMAX), (seg_waves<G>())) void k_seg_grad_flux(
+    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles,
+    const InstDev *__restrict__ inst, const double *q, const TG *grad, const double *met, double *F, int64_t NT)
 {
     SEG_PROLOGUE
-    SrcPrim src{q, NT, prim};
-    SinkOut<4, TG> sink{grad + 4 * d * NT, NT};
-    seg_tile<4, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles.list[tix], d, 0, tiles.SP, src, sink, lds);
+    const Tile t = tiles.list[tix];
+    SrcPrim src{q, NT};
+    SinkVisc<TG> sink{inst + blks[t.b].inst, q, grad, met, F, NT};
+    seg_tile<4, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
 }
 
-// Gradients along d (eta, zeta) of the primitive v = blockIdx.y that the xi
-// gradient sweep stored (prim, four fields NT apart), into grad as TG.
+// Gradients along d (eta, zeta) of the primitive v = blockIdx.y (prim, four
+// fields NT apart), into grad as TG.
 template <class G, class TG>
 __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_grad_prim(
     const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles, const double *prim, TG *grad,
