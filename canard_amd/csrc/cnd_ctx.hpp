@@ -160,14 +160,15 @@ inline dim3 pts_grid(cnd_ctx *c) { return dim3(unsigned(c->hpt.size())); }
 
 
 inline int ntiles(cnd_ctx *c, int d) { return int(c->htiles[d].size()); }
-// LDS bytes of a segmented launch (cnd_seg.hpp SegShape::lds_bytes).
+// LDS bytes of a segmented launch (cnd_seg.hpp SegShape).
 inline size_t seg_lds_bytes(const ShapeInfo &G, int nv, int sp, int nmax, bool has_part)
 {
     const size_t chunk = size_t(G.C) * nv * sp * G.P, part = size_t(2) * kSegEndRows * nv * G.P,
                  ex = size_t(4) * nv * sp * G.P, lu = size_t(5) * G.L * sp;
     const size_t tile = size_t(nv) * G.P * size_t(nmax | 1);   // pencils n | 1 apart (SegShape::pencil_stride)
-    if (G.XI) return sizeof(double) * (std::max(tile, lu + ex) + size_t(8) * G.SPMAX + (has_part ? part : 0));
-    return sizeof(double) * (std::max(std::max(chunk, part), ex) + lu + part + size_t(8) * G.SPMAX);
+    const size_t coef = size_t(8) * sp;
+    if (G.XI) return sizeof(double) * (std::max(tile, lu + ex) + coef + (has_part ? part : 0));
+    return sizeof(double) * (std::max(std::max(chunk, part), ex) + lu + part + coef);
 }
 
 // One segmented launch: shape, tiles, workgroup size and LDS.
@@ -202,7 +203,7 @@ inline SegLaunch seg_launch(const cnd_ctx *c, int kind, int d, int nv, bool join
     const int sp = joint ? std::max(c->seg_sp[kind][1], c->seg_sp[kind][2]) : c->seg_sp[kind][d];
     const int nmax = joint ? std::max(c->nmax[1], c->nmax[2]) : c->nmax[d];
     const bool part = c->part_other[d] || (joint && c->part_other[2]);
-    return SegLaunch{sh, SegTiles{c->dstiles[pi][d], n + n2, sp, d, n}, unsigned(nv * kShapes[sh].P * sp),
+    return SegLaunch{sh, SegTiles{c->nblk == 1 ? nullptr : c->dstiles[pi][d], n + n2, sp, d, n}, unsigned(nv * kShapes[sh].P * sp),
                      seg_lds_bytes(kShapes[sh], nv, sp, nmax, part)};
 }
 

@@ -89,24 +89,15 @@ struct SegShape {
         const int m = chunk > part ? chunk : part;
         return m > ex ? m : ex;
     }
-    // then the segment transfer values [SPM][8] and the LU rows of the
+    // then the segment transfer values [SP][8] and the LU rows of the
     // launch's SP segments as their lanes hold them [SP][L][5]
     __host__ __device__ static constexpr int ends_doubles() { return 2 * kSegEndRows * NV * P; }
     // (xi: the whole tile's sources [NV][P][nmax | 1] replace the work area; once
     // the closure rows are formed, the LU rows and then the exchange buffer
     // [4][NV][SP][P] overlay the tile; the partner points [2][13][NV][P]
-    // come last and only when has_part, some block having another block as
-    // its partner along the sweep direction.)
-    __host__ __device__ static constexpr size_t lds_bytes(int SP, int spm, int nmax, bool has_part)
-    {
-        const size_t tile = size_t(NV) * P * pencil_stride(nmax), ex4 = size_t(4) * NV * SP * P,
-                     lu = size_t(5) * L * SP;
-        const size_t over = lu + ex4;
-        if (XI)
-            return sizeof(double) * ((tile > over ? tile : over) + size_t(8) * spm +
-                                     (has_part ? size_t(ends_doubles()) : size_t(0)));
-        return sizeof(double) * (size_t(work_doubles(SP)) + lu + size_t(ends_doubles()) + size_t(8) * spm);
-    }
+    // come last and only when some block has another block as its partner
+    // along the sweep direction.)
+    // Total bytes: seg_lds_bytes.
 };
 
 // Chunk slot -> (o, s, p): xi runs along the pencil, eta/zeta across pencils.
@@ -150,38 +141,42 @@ __host__ __device__ constexpr double seg_pass_row(int c) { return c == 0 || c ==
 // passes run over all L registers with no branches: the segment's last row
 // is always register L - 1, and the kb pass-through registers carry the
 // state across the front of the segment (swapped kb times, which the start
-// or end values undo).
-template <int L, int SPM>
+// or end values undo).  A pencil of one segment (S is the same for the whole
+// workgroup) needs no pass 1: with it, and with the block's codes read in the
+// first round of loads, a step of 16^3 points went from 50.4 to 45.5 us.
+template <int L>
 __device__ __forceinline__ void seg_solve(double (&Y)[L], const SegLane &ln, const double *LUs, const double *SM,
                                           double *ex)
 {
     const int s = ln.s;
     const bool odd = (ln.kb & 1) != 0;
     const double *lu = LUs + 5 * L * s;
-    // forward, pass 1: zero incoming values, outgoing values only
-    {
-        double ya = 0.0, yb = 0.0;
-#pragma unroll
-        for (int k = 0; k < L; ++k) {
-            const double y = (Y[k] - lu[5 * k] * ya) - lu[5 * k + 1] * yb;
-            ya = yb;
-            yb = y;
-        }
-        __syncthreads();
-        ex[ln.exi] = ya;
-        ex[ln.exs + ln.exi] = yb;
-        __syncthreads();
-    }
-    // incoming values y(a-2), y(a-1): scan over the segments before this one
     double t0 = 0.0, t1 = 0.0;
-    if (ln.ok) {
-        for (int sp = 0; sp < s; ++sp) {
-            const double *m = SM + 8 * sp;
-            const int xi = ln.exi + (sp - s) * ln.P;
-            const double n0 = (m[0] * t0 + m[1] * t1) + ex[xi];
-            const double n1 = (m[2] * t0 + m[3] * t1) + ex[ln.exs + xi];
-            t0 = n0;
-            t1 = n1;
+    if (ln.S > 1) {
+        // forward, pass 1: zero incoming values, outgoing values only
+        {
+            double ya = 0.0, yb = 0.0;
+#pragma unroll
+            for (int k = 0; k < L; ++k) {
+                const double y = (Y[k] - lu[5 * k] * ya) - lu[5 * k + 1] * yb;
+                ya = yb;
+                yb = y;
+            }
+            __syncthreads();
+            ex[ln.exi] = ya;
+            ex[ln.exs + ln.exi] = yb;
+            __syncthreads();
+        }
+        // incoming values y(a-2), y(a-1): scan over the segments before this one
+        if (ln.ok) {
+            for (int sp = 0; sp < s; ++sp) {
+                const double *m = SM + 8 * sp;
+                const int xi = ln.exi + (sp - s) * ln.P;
+                const double n0 = (m[0] * t0 + m[1] * t1) + ex[xi];
+                const double n1 = (m[2] * t0 + m[3] * t1) + ex[ln.exs + xi];
+                t0 = n0;
+                t1 = n1;
+            }
         }
     }
     // forward, pass 2: from the true incoming values
@@ -195,30 +190,32 @@ __device__ __forceinline__ void seg_solve(double (&Y)[L], const SegLane &ln, con
             yb = y;
         }
     }
-    // backward, pass 1: zero incoming values, outgoing values only
-    {
-        double xa = 0.0, xb = 0.0;
-#pragma unroll
-        for (int k = L - 1; k >= 0; --k) {
-            const double x = (lu[5 * k + 2] * Y[k] - lu[5 * k + 3] * xa) - lu[5 * k + 4] * xb;
-            xb = xa;
-            xa = x;
-        }
-        __syncthreads();
-        ex[ln.exi] = odd ? xb : xa;
-        ex[ln.exs + ln.exi] = odd ? xa : xb;
-        __syncthreads();
-    }
-    // incoming values x(b), x(b+1): scan over the segments after this one
     double h0 = 0.0, h1 = 0.0;
-    if (ln.ok) {
-        for (int sp = ln.S - 1; sp > s; --sp) {
-            const double *m = SM + 8 * sp + 4;
-            const int xi = ln.exi + (sp - s) * ln.P;
-            const double n0 = (m[0] * h0 + m[1] * h1) + ex[xi];
-            const double n1 = (m[2] * h0 + m[3] * h1) + ex[ln.exs + xi];
-            h0 = n0;
-            h1 = n1;
+    if (ln.S > 1) {
+        // backward, pass 1: zero incoming values, outgoing values only
+        {
+            double xa = 0.0, xb = 0.0;
+#pragma unroll
+            for (int k = L - 1; k >= 0; --k) {
+                const double x = (lu[5 * k + 2] * Y[k] - lu[5 * k + 3] * xa) - lu[5 * k + 4] * xb;
+                xb = xa;
+                xa = x;
+            }
+            __syncthreads();
+            ex[ln.exi] = odd ? xb : xa;
+            ex[ln.exs + ln.exi] = odd ? xa : xb;
+            __syncthreads();
+        }
+        // incoming values x(b), x(b+1): scan over the segments after this one
+        if (ln.ok) {
+            for (int sp = ln.S - 1; sp > s; --sp) {
+                const double *m = SM + 8 * sp + 4;
+                const int xi = ln.exi + (sp - s) * ln.P;
+                const double n0 = (m[0] * h0 + m[1] * h1) + ex[xi];
+                const double n1 = (m[2] * h0 + m[3] * h1) + ex[ln.exs + xi];
+                h0 = n0;
+                h1 = n1;
+            }
         }
     }
     // backward, pass 2
@@ -257,7 +254,7 @@ template <class S> struct sink_pre<S, std::void_t<typename S::Pre>> : std::true_
 //        put_raw: write such a value (eta/zeta sweeps of plain fields, which
 //        still hold the source in registers, use these instead of put);
 //        optionally Pre, pre and put_pre (sink_pre)
-template <int NV, int SCH, int L, int P, int C, bool XI, int SPM, class Src, class Sink>
+template <int NV, int SCH, int L, int P, int C, bool XI, class Src, class Sink>
 __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs,
                                          const SegTabs &tb, Tile tile, int d, int n45, int SP, const Src &src,
                                          Sink &sink, double *lds)
@@ -272,8 +269,12 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     const int b = tile.b;
     const BlkDev &B = blks[b];
     const TabDev &T = tabs[B.inst];
+    const double fa = SCH == 1 ? T.fa : 0.0, fb = SCH == 1 ? T.fb : 0.0, fc = SCH == 1 ? T.fc : 0.0;
     const int npen = npencils(B, d);
     const int n = B.n[d], N = n - 1;
+    // (read here, with the first round of loads, not at the uses behind the barriers)
+    const int qds[2] = {B.qd[d][0], B.qd[d][1]}, parts[2] = {B.part[d][0], B.part[d][1]};
+    const int codes[2] = {B.bc[d][0], B.bc[d][1]};
     const int S = seg_count(n, L);
     const double *LU = tb.lu + 5 * int64_t(B.lu[SCH][d]);
     const double *ST = tb.seg + 4 * int64_t(B.lu[SCH][d]);
@@ -285,20 +286,20 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     const int nlu = 5 * L * SP;
     double *buf = lds;
     double *ends = nullptr, *part = nullptr, *LUs = nullptr, *ex = nullptr;
-    double *SM = nullptr;   // [SPM][8]
+    double *SM = nullptr;   // [SP][8]
     if constexpr (XI) {
         const int fsz = NV * P * Sh::pencil_stride(n), exs4 = 4 * NV * SP * P;
         LUs = lds;
         ex = lds + nlu;
         SM = lds + (fsz > nlu + exs4 ? fsz : nlu + exs4);
-        part = SM + 8 * SPM;
+        part = SM + 8 * SP;
         ends = part;
     } else {
         ends = lds + Sh::work_doubles(SP);
         part = buf;
         ex = buf;
         SM = ends + Sh::ends_doubles();
-        LUs = SM + 8 * SPM;
+        LUs = SM + 8 * SP;
     }
     // xi: staged source of the lane's variable and pencil at row; the place
     // of tile point e (pencil e / n, row e % n) of variable 0; variable m
@@ -427,8 +428,8 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
                 rr = kAa * (w[3] - w[1]) + kAb * (w[4] - w[0]);
             } else {
                 const double resk = w[3] + w[3];
-                rr = (T.fa * ((w[2] + w[4]) - resk) + T.fb * ((w[1] + w[5]) - resk)) +
-                     T.fc * ((w[0] + w[6]) - resk);
+                rr = (fa * ((w[2] + w[4]) - resk) + fb * ((w[1] + w[5]) - resk)) +
+                     fc * ((w[0] + w[6]) - resk);
             }
             Y[k] = rr;
         }
@@ -468,8 +469,8 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
                 rr = kAa * (W[k + 3] - W[k + 1]) + kAb * (W[k + 4] - W[k]);
             } else {
                 const double resk = W[k + 3] + W[k + 3];
-                rr = (T.fa * ((W[k + 2] + W[k + 4]) - resk) + T.fb * ((W[k + 1] + W[k + 5]) - resk)) +
-                     T.fc * ((W[k] + W[k + 6]) - resk);
+                rr = (fa * ((W[k + 2] + W[k + 4]) - resk) + fb * ((W[k + 1] + W[k + 5]) - resk)) +
+                     fc * ((W[k] + W[k + 6]) - resk);
             }
             Y[k] = rr;
         }
@@ -566,8 +567,8 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
                 rr = kAa * (w[3] - w[1]) + kAb * (w[4] - w[0]);
             } else {
                 const double resk = w[3] + w[3];
-                rr = (T.fa * ((w[2] + w[4]) - resk) + T.fb * ((w[1] + w[5]) - resk)) +
-                     T.fc * ((w[0] + w[6]) - resk);
+                rr = (fa * ((w[2] + w[4]) - resk) + fb * ((w[1] + w[5]) - resk)) +
+                     fc * ((w[0] + w[6]) - resk);
             }
             Y[k] = rr;
         }
@@ -583,16 +584,16 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
 
     // ---- 2. partner points of interfaces with another block (one round) ------
     bool self[2];
-    for (int side = 0; side < 2; ++side) self[side] = B.qd[d][side] != 0 && B.part[d][side] == b;
-    const bool stage_part = (B.qd[d][0] != 0 && !self[0]) || (B.qd[d][1] != 0 && !self[1]);
+    for (int side = 0; side < 2; ++side) self[side] = qds[side] != 0 && parts[side] == b;
+    const bool stage_part = (qds[0] != 0 && !self[0]) || (qds[1] != 0 && !self[1]);
     __syncthreads();
     if (stage_part) {
         for (int slot = t; slot < 2 * kSegEndRows * P; slot += nthr) {
             const int pp = slot % P, o = (slot / P) % kSegEndRows, side = slot / (P * kSegEndRows);
-            if (tile.q0 + pp >= npen || B.qd[d][side] == 0 || self[side]) continue;
-            const int Pb = B.part[d][side];
+            if (tile.q0 + pp >= npen || qds[side] == 0 || self[side]) continue;
+            const int Pb = parts[side];
             const BlkDev &BP = blks[Pb];
-            const int ps = 1 - side, code = BP.bc[d][ps];
+            const int ps = 1 - side, code = codes[side];
             const int iik = code == 40 ? 0 : 1;
             const int NP = BP.n[d] - 1;
             const int idx = o == kSegEnd ? (ps == 0 ? 0 : NP) : (ps == 0 ? o + iik : NP - (o + iik));
@@ -615,11 +616,10 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
         if (!(lane_ok && s == (side == 0 ? 0 : S - 1))) continue;
         // distance i from this end
         auto f = [&](int i) { return XI ? F(side == 0 ? i : N - i) : ends[eidx(side, i, v, p)]; };
-        const bool qd = B.qd[d][side] != 0;
+        const bool qd = qds[side] != 0;
         double rows[3] = {0.0, 0.0, 0.0};
         if (qd) {
-            const int Pb = B.part[d][side];
-            const int ps = 1 - side, code = blks[Pb].bc[d][ps];
+            const int ps = 1 - side, code = codes[side];   // the partner's opposite face has the same
             const int iik = code == 40 ? 0 : 1;
             const double ra0k = code == 45 ? double(n45) : 0.0;
             // partner point o (o = 12: the partner's face point)
@@ -641,7 +641,7 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
             r0 = r0 - resk * T.qsum[SCH][0];
             r1 = r1 - resk * T.qsum[SCH][1];
             double r2 = sap0 - resk;
-            if (n45 == 1 && B.bc[d][side] == 45) {
+            if (n45 == 1 && codes[side] == 45) {
                 const double fo = f(0);
                 r0 = r0 + fo * T.qsum[SCH][0];
                 r1 = r1 + fo * T.qsum[SCH][1];
@@ -660,11 +660,11 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
                 rows[1] = a1 + r1;
                 const double ra2k = f(2) + f(2);
                 if (side == 0)
-                    rows[2] = (T.fa * ((f(1) + f(3)) - ra2k) + T.fb * ((f(0) + f(4)) - ra2k)) +
-                              T.fc * ((r2 + f(5)) - ra2k);
+                    rows[2] = (fa * ((f(1) + f(3)) - ra2k) + fb * ((f(0) + f(4)) - ra2k)) +
+                              fc * ((r2 + f(5)) - ra2k);
                 else
-                    rows[2] = (T.fa * ((f(3) + f(1)) - ra2k) + T.fb * ((f(4) + f(0)) - ra2k)) +
-                              T.fc * ((f(5) + r2) - ra2k);
+                    rows[2] = (fa * ((f(3) + f(1)) - ra2k) + fb * ((f(4) + f(0)) - ra2k)) +
+                              fc * ((f(5) + r2) - ra2k);
             }
         } else if (SCH == 0) {
             double sum = 0.0;
@@ -720,7 +720,7 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
 
     // ---- 4. solve ---------------------------------------------------------------
     const SegLane ln{a, len, kb, s, S, n, L, lane_ok, (v * SP + s) * P + p, NV * SP * P, v, p, P, SP};
-    seg_solve<L, SPM>(Y, ln, LUs, SM, ex);
+    seg_solve<L>(Y, ln, LUs, SM, ex);
     if (lane_ok && s == 0) {
         double x0 = 0.0;
 #pragma unroll

@@ -455,10 +455,16 @@ __host__ __device__ constexpr int l_index(int L) { return L == 17 ? 0 : 1; }
 
 // Tiles of one direction d (split = ntiles), or of eta and zeta in one launch
 // (d = 1; tiles from split on are zeta's).
+// list null: the tiles of a context of one block, whose place follows from
+// their number (a dependent load less at the start of every workgroup).
 struct SegTiles {
     const Tile *list;
     int n, SP, d, split;
     __device__ int dir(int tix) const { return d + (tix >= split ? 1 : 0); }
+    __device__ Tile at(int tix, int P) const
+    {
+        return list ? list[tix] : Tile{0, (tix - (tix >= split ? split : 0)) * P};
+    }
 };
 #define SEG_PROLOGUE                       \
     const int tix = xcd_tile(tiles.n);     \
@@ -474,7 +480,7 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
     const int v = blockIdx.y;
     SrcField<1> src{in + v * in_vstride, 0};
     SinkOut<1> sink{out + v * out_vstride, 0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles.list[tix], d, n45, tiles.SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::C, G::XI>(blks, tabs, tb, tiles.at(tix, G::P), d, n45, tiles.SP, src, sink, lds);
 }
 
 template <class G>
@@ -485,7 +491,7 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
     const int v = blockIdx.y;
     SrcField<1> src{in + v * vstride, 0};
     SinkFilt<1> sink{out + v * vstride, in + v * vstride, 0};
-    seg_tile<1, 1, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles.list[tix], d, 0, tiles.SP, src, sink, lds);
+    seg_tile<1, 1, G::L, G::P, G::C, G::XI>(blks, tabs, tb, tiles.at(tix, G::P), d, 0, tiles.SP, src, sink, lds);
 }
 
 // Xi gradients of u, v, w, T and, from them and the stored eta and zeta ones
@@ -502,10 +508,10 @@ __global__ __launch_bounds__(wg_bound(4 * G::P * G::SPMAX), (seg_waves<G>())) vo
     const InstDev *__restrict__ inst, const double *q, const TG *grad, const double *met, double *F, int64_t NT)
 {
     SEG_PROLOGUE
-    const Tile t = tiles.list[tix];
+    const Tile t = tiles.at(tix, G::P);
     SrcPrim src{q, NT};
     SinkVisc<TG> sink{inst + blks[t.b].inst, q, grad, met, F, NT};
-    seg_tile<4, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
+    seg_tile<4, 0, G::L, G::P, G::C, G::XI>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
 }
 
 // Gradients along d (eta, zeta) of the primitive v = blockIdx.y (prim, four
@@ -519,7 +525,7 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
     const int v = blockIdx.y;
     SrcField<1> src{prim + v * NT, 0};
     SinkOut<1, TG> sink{grad + (4 * d + v) * NT, 0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, tiles.list[tix], d, 0, tiles.SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::C, G::XI>(blks, tabs, tb, tiles.at(tix, G::P), d, 0, tiles.SP, src, sink, lds);
 }
 
 // Pencil-end derivatives of the three directions, and their face strides.
@@ -533,10 +539,10 @@ __global__ __launch_bounds__(wg_bound(5 * G::P * G::SPMAX), (seg_waves<G>())) vo
     const InstDev *__restrict__ inst, const double *q, const double *met, double *de, const Ends3 ends, int64_t NT)
 {
     SEG_PROLOGUE
-    const Tile t = tiles.list[tix];
+    const Tile t = tiles.at(tix, G::P);
     SrcFlux src{q, met, blks, inst, NT, d};
     SinkFlux sink{de + 5 * d * NT, ends.drva[d], NT, ends.FT[d], blks[t.b].foff[d] + t.q0};
-    seg_tile<5, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
+    seg_tile<5, 0, G::L, G::P, G::C, G::XI>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
 }
 
 // ... or component v = blockIdx.y of the stored ones.
@@ -547,10 +553,10 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
 {
     SEG_PROLOGUE
     const int v = blockIdx.y;
-    const Tile t = tiles.list[tix];
+    const Tile t = tiles.at(tix, G::P);
     SrcField<1> src{F + (5 * d + v) * NT, 0};
     SinkFluxV sink{de + (5 * d + v) * NT, ends.drva[d], v, ends.FT[d], blks[t.b].foff[d] + t.q0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::C, G::XI>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
 }
 
 // Last flux sweep of a stage fused with the RK update: sweep of the stored
@@ -568,14 +574,14 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
     if (w >= 5 * tiles.n) return;
     extern __shared__ double lds[];
     const int tix = w / 5, v = w % 5, d = tiles.d;
-    const Tile t = tiles.list[tix];
+    const Tile t = tiles.at(tix, G::P);
     SrcField<1> src{F + (5 * d + v) * NT, 0};
     const double dtk = inst[blks[t.b].inst].dt / double(4 - nk + 1);
     // the two other directions' right-hand sides
     const double *da = de + ((G::XI ? 5 : 0) + v) * NT, *db = de + ((G::XI ? 10 : 5) + v) * NT;
     SinkUpdateV<G::XI> sink{qa + v * NT, ends.drva[d], qo + v * NT, da, db, met, dtk, v, NT, ends.FT[d],
                             blks[t.b].foff[d] + t.q0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI, G::SPMAX>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::C, G::XI>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
 }
 
 }  // namespace cnd
