@@ -38,6 +38,11 @@ struct JuncDev {
     double *scale = nullptr, *tmp = nullptr;
 };
 
+// Tiles of a direction that one launch takes (blocks of like pencil length):
+// where they start in the direction's list, and their longest pencil.
+struct SegClass { int t0, n, S, nmax; };
+constexpr int kMaxClasses = 4, kClassTiles = 512;
+
 struct cnd_ctx {
     int ninst = 0, nblk = 0, precision = CND_FP64;
     std::vector<cnd_params> prm;
@@ -62,7 +67,8 @@ struct cnd_ctx {
     Tile *dtiles[3] = {nullptr, nullptr, nullptr};
     // segmented sweeps: tiles per direction, segments per pencil (rounded to
     // whole waves; 0: the direction uses the tiled sweeps), homogeneous tables
-    std::vector<Tile> hstiles[kNumP][3];            // tiles of P pencils
+    std::vector<Tile> hstiles[kNumP][3];            // tiles of P pencils, longest pencils first
+    std::vector<SegClass> classes[kNumL][kNumP][3];   // launches of segments of L points (seg_classes)
     Tile *dstiles[kNumP][3] = {};
     double *dseg[kNumL] = {};                       // homogeneous solutions per L
     // sweep shape per kind (CND_KIND_*) and direction: index into kShapes
@@ -189,27 +195,49 @@ inline bool eta_zeta_joint(const cnd_ctx *c, int kind)
     const int sh = c->shape[kind][1];
     if (sh == kTiled || sh != c->shape[kind][2]) return false;
     const int pi = p_index(kShapes[sh].P), li = l_index(kShapes[sh].L);
+    if (c->classes[li][pi][1].size() > 1 || c->classes[li][pi][2].size() > 1) return false;
     const int a = c->segs[li][1], b = c->segs[li][2], m = std::max(a, b);
     const int64_t na = int64_t(c->hstiles[pi][1].size()), nb = int64_t(c->hstiles[pi][2].size());
     return 4 * ((m - a) * na + (m - b) * nb) <= m * (na + nb);
 }
 
-// Launch of nv variables per workgroup for kind along d; joint: of eta (d = 1)
-// and zeta together.
-inline SegLaunch seg_launch(const cnd_ctx *c, int kind, int d, int nv, bool joint = false)
+// Segments per pencil of a workgroup whose pencils have at most S: rounded up
+// to whole waves per variable where that fits the shape.
+inline int round_sp(const ShapeInfo &G, int S)
+{
+    const int per_wave = 64 / G.P, up = (S + per_wave - 1) / per_wave * per_wave;
+    return up <= G.SPMAX ? up : S;
+}
+
+// Launches of nv variables per workgroup for kind along d, one per class of
+// pencil lengths; joint: of eta (d = 1) and zeta together.
+struct SegLaunches {
+    SegLaunch at[kMaxClasses];
+    int n = 0;
+    const SegLaunch *begin() const { return at; }
+    const SegLaunch *end() const { return at + n; }
+};
+inline SegLaunches seg_launches(const cnd_ctx *c, int kind, int d, int nv, bool joint = false)
 {
     const int sh = c->shape[kind][d], pi = p_index(kShapes[sh].P);
-    const int n = int(c->hstiles[pi][d].size()), n2 = joint ? int(c->hstiles[pi][2].size()) : 0;
-    const int sp = joint ? std::max(c->seg_sp[kind][1], c->seg_sp[kind][2]) : c->seg_sp[kind][d];
-    const int nmax = joint ? std::max(c->nmax[1], c->nmax[2]) : c->nmax[d];
-    const bool part = c->part_other[d] || (joint && c->part_other[2]);
-    return SegLaunch{sh, SegTiles{c->nblk == 1 ? nullptr : c->dstiles[pi][d], n + n2, sp, d, n}, unsigned(nv * kShapes[sh].P * sp),
-                     seg_lds_bytes(kShapes[sh], nv, sp, nmax, part)};
+    const ShapeInfo &G = kShapes[sh];
+    SegLaunches out;
+    for (const SegClass &C : c->classes[l_index(G.L)][pi][d]) {
+        // (a joint launch has one class per direction)
+        const int n2 = joint ? int(c->hstiles[pi][2].size()) : 0;
+        const int sp = joint ? std::max(c->seg_sp[kind][1], c->seg_sp[kind][2]) : round_sp(G, C.S);
+        const int nmax = joint ? std::max(c->nmax[1], c->nmax[2]) : C.nmax;
+        const bool part = c->part_other[d] || (joint && c->part_other[2]);
+        out.at[out.n++] = SegLaunch{sh, SegTiles{c->nblk == 1 ? nullptr : c->dstiles[pi][d] + C.t0, C.n + n2, sp, d, C.n},
+                                    unsigned(nv * G.P * sp), seg_lds_bytes(G, nv, sp, nmax, part)};
+    }
+    return out;
 }
 
 // Launch the segmented sweep K (a template-id of the shape G, in parentheses)
 // as SL (a SegLaunch) says, over xm x its tiles x y workgroups (kernels with xm > 1 split a
 // tile's work themselves); the arguments after the common ones follow.
+// LAUNCH_SEG*: every launch of SLS (SegLaunches).
 #define SEG_CASE(i, K, c, SL, y, ...)                                                                       \
     case i: {                                                                                              \
         using G = Sh##i;                                                                                   \
@@ -217,8 +245,8 @@ inline SegLaunch seg_launch(const cnd_ctx *c, int kind, int d, int nv, bool join
                            (SL).lds, (c)->st, (c)->dblk, (c)->dtab, seg_tabs(c, G::L), (SL).tiles, __VA_ARGS__); \
     } break;
 // xi shapes, eta / zeta shapes
-#define LAUNCH_SEG_XI(K, c, SL, xm, y, ...)                                                                 \
-    do {                                                                                                   \
+#define LAUNCH_SEG_XI(K, c, SLS, xm, y, ...)                                                                \
+    for (const SegLaunch &SL : SLS) {                                                                      \
         constexpr int seg_xm = xm;                                                                         \
         switch ((SL).shape) {                                                                               \
             SEG_CASE(0, K, c, SL, y, __VA_ARGS__) \
@@ -234,9 +262,9 @@ inline SegLaunch seg_launch(const cnd_ctx *c, int kind, int d, int nv, bool join
             SEG_CASE(19, K, c, SL, y, __VA_ARGS__) \
             default: break;                                                                                \
         }                                                                                                  \
-    } while (0)
-#define LAUNCH_SEG_EZ(K, c, SL, xm, y, ...)                                                                 \
-    do {                                                                                                   \
+    }
+#define LAUNCH_SEG_EZ(K, c, SLS, xm, y, ...)                                                                \
+    for (const SegLaunch &SL : SLS) {                                                                      \
         constexpr int seg_xm = xm;                                                                         \
         switch ((SL).shape) {                                                                               \
             SEG_CASE(2, K, c, SL, y, __VA_ARGS__) \
@@ -251,11 +279,12 @@ inline SegLaunch seg_launch(const cnd_ctx *c, int kind, int d, int nv, bool join
             SEG_CASE(20, K, c, SL, y, __VA_ARGS__) \
             default: break;                                                                                \
         }                                                                                                  \
-    } while (0)
-#define LAUNCH_SEG(K, c, SL, xm, y, ...)                                                                    \
+    }
+#define LAUNCH_SEG(K, c, SLS, xm, y, ...)                                                                   \
     do {                                                                                                   \
-        if ((SL).tiles.d == 0) LAUNCH_SEG_XI(K, c, SL, xm, y, __VA_ARGS__);                                  \
-        else LAUNCH_SEG_EZ(K, c, SL, xm, y, __VA_ARGS__);                                                   \
+        const SegLaunches sls = SLS;                                                                        \
+        if (sls.at[0].tiles.d == 0) { LAUNCH_SEG_XI(K, c, sls, xm, y, __VA_ARGS__) }                         \
+        else { LAUNCH_SEG_EZ(K, c, sls, xm, y, __VA_ARGS__) }                                                \
     } while (0)
 
 inline SegTabs seg_tabs(cnd_ctx *c, int L)

@@ -39,11 +39,11 @@ int run_prims(cnd_ctx *c, const double *cur)
 int run_grad(cnd_ctx *c, int d, const double *cur, bool joint)
 {
     const int K = CND_KIND_GRAD;
-    if (d > 0 && c->precision == CND_MIXED)   // FP32 gradients (segmented only)
-        LAUNCH_SEG_EZ((k_seg_grad_prim<G, float>), c, seg_launch(c, K, d, 1, joint), 1, 4, c->fl, c->gradf, c->NT);
-    else if (d > 0 && seg_on(c, K, d))
-        LAUNCH_SEG_EZ((k_seg_grad_prim<G, double>), c, seg_launch(c, K, d, 1, joint), 1, 4, c->fl, c->grad, c->NT);
-    else
+    if (d > 0 && c->precision == CND_MIXED) {   // FP32 gradients (segmented only)
+        LAUNCH_SEG_EZ((k_seg_grad_prim<G, float>), c, seg_launches(c, K, d, 1, joint), 1, 4, c->fl, c->gradf, c->NT)
+    } else if (d > 0 && seg_on(c, K, d)) {
+        LAUNCH_SEG_EZ((k_seg_grad_prim<G, double>), c, seg_launches(c, K, d, 1, joint), 1, 4, c->fl, c->grad, c->NT)
+    } else
         LAUNCH_SWEEP(k_fd_grad, 4, c, d, 1, 4 * kTile, c->dblk, c->dtab, c->dlu, c->dtiles[d], ntiles(c, d), d,
                      c->nmax[d], c->ys, cur, c->grad, c->NT);
     return check_launch(c);
@@ -51,11 +51,12 @@ int run_grad(cnd_ctx *c, int d, const double *cur, bool joint)
 
 int run_grad_flux(cnd_ctx *c, const double *cur)
 {
-    const SegLaunch SL = seg_launch(c, CND_KIND_GRAD, 0, 4);
-    if (c->precision == CND_MIXED)
-        LAUNCH_SEG_XI((k_seg_grad_flux<G, float>), c, SL, 1, 1, c->dinst, cur, c->gradf, c->met, c->fl, c->NT);
-    else
-        LAUNCH_SEG_XI((k_seg_grad_flux<G, double>), c, SL, 1, 1, c->dinst, cur, c->grad, c->met, c->fl, c->NT);
+    const SegLaunches sls = seg_launches(c, CND_KIND_GRAD, 0, 4);
+    if (c->precision == CND_MIXED) {
+        LAUNCH_SEG_XI((k_seg_grad_flux<G, float>), c, sls, 1, 1, c->dinst, cur, c->gradf, c->met, c->fl, c->NT)
+    } else {
+        LAUNCH_SEG_XI((k_seg_grad_flux<G, double>), c, sls, 1, 1, c->dinst, cur, c->grad, c->met, c->fl, c->NT)
+    }
     return check_launch(c);
 }
 

@@ -143,7 +143,7 @@ __host__ __device__ constexpr double seg_pass_row(int c) { return c == 0 || c ==
 // state across the front of the segment (swapped kb times, which the start
 // or end values undo).  A pencil of one segment (S is the same for the whole
 // workgroup) needs no pass 1: with it, and with the block's codes read in the
-// first round of loads, a step of 16^3 points went from 50.4 to 45.5 us.
+// first round of loads, a step of 16^3 points went from 252 to 228 us.
 template <int L>
 __device__ __forceinline__ void seg_solve(double (&Y)[L], const SegLane &ln, const double *LUs, const double *SM,
                                           double *ex)

@@ -1,0 +1,83 @@
+"""How the segmented sweeps of a stage are grouped into launches: blocks of
+like pencil length together, the others on their own, against the tiled
+sweeps, which take one launch per direction.  Sweeps agree to 1e-13 of the
+field maximum (both solve the same pentadiagonal lines, in another order of
+operations), whole steps to 1e-12 per conserved variable."""
+import numpy as np
+import pytest
+
+from canard_amd import cases
+from canard_amd.solver import CanardError, Case, shapes
+from helpers import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _blocks(sizes):
+    """Triply periodic blocks, each its own partner, with a perturbed Taylor-Green state."""
+    blocks, grids, states = [], [], []
+    for i, (lx, ly, lz) in enumerate(sizes):
+        blocks.append(dict(lxi=lx, let=ly, lze=lz, nbc=[[45, 45]] * 3, mcd=[[i, i]] * 3))
+        grids.append(cases.gridtoy(lx, ly, lz, doml0=0.0, doml1=2 * np.pi, domh=np.pi, span=2 * np.pi))
+        states.append(cases.tgv_state(grids[-1], (lx + 1, ly + 1, lz + 1), mach=0.1, pert=1e-3, seed=5 + i))
+    return blocks, grids, states, dict(fltk=0.49, fltrbc=0.9, reoo=1.6e4, cfl=0.8, viscous=1)
+
+
+# more than 512 workgroups of 4 to 16 pencils per class, in two and in four
+# classes, the longest pencils first, last and in between; one class whose
+# short block has too few pencils
+@pytest.mark.parametrize("sizes", [[(40, 92, 90), (150, 92, 90)],
+                                   [(99, 90, 66), (290, 40, 66), (150, 68, 64), (31, 92, 91)],
+                                   [(120, 60, 60), (30, 20, 18)]])
+def test_blocks_of_unlike_length_match_the_tiled_sweeps(sizes):
+    blocks, grids, states, params = _blocks(sizes)
+    rng = np.random.default_rng(11)
+    fields = [np.sin(g[0]) * np.cos(2 * g[1]) + 0.3 * rng.standard_normal(g.shape[1]) for g in grids]
+    c = Case(blocks, params)
+    c.set_grids(grids)
+    c.set_states(states)
+    for d in range(3):
+        for kind in ("field", "filter"):
+            c.set_shape(kind, d, -1)
+        want_d, want_f = c.deriv(d, fields), c.filter_sweep(d, fields)
+        for sh in [i for i, s in enumerate(shapes()) if s["xi"] == (d == 0)]:
+            try:
+                c.set_shape("field", d, sh)
+                c.set_shape("filter", d, sh)
+            except CanardError:   # does not fit these pencils
+                continue
+            print(f"[classes] {sizes} d={d} shape={sh}", flush=True)
+            for got, want in ((c.deriv(d, fields), want_d), (c.filter_sweep(d, fields), want_f)):
+                for b in range(len(blocks)):
+                    assert np.max(np.abs(got[b] - want[b])) <= 1e-13 * np.max(np.abs(want[b])), (d, sh, b)
+    c.close()
+
+
+@pytest.mark.parametrize("short", [False, True])
+def test_steps_of_blocks_of_unlike_length_match_the_tiled_sweeps(short):
+    """short: the shapes of few pencils per workgroup, which split into most classes."""
+    blocks, grids, states, params = _blocks([(99, 90, 66), (260, 40, 66), (31, 92, 91)])
+    out = []
+    for tiled in (True, False):
+        c = Case(blocks, params)
+        c.set_grids(grids)
+        c.set_states(states)
+        c.set_clock()
+        for d in range(3):
+            picks = [-1] if tiled else [i for i, s in enumerate(shapes()) if s["xi"] == (d == 0)]
+            picks.sort(key=lambda i: shapes()[i]["pencils"] * (1 if short else -1) if i >= 0 else 0)
+            for kind in ("filter", "grad", "flux"):
+                for sh in picks:
+                    try:
+                        c.set_shape(kind, d, sh)
+                        break
+                    except CanardError:
+                        continue
+        print(f"[classes] steps tiled={tiled} short={short}", flush=True)
+        c.step(3)
+        out.append([c.state(b) for b in range(len(blocks))])
+        c.close()
+    for b in range(len(blocks)):
+        err = rel_err(out[1][b], out[0][b])
+        print("  rel err per variable", err, flush=True)
+        assert np.all(err < 1e-12), (b, err)
