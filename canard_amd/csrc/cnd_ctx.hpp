@@ -108,6 +108,9 @@ struct cnd_ctx {
     unsigned *tstep_done = nullptr;   // workgroups of k_tstep that are through
     bool gcbc_dir[3] = {}, wall_dir[3] = {};   // directions with such faces
     bool any_frame = false;   // some instance's frame accelerates (nsmf = 0)
+    // staging of large reads (read_to_host), allocated by the first
+    char *stage = nullptr;
+    hipEvent_t stage_ev[3] = {};
     bool use_graph = false;
     hipGraphExec_t gexec = nullptr;
     // section timers
@@ -344,6 +347,12 @@ int run_flux(cnd_ctx *c, int d, const double *cur, bool joint = false);
 // RK update of stage nk, written to qa; the other two directions' buffers
 // must be complete.
 int run_flux_update(cnd_ctx *c, int nk, double *qa);
+
+// Synchronous copies of device arrays to the caller's host memory, in order
+// with st (cnd_read.hip); read_release frees the staging memory (cnd_destroy).
+struct HostCopy { void *dst; const void *src; size_t bytes; };
+int read_to_host(cnd_ctx *c, const HostCopy *copies, int n);
+void read_release(cnd_ctx *c);
 
 // Joins an output write in flight and frees the output buffers (cnd_destroy).
 void output_release(cnd_ctx *c);

@@ -1420,6 +1420,7 @@ void cnd_destroy(cnd_ctx *c)
     if (c->st) hipStreamSynchronize(c->st);
     if (c->st2) hipStreamSynchronize(c->st2);
     output_release(c);
+    read_release(c);
     if (c->gexec) hipGraphExecDestroy(c->gexec);
     for (auto &m : c->marks) { hipEventDestroy(m.a); hipEventDestroy(m.b); }
     for (hipEvent_t e : c->pool) hipEventDestroy(e);
@@ -1519,10 +1520,9 @@ int cnd_get_state(cnd_ctx *c, int b, double *q)
     if (!c || !q || b < 0 || b >= c->nblk) return fail(c, CND_EINVAL, "cnd_get_state: bad argument");
     const int64_t n = int64_t(c->spec[b].n[0]) * c->spec[b].n[1] * c->spec[b].n[2];
     const double *srcp = c->state_in_qo ? c->qo : c->qa;
-    for (int m = 0; m < 5; ++m)
-        HIPX(c, hipMemcpyAsync(q + m * n, srcp + m * c->NT + c->off[b], sizeof(double) * n, hipMemcpyDeviceToHost, c->st));
-    HIPX(c, hipStreamSynchronize(c->st));
-    return CND_OK;
+    HostCopy parts[5];
+    for (int m = 0; m < 5; ++m) parts[m] = HostCopy{q + m * n, srcp + m * c->NT + c->off[b], sizeof(double) * n};
+    return read_to_host(c, parts, 5);
 }
 
 int cnd_set_clock(cnd_ctx *c, int inst, int n, int ndt, double dt, double dts, double dte, double timo)
