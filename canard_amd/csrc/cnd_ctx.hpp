@@ -297,23 +297,22 @@ inline SegTabs seg_tabs(cnd_ctx *c, int L)
 inline bool seg_on(const cnd_ctx *c, int kind, int d) { return c->shape[kind][d] != kTiled; }
 
 
-// Variables per workgroup of a sweep kind along d (viscous flux sweeps run
-// one workgroup column per component of the stored fluxes; the eta and zeta
-// gradient sweeps, one per primitive the xi sweep stored).
-inline int kind_nv(const cnd_ctx *c, int kind, int d)
+// Variables per workgroup of a sweep kind along d (flux sweeps run one
+// workgroup column per component of the stored fluxes; the eta and zeta
+// gradient sweeps, one per stored primitive).
+inline int kind_nv(int kind, int d)
 {
-    if (kind == CND_KIND_GRAD) return d > 0 ? 1 : 4;
-    return kind == CND_KIND_FLUX && !c->any_visc ? 5 : 1;
+    return kind == CND_KIND_GRAD && d == 0 ? 4 : 1;
 }
 
 
-// Viscous stages without characteristic faces or sponge fold the update
+// Stages without characteristic faces or sponge fold the update
 // into the flux sweep of direction fuse_dir, run after the other two, when
 // that sweep is segmented (GCBC needs all three flux derivatives before the
 // update; the sponge stays in k_update).
 inline bool fuse_possible(const cnd_ctx *c)
 {
-    return c->fuse_update && c->any_visc && !c->any_gcbc && !c->any_sponge;
+    return c->fuse_update && !c->any_gcbc && !c->any_sponge;
 }
 
 
@@ -342,7 +341,7 @@ int run_grad(cnd_ctx *c, int d, const double *cur, bool joint = false);
 int run_grad_flux(cnd_ctx *c, const double *cur);
 // Flux sweep along d into the d-th right-hand-side buffer (kind
 // CND_KIND_FLUX); joint as for run_grad.
-int run_flux(cnd_ctx *c, int d, const double *cur, bool joint = false);
+int run_flux(cnd_ctx *c, int d, bool joint = false);
 // Flux sweep of the stored fluxes along fuse_dir (xi, or zeta) fused with the
 // RK update of stage nk, written to qa; the other two directions' buffers
 // must be complete.

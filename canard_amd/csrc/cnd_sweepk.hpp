@@ -34,6 +34,16 @@ struct SrcField {   // NV plain fields, vs apart
     }
 };
 
+// u, v, w, T of the state q.
+__device__ __forceinline__ void prims_of(const double (&q)[5], double (&o)[4])
+{
+    const double ri = 1.0 / q[0];
+    const double u = q[1] * ri, v = q[2] * ri, w = q[3] * ri;
+    const double p = kGm1 * (q[4] - 0.5 * ((q[1] * u + q[2] * v) + q[3] * w));
+    o[0] = u; o[1] = v; o[2] = w;
+    o[3] = (kGam * p) * ri;
+}
+
 // u, v, w, T of a state, exactly as the reference's primitives step
 // (src/mo_canard_driver.f90:267-274).
 // values they stage to po (four fields NT apart), for the eta and zeta
@@ -51,12 +61,7 @@ struct SrcPrim {
     }
     __device__ void finish(const Raw &r, int, double (&o)[4]) const
     {
-        const double ri = 1.0 / r.q[0];
-        const double q2 = r.q[1], q3 = r.q[2], q4 = r.q[3];
-        const double u = q2 * ri, v = q3 * ri, w = q4 * ri;
-        const double p = kGm1 * (r.q[4] - 0.5 * ((q2 * u + q3 * v) + q4 * w));
-        o[0] = u; o[1] = v; o[2] = w;
-        o[3] = (kGam * p) * ri;
+        prims_of(r.q, o);
     }
 };
 
@@ -142,34 +147,23 @@ __device__ __forceinline__ void visc_point(const InstDev &I, int64_t g, const do
     }
 }
 
-// Inviscid fluxes of direction d evaluated in the sweep from q and the
-// metric row of d (viscous runs differentiate the stored fluxes instead).
-struct SrcFlux {
-    const double *q;
-    const double *met;
-    const BlkDev *blks;
-    const InstDev *inst;
-    int64_t NT;
-    int d;
-    struct Raw { double q[5], m[3]; };
-    static constexpr bool kDirect = false;
-    __device__ double field(int64_t, int) const { return 0.0; }
-    __device__ void load(int64_t g, int, Raw &r) const
-    {
+// Inviscid fluxes (src/mo_physics.f90:319-382) of all three directions of the
+// state q1..q5 at point g into F[5 d + m].
+__device__ __forceinline__ void inv_point(const InstDev &I, int64_t g, const double (&q)[5], const double *met,
+                                          double *F, int64_t NT)
+{
+    const double ri = 1.0 / q[0];
+    const double u = q[1] * ri, v = q[2] * ri, w = q[3] * ri;
+    const double p = kGm1 * (q[4] - 0.5 * ((q[1] * u + q[2] * v) + q[3] * w));
 #pragma unroll
-        for (int k = 0; k < 5; ++k) r.q[k] = q[k * NT + g];
+    for (int d = 0; d < 3; ++d) {
+        const double m[3] = {met[(3 * d) * NT + g], met[(3 * d + 1) * NT + g], met[(3 * d + 2) * NT + g]};
+        double o[5];
+        dir_flux<false>(q[0], q[1], q[2], q[3], q[4], u, v, w, p, m, I.umf, nullptr, o);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) r.m[k] = met[(3 * d + k) * NT + g];
+        for (int c = 0; c < 5; ++c) F[(5 * d + c) * NT + g] = o[c];
     }
-    __device__ void finish(const Raw &r, int b, double (&o)[5]) const
-    {
-        const double q1 = r.q[0], q2 = r.q[1], q3 = r.q[2], q4 = r.q[3], q5 = r.q[4];
-        const double ri = 1.0 / q1;
-        const double u = q2 * ri, v = q3 * ri, w = q4 * ri;
-        const double p = kGm1 * (q5 - 0.5 * ((q2 * u + q3 * v) + q4 * w));
-        dir_flux<false>(q1, q2, q3, q4, q5, u, v, w, p, r.m, inst[blks[b].inst].umf, nullptr, o);
-    }
-};
+}
 
 // ---- sinks ----------------------------------------------------------------
 // store / put write results; fold(f, x) is the value to write for source f
@@ -222,22 +216,6 @@ struct SinkFilt {  // out = f + correction
     __device__ double fold(double fv, double x) const { return fv + x; }
     __device__ void put_raw(int64_t g, int, int k, double x) { o[k * vs + g] = x; }
     __device__ void ends(int, int, int, double) {}
-};
-
-struct SinkFlux {  // the five components of dF/dxi_d; pencil ends to drva
-    double *de, *drva;
-    int64_t NT, FT, fi0;
-    __device__ void store(int64_t g, int, const double (&x)[5])
-    {
-#pragma unroll
-        for (int m = 0; m < 5; ++m) de[m * NT + g] = x[m];
-    }
-    __device__ void put(int64_t g, int, int m, double x) { de[m * NT + g] = x; }
-    static constexpr bool kReadBack = false;
-    __device__ double src(int64_t, int) const { return 0.0; }
-    __device__ double fold(double, double x) const { return x; }
-    __device__ void put_raw(int64_t g, int b, int m, double x) { put(g, b, m, x); }
-    __device__ void ends(int side, int lane, int m, double x) { drva[(side * 5 + m) * FT + fi0 + lane] = x; }
 };
 
 struct SinkFluxV {  // component v of dF/dxi_d; pencil ends to drva
@@ -344,23 +322,8 @@ __global__ __launch_bounds__(4 * kTile) void k_fd_grad(const BlkDev *__restrict_
     sweep_tile<4, 0, C>(blks, tabs, lu, tiles[tix], tix, d, 0, nmax, ys, src, sink, lds);
 }
 
-// Flux derivatives along d (src/mo_physics.f90:385-399) into the d-th
-// right-hand-side buffer de: inviscid fluxes evaluated in the sweep ...
-template <int C>
-__global__ __launch_bounds__(5 * kTile) void k_fd_flux(const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs,
-                                                  const InstDev *__restrict__ inst, const double *__restrict__ lu,
-                                                  const Tile *__restrict__ tiles, int ntiles, int d, int nmax,
-                                                  double *ys, const double *q, const double *met, double *de,
-                                                  double *drva, int64_t NT, int64_t FT)
-{
-    SWEEP_TILE_PROLOGUE(ntiles)
-    const Tile t = tiles[tix];
-    SrcFlux src{q, met, blks, inst, NT, d};
-    SinkFlux sink{de, drva, NT, FT, blks[t.b].foff[d] + t.q0};
-    sweep_tile<5, 0, C>(blks, tabs, lu, t, tix, d, 0, nmax, ys, src, sink, lds);
-}
-
-// ... or stored fluxes F (component v = blockIdx.y), the viscous case.
+// Flux derivatives along d (src/mo_physics.f90:385-399) of the stored fluxes F
+// (component v = blockIdx.y) into the d-th right-hand-side buffer de.
 template <int C>
 __global__ __launch_bounds__(kTile) void k_fd_flux_field(const BlkDev *__restrict__ blks,
                                                         const TabDev *__restrict__ tabs,
@@ -531,21 +494,8 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
 // Pencil-end derivatives of the three directions, and their face strides.
 struct Ends3 { double *drva[3]; int64_t FT[3]; };
 
-// Flux derivatives along d into the d-th right-hand-side buffer of de:
-// inviscid fluxes evaluated in the sweep ...
-template <class G>
-__global__ __launch_bounds__(wg_bound(5 * G::P * G::SPMAX), (seg_waves<G>())) void k_seg_flux(
-    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles,
-    const InstDev *__restrict__ inst, const double *q, const double *met, double *de, const Ends3 ends, int64_t NT)
-{
-    SEG_PROLOGUE
-    const Tile t = tiles.at(tix, G::P);
-    SrcFlux src{q, met, blks, inst, NT, d};
-    SinkFlux sink{de + 5 * d * NT, ends.drva[d], NT, ends.FT[d], blks[t.b].foff[d] + t.q0};
-    seg_tile<5, 0, G::L, G::P, G::C, G::XI>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
-}
-
-// ... or component v = blockIdx.y of the stored ones.
+// Derivatives along d of the stored fluxes (component v = blockIdx.y) into the
+// d-th right-hand-side buffer of de.
 template <class G>
 __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_flux_field(
     const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles,

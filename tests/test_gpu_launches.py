@@ -2,13 +2,14 @@
 like pencil length together, the others on their own, against the tiled
 sweeps, which take one launch per direction.  Sweeps agree to 1e-13 of the
 field maximum (both solve the same pentadiagonal lines, in another order of
-operations), whole steps to 1e-12 per conserved variable."""
+operations), whole steps to 1e-12 per conserved variable.  Also the inviscid stage, whose
+fluxes are stored before the sweeps."""
 import numpy as np
 import pytest
 
 from canard_amd import cases
 from canard_amd.solver import CanardError, Case, shapes
-from helpers import rel_err
+from helpers import oracle_for, rel_err, tgv_case
 
 pytestmark = pytest.mark.gpu
 
@@ -81,3 +82,32 @@ def test_steps_of_blocks_of_unlike_length_match_the_tiled_sweeps(short):
         err = rel_err(out[1][b], out[0][b])
         print("  rel err per variable", err, flush=True)
         assert np.all(err < 1e-12), (b, err)
+
+
+# stored inviscid fluxes: pointwise kernel, flux sweeps, and the update fused
+# into the xi one, its own kernel, or after tiled sweeps
+@pytest.mark.parametrize("nxyz", [(12, 13, 16), (40, 36, 34), (67, 33, 20)])
+def test_inviscid_steps_match_oracle_fused_separate_and_tiled(monkeypatch, nxyz):
+    blocks, grids, states, params = tgv_case(0, nxyz=nxyz, pert=1e-3)
+    params["viscous"] = 0
+    o = oracle_for(blocks, grids, states, params)
+    o.run(5)
+    got = {}
+    for name, env in (("fused", {}), ("separate", {"CANARD_FUSE_UPDATE": "0"}), ("tiled", {"CANARD_SWEEP": "tiled"})):
+        with monkeypatch.context() as m:
+            m.setenv("CANARD_TUNE", "0")
+            for k, v in env.items():
+                m.setenv(k, v)
+            print(f"[inviscid] {nxyz} {name}", flush=True)
+            c = Case(blocks, params)
+        c.set_grids(grids)
+        c.set_states(states)
+        c.set_clock()
+        c.step(5)
+        got[name] = c.state(0)
+        c.close()
+        err = rel_err(got[name], o.state(0))
+        print("  rel err per variable", err, flush=True)
+        assert np.all(err < 1e-12), (name, err)
+    assert np.array_equal(got["fused"], got["separate"])
+    o.close()
