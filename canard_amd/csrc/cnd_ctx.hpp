@@ -172,12 +172,11 @@ inline int ntiles(cnd_ctx *c, int d) { return int(c->htiles[d].size()); }
 // LDS bytes of a segmented launch (cnd_seg.hpp SegShape).
 inline size_t seg_lds_bytes(const ShapeInfo &G, int nv, int sp, int nmax, bool has_part)
 {
-    const size_t chunk = size_t(G.C) * nv * sp * G.P, part = size_t(2) * kSegEndRows * nv * G.P,
-                 ex = size_t(4) * nv * sp * G.P, lu = size_t(5) * G.L * sp;
+    const size_t ends = size_t(2) * kSegEndRows * nv * G.P, part = has_part ? ends : 0;
+    const size_t ex = size_t(2) * nv * sp * G.P, lu = size_t(5) * G.L * sp, coef = size_t(8) * sp;
     const size_t tile = size_t(nv) * G.P * size_t(nmax | 1);   // pencils n | 1 apart (SegShape::pencil_stride)
-    const size_t coef = size_t(8) * sp;
-    if (G.XI) return sizeof(double) * (std::max(tile, lu + ex) + coef + (has_part ? part : 0));
-    return sizeof(double) * (std::max(std::max(chunk, part), ex) + lu + part + coef);
+    if (G.XI) return sizeof(double) * (std::max(tile, lu + ex) + coef + part);
+    return sizeof(double) * (std::max(ends, ex) + coef + lu + part);
 }
 
 // One segmented launch: shape, tiles, workgroup size and LDS.
@@ -263,6 +262,10 @@ inline SegLaunches seg_launches(const cnd_ctx *c, int kind, int d, int nv, bool 
             SEG_CASE(17, K, c, SL, y, __VA_ARGS__) \
             SEG_CASE(18, K, c, SL, y, __VA_ARGS__) \
             SEG_CASE(19, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(21, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(22, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(23, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(24, K, c, SL, y, __VA_ARGS__) \
             default: break;                                                                                \
         }                                                                                                  \
     }
@@ -280,6 +283,10 @@ inline SegLaunches seg_launches(const cnd_ctx *c, int kind, int d, int nv, bool 
             SEG_CASE(12, K, c, SL, y, __VA_ARGS__) \
             SEG_CASE(13, K, c, SL, y, __VA_ARGS__) \
             SEG_CASE(20, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(25, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(26, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(27, K, c, SL, y, __VA_ARGS__) \
+            SEG_CASE(28, K, c, SL, y, __VA_ARGS__) \
             default: break;                                                                                \
         }                                                                                                  \
     }

@@ -18,14 +18,11 @@
 // recurrence state exactly), so every lane runs the same branch-free code.
 //
 // Workgroup: NV * P * SP threads.  Thread t: variable v = t / (P * SP),
-// pencil p = t % P, segment s = (t / P) % SP.  Sources reach the lanes in
-// one of three ways: xi tiles (P contiguous pencils) are staged whole into
-// LDS with consecutive threads on consecutive points; eta/zeta sweeps of
-// plain fields load each lane's rows directly (the lanes of a wave hold P
-// neighbouring pencils, so every load reads runs of P consecutive points);
-// eta/zeta sweeps of derived sources (primitives, inviscid fluxes) evaluate
-// them cooperatively chunk by chunk (C rows of every segment) into LDS and
-// each lane picks its variable.  The lanes holding a pencil end keep the 13
+// pencil p = t % P, segment s = (t / P) % SP.  xi tiles (P contiguous
+// pencils) are staged whole into LDS with consecutive threads on consecutive
+// points; eta/zeta sweeps, of one plain field a workgroup, load each lane's
+// rows directly (the lanes of a wave hold P neighbouring pencils, so every
+// load reads runs of P consecutive points).  The lanes near a pencil end keep the 13
 // source values next to it in LDS (xi: they stay in the staged tile); the
 // closure rows are formed from them after the stream (and, for a block that
 // is its own periodic partner, the partner sums too, so no extra loads).
@@ -42,8 +39,9 @@ namespace cnd {
 constexpr int kSegEnd = 12;
 constexpr int kSegEndRows = kSegEnd + 1;
 
-// Fewest rows of a segment (seg_count) and of a whole pencil (13).
-constexpr int kSegMinRows = 12;
+// Fewest rows of a segment of at most L (seg_count); a whole pencil has 13 or
+// more.
+__host__ __device__ constexpr int seg_min_rows(int L) { return L < 17 ? 6 : 12; }
 
 // LU values a thread stages per round trip.
 constexpr int kLuBatch = 12;
@@ -57,7 +55,7 @@ constexpr int kOutBatch = 8;
 __host__ __device__ inline int seg_count(int n, int L)
 {
     const int S = (n + L - 1) / L;
-    if (S > 1 && n / S < kSegMinRows) return 0;
+    if (S > 1 && n / S < seg_min_rows(L)) return 0;
     return S;
 }
 
@@ -69,44 +67,28 @@ __host__ __device__ inline void seg_bounds(int n, int, int S, int s, int &a, int
 }
 
 
-template <int NV, int SCH, int L, int P, int C, bool XI>
+template <int NV, int SCH, int L, int P, bool XI>
 struct SegShape {
     static constexpr int H = SCH == 0 ? 2 : 3;          // stencil half width
     static constexpr int NB = SCH == 0 ? 2 : 3;         // closure rows per end
     static constexpr int KR = L + 2 * H;                // rows streamed per lane
-    static constexpr int NCH = (KR + C - 1) / C;        // staging chunks
     // xi tiles in LDS: pencil after pencil, each n | 1 points long (an odd
     // stride puts the lanes of neighbouring pencils in different banks),
     // variable after variable; for odd n a point's place is its index in
     // the tile
     __host__ __device__ static constexpr int pencil_stride(int n) { return n | 1; }
-    // LDS: a work area (chunk buffer [C][NV][SP][P], then partner points
-    // [2][13][NV][P], then the exchange buffer [4][NV][SP][P]) and the
-    // pencil-end values [2][13][NV][P].
-    __host__ __device__ static constexpr int work_doubles(int SP)
-    {
-        const int chunk = C * NV * SP * P, part = 2 * kSegEndRows * NV * P, ex = 4 * NV * SP * P;
-        const int m = chunk > part ? chunk : part;
-        return m > ex ? m : ex;
-    }
-    // then the segment transfer values [SP][8] and the LU rows of the
-    // launch's SP segments as their lanes hold them [SP][L][5]
-    __host__ __device__ static constexpr int ends_doubles() { return 2 * kSegEndRows * NV * P; }
-    // (xi: the whole tile's sources [NV][P][nmax | 1] replace the work area; once
-    // the closure rows are formed, the LU rows and then the exchange buffer
-    // [4][NV][SP][P] overlay the tile; the partner points [2][13][NV][P]
-    // come last and only when some block has another block as its partner
-    // along the sweep direction.)
-    // Total bytes: seg_lds_bytes.
+    // LDS.  eta/zeta: the pencil-end values [2][13][P], and over them, once the
+    // closure rows are formed, the exchange buffer [2][SP][P]; the segment
+    // transfer values [SP][8]; the LU rows of the launch's SP segments as
+    // their lanes hold them [SP][L][5].  xi: the whole tile's sources
+    // [NV][P][nmax | 1], and over them, once the closure rows are formed, the
+    // LU rows and the exchange buffer [2][NV][SP][P]; the transfer values.
+    // Last, both, and only when some block has another block as its partner
+    // along the sweep direction: the partner points [2][13][NV][P].
+    // Total bytes: seg_lds_bytes.  (With a staging chunk, partner points and
+    // both buffers side by side eta and zeta took twice as much: the filters
+    // of 257^3 points 354 and 377 us, with this 329 and 347.)
 };
-
-// Chunk slot -> (o, s, p): xi runs along the pencil, eta/zeta across pencils.
-template <int P, int C, bool XI>
-__device__ __forceinline__ void seg_slot(int slot, int SP, int &o, int &s, int &p)
-{
-    if (XI) { o = slot % C; p = (slot / C) % P; s = slot / (C * P); }
-    else { p = slot % P; s = (slot / P) % SP; o = slot / (P * SP); }
-}
 
 // xi sweeps (XI shapes run along xi only): the P pencils of a tile are
 // consecutive rows of the block, so point e of the tile (pencil e / n, row
@@ -251,15 +233,15 @@ template <class S> struct sink_pre<S, std::void_t<typename S::Pre>> : std::true_
 //  Src: load(g, b, Raw&), finish(Raw, b, double (&)[NV])
 //  Sink: store(g, b, const double (&)[NV]), put(g, b, v, x), ends(side, pencil, v, x);
 //        fold(f, x): the value to write given the source f and the result x,
-//        put_raw: write such a value (eta/zeta sweeps of plain fields, which
-//        still hold the source in registers, use these instead of put);
+//        put_raw: write such a value (eta/zeta sweeps, which still hold the
+//        source in registers, use these instead of put);
 //        optionally Pre, pre and put_pre (sink_pre)
-template <int NV, int SCH, int L, int P, int C, bool XI, class Src, class Sink>
+template <int NV, int SCH, int L, int P, bool XI, class Src, class Sink>
 __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs,
                                          const SegTabs &tb, Tile tile, int d, int n45, int SP, const Src &src,
                                          Sink &sink, double *lds)
 {
-    using Sh = SegShape<NV, SCH, L, P, C, XI>;
+    using Sh = SegShape<NV, SCH, L, P, XI>;
     constexpr int H = Sh::H;
     const int nthr = NV * P * SP;
     const int t = threadIdx.x;
@@ -278,28 +260,25 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     const int S = seg_count(n, L);
     const double *LU = tb.lu + 5 * int64_t(B.lu[SCH][d]);
     const double *ST = tb.seg + 4 * int64_t(B.lu[SCH][d]);
-    // LDS.  eta/zeta: work area (chunk buffer, then partner points, then the
-    // exchange buffer), the pencil-end values, SM, LU rows.  xi: the whole
-    // tile's sources [NV][P][n | 1] (once the closure rows are formed: the LU rows
-    // and the exchange buffer; at the end: the results), SM, and the
-    // partner points where some block has another block as partner along d.
     const int nlu = 5 * L * SP;
-    double *buf = lds;
+    double *buf = lds;   // xi: the tile
     double *ends = nullptr, *part = nullptr, *LUs = nullptr, *ex = nullptr;
     double *SM = nullptr;   // [SP][8]
+    const int exs2 = 2 * NV * SP * P;
     if constexpr (XI) {
-        const int fsz = NV * P * Sh::pencil_stride(n), exs4 = 4 * NV * SP * P;
+        const int fsz = NV * P * Sh::pencil_stride(n);
         LUs = lds;
         ex = lds + nlu;
-        SM = lds + (fsz > nlu + exs4 ? fsz : nlu + exs4);
+        SM = lds + (fsz > nlu + exs2 ? fsz : nlu + exs2);
         part = SM + 8 * SP;
-        ends = part;
     } else {
-        ends = lds + Sh::work_doubles(SP);
-        part = buf;
-        ex = buf;
-        SM = ends + Sh::ends_doubles();
+        static_assert(NV == 1, "an eta or zeta workgroup sweeps one field");
+        constexpr int esz = 2 * kSegEndRows * P;
+        ends = lds;
+        ex = lds;
+        SM = lds + (esz > exs2 ? esz : exs2);
         LUs = SM + 8 * SP;
+        part = LUs + nlu;
     }
     // xi: staged source of the lane's variable and pencil at row; the place
     // of tile point e (pencil e / n, row e % n) of variable 0; variable m
@@ -379,7 +358,6 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     double w[2 * H + 1];
 #pragma unroll
     for (int m = 0; m <= 2 * H; ++m) w[m] = 0.0;
-    const int nslots = C * SP * P;
     if constexpr (XI) {
         // stage all points of the tile at once, consecutive threads on
         // consecutive points: a thread has P n / (NV P SP) <= L / NV points
@@ -433,8 +411,8 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
             }
             Y[k] = rr;
         }
-    } else if constexpr (Src::kDirect) {
-        // eta/zeta, plain fields: each lane loads its own rows, all at once.
+    } else {
+        // eta/zeta: each lane loads its own rows, all at once.
         // The lanes of a wave hold P neighbouring pencils, so one load
         // instruction reads runs of P consecutive points.  Rows outside the
         // lane's window are clamped into it (loaded but never used).
@@ -450,14 +428,15 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
             row = row < rlo ? rlo : (row > rhi ? rhi : row);
             W[kr] = src.field(pb + int64_t(row) * st, v);
         }
-        // the 13 points next to each pencil end, for the closure rows
-        if (lane_ok && (s == 0 || s == S - 1)) {
+        // the 13 points next to each pencil end, for the closure rows, from the
+        // lanes whose rows they are
+        if (lane_ok && (a <= kSegEnd || N - (a + len - 1) <= kSegEnd)) {
 #pragma unroll
-            for (int kr = 0; kr < Sh::KR; ++kr) {
-                const int row = r0 + kr;
-                if (row < rlo || row > rhi) continue;
-                if (s == 0 && row <= kSegEnd) ends[eidx(0, row, v, p)] = W[kr];
-                if (s == S - 1 && N - row <= kSegEnd) ends[eidx(1, N - row, v, p)] = W[kr];
+            for (int k = 0; k < L; ++k) {
+                const int row = a - kb + k;
+                if (k < kb) continue;
+                if (row <= kSegEnd) ends[eidx(0, row, v, p)] = W[k + H];
+                if (N - row <= kSegEnd) ends[eidx(1, N - row, v, p)] = W[k + H];
             }
         }
         // row a - kb + k: stencil W[k .. k + 2H] (interior rows; the closure
@@ -474,112 +453,12 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
             }
             Y[k] = rr;
         }
-    } else {
-    constexpr int CPT = (C + NV - 1) / NV;   // staging slots per thread and chunk (= C / NV rounded up)
-    // slots whose loads are issued together: as many as keep the loaded
-    // values within about 24 doubles of registers
-    constexpr int RAWD = int(sizeof(typename Src::Raw) / sizeof(double));
-    constexpr int BAT = (24 / RAWD) < 1 ? 1 : ((24 / RAWD) < CPT ? 24 / RAWD : CPT);
-    // Slot k of a thread stages, chunk after chunk, rows r0 + c C of one
-    // segment's window [lo, hi] of pencil pb (stride st): these are the same
-    // for every chunk and computed once.  The loads of slot k of chunk c
-    // (addresses clamped into the block, so they are valid for every slot)
-    // and the LDS place of its sources (-1: nothing to stage).
-    constexpr int CPTB = (CPT + BAT - 1) / BAT * BAT;   // slots the batches below visit
-    int64_t spb[CPTB];
-    int sr0[CPTB], slo[CPTB], shi[CPTB], sdst[CPTB];
-    int64_t sst = 0;
-#pragma unroll
-    for (int k = 0; k < CPTB; ++k) {
-        const int slot = k < CPT ? t + k * nthr : nslots;
-        int o, ss, pp;
-        seg_slot<P, C, XI>(slot < nslots ? slot : 0, SP, o, ss, pp);
-        const int ssc = ss < S ? ss : S - 1;
-        int sa, sl;
-        seg_bounds(n, L, S, ssc, sa, sl);
-        const bool valid = slot < nslots && ss < S && tile.q0 + pp < npen;
-        sr0[k] = sa - (L - sl) - H + o;
-        slo[k] = sa - H > 0 ? sa - H : 0;
-        shi[k] = sa + sl + H - 1 < N ? sa + sl + H - 1 : N;
-        sdst[k] = valid ? ((o * NV) * SP + ss) * P + pp : -1;
-        pencil_of(B, d, tile.q0 + (tile.q0 + pp < npen ? pp : npen - 1 - tile.q0), spb[k], sst);
-    }
-    auto issue = [&](int c, int k, typename Src::Raw &raw, int &dst) {
-        const int row = sr0[k] + c * C;
-        const int rowc = row < 0 ? 0 : (row > N ? N : row);
-        src.load(spb[k] + int64_t(rowc) * sst, b, raw);
-        dst = (sdst[k] >= 0 && row >= slo[k] && row <= shi[k]) ? sdst[k] : -1;
-    };
-    auto deposit = [&](const typename Src::Raw &raw, int dst) {
-        if (dst < 0) return;
-        double f[NV];
-        src.finish(raw, b, f);
-#pragma unroll
-        for (int m = 0; m < NV; ++m) buf[dst + m * SP * P] = f[m];
-    };
-    // one batch per chunk: the next chunk's loads are issued before this
-    // chunk's rows are consumed, so they are in flight meanwhile
-    typename Src::Raw rawp[BAT];
-    int dstp[BAT];
-    if constexpr (BAT == CPT) {
-#pragma unroll
-        for (int kk = 0; kk < CPT; ++kk) issue(0, kk, rawp[kk], dstp[kk]);
-    }
-#pragma unroll
-    for (int c = 0; c < Sh::NCH; ++c) {
-        __syncthreads();
-        if constexpr (BAT == CPT) {
-#pragma unroll
-            for (int kk = 0; kk < CPT; ++kk) deposit(rawp[kk], dstp[kk]);
-            if (c + 1 < Sh::NCH) {
-#pragma unroll
-                for (int kk = 0; kk < CPT; ++kk) issue(c + 1, kk, rawp[kk], dstp[kk]);
-            }
-        } else {
-#pragma unroll
-            for (int k0 = 0; k0 < CPT; k0 += BAT) {
-                typename Src::Raw raw[BAT];
-                int dst[BAT];
-#pragma unroll
-                for (int kk = 0; kk < BAT; ++kk) issue(c, k0 + kk, raw[kk], dst[kk]);
-#pragma unroll
-                for (int kk = 0; kk < BAT; ++kk) deposit(raw[kk], dst[kk]);
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int o = 0; o < C; ++o) {
-            const int kr = c * C + o;            // streamed point a - kb - H + kr
-            if (kr >= Sh::KR) break;
-            const double fv = buf[((o * NV + v) * SP + s) * P + p];
-            const int row = a - kb - H + kr;
-            if (lane_ok && row >= 0 && row <= N && row >= a - H && row < a + len + H) {
-                if (s == 0 && row <= kSegEnd) ends[eidx(0, row, v, p)] = fv;
-                if (s == S - 1 && N - row <= kSegEnd) ends[eidx(1, N - row, v, p)] = fv;
-            }
-#pragma unroll
-            for (int m = 0; m < 2 * H; ++m) w[m] = w[m + 1];
-            w[2 * H] = fv;
-            const int k = kr - 2 * H;            // row a - kb + k has its stencil complete
-            if (k < 0 || k >= L) continue;
-            double rr;
-            if constexpr (SCH == 0) {
-                rr = kAa * (w[3] - w[1]) + kAb * (w[4] - w[0]);
-            } else {
-                const double resk = w[3] + w[3];
-                rr = (fa * ((w[2] + w[4]) - resk) + fb * ((w[1] + w[5]) - resk)) +
-                     fc * ((w[0] + w[6]) - resk);
-            }
-            Y[k] = rr;
-        }
-    }
-
     }
 
     // the pass-through registers start at zero (a segment has at least
-    // kSegMinRows rows, so only the first L - kSegMinRows can be such)
+    // seg_min_rows(L) rows, so only the first L - seg_min_rows(L) can be such)
 #pragma unroll
-    for (int k = 0; k < L - kSegMinRows; ++k)
+    for (int k = 0; k < L - seg_min_rows(L); ++k)
         if (k < kb) Y[k] = 0.0;
 
     // ---- 2. partner points of interfaces with another block (one round) ------
@@ -704,7 +583,7 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
 #pragma unroll
         for (int r = 0; r < Sh::NB; ++r)
 #pragma unroll
-            for (int k = 0; k <= L - kSegMinRows + r; ++k)
+            for (int k = 0; k <= L - seg_min_rows(L) + r; ++k)
                 if (k == kb + r) Y[k] = lo[r];
     }
     if (lane_ok && s == S - 1) {   // row N is Y[L - 1]
@@ -724,7 +603,7 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     if (lane_ok && s == 0) {
         double x0 = 0.0;
 #pragma unroll
-        for (int k = 0; k <= L - kSegMinRows; ++k)
+        for (int k = 0; k <= L - seg_min_rows(L); ++k)
             if (k == kb) x0 = Y[k];
         sink.ends(0, p, v, x0);
     }
@@ -752,12 +631,7 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
             } else {
 #pragma unroll
                 for (int k = 0; k < L; ++k)
-                    if (have(k)) {
-                        if constexpr (Src::kDirect)
-                            sink.put_raw(pb + int64_t(k) * st, b, v, sink.fold(W[k + H], Y[k]));
-                        else
-                            sink.put(pb + int64_t(k) * st, b, v, Y[k]);
-                    }
+                    if (have(k)) sink.put_raw(pb + int64_t(k) * st, b, v, sink.fold(W[k + H], Y[k]));
             }
         }
     } else {

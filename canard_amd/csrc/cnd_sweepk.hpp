@@ -20,7 +20,6 @@ struct SrcField {   // NV plain fields, vs apart
     const double *a;
     int64_t vs;
     struct Raw { double v[NV]; };
-    static constexpr bool kDirect = true;   // variable v reads field v only
     __device__ double field(int64_t g, int v) const { return a[v * vs + g]; }
     __device__ void load(int64_t g, int, Raw &r) const
     {
@@ -52,8 +51,6 @@ struct SrcPrim {
     const double *q;
     int64_t NT;
     struct Raw { double q[5]; };
-    static constexpr bool kDirect = false;
-    __device__ double field(int64_t, int) const { return 0.0; }
     __device__ void load(int64_t g, int, Raw &r) const
     {
 #pragma unroll
@@ -341,14 +338,19 @@ __global__ __launch_bounds__(kTile) void k_fd_flux_field(const BlkDev *__restric
 
 // ---- segmented sweeps (cnd_seg.hpp) ---------------------------------------
 // Compiled shapes: L points per segment (lanes per pencil = segments =
-// ceil(n / L)), P pencils per workgroup, C-point staging runs, at most SPMAX
-// segments per pencil; XI shapes stage runs along the pencil (xi sweeps),
-// the others across P neighbouring pencils (eta, zeta sweeps).  The
-// autotuner picks one per sweep kind and direction.
+// ceil(n / L)), P pencils per workgroup, at most SPMAX segments per pencil; XI
+// shapes stage runs along the pencil (xi sweeps), the others take P
+// neighbouring pencils (eta, zeta sweeps).  C is the run length reported with
+// a shape; no sweep stages in runs of it any more, so shapes that differ in C
+// only are the same.  The autotuner picks one per sweep kind and direction.
+// Short segments suit small blocks, where a sweep is one wave's chain of
+// instructions (17 -> 9 points: eta and zeta filters 9.7 -> 7.3 us at 17^3,
+// 10.2 -> 8.2 us at 33^3, 14.2 -> 12.0 us at 101 x 61 x 41); long ones run
+// fewer scans and closure rows per point (257^3: 33 points).
 template <int L_, int P_, int C_, int SPMAX_, bool XI_>
 struct SegG { static constexpr int L = L_, P = P_, C = C_, SPMAX = SPMAX_; static constexpr bool XI = XI_; };
 struct ShapeInfo { int L, P, C, SPMAX; bool XI; };
-constexpr int kNumShapes = 21;
+constexpr int kNumShapes = 29;
 constexpr ShapeInfo kShapes[kNumShapes] = {
     {17, 4, 16, 16, true},    // 0: xi default (pencils up to 272 points)
     {33, 4, 16, 8, true},     // 1
@@ -374,7 +376,15 @@ constexpr ShapeInfo kShapes[kNumShapes] = {
     {17, 16, 16, 32, true},   // 17
     {17, 8, 16, 32, true},    // 18
     {17, 4, 16, 32, true},    // 19
-    {17, 16, 8, 32, false}};  // 20
+    {17, 16, 8, 32, false},   // 20
+    {9, 4, 16, 16, true},     // 21
+    {9, 8, 16, 16, true},     // 22
+    {9, 16, 16, 16, true},    // 23
+    {9, 32, 16, 16, true},    // 24
+    {9, 8, 8, 16, false},     // 25
+    {9, 16, 8, 16, false},    // 26
+    {9, 32, 8, 16, false},    // 27
+    {9, 64, 8, 16, false}};   // 28
 using Sh0 = SegG<17, 4, 16, 16, true>;
 using Sh1 = SegG<33, 4, 16, 8, true>;
 using Sh2 = SegG<33, 16, 8, 8, false>;
@@ -396,25 +406,35 @@ using Sh17 = SegG<17, 16, 16, 32, true>;
 using Sh18 = SegG<17, 8, 16, 32, true>;
 using Sh19 = SegG<17, 4, 16, 32, true>;
 using Sh20 = SegG<17, 16, 8, 32, false>;
+using Sh21 = SegG<9, 4, 16, 16, true>;
+using Sh22 = SegG<9, 8, 16, 16, true>;
+using Sh23 = SegG<9, 16, 16, 16, true>;
+using Sh24 = SegG<9, 32, 16, 16, true>;
+using Sh25 = SegG<9, 8, 8, 16, false>;
+using Sh26 = SegG<9, 16, 8, 16, false>;
+using Sh27 = SegG<9, 32, 8, 16, false>;
+using Sh28 = SegG<9, 64, 8, 16, false>;
 // workgroup size bound of a kernel (shapes whose NV * P * SPMAX exceeds the
 // 1024-thread limit are rejected at launch time by shape_sp)
 __host__ __device__ constexpr int wg_bound(int x) { return x > 1024 ? 1024 : x; }
-// waves per SIMD a segmented sweep is compiled for: shapes of 17-point
-// segments are held to 128 VGPRs (4 waves, so two 512-thread workgroups
-// share a CU), which their LDS also allows and which costs no spills; the
-// others are left to the compiler
-template <class G>
-__host__ __device__ constexpr int seg_waves() { return G::L <= 17 ? 4 : 1; }
+// waves per SIMD a segmented sweep is compiled for: eta / zeta sweeps of
+// 17-point segments are held to 96 VGPRs (5 waves) where that costs no spills,
+// not in the fused update, whose operand batches need more; other shapes of
+// up to 17 points to 128 (4 waves; those of 9 points need 84 to 102 anyway,
+// and forcing 80 spills), the others are left to the compiler.  4 -> 5 waves,
+// 129^3: joint gradient sweeps 59 -> 53 us, flux sweeps 87 -> 86 us.
+template <class G, bool OPERANDS = false>
+__host__ __device__ constexpr int seg_waves() { return G::L > 17 ? 1 : (G::L == 17 && !G::XI && !OPERANDS ? 5 : 4); }
 constexpr int kSegMaxPoints = 528;   // longest pencil of a segmented sweep
 constexpr int kTiled = -1;   // shape index of the tiled sweep
 // pencils-per-workgroup values (tile lists) and segment lengths (tables)
 constexpr int kNumP = 7, kPs[kNumP] = {4, 8, 16, 32, 64, 20, 24};
-constexpr int kNumL = 2, kLs[kNumL] = {17, 33};
+constexpr int kNumL = 3, kLs[kNumL] = {17, 33, 9};
 __host__ __device__ constexpr int p_index(int P)
 {
     return P == 4 ? 0 : (P == 8 ? 1 : (P == 16 ? 2 : (P == 32 ? 3 : (P == 64 ? 4 : (P == 20 ? 5 : 6)))));
 }
-__host__ __device__ constexpr int l_index(int L) { return L == 17 ? 0 : 1; }
+__host__ __device__ constexpr int l_index(int L) { return L == 17 ? 0 : (L == 33 ? 1 : 2); }
 
 // Tiles of one direction d (split = ntiles), or of eta and zeta in one launch
 // (d = 1; tiles from split on are zeta's).
@@ -443,7 +463,7 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
     const int v = blockIdx.y;
     SrcField<1> src{in + v * in_vstride, 0};
     SinkOut<1> sink{out + v * out_vstride, 0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI>(blks, tabs, tb, tiles.at(tix, G::P), d, n45, tiles.SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::XI>(blks, tabs, tb, tiles.at(tix, G::P), d, n45, tiles.SP, src, sink, lds);
 }
 
 template <class G>
@@ -454,7 +474,7 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
     const int v = blockIdx.y;
     SrcField<1> src{in + v * vstride, 0};
     SinkFilt<1> sink{out + v * vstride, in + v * vstride, 0};
-    seg_tile<1, 1, G::L, G::P, G::C, G::XI>(blks, tabs, tb, tiles.at(tix, G::P), d, 0, tiles.SP, src, sink, lds);
+    seg_tile<1, 1, G::L, G::P, G::XI>(blks, tabs, tb, tiles.at(tix, G::P), d, 0, tiles.SP, src, sink, lds);
 }
 
 // Xi gradients of u, v, w, T and, from them and the stored eta and zeta ones
@@ -474,7 +494,7 @@ __global__ __launch_bounds__(wg_bound(4 * G::P * G::SPMAX), (seg_waves<G>())) vo
     const Tile t = tiles.at(tix, G::P);
     SrcPrim src{q, NT};
     SinkVisc<TG> sink{inst + blks[t.b].inst, q, grad, met, F, NT};
-    seg_tile<4, 0, G::L, G::P, G::C, G::XI>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
+    seg_tile<4, 0, G::L, G::P, G::XI>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
 }
 
 // Gradients along d (eta, zeta) of the primitive v = blockIdx.y (prim, four
@@ -488,7 +508,7 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
     const int v = blockIdx.y;
     SrcField<1> src{prim + v * NT, 0};
     SinkOut<1, TG> sink{grad + (4 * d + v) * NT, 0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI>(blks, tabs, tb, tiles.at(tix, G::P), d, 0, tiles.SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::XI>(blks, tabs, tb, tiles.at(tix, G::P), d, 0, tiles.SP, src, sink, lds);
 }
 
 // Pencil-end derivatives of the three directions, and their face strides.
@@ -506,14 +526,14 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
     const Tile t = tiles.at(tix, G::P);
     SrcField<1> src{F + (5 * d + v) * NT, 0};
     SinkFluxV sink{de + (5 * d + v) * NT, ends.drva[d], v, ends.FT[d], blks[t.b].foff[d] + t.q0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::XI>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
 }
 
 // Last flux sweep of a stage fused with the RK update: sweep of the stored
 // flux component v along d (xi or zeta), written as the updated state qa.
 // Grid x: five workgroups (components) per tile.
 template <class G>
-__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_flux_update(
+__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G, true>())) void k_seg_flux_update(
     const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles,
     const InstDev *__restrict__ inst, const double *F, const double *de, const double *__restrict__ qo,
     const double *__restrict__ met, double *qa, const Ends3 ends, int64_t NT, int nk)
@@ -531,7 +551,7 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
     const double *da = de + ((G::XI ? 5 : 0) + v) * NT, *db = de + ((G::XI ? 10 : 5) + v) * NT;
     SinkUpdateV<G::XI> sink{qa + v * NT, ends.drva[d], qo + v * NT, da, db, met, dtk, v, NT, ends.FT[d],
                             blks[t.b].foff[d] + t.q0};
-    seg_tile<1, 0, G::L, G::P, G::C, G::XI>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
+    seg_tile<1, 0, G::L, G::P, G::XI>(blks, tabs, tb, t, d, 0, tiles.SP, src, sink, lds);
 }
 
 }  // namespace cnd

@@ -111,3 +111,40 @@ def test_inviscid_steps_match_oracle_fused_separate_and_tiled(monkeypatch, nxyz)
         assert np.all(err < 1e-12), (name, err)
     assert np.array_equal(got["fused"], got["separate"])
     o.close()
+
+
+# pencils of the fewest points (13), of one point more or less than whole
+# segments of 9, 17 and 33 points, and between blocks whose partner along d is
+# another block (its points staged beside the sweep's own LDS) or themselves
+@pytest.mark.parametrize("other", [False, True])
+@pytest.mark.parametrize("na,nb", [(13, 18), (19, 27), (28, 17), (34, 67), (101, 55)])
+def test_every_shape_at_segment_edges_matches_the_tiled_sweeps(na, nb, other):
+    rng = np.random.default_rng(na)
+    for d in range(3):
+        blocks, fields = [], []
+        for i, n in enumerate((na, nb)):
+            size = [21, 19, 23]
+            size[d] = n
+            mcd = [[i, i] for _ in range(3)]
+            if other:
+                mcd[d] = [1 - i, 1 - i]
+            blocks.append(dict(lxi=size[0] - 1, let=size[1] - 1, lze=size[2] - 1, nbc=[[45, 45]] * 3, mcd=mcd))
+            fields.append(rng.standard_normal(size[0] * size[1] * size[2]))
+        c = Case(blocks, dict(fltk=0.49, fltrbc=0.9))
+        for kind in ("field", "filter"):
+            c.set_shape(kind, d, -1)
+        want_d, want_f = c.deriv(d, fields), c.filter_sweep(d, fields)
+        tried = 0
+        for sh in [i for i, s in enumerate(shapes()) if s["xi"] == (d == 0)]:
+            try:
+                c.set_shape("field", d, sh)
+                c.set_shape("filter", d, sh)
+            except CanardError:   # segments too short or too many
+                continue
+            tried += 1
+            print(f"[edges] {na} {nb} other={other} d={d} shape={sh}", flush=True)
+            for got, want in ((c.deriv(d, fields), want_d), (c.filter_sweep(d, fields), want_f)):
+                for b in range(2):
+                    assert np.max(np.abs(got[b] - want[b])) <= 1e-13 * np.max(np.abs(want[b])), (d, sh, b)
+        assert tried > 0
+        c.close()
