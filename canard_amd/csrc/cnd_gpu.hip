@@ -645,54 +645,51 @@ __global__ __launch_bounds__(kLine) void k_surf_avg(const BlkDev *__restrict__ b
 
 // End of a stage where every averaged face's partner is its own block (each
 // instance one periodic block): a point on such faces and its copies across
-// them form a group of 2, 4 or 8 that no other group touches, so the lane of
-// the group's member on the low faces applies every copy's running means
-// (those of k_surf_avg) in place, with no snapshot.  In the same launch the
+// them form a group of 2, 4 or 8 that no other group touches, found at its
+// member on the low faces, so every copy's running means (those of
+// k_surf_avg) are applied in place, with no snapshot.  In the same launch the
 // primitives u, v, w, T of the new state for the next stage's gradient sweeps
 // (prim, or null) and the end of the step (end_step): from 17^3 to 65^3 points
 // each of these was a launch of its own of 2-6 us.  Workgroups below nfb take
-// four face tiles (side 0) each, the others one point tile.
+// half a face tile (side 0) each, the others one point tile.
+//
+// A chain of latencies: eight lanes share a group, five averaging a variable
+// each, then one per copy forming its primitives.  With a lane for a whole
+// group (186 VGPRs, three variants of straight code one after the other) 17^3
+// points took 10.2 us instead of 4.2, 65^3 12.9 instead of 7.1.
+constexpr int kAvgLanes = 8, kAvgGroups = kPts / kAvgLanes;   // lanes of a group, groups of a workgroup
+
+// Means of one variable q over the copies of the group at g (NS directions,
+// copies off apart), also left in LDS (6 apart).
 template <int NS>
-__device__ __forceinline__ void avg_group(double *q, double *prim, int64_t NT, int64_t g, const int64_t (&off)[3])
+__device__ __forceinline__ void avg_group(double *q, double *mean, int64_t g, const int64_t (&off)[3])
 {
     constexpr int NC = 1 << NS;
-    double o[NC][5];
+    double o[NC];
     int64_t at[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         at[c] = g;
 #pragma unroll
         for (int k = 0; k < NS; ++k) at[c] += (c >> k & 1) ? off[k] : 0;
-#pragma unroll
-        for (int m = 0; m < 5; ++m) o[c][m] = q[m * NT + at[c]];
+        o[c] = q[at[c]];
     }
-    SrcPrim src{q, NT};
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-        SrcPrim::Raw raw;
+        double v = o[c], cnt = 1.0;
 #pragma unroll
-        for (int m = 0; m < 5; ++m) {
-            double v = o[c][m], cnt = 1.0;
-#pragma unroll
-            for (int k = 0; k < NS; ++k) {
-                cnt = cnt + 1.0;
-                const double r2 = 1.0 / cnt;
-                v = r2 * ((cnt - 1.0) * v + o[c ^ (1 << k)][m]) + 0.0 * v;
-            }
-            raw.q[m] = v;
-            q[m * NT + at[c]] = v;
+        for (int k = 0; k < NS; ++k) {
+            cnt = cnt + 1.0;
+            const double r2 = 1.0 / cnt;
+            v = r2 * ((cnt - 1.0) * v + o[c ^ (1 << k)]) + 0.0 * v;
         }
-        if (prim) {
-            double f[4];
-            src.finish(raw, 0, f);
-#pragma unroll
-            for (int m = 0; m < 4; ++m) prim[m * NT + at[c]] = f[m];
-        }
+        q[at[c]] = v;
+        mean[6 * c] = v;
     }
 }
 
 __global__ __launch_bounds__(kPts) void k_self_avg(const BlkDev *__restrict__ blks, InstDev *__restrict__ inst,
-                                                  int ninst, const FaceSet fs, int nft, int nfb,
+                                                  int ninst, const FaceSet fs, int nfb,
                                                   const Tile *__restrict__ tiles, double *q, double *prim, int64_t NT,
                                                   int end_step)
 {
@@ -710,38 +707,54 @@ __global__ __launch_bounds__(kPts) void k_self_avg(const BlkDev *__restrict__ bl
         for (int d = 0; d < 3; ++d)
             if (is_avg(B.bc[d][0]) && (idx[d] == 0 || int(idx[d]) == B.n[d] - 1)) return;
         const int64_t g = B.off + lp;
-        SrcPrim src{q, NT};
-        SrcPrim::Raw raw;
-        src.load(g, t.b, raw);
-        double f[4];
-        src.finish(raw, t.b, f);
+        double x[5], f[4];
+#pragma unroll
+        for (int m = 0; m < 5; ++m) x[m] = q[m * NT + g];
+        prims_of(x, f);
 #pragma unroll
         for (int m = 0; m < 4; ++m) prim[m * NT + g] = f[m];
         return;
     }
-    const int ft = int(blockIdx.x) * (kPts / kLine) + int(threadIdx.x) / kLine;
-    if (ft >= nft) return;
+    static_assert(kLine == 2 * kAvgGroups);
+    __shared__ double means[kAvgGroups * 8 * 6];
     int d;
-    const Tile t = fs.tile(ft, d);
+    const Tile t = fs.tile(int(blockIdx.x) / 2, d);
     const BlkDev &B = blks[t.b];
-    const int qq = t.q0 + int(threadIdx.x) % kLine;
-    if (qq >= npencils(B, d) || !is_avg(B.bc[d][0])) return;
-    const int w = d == 0 ? B.n[1] : B.n[0], qa = qq % w, qb = qq / w;
-    const int idx[3] = {d == 0 ? 0 : qa, d == 1 ? 0 : (d == 0 ? qa : qb), d == 2 ? 0 : qb};
-    const int64_t stride[3] = {1, B.n[0], int64_t(B.n[0]) * B.n[1]};
-    // the averaged directions the point lies on, in order; another lane has
-    // the group if one of them is at its high face or comes before d
-    int64_t off[3] = {0, 0, 0};
-    int ns = 0;
-    for (int dd = 0; dd < 3; ++dd) {
-        if (!is_avg(B.bc[dd][0])) continue;
-        if (idx[dd] == B.n[dd] - 1 || (dd < d && idx[dd] == 0)) return;
-        if (idx[dd] == 0) off[ns++] = (B.n[dd] - 1) * stride[dd];
+    const int gr = int(threadIdx.x) / kAvgLanes, l = int(threadIdx.x) % kAvgLanes;
+    const int qq = t.q0 + (int(blockIdx.x) % 2) * kAvgGroups + gr;
+    int64_t off[3] = {0, 0, 0}, g = 0;
+    int ns = 0;   // averaged directions the group extends in, 0: none here
+    if (qq < npencils(B, d) && is_avg(B.bc[d][0])) {
+        const int w = d == 0 ? B.n[1] : B.n[0], qa = qq % w, qb = qq / w;
+        const int idx[3] = {d == 0 ? 0 : qa, d == 1 ? 0 : (d == 0 ? qa : qb), d == 2 ? 0 : qb};
+        const int64_t stride[3] = {1, B.n[0], int64_t(B.n[0]) * B.n[1]};
+        // in order; other lanes have the group if one of its directions is at
+        // the high face here or comes before d
+        bool here = true;
+        for (int dd = 0; dd < 3; ++dd) {
+            if (!is_avg(B.bc[dd][0])) continue;
+            if (idx[dd] == B.n[dd] - 1 || (dd < d && idx[dd] == 0)) here = false;
+            if (idx[dd] == 0) off[ns++] = (B.n[dd] - 1) * stride[dd];
+        }
+        if (!here) ns = 0;
+        g = B.off + idx[0] + idx[1] * stride[1] + idx[2] * stride[2];
     }
-    const int64_t g = B.off + idx[0] + idx[1] * stride[1] + idx[2] * stride[2];
-    if (ns == 1) avg_group<1>(q, prim, NT, g, off);
-    else if (ns == 2) avg_group<2>(q, prim, NT, g, off);
-    else avg_group<3>(q, prim, NT, g, off);
+    double *mean = means + gr * 8 * 6;
+    if (l < 5) {
+        if (ns == 1) avg_group<1>(q + l * NT, mean + l, g, off);
+        else if (ns == 2) avg_group<2>(q + l * NT, mean + l, g, off);
+        else if (ns == 3) avg_group<3>(q + l * NT, mean + l, g, off);
+    }
+    __syncthreads();
+    if (prim && ns > 0 && l < (1 << ns)) {
+        double x[5], f[4];
+#pragma unroll
+        for (int m = 0; m < 5; ++m) x[m] = mean[6 * l + m];
+        prims_of(x, f);
+        const int64_t at = g + (l & 1 ? off[0] : 0) + (l & 2 ? off[1] : 0) + (l & 4 ? off[2] : 0);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) prim[m * NT + at] = f[m];
+    }
 }
 
 // ---- grid metrics (mo_grid.f90:107-186) ----------------------------------------
@@ -1118,11 +1131,11 @@ int enqueue_stage(cnd_ctx *c, int nk, bool whole)
     }
     if (c->avg_self) {
         const FaceSet fs = face_set(c, c->surf);
-        const int nft = fs.n01 + ntiles(c, 2), nfb = (nft + kPts / kLine - 1) / (kPts / kLine);
+        const int nfb = 2 * (fs.n01 + ntiles(c, 2));
         const bool prims = whole && nk < 4 && prims_wanted(c);
         c->ended = whole && nk == 4 && !c->any_frame;
         hipLaunchKernelGGL(k_self_avg, dim3(unsigned(nfb + (prims ? int(c->hpt.size()) : 0))), dim3(kPts), 0, c->st,
-                           c->dblk, c->dinst, c->ninst, fs, nft, nfb, c->dpt, c->qa, prims ? c->fl : nullptr, c->NT,
+                           c->dblk, c->dinst, c->ninst, fs, nfb, c->dpt, c->qa, prims ? c->fl : nullptr, c->NT,
                            c->ended ? 1 : 0);
     } else if (c->any_avg) {
         const FaceSet fs = face_set(c, c->surf);
