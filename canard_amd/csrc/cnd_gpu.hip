@@ -421,41 +421,35 @@ __global__ __launch_bounds__(kLine) void k_gcbc_setup(const BlkDev *__restrict__
     }
 }
 
-// gcbc_update of both faces of direction d (blockIdx.y; their bands of
-// kGcbcBand points never meet, a block having 13 points or more); the
-// directions follow each other in the reference's order.  Bound by latency:
-// a face has few points, each a long chain of loads and divisions, so every
-// point of the band has its own lane (threadIdx.y, one wave each) that forms
-// the face's correction itself, instead of one lane walking the band (13 us
-// a launch on faces of 80 x 70 points, at six launches a stage).
+// Number of characteristic faces along direction dd whose band of kGcbcBand
+// points holds the point of index i (at most one: a block has 13 points or
+// more), and its side.
 constexpr int kGcbcBand = 5;
-__global__ __launch_bounds__(kLine * kGcbcBand) void k_gcbc_update(const BlkDev *__restrict__ blks,
-                                                                  const InstDev *__restrict__ inst,
-                                                                  const TabDev *__restrict__ tabs,
-                                                                  const Tile *__restrict__ tiles, int d,
-                                                                  const double *q, double *de, const double *met,
-                                                                  const double *cmf, const double *drva, int64_t NT,
-                                                                  int64_t FT)
+__device__ __forceinline__ int gcbc_bands(const BlkDev &B, int dd, int i, int &side)
 {
-    const Tile t = tiles[blockIdx.x];
-    const BlkDev &B = blks[t.b];
-    const int side = blockIdx.y, qq = t.q0 + threadIdx.x, ii = threadIdx.y;
+    if (is_gcbc(B.bc[dd][0]) && i < kGcbcBand) { side = 0; return 1; }
+    if (is_gcbc(B.bc[dd][1]) && B.n[dd] - 1 - i < kGcbcBand) { side = 1; return 1; }
+    return 0;
+}
+
+// Correction of the right-hand side by the characteristic face (d, side) of
+// pencil qq of block B, before the spreading weight; res: 1 / yaco at the face
+// point.
+__device__ __forceinline__ void gcbc_correction(const BlkDev *__restrict__ blks, const BlkDev &B, const InstDev &I,
+                                                int d, int side, int qq, const double *q, const double *met,
+                                                const double *cmf, const double *drva, int64_t NT, int64_t FT,
+                                                double (&dha)[5], double &res)
+{
     const int code = B.bc[d][side];
-    if (qq >= npencils(B, d) || !is_gcbc(code)) return;
-    const InstDev &I = inst[B.inst];
-    int64_t base, st;
-    pencil_of(B, d, qq, base, st);
-    const int i0 = side == 0 ? 0 : B.n[d] - 1, ip = side == 0 ? ii : i0 - ii;
-    const int64_t g = base + int64_t(i0) * st, gl = base + int64_t(ip) * st;
-    // the right-hand side of the lane's own point, loaded with the face's data
-    double tot[5];
-    for (int c = 0; c < 5; ++c) tot[c] = (de[c * NT + gl] + de[(5 + c) * NT + gl]) + de[(10 + c) * NT + gl];
+    int64_t g, st;
+    face_point(B, d, qq, side, g, st);
     const int64_t fi = B.foff[d] + qq;
     const double ra0 = side == 0 ? 1.0 : -1.0;
-    double cm[3], q24[3], cha[5], dha[5], dif[5], xt[5][5];
+    double cm[3], q24[3], cha[5], dif[5], xt[5][5];
     for (int c = 0; c < 3; ++c) { cm[c] = cmf[(side * 3 + c) * FT + fi]; q24[c] = q[(c + 1) * NT + g]; }
-    const Elem e = eleme(cm, q[g], q24, pressure(q, NT, g), I.umf);
     for (int c = 0; c < 5; ++c) cha[c] = drva[(side * 5 + c) * FT + fi];
+    res = 1.0 / met[9 * NT + g];
+    const Elem e = eleme(cm, q[g], q24, pressure(q, NT, g), I.umf);
     for (int c = 0; c < 5; ++c) dif[c] = cha[c];
     if (code == 10) {
         if (ra0 * ((e.vn + e.vs) + e.ao) > 0.0) cha[3] = 0.0;
@@ -480,25 +474,62 @@ __global__ __launch_bounds__(kLine * kGcbcBand) void k_gcbc_update(const BlkDev 
         for (int c = 0; c < 5; ++c) s = s + xt[r][c] * dif[c];
         dha[r] = s;
     }
-    // spreading weights (gcbc_init, mo_gcbc.f90:82-129): 1/yaco of the face
-    // point, scaled by sbci for inward points, divided by the number of
-    // characteristic faces whose 5-point band covers the point.
-    const double res = 1.0 / met[9 * NT + g];
+}
+
+// gcbc_update of the characteristic faces of all directions: grid (face
+// tiles, side), block (pencils, band), a lane per point of a band.  A
+// correction reads its face's data only, and the right-hand side of its own
+// point, so a point in the bands of several directions takes their
+// corrections one after the other in the reference's order, from the lane of
+// the first.  Bound by latency: few points, each a long chain of loads and
+// divisions; with a launch per direction, 81 x 71 x 51 points with two such
+// directions took 2 x 11.2 us instead of 18.8, 15 M points 2 x 82 instead of 149.
+__global__ __launch_bounds__(kLine * kGcbcBand) void k_gcbc_update(const BlkDev *__restrict__ blks,
+                                                                  const InstDev *__restrict__ inst,
+                                                                  const TabDev *__restrict__ tabs, const FaceSet fs,
+                                                                  const Faces3 cmf3, const double *q, double *de,
+                                                                  const double *met, int64_t NT)
+{
+    int d;
+    const Tile t = fs.tile(blockIdx.x, d);
+    const BlkDev &B = blks[t.b];
+    const int qq = t.q0 + threadIdx.x, ii = threadIdx.y;
+    int side = blockIdx.y;
+    if (qq >= npencils(B, d) || !is_gcbc(B.bc[d][side])) return;
+    const int ip = side == 0 ? ii : B.n[d] - 1 - ii;
     const int w = d == 0 ? B.n[1] : B.n[0], qa = qq % w, qb = qq / w;   // pencil_of's transverse indices
     const int idx[3] = {d == 0 ? ip : qa, d == 1 ? ip : (d == 0 ? qa : qb), d == 2 ? ip : qb};
-    int cnt = 0;
-    for (int dd = 0; dd < 3; ++dd)
-        for (int s = 0; s < 2; ++s)
-            if (is_gcbc(B.bc[dd][s])) {
-                const int dist = s == 0 ? idx[dd] : B.n[dd] - 1 - idx[dd];
-                if (dist < kGcbcBand) ++cnt;
-            }
-    const double wv = ii == 0 ? res : res * tabs[B.inst].gcbc_w[ii - 1];
-    const double sbcc = wv / double(cnt);
+    // directions whose bands hold the point, and how many
+    int sd[3] = {0, 0, 0}, in[3], cnt = 0;
+    for (int dd = 0; dd < 3; ++dd) cnt += in[dd] = gcbc_bands(B, dd, idx[dd], sd[dd]);
+    for (int dd = 0; dd < d; ++dd)
+        if (in[dd]) return;
+    const InstDev &I = inst[B.inst];
+    const int64_t gl = B.off + idx[0] + int64_t(B.n[0]) * (idx[1] + int64_t(B.n[1]) * idx[2]);
+    double tot[5];
+    for (int c = 0; c < 5; ++c) tot[c] = (de[c * NT + gl] + de[(5 + c) * NT + gl]) + de[(10 + c) * NT + gl];
+#pragma unroll 1
+    for (int dd = d; dd < 3; ++dd) {
+        // (selects: a run-time index would put the arrays into scratch memory)
+        auto of = [&](auto x0, auto x1, auto x2) { return dd == 0 ? x0 : (dd == 1 ? x1 : x2); };
+        if (!of(in[0], in[1], in[2])) continue;
+        const int sf = of(sd[0], sd[1], sd[2]), i = of(idx[0], idx[1], idx[2]);
+        const int qd = of(idx[1] + B.n[1] * idx[2], idx[0] + B.n[0] * idx[2], idx[0] + B.n[0] * idx[1]);
+        double dha[5], res;
+        gcbc_correction(blks, B, I, dd, sf, qd, q, met, of(cmf3.p[0], cmf3.p[1], cmf3.p[2]),
+                        of(fs.sv[0], fs.sv[1], fs.sv[2]), NT, of(fs.FT[0], fs.FT[1], fs.FT[2]), dha, res);
+        // spreading weights (gcbc_init, mo_gcbc.f90:82-129): 1/yaco of the face
+        // point, scaled by sbci for inward points, divided by the number of
+        // characteristic faces whose band covers the point
+        const int dist = sf == 0 ? i : B.n[dd] - 1 - i;
+        const double wv = dist == 0 ? res : res * tabs[B.inst].gcbc_w[dist - 1];
+        const double sbcc = wv / double(cnt);
+        for (int c = 0; c < 5; ++c) tot[c] = tot[c] + sbcc * dha[c];
+    }
     // the right-hand side is the sum of the three direction buffers: the
     // corrected sum goes to the first, the others are cleared
     for (int c = 0; c < 5; ++c) {
-        de[c * NT + gl] = tot[c] + sbcc * dha[c];
+        de[c * NT + gl] = tot[c];
         de[(5 + c) * NT + gl] = 0.0;
         de[(10 + c) * NT + gl] = 0.0;
     }
@@ -1097,14 +1128,12 @@ int enqueue_stage(cnd_ctx *c, int nk, bool whole)
     }
     if (c->any_gcbc) {
         const FaceSet fs = face_set(c, c->drva);
-        Section sec(c, CND_SEC_GCBC, 1 + c->gcbc_dir[0] + c->gcbc_dir[1] + c->gcbc_dir[2]);
+        const Faces3 cmf3{{c->cmf[0], c->cmf[1], c->cmf[2]}};
+        Section sec(c, CND_SEC_GCBC, 2);
         hipLaunchKernelGGL(k_gcbc_setup, faces_grid(c), dim3(kLine), 0, c->st, c->dblk, c->dinst, fs,
-                           Faces3{{c->cmf[0], c->cmf[1], c->cmf[2]}}, cur, c->de, c->met, c->NT);
-        for (int d = 0; d < 3; ++d)
-            if (c->gcbc_dir[d])
-                hipLaunchKernelGGL(k_gcbc_update, tiles_grid(c, d, 2), dim3(kLine, kGcbcBand), 0, c->st, c->dblk,
-                                   c->dinst, c->dtab, c->dtiles[d], d, cur, c->de, c->met, c->cmf[d], c->drva[d],
-                                   c->NT, c->FT[d]);
+                           cmf3, cur, c->de, c->met, c->NT);
+        hipLaunchKernelGGL(k_gcbc_update, faces_grid(c), dim3(kLine, kGcbcBand), 0, c->st, c->dblk, c->dinst, c->dtab,
+                           fs, cmf3, cur, c->de, c->met, c->NT);
     }
     if (fused) {
         Section sec(c, CND_SEC_UPDATE, 1);
@@ -1245,7 +1274,7 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
                 B.qd[d][e] = (cd == kInterStraight || cd == kInterSub || cd == kPeriodic) ? 1 : 0;
                 if (B.qd[d][e] && B.part[d][e] != b) c->part_other[d] = true;
                 if (cd == kNonReflective || cd == kWallInviscid || cd == kWallViscous || cd == kInterCurv) {
-                    c->any_gcbc = c->gcbc_dir[d] = true; B.gcbc_any = 1;
+                    c->any_gcbc = true; B.gcbc_any = 1;
                 }
                 if (cd == kWallInviscid || cd == kWallViscous) c->any_wall = c->wall_dir[d] = true;
                 if (cd == kInterCurv || cd == kInterStraight || cd == kPeriodic) {
