@@ -70,7 +70,7 @@ struct cnd_ctx {
     std::vector<Tile> hstiles[kNumP][3];            // tiles of P pencils, longest pencils first
     std::vector<SegClass> classes[kNumL][kNumP][3];   // launches of segments of L points (seg_classes)
     Tile *dstiles[kNumP][3] = {};
-    double *dseg[kNumL] = {};                       // homogeneous solutions per L
+    double *dpk[kNumL] = {};                        // coefficients per L (SegTabs)
     // sweep shape per kind (CND_KIND_*) and direction: index into kShapes
     // or kTiled, with the segments per pencil of the launch (seg_sp)
     int shape[CND_NKIND][3] = {};
@@ -174,7 +174,7 @@ inline size_t seg_lds_bytes(const ShapeInfo &G, int nv, int sp, int nmax, bool h
 {
     const size_t ends = size_t(2) * kSegEndRows * nv * G.P, part = has_part ? ends : 0;
     const size_t ex = size_t(2) * nv * sp * G.P, lu = size_t(5) * G.L * sp, coef = size_t(8) * sp;
-    const size_t tile = size_t(nv) * G.P * size_t(nmax | 1);   // pencils n | 1 apart (SegShape::pencil_stride)
+    const size_t tile = size_t(nv) * G.P * size_t(nmax | 1) + 2 * kTilePad;   // pencils n | 1 apart (SegShape::pencil_stride)
     if (G.XI) return sizeof(double) * (std::max(tile, lu + ex) + coef + part);
     return sizeof(double) * (std::max(ends, ex) + coef + lu + part);
 }
@@ -297,10 +297,7 @@ inline SegLaunches seg_launches(const cnd_ctx *c, int kind, int d, int nv, bool 
         else { LAUNCH_SEG_EZ(K, c, sls, xm, y, __VA_ARGS__) }                                                \
     } while (0)
 
-inline SegTabs seg_tabs(cnd_ctx *c, int L)
-{
-    return SegTabs{c->dlu, c->dseg[l_index(L)]};
-}
+inline SegTabs seg_tabs(cnd_ctx *c, int L) { return SegTabs{c->dpk[l_index(L)]}; }
 inline bool seg_on(const cnd_ctx *c, int kind, int d) { return c->shape[kind][d] != kTiled; }
 
 

@@ -30,6 +30,7 @@ struct BlkDev {
     int64_t off;        // first global point index
     int64_t foff[3];    // first pencil of this block in per-direction face buffers
     int lu[2][3];       // first LU row (scheme, direction) in the LU table
+    int pk[3][2][3];    // the same in the segmented sweeps' table of each segment length (SegTabs)
 };
 
 // Per-instance scheme constants.

@@ -954,6 +954,31 @@ int shape_sp(cnd_ctx *c, int sh, int d, int nv)
     return sp;
 }
 
+// Appends the coefficients of a pencil of n points in segments of at most L
+// (SegTabs) from its LU rows; nothing where no partition fits.
+void seg_pack(const double *lu, int n, int L, std::vector<double> &out)
+{
+    const int S = seg_count(n, L);
+    if (S == 0) return;
+    std::vector<double> hom(4 * size_t(n), 0.0);
+    seg_tables(lu, S, [&](int k, int &a0, int &l0) { seg_bounds(n, L, S, k, a0, l0); }, hom.data());
+    const size_t at = out.size();
+    out.resize(at + size_t(S) * (5 * L + 8));
+    double *rows = out.data() + at, *sm = rows + size_t(S) * 5 * L;
+    for (int sg = 0; sg < S; ++sg) {
+        int a, len;
+        seg_bounds(n, L, S, sg, a, len);
+        for (int k = 0; k < L; ++k)
+            for (int c = 0; c < 5; ++c)
+                *rows++ = k < L - len ? seg_pass_row(c) : lu[5 * (a - (L - len) + k) + c];
+        for (int e = 0; e < 8; ++e) {
+            // phi at the last two rows (e 0..3), psi at the first two (e 4..7)
+            const int r = e < 4 ? a + len - 2 + (e >> 1) : a + ((e - 4) >> 1), c = e < 4 ? (e & 1) : 2 + (e & 1);
+            *sm++ = r >= 0 && r < n ? hom[4 * size_t(r) + c] : 0.0;
+        }
+    }
+}
+
 // Tiles of the segmented sweeps along d, blocks of longer pencils first, and
 // the classes that are launched together.  The lanes of a workgroup are those
 // its launch's longest pencil needs, so where blocks differ in length, lanes of
@@ -1300,14 +1325,9 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
                 const size_t at = lu.size();
                 lu.resize(at + 5 * size_t(s.n[d]));
                 lu_factors(c->htab[s.inst], sch, s.n[d], B.qd[d][0] != 0, B.qd[d][1] != 0, lu.data() + at);
-                const int nd = s.n[d];
                 for (int li = 0; li < kNumL; ++li) {
-                    const int SL = kLs[li], S = seg_count(nd, SL);
-                    segtab[li].resize(4 * (at / 5 + size_t(nd)), 0.0);
-                    if (S > 0)
-                        seg_tables(lu.data() + at, S,
-                                   [&](int k, int &a0, int &l0) { seg_bounds(nd, SL, S, k, a0, l0); },
-                                   segtab[li].data() + 4 * (at / 5));
+                    B.pk[li][sch][d] = int(segtab[li].size());
+                    seg_pack(lu.data() + at, s.n[d], kLs[li], segtab[li]);
                 }
             }
         }
@@ -1397,7 +1417,7 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
                 ok(dalloc(c, &c->de, 15 * NT)) && ok(dalloc(c, &c->grad, 12 * NT)) && ok(dalloc(c, &c->fl, 15 * NT)) &&
                 ok(dalloc(c, &c->met, 10 * NT)) && ok(dalloc(c, &c->ys, c->ys_len)) && ok(dalloc(c, &c->xyz, 3 * NT)) &&
                 ok(dalloc(c, &c->sp_par, 5 * ninst)) && ok(dalloc(c, &c->tstep_done, 1));
-    for (int li = 0; good && li < kNumL; ++li) good = ok(dalloc(c, &c->dseg[li], segtab[li].size()));
+    for (int li = 0; good && li < kNumL; ++li) good = ok(dalloc(c, &c->dpk[li], segtab[li].size()));
     if (good && c->any_sponge) good = ok(dalloc(c, &c->sponge, 2 * NT));
     if (good && precision == CND_MIXED) good = ok(dalloc(c, &c->gradf, 12 * NT));
     for (int d = 0; good && d < 3; ++d)
@@ -1442,7 +1462,7 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
     for (int pi = 0; pi < kNumP; ++pi)
         for (int d = 0; d < 3; ++d)
             up(c->dstiles[pi][d], c->hstiles[pi][d].data(), sizeof(Tile) * c->hstiles[pi][d].size());
-    for (int li = 0; li < kNumL; ++li) up(c->dseg[li], segtab[li].data(), sizeof(double) * segtab[li].size());
+    for (int li = 0; li < kNumL; ++li) up(c->dpk[li], segtab[li].data(), sizeof(double) * segtab[li].size());
     up(c->dpt, c->hpt.data(), sizeof(Tile) * c->hpt.size());
     if (!r) r = upload_inst(c);
     if (!r) {
@@ -1493,7 +1513,7 @@ void cnd_destroy(cnd_ctx *c)
                     c->jn.first, c->jn.tc, c->jn.sc, c->jn.write, c->jn.scale, c->jn.tmp, c->qb, c->tstep_done};
     for (void *p : ptrs) if (p) hipFree(p);
     for (int li = 0; li < kNumL; ++li)
-        if (c->dseg[li]) hipFree(c->dseg[li]);
+        if (c->dpk[li]) hipFree(c->dpk[li]);
     for (int d = 0; d < 3; ++d) {
         if (c->dtiles[d]) hipFree(c->dtiles[d]);
         for (int pi = 0; pi < kNumP && d != 2; ++pi)   // zeta's lists are part of eta's

@@ -39,9 +39,18 @@ namespace cnd {
 constexpr int kSegEnd = 12;
 constexpr int kSegEndRows = kSegEnd + 1;
 
+// Compiled segment lengths (coefficient tables).
+constexpr int kNumL = 3, kLs[kNumL] = {17, 33, 9};
+__host__ __device__ constexpr int l_index(int L) { return L == 17 ? 0 : (L == 33 ? 1 : 2); }
+
 // Fewest rows of a segment of at most L (seg_count); a whole pencil has 13 or
 // more.
 __host__ __device__ constexpr int seg_min_rows(int L) { return L < 17 ? 6 : 12; }
+
+// Doubles in front of and behind a xi tile in LDS: a lane reads its rows
+// without clamping those outside its line (they only reach rows that the
+// closure rows replace), at most 33 - 12 + 3 of them.
+constexpr int kTilePad = 24;
 
 // LU values a thread stages per round trip.
 constexpr int kLuBatch = 12;
@@ -82,7 +91,8 @@ struct SegShape {
     // transfer values [SP][8]; the LU rows of the launch's SP segments as
     // their lanes hold them [SP][L][5].  xi: the whole tile's sources
     // [NV][P][nmax | 1], and over them, once the closure rows are formed, the
-    // LU rows and the exchange buffer [2][NV][SP][P]; the transfer values.
+    // LU rows and the exchange buffer [2][NV][SP][P] (kTilePad doubles on
+    // either side of the tile); the transfer values.
     // Last, both, and only when some block has another block as its partner
     // along the sweep direction: the partner points [2][13][NV][P].
     // Total bytes: seg_lds_bytes.  (With a staging chunk, partner points and
@@ -217,10 +227,13 @@ __device__ __forceinline__ void seg_solve(double (&Y)[L], const SegLane &ln, con
     for (int k = 0; k < L; ++k) asm volatile("" : "+v"(Y[k]));
 }
 
-// Coefficient tables of the segmented sweeps, indexed like the LU rows:
-// LU factors and homogeneous solutions.
+// Coefficients of the segmented sweeps of one segment length L: at
+// BlkDev.pk, per block, scheme and direction, the LU rows as the lanes hold
+// them [S][L][5] (pass-through rows in front of a short segment's), then the
+// transfer values [S][8].  Laid out once by the host: formed entry by entry
+// in the sweep they took 400 of the 3500 instructions of a xi wave.
 struct SegTabs {
-    const double *lu, *seg;
+    const double *pk;
 };
 
 // Sinks that read operands of their own at each point (type Pre, filled by
@@ -258,15 +271,15 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     const int qds[2] = {B.qd[d][0], B.qd[d][1]}, parts[2] = {B.part[d][0], B.part[d][1]};
     const int codes[2] = {B.bc[d][0], B.bc[d][1]};
     const int S = seg_count(n, L);
-    const double *LU = tb.lu + 5 * int64_t(B.lu[SCH][d]);
-    const double *ST = tb.seg + 4 * int64_t(B.lu[SCH][d]);
-    const int nlu = 5 * L * SP;
+    const double *PK = tb.pk + B.pk[l_index(L)][SCH][d];
+    const int nlu = 5 * L * SP, nluS = 5 * L * S;   // (idle lanes' rows are not set)
     double *buf = lds;   // xi: the tile
     double *ends = nullptr, *part = nullptr, *LUs = nullptr, *ex = nullptr;
     double *SM = nullptr;   // [SP][8]
     const int exs2 = 2 * NV * SP * P;
     if constexpr (XI) {
-        const int fsz = NV * P * Sh::pencil_stride(n);
+        const int fsz = NV * P * Sh::pencil_stride(n) + 2 * kTilePad;
+        buf = lds + kTilePad;
         LUs = lds;
         ex = lds + nlu;
         SM = lds + (fsz > nlu + exs2 ? fsz : nlu + exs2);
@@ -285,13 +298,16 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     // follows FS doubles further on
     const int NS = Sh::pencil_stride(n), FS = P * NS;
     auto F = [&](int row) { return buf[(v * P + p) * NS + row]; };
-    auto place = [&](int e) { return (n & 1) ? e : e + e / n; };
+    // (e + e / n for even n: exact for e < 2^32 / n, one multiplication)
+    const unsigned inv_n = (n & 1) ? 0u : 0xffffffffu / unsigned(n) + 1u;
+    auto place = [&](int e) { return e + int(__umulhi(unsigned(e), inv_n)); };
     const bool pen_ok = tile.q0 + p < npen;
     const bool lane_ok = pen_ok && s < S;
     int a = 0, len = 0;
     if (s < S) seg_bounds(n, L, S, s, a, len);
     const int kb = L - len;                 // row a - kb + k is held in Y[k], kb <= k < L
-    auto have = [&](int k) { return k >= kb; };
+// (a segment has at least seg_min_rows(L) rows)
+    auto have = [&](int k) { return k >= L - seg_min_rows(L) || k >= kb; };
     auto pt = [&](int pp, int i) -> int64_t {
         int64_t pb, st;
         pencil_of(B, d, tile.q0 + pp, pb, st);
@@ -303,15 +319,6 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     //         pass-through rows, then the segment's rows; a thread's loads are
     //         issued together, kLuBatch per round trip) and the segments'
     //         transfer values into LDS
-    const int sq = n / (S > 0 ? S : 1), sr = n % (S > 0 ? S : 1);
-    auto lu_value = [&](int i) {   // entry i of the [SP][L][5] table
-        const int sg = i / (5 * L), k = (i / 5) % L, c = i % 5;
-        const int sl = sg < S ? sq + (sg < sr ? 1 : 0) : 0;
-        const int sa = sg * sq + (sg < sr ? sg : sr);
-        const bool real = k >= L - sl;
-        const double x = LU[real ? 5 * (sa - (L - sl) + k) + c : 0];
-        return real ? x : seg_pass_row(c);
-    };
     // xi: the first KPRE values per thread are loaded once the tile is
     // staged (their latency overlaps the right-hand sides and closure rows)
     // and written over the tile afterwards
@@ -320,34 +327,27 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     double lv[KPRE];
     auto lu_fetch = [&]() {
 #pragma unroll
-        for (int u = 0; u < KPRE; ++u) lv[u] = lu_value(t + u * nthr < nlu ? t + u * nthr : nlu - 1);
+        for (int u = 0; u < KPRE; ++u) lv[u] = PK[t + u * nthr < nluS ? t + u * nthr : nluS - 1];
     };
     auto lu_store = [&]() {
 #pragma unroll
         for (int u = 0; u < KPRE; ++u)
-            if (t + u * nthr < nlu) LUs[t + u * nthr] = lv[u];
-        for (int i0 = t + KPRE * nthr; i0 < nlu; i0 += kLuBatch * nthr) {
-            double w2[kLuBatch];
+            if (t + u * nthr < nluS) LUs[t + u * nthr] = lv[u];
+        if constexpr (KPRE0 > kLuBatch)
+            for (int i0 = t + KPRE * nthr; i0 < nluS; i0 += kLuBatch * nthr) {
+                double w2[kLuBatch];
 #pragma unroll
-            for (int u = 0; u < kLuBatch; ++u) w2[u] = lu_value(i0 + u * nthr < nlu ? i0 + u * nthr : nlu - 1);
+                for (int u = 0; u < kLuBatch; ++u) w2[u] = PK[i0 + u * nthr < nluS ? i0 + u * nthr : nluS - 1];
 #pragma unroll
-            for (int u = 0; u < kLuBatch; ++u)
-                if (i0 + u * nthr < nlu) LUs[i0 + u * nthr] = w2[u];
-        }
+                for (int u = 0; u < kLuBatch; ++u)
+                    if (i0 + u * nthr < nluS) LUs[i0 + u * nthr] = w2[u];
+            }
     };
     if constexpr (!XI) {
         lu_fetch();
         lu_store();
     }
-    for (int i = t; i < 8 * S; i += nthr) {
-        const int sp = i / 8, e = i % 8;
-        int sa, sl;
-        seg_bounds(n, L, S, sp, sa, sl);
-        // phi at the last two rows (e 0..3), psi at the first two (e 4..7)
-        const int r = e < 4 ? sa + sl - 2 + (e >> 1) : sa + ((e - 4) >> 1);
-        const int c = e < 4 ? (e & 1) : 2 + (e & 1);
-        SM[i] = (r >= 0 && r < n) ? ST[4 * r + c] : 0.0;
-    }
+    for (int i = t; i < 8 * S; i += nthr) SM[i] = PK[nluS + i];
 
     // ---- 1. stream the segment (with H halo points each side): interior
     //         right-hand sides into registers, end values into LDS
@@ -388,12 +388,11 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
         }
         __syncthreads();
         lu_fetch();
+        // (lanes without a segment read the line's first rows and store nothing)
+        const double *rows_in = &buf[(v * P + p) * NS + (s < S ? a - kb - H : 0)];
 #pragma unroll
         for (int kr = 0; kr < Sh::KR; ++kr) {
-            const int row = a - kb - H + kr;
-            // rows outside the line only reach the rows the closure rows
-            // replace (and lanes that store nothing): a clamped row serves
-            const double fv = F(row < 0 ? 0 : (row > N ? N : row));
+            const double fv = rows_in[kr];
 #pragma unroll
             for (int m = 0; m < 2 * H; ++m) w[m] = w[m + 1];
             w[2 * H] = fv;

@@ -427,14 +427,12 @@ template <class G, bool OPERANDS = false>
 __host__ __device__ constexpr int seg_waves() { return G::L > 17 ? 1 : (G::L == 17 && !G::XI && !OPERANDS ? 5 : 4); }
 constexpr int kSegMaxPoints = 528;   // longest pencil of a segmented sweep
 constexpr int kTiled = -1;   // shape index of the tiled sweep
-// pencils-per-workgroup values (tile lists) and segment lengths (tables)
+// pencils-per-workgroup values (tile lists)
 constexpr int kNumP = 7, kPs[kNumP] = {4, 8, 16, 32, 64, 20, 24};
-constexpr int kNumL = 3, kLs[kNumL] = {17, 33, 9};
 __host__ __device__ constexpr int p_index(int P)
 {
     return P == 4 ? 0 : (P == 8 ? 1 : (P == 16 ? 2 : (P == 32 ? 3 : (P == 64 ? 4 : (P == 20 ? 5 : 6)))));
 }
-__host__ __device__ constexpr int l_index(int L) { return L == 17 ? 0 : (L == 33 ? 1 : 2); }
 
 // Tiles of one direction d (split = ntiles), or of eta and zeta in one launch
 // (d = 1; tiles from split on are zeta's).
