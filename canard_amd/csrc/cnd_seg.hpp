@@ -303,10 +303,10 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     auto place = [&](int e) { return e + int(__umulhi(unsigned(e), inv_n)); };
     const bool pen_ok = tile.q0 + p < npen;
     const bool lane_ok = pen_ok && s < S;
-    int a = 0, len = 0;
-    if (s < S) seg_bounds(n, L, S, s, a, len);
+    int a, len;   // (lanes without a segment: the last one's, so that what they load is in the block)
+    seg_bounds(n, L, S, s < S ? s : S - 1, a, len);
     const int kb = L - len;                 // row a - kb + k is held in Y[k], kb <= k < L
-// (a segment has at least seg_min_rows(L) rows)
+    // (a segment has at least seg_min_rows(L) rows)
     auto have = [&](int k) { return k >= L - seg_min_rows(L) || k >= kb; };
     auto pt = [&](int pp, int i) -> int64_t {
         int64_t pb, st;
@@ -354,7 +354,8 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     double Y[L];
 #pragma unroll
     for (int k = 0; k < L; ++k) Y[k] = 0.0;
-    double W[Sh::KR];   // eta/zeta plain fields: the lane's source rows
+    double W[Sh::KR];   // eta/zeta: the lane's source rows
+    int64_t pb = 0, st = 0;   // and its pencil
     double w[2 * H + 1];
 #pragma unroll
     for (int m = 0; m <= 2 * H; ++m) w[m] = 0.0;
@@ -388,8 +389,7 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
         }
         __syncthreads();
         lu_fetch();
-        // (lanes without a segment read the line's first rows and store nothing)
-        const double *rows_in = &buf[(v * P + p) * NS + (s < S ? a - kb - H : 0)];
+        const double *rows_in = &buf[(v * P + p) * NS + (a - kb - H)];
 #pragma unroll
         for (int kr = 0; kr < Sh::KR; ++kr) {
             const double fv = rows_in[kr];
@@ -414,18 +414,25 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
         // eta/zeta: each lane loads its own rows, all at once.
         // The lanes of a wave hold P neighbouring pencils, so one load
         // instruction reads runs of P consecutive points.  Rows outside the
-        // lane's window are clamped into it (loaded but never used).
+        // lane's window are clamped into it (loaded but never used); those of
+        // the fewest rows a segment has need no clamp, and their places differ
+        // by the same offsets in all lanes.
         const int ppc = tile.q0 + p < npen ? p : npen - 1 - tile.q0;
-        int64_t pb, st;
         pencil_of(B, d, tile.q0 + ppc, pb, st);
         const int r0 = a - kb - H;                 // row held in W[0]
         const int rlo = (a - H) > 0 ? a - H : 0;
         const int rhi = (a + len + H - 1) < N ? a + len + H - 1 : N;
+        const int64_t g0 = pb + int64_t(r0) * st;
 #pragma unroll
         for (int kr = 0; kr < Sh::KR; ++kr) {
-            int row = r0 + kr;
-            row = row < rlo ? rlo : (row > rhi ? rhi : row);
-            W[kr] = src.field(pb + int64_t(row) * st, v);
+            if (kr >= L - seg_min_rows(L) + H && kr < L + H) {
+                W[kr] = src.field(g0 + int64_t(kr) * st, v);
+            } else {
+                // (n >= 13 along the other directions: st < 2^31)
+                int row = r0 + kr;
+                row = row < rlo ? rlo : (row > rhi ? rhi : row);
+                W[kr] = src.field(pb + int64_t(uint64_t(unsigned(row)) * unsigned(st)), v);
+            }
         }
         // the 13 points next to each pencil end, for the closure rows, from the
         // lanes whose rows they are
@@ -612,8 +619,6 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     if constexpr (!XI) {
         // eta/zeta: lanes of a wave hold P neighbouring pencils, stores coalesce
         if (lane_ok) {
-            int64_t pb, st;
-            pencil_of(B, d, tile.q0 + p, pb, st);
             pb += int64_t(a - kb) * st;
             if constexpr (sink_pre<Sink>::value) {
                 static_assert(!Sink::kReadBack, "prefetching sinks write results as they are");

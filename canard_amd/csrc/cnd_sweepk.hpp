@@ -419,7 +419,7 @@ using Sh28 = SegG<9, 64, 8, 16, false>;
 __host__ __device__ constexpr int wg_bound(int x) { return x > 1024 ? 1024 : x; }
 // waves per SIMD a segmented sweep is compiled for: eta / zeta sweeps of
 // 17-point segments are held to 96 VGPRs (5 waves) where that costs no spills,
-// not in the fused update, whose operand batches need more; other shapes of
+// not in the filter and the fused update, whose operands need more; other shapes of
 // up to 17 points to 128 (4 waves; those of 9 points need 84 to 102 anyway,
 // and forcing 80 spills), the others are left to the compiler.  4 -> 5 waves,
 // 129^3: joint gradient sweeps 59 -> 53 us, flux sweeps 87 -> 86 us.
@@ -465,7 +465,7 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
 }
 
 template <class G>
-__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_filter_field(
+__global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G, true>())) void k_seg_filter_field(
     const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles, const double *in, double *out, int64_t vstride)
 {
     SEG_PROLOGUE
