@@ -76,7 +76,7 @@ struct cnd_ctx {
     int shape[CND_NKIND][3] = {};
     int seg_sp[CND_NKIND][3] = {};
     bool tuned = false, tune_on = true, tiled_only = false;
-    bool fuse_update = true;   // last viscous flux sweep writes the RK update (CANARD_FUSE_UPDATE=0: separate)
+    bool fuse_update = true;   // last flux sweep writes the RK update (CANARD_FUSE_UPDATE=0: separate)
     int fuse_dir = 0;          // the direction of that sweep, 0 (xi) or 2 (zeta; CANARD_FUSE_DIR=2)
     bool recording = false;    // cnd_record: time averages accumulated in qb
     double *qb = nullptr;
@@ -85,8 +85,8 @@ struct cnd_ctx {
     std::vector<Tile> hpt;
     Tile *dpt = nullptr;
     // de: right-hand side as three 5-field buffers, one per flux direction
-    // (summed in the update); fl: the 15 stored fluxes F[5 d + m] of viscous
-    // stages, scratch for metrics, single sweeps and the autotuner otherwise
+    // (summed in the update); fl: the 15 stored fluxes F[5 d + m], before
+    // them a viscous stage's primitives; scratch for metrics, single sweeps and the autotuner otherwise
     double *qa = nullptr, *qo = nullptr, *de = nullptr, *grad = nullptr, *fl = nullptr, *met = nullptr;
     double *ys = nullptr, *xyz = nullptr, *sponge = nullptr, *sp_par = nullptr;
     int nmax[3] = {0, 0, 0};   // longest pencil per direction

@@ -43,9 +43,9 @@ namespace {
 // Evaluated in the sweeps instead, with all five components of a tile in one
 // workgroup and an update of its own after them, they saved 13 % of the
 // traffic but ran the sweeps at a third of the memory rate; a step of
-// 128^3 points 1.96 -> 1.48 ms, of 101 x 61 x 41 points 0.36 -> 0.30.  Writing them at the end of a stage with the averaging
-// (as the primitives are) took 38 us a launch of 101 x 61 x 41 points instead
-// of 11 + 10: the groups' lanes then hold 246 VGPRs.
+// 128^3 points 1.96 -> 1.48 ms, of 101 x 61 x 41 points 0.36 -> 0.30.  Writing
+// them at the end of a stage with the averaging, as the primitives are, made a
+// step of 128^3 points 5 % slower.
 __global__ __launch_bounds__(kPts) void k_inv_flux(const BlkDev *__restrict__ blks, const InstDev *__restrict__ inst,
                                                   const Tile *__restrict__ tiles, const double *__restrict__ q,
                                                   const double *__restrict__ met, double *__restrict__ F, int64_t NT)
@@ -87,8 +87,8 @@ __device__ __forceinline__ double wave_max(double v)
 //
 // Nine launches of ten find no instance due, so the grid is at most
 // kTstepBlocks workgroups that walk the tiles, and they leave after one look
-// at the instances: one workgroup per tile spent 40 us of a 257^3 step on
-// 66 k workgroups that only returned.
+// at the instances (one workgroup per tile of 257^3 points, 66 k of them only
+// to return: 86 us a step on average, now 77).
 constexpr unsigned kTstepBlocks = 2048;   // 8 workgroups of 4 waves on each of 256 CUs
 
 __device__ __forceinline__ void tstep_tile(const Tile t, const BlkDev *__restrict__ blks, InstDev *__restrict__ inst,

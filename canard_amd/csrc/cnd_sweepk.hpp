@@ -455,7 +455,8 @@ struct SegTiles {
 
 template <class G>
 __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k_seg_fd_field(
-    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles, int n45, const double *in, int64_t in_vstride, double *out, int64_t out_vstride)
+    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles, int n45,
+    const double *in, int64_t in_vstride, double *out, int64_t out_vstride)
 {
     SEG_PROLOGUE
     const int v = blockIdx.y;
@@ -466,7 +467,8 @@ __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G>())) void k
 
 template <class G>
 __global__ __launch_bounds__(wg_bound(G::P * G::SPMAX), (seg_waves<G, true>())) void k_seg_filter_field(
-    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles, const double *in, double *out, int64_t vstride)
+    const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs, SegTabs tb, const SegTiles tiles,
+    const double *in, double *out, int64_t vstride)
 {
     SEG_PROLOGUE
     const int v = blockIdx.y;

@@ -148,3 +148,47 @@ def test_every_shape_at_segment_edges_matches_the_tiled_sweeps(na, nb, other):
                     assert np.max(np.abs(got[b] - want[b])) <= 1e-13 * np.max(np.abs(want[b])), (d, sh, b)
         assert tried > 0
         c.close()
+
+
+# averaging groups of 2 (one periodic direction), 4 (two) and 8 points (three),
+# faces of fewer and more pencils than a workgroup takes, two instances; whole
+# steps, whose stages prepare each other, against stages called one by one
+@pytest.mark.parametrize("viscous", [1, 0])
+@pytest.mark.parametrize("periodic", [(0,), (1,), (2,), (0, 1), (0, 2), (1, 2), (0, 1, 2)])
+def test_whole_steps_equal_single_stages_and_oracle(monkeypatch, periodic, viscous):
+    monkeypatch.setenv("CANARD_TUNE", "0")   # the same shapes in both
+    blocks, grids, states = [], [], []
+    for i, (lx, ly, lz) in enumerate([(12, 15, 14), (33, 20, 17)]):
+        per = [d in periodic for d in range(3)]
+        blocks.append(dict(lxi=lx, let=ly, lze=lz, nbc=[[45, 45] if p else [10, 10] for p in per],
+                           mcd=[[i, i] if p else [-1, -1] for p in per], inst=i))
+        grids.append(cases.gridtoy(lx, ly, lz, doml0=0.0, doml1=2 * np.pi, domh=np.pi, span=2 * np.pi))
+        states.append(cases.tgv_state(grids[-1], (lx + 1, ly + 1, lz + 1), mach=0.1, pert=1e-3, seed=7 + i))
+    params = dict(fltk=0.49, fltrbc=0.9, reoo=1.6e4, cfl=0.8, viscous=viscous)
+    out = []
+    for whole in (True, False):
+        print(f"[stages] periodic={periodic} viscous={viscous} whole={whole}", flush=True)
+        c = Case(blocks, [params, params])
+        c.set_grids(grids)
+        c.set_states(states)
+        for i in range(2):
+            c.set_clock(inst=i)
+        if whole:
+            c.step(4)
+        else:
+            for _ in range(4):
+                c.filter()
+                for nk in range(1, 5):
+                    c.rk_stage(nk)
+                c.end_step()
+        out.append([c.state(b) for b in range(2)])
+        c.close()
+    for b in range(2):
+        assert np.array_equal(out[0][b], out[1][b]), b
+        blk = dict(blocks[b], mcd=[[0, 0] if m[0] >= 0 else [-1, -1] for m in blocks[b]["mcd"]])
+        o = oracle_for([blk], [grids[b]], [states[b]], params)
+        o.run(4)
+        err = rel_err(out[0][b], o.state(0))
+        print("  rel err per variable", err, flush=True)
+        assert np.all(err < 1e-12), (b, err)
+        o.close()
