@@ -106,7 +106,6 @@ struct cnd_ctx {
     bool avg_self = false;    // averaged faces, each between a block and itself
     bool ended = false;       // the step's last averaging has ended the step
     unsigned *tstep_done = nullptr;   // workgroups of k_tstep that are through
-    bool wall_dir[3] = {};   // directions with wall faces
     bool any_frame = false;   // some instance's frame accelerates (nsmf = 0)
     // staging of large reads (read_to_host), allocated by the first
     char *stage = nullptr;
