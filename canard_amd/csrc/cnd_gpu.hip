@@ -1473,9 +1473,12 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
     up(c->dpt, c->hpt.data(), sizeof(Tile) * c->hpt.size());
     if (!r) r = upload_inst(c);
     if (!r) {
-        hipError_t e = hipMemset(c->de, 0, sizeof(double) * 15 * NT);
-        if (e == hipSuccess) e = hipMemset(c->fl, 0, sizeof(double) * 15 * NT);
-        if (e == hipSuccess) e = hipMemset(c->tstep_done, 0, sizeof(unsigned));
+        // on the context's own stream: a hipMemset returns before the device is
+        // through, and the null stream is not ordered with a non-blocking one,
+        // so the clearing of fl could meet the metrics that follow in it
+        hipError_t e = hipMemsetAsync(c->de, 0, sizeof(double) * 15 * NT, c->st);
+        if (e == hipSuccess) e = hipMemsetAsync(c->fl, 0, sizeof(double) * 15 * NT, c->st);
+        if (e == hipSuccess) e = hipMemsetAsync(c->tstep_done, 0, sizeof(unsigned), c->st);
         if (e != hipSuccess) r = fail(c, CND_EDEVICE, "memset");
     }
     // junction averaging (search_point / search_line, average_point / average_line)
