@@ -343,8 +343,16 @@ int run_prims(cnd_ctx *c, const double *cur);
 int run_grad(cnd_ctx *c, int d, const double *cur, bool joint = false);
 int run_grad_flux(cnd_ctx *c, const double *cur);
 // Flux sweep along d into the d-th right-hand-side buffer (kind
-// CND_KIND_FLUX); joint as for run_grad.
-int run_flux(cnd_ctx *c, int d, bool joint = false);
+// CND_KIND_FLUX) of the stored fluxes, or, where it is a tiled one of an
+// inviscid context, of the state cur; joint as for run_grad.
+int run_flux(cnd_ctx *c, int d, const double *cur, bool joint = false);
+// The directions (bits) whose sweeps take an inviscid stage's stored fluxes.
+inline unsigned inv_flux_dirs(const cnd_ctx *c)
+{
+    unsigned m = 0;
+    for (int d = 0; d < 3; ++d) m |= seg_on(c, CND_KIND_FLUX, d) ? 1u << d : 0u;
+    return m;
+}
 // Flux sweep of the stored fluxes along fuse_dir (xi, or zeta) fused with the
 // RK update of stage nk, written to qa; the other two directions' buffers
 // must be complete.

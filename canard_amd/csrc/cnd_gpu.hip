@@ -39,22 +39,26 @@ namespace {
     if (lp >= npt) return;                                               \
     const int64_t g = B.off + lp;
 
-// Inviscid fluxes of all three directions, stored for the flux sweeps.
-// Evaluated in the sweeps instead, with all five components of a tile in one
-// workgroup and an update of its own after them, they saved 13 % of the
+// Inviscid fluxes stored for the segmented flux sweeps: of all three
+// directions, or (not ALL) of those in dirs, where tiled sweeps evaluate the
+// others' themselves (k_fd_flux).
+// Evaluated in the segmented sweeps too, with all five components of a tile in
+// one workgroup and an update of its own after them, they saved 13 % of the
 // traffic but ran the sweeps at a third of the memory rate; a step of
 // 128^3 points 1.96 -> 1.48 ms, of 101 x 61 x 41 points 0.36 -> 0.30.  Writing
 // them at the end of a stage with the averaging, as the primitives are, made a
 // step of 128^3 points 5 % slower.
+template <bool ALL>
 __global__ __launch_bounds__(kPts) void k_inv_flux(const BlkDev *__restrict__ blks, const InstDev *__restrict__ inst,
                                                   const Tile *__restrict__ tiles, const double *__restrict__ q,
-                                                  const double *__restrict__ met, double *__restrict__ F, int64_t NT)
+                                                  const double *__restrict__ met, double *__restrict__ F, int64_t NT,
+                                                  unsigned dirs)
 {
     POINT_PROLOGUE
     double v[5];
 #pragma unroll
     for (int m = 0; m < 5; ++m) v[m] = q[m * NT + g];
-    inv_point(inst[B.inst], g, v, met, F, NT);
+    inv_point<ALL>(inst[B.inst], g, v, met, F, NT, dirs);
 }
 
 // Viscous stresses, heat flux and fluxes (visc_point) from stored gradients of
@@ -1131,10 +1135,10 @@ int enqueue_stage(cnd_ctx *c, int nk, bool whole)
         }
         Section sec(c, CND_SEC_STRESS, xi_tiled ? 2 : 1);
         if ((r = run_xi_grad_flux(c, cur))) return r;
-    } else {
+    } else if (const unsigned dirs = inv_flux_dirs(c)) {
         Section sec(c, CND_SEC_STRESS, 1);
-        hipLaunchKernelGGL(k_inv_flux, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dinst, c->dpt, cur, c->met, c->fl,
-                           c->NT);
+        hipLaunchKernelGGL(dirs == 7u ? k_inv_flux<true> : k_inv_flux<false>, pts_grid(c), dim3(kPts), 0, c->st,
+                           c->dblk, c->dinst, c->dpt, cur, c->met, c->fl, c->NT, dirs);
     }
     const bool fused = fuse_possible(c) && seg_on(c, CND_KIND_FLUX, c->fuse_dir);
     {
@@ -1145,21 +1149,21 @@ int enqueue_stage(cnd_ctx *c, int nk, bool whole)
     const int other = fused && c->fuse_dir == 0 ? 2 : 0;
     if (joint) {
         if (fused) {
-            if ((r = run_flux(c, 1, true))) return r;
+            if ((r = run_flux(c, 1, cur, true))) return r;
         } else if (c->overlap) {
-            if ((r = on_side(c, [&] { return run_flux(c, 1, true); })) || (r = run_flux(c, 0)) ||
+            if ((r = on_side(c, [&] { return run_flux(c, 1, cur, true); })) || (r = run_flux(c, 0, cur)) ||
                 (r = join_side(c)))
                 return r;
-        } else if ((r = run_flux(c, 0)) || (r = run_flux(c, 1, true))) {
+        } else if ((r = run_flux(c, 0, cur)) || (r = run_flux(c, 1, cur, true))) {
             return r;
         }
     } else if (c->overlap && seg_on(c, CND_KIND_FLUX, 1)) {
-        if ((r = on_side(c, [&] { return run_flux(c, 1); })) || (r = run_flux(c, other)) ||
-            (!fused && (r = run_flux(c, 2))) || (r = join_side(c)))
+        if ((r = on_side(c, [&] { return run_flux(c, 1, cur); })) || (r = run_flux(c, other, cur)) ||
+            (!fused && (r = run_flux(c, 2, cur))) || (r = join_side(c)))
             return r;
     } else {
         for (int d = 0; d < 3; ++d)
-            if ((!fused || d != c->fuse_dir) && (r = run_flux(c, d))) return r;
+            if ((!fused || d != c->fuse_dir) && (r = run_flux(c, d, cur))) return r;
     }
     }
     if (c->any_gcbc) {
@@ -1676,7 +1680,7 @@ static int tune(cnd_ctx *c)
         if (kind == CND_KIND_GRAD && d == 0) return run_xi_grad_flux(c, c->qa);
         if (kind == CND_KIND_GRAD) return run_grad(c, d, c->qa, joint);
         if (d == c->fuse_dir && fz) return run_flux_update(c, 1, c->grad);
-        return run_flux(c, d, joint);
+        return run_flux(c, d, c->qa, joint);
     };
     auto set = [&](int kind, int d, int sh) {
         c->shape[kind][d] = sh;

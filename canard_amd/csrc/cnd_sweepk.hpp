@@ -144,16 +144,19 @@ __device__ __forceinline__ void visc_point(const InstDev &I, int64_t g, const do
     }
 }
 
-// Inviscid fluxes (src/mo_physics.f90:319-382) of all three directions of the
-// state q1..q5 at point g into F[5 d + m].
+// Inviscid fluxes (src/mo_physics.f90:319-382) of the state q1..q5 at point g
+// into F[5 d + m]: of all three directions, or (not ALL) of those whose bit is
+// set in dirs.
+template <bool ALL>
 __device__ __forceinline__ void inv_point(const InstDev &I, int64_t g, const double (&q)[5], const double *met,
-                                          double *F, int64_t NT)
+                                          double *F, int64_t NT, unsigned dirs)
 {
     const double ri = 1.0 / q[0];
     const double u = q[1] * ri, v = q[2] * ri, w = q[3] * ri;
     const double p = kGm1 * (q[4] - 0.5 * ((q[1] * u + q[2] * v) + q[3] * w));
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
+        if (!ALL && !(dirs >> d & 1)) continue;
         const double m[3] = {met[(3 * d) * NT + g], met[(3 * d + 1) * NT + g], met[(3 * d + 2) * NT + g]};
         double o[5];
         dir_flux<false>(q[0], q[1], q[2], q[3], q[4], u, v, w, p, m, I.umf, nullptr, o);
@@ -161,6 +164,33 @@ __device__ __forceinline__ void inv_point(const InstDev &I, int64_t g, const dou
         for (int c = 0; c < 5; ++c) F[(5 * d + c) * NT + g] = o[c];
     }
 }
+
+// Inviscid fluxes of direction d evaluated in a tiled sweep from q and the
+// metric row of d, with inv_point's arithmetic.
+struct SrcFlux {
+    const double *q;
+    const double *met;
+    const BlkDev *blks;
+    const InstDev *inst;
+    int64_t NT;
+    int d;
+    struct Raw { double q[5], m[3]; };
+    __device__ void load(int64_t g, int, Raw &r) const
+    {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) r.q[k] = q[k * NT + g];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) r.m[k] = met[(3 * d + k) * NT + g];
+    }
+    __device__ void finish(const Raw &r, int b, double (&o)[5]) const
+    {
+        const double q1 = r.q[0], q2 = r.q[1], q3 = r.q[2], q4 = r.q[3], q5 = r.q[4];
+        const double ri = 1.0 / q1;
+        const double u = q2 * ri, v = q3 * ri, w = q4 * ri;
+        const double p = kGm1 * (q5 - 0.5 * ((q2 * u + q3 * v) + q4 * w));
+        dir_flux<false>(q1, q2, q3, q4, q5, u, v, w, p, r.m, inst[blks[b].inst].umf, nullptr, o);
+    }
+};
 
 // ---- sinks ----------------------------------------------------------------
 // store / put write results; fold(f, x) is the value to write for source f
@@ -213,6 +243,17 @@ struct SinkFilt {  // out = f + correction
     __device__ double fold(double fv, double x) const { return fv + x; }
     __device__ void put_raw(int64_t g, int, int k, double x) { o[k * vs + g] = x; }
     __device__ void ends(int, int, int, double) {}
+};
+
+struct SinkFlux {  // the five components of dF/dxi_d; pencil ends to drva
+    double *de, *drva;
+    int64_t NT, FT, fi0;
+    __device__ void store(int64_t g, int, const double (&x)[5])
+    {
+#pragma unroll
+        for (int m = 0; m < 5; ++m) de[m * NT + g] = x[m];
+    }
+    __device__ void ends(int side, int lane, int m, double x) { drva[(side * 5 + m) * FT + fi0 + lane] = x; }
 };
 
 struct SinkFluxV {  // component v of dF/dxi_d; pencil ends to drva
@@ -319,8 +360,27 @@ __global__ __launch_bounds__(4 * kTile) void k_fd_grad(const BlkDev *__restrict_
     sweep_tile<4, 0, C>(blks, tabs, lu, tiles[tix], tix, d, 0, nmax, ys, src, sink, lds);
 }
 
-// Flux derivatives along d (src/mo_physics.f90:385-399) of the stored fluxes F
-// (component v = blockIdx.y) into the d-th right-hand-side buffer de.
+// Flux derivatives along d (src/mo_physics.f90:385-399) into the d-th
+// right-hand-side buffer de: inviscid fluxes evaluated in the sweep, five
+// waves on one tile.  With stored fluxes in a sweep per component, as the
+// segmented sweeps take them, a step of 601 x 561 x 541 points went from 154
+// to 177 ms: the forward values' scratch makes these sweeps bound by their
+// bytes, and the stored fluxes add 20 fields a stage to them.
+template <int C>
+__global__ __launch_bounds__(5 * kTile) void k_fd_flux(const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs,
+                                                  const InstDev *__restrict__ inst, const double *__restrict__ lu,
+                                                  const Tile *__restrict__ tiles, int ntiles, int d, int nmax,
+                                                  double *ys, const double *q, const double *met, double *de,
+                                                  double *drva, int64_t NT, int64_t FT)
+{
+    SWEEP_TILE_PROLOGUE(ntiles)
+    const Tile t = tiles[tix];
+    SrcFlux src{q, met, blks, inst, NT, d};
+    SinkFlux sink{de, drva, NT, FT, blks[t.b].foff[d] + t.q0};
+    sweep_tile<5, 0, C>(blks, tabs, lu, t, tix, d, 0, nmax, ys, src, sink, lds);
+}
+
+// ... or stored fluxes F (component v = blockIdx.y), the viscous case.
 template <int C>
 __global__ __launch_bounds__(kTile) void k_fd_flux_field(const BlkDev *__restrict__ blks,
                                                         const TabDev *__restrict__ tabs,
