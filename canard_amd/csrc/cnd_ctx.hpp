@@ -114,6 +114,7 @@ struct cnd_ctx {
     hipGraphExec_t gexec = nullptr;
     // section timers
     bool prof = false, capturing = false;
+    long long launched = 0;    // kernels launched through LAUNCH
     struct Mark { int sec; hipEvent_t a, b; int launches; };
     std::vector<Mark> marks;
     std::vector<hipEvent_t> pool;
@@ -154,14 +155,21 @@ inline int check_launch(cnd_ctx *c)
 inline dim3 tiles_grid(cnd_ctx *c, int d, int y) { return dim3(unsigned(c->htiles[d].size()), unsigned(y)); }
 inline dim3 sweep_grid(cnd_ctx *c, int d, int y) { return dim3(unsigned(xcd_width(int(c->htiles[d].size()))), unsigned(y)); }
 
+// A kernel launch, counted for the section timers.
+#define LAUNCH(c, ...)                                                                                     \
+    do {                                                                                                   \
+        ++(c)->launched;                                                                                   \
+        hipLaunchKernelGGL(__VA_ARGS__);                                                                   \
+    } while (0)
+
 // Launch a sweep kernel template K<C> with the chunk length of direction d.
 #define LAUNCH_SWEEP(K, NV, c, d, y, block, ...)                                                           \
     do {                                                                                                   \
         if ((d) == 0)                                                                                      \
-            hipLaunchKernelGGL(K<kChunkXi>, sweep_grid(c, d, y), dim3(block),                              \
+            LAUNCH(c, K<kChunkXi>, sweep_grid(c, d, y), dim3(block),                                       \
                                (sweep_lds_bytes<NV, kChunkXi>()), (c)->st, __VA_ARGS__);                    \
         else                                                                                               \
-            hipLaunchKernelGGL(K<kChunkEta>, sweep_grid(c, d, y), dim3(block),                             \
+            LAUNCH(c, K<kChunkEta>, sweep_grid(c, d, y), dim3(block),                                      \
                                (sweep_lds_bytes<NV, kChunkEta>()), (c)->st, __VA_ARGS__);                   \
     } while (0)
 inline dim3 pts_grid(cnd_ctx *c) { return dim3(unsigned(c->hpt.size())); }
@@ -242,7 +250,7 @@ inline SegLaunches seg_launches(const cnd_ctx *c, int kind, int d, int nv, bool 
 #define SEG_CASE(i, K, c, SL, y, ...)                                                                       \
     case i: {                                                                                              \
         using G = Sh##i;                                                                                   \
-        hipLaunchKernelGGL(K, dim3(unsigned(xcd_width(seg_xm * (SL).tiles.n)), unsigned(y)), dim3((SL).threads), \
+        LAUNCH(c, K, dim3(unsigned(xcd_width(seg_xm * (SL).tiles.n)), unsigned(y)), dim3((SL).threads),      \
                            (SL).lds, (c)->st, (c)->dblk, (c)->dtab, seg_tabs(c, G::L), (SL).tiles, __VA_ARGS__); \
     } break;
 // xi shapes, eta / zeta shapes

@@ -932,9 +932,10 @@ hipEvent_t pool_event(cnd_ctx *c)
 // Bracket a kernel group of section sec (no-op unless profiling eagerly).
 struct Section {
     cnd_ctx *c;
-    int sec, launches;
+    int sec;
+    long long first;   // launches before the group
     hipEvent_t a = nullptr;
-    Section(cnd_ctx *c_, int s, int n) : c(c_), sec(s), launches(n)
+    Section(cnd_ctx *c_, int s) : c(c_), sec(s), first(c_->launched)
     {
         if (c->prof && !c->capturing && (a = pool_event(c))) (void)hipEventRecord(a, c->st);
     }
@@ -944,7 +945,7 @@ struct Section {
         hipEvent_t b = pool_event(c);
         if (!b) { c->pool.push_back(a); return; }
         (void)hipEventRecord(b, c->st);
-        c->marks.push_back({sec, a, b, launches});
+        c->marks.push_back({sec, a, b, int(c->launched - first)});
     }
 };
 
@@ -1034,7 +1035,7 @@ void seg_classes(cnd_ctx *c, int d)
 // filtered state (which is also qo) ends in qo.
 int enqueue_filter(cnd_ctx *c)
 {
-    Section sec(c, CND_SEC_FILTER, 3);
+    Section sec(c, CND_SEC_FILTER);
     int r;
     if ((r = run_filter_field(c, 1, c->qa, c->qo, 5))) return r;
     if ((r = run_filter_field(c, 2, c->qo, c->qa, 5))) return r;
@@ -1081,7 +1082,7 @@ int run_xi_grad_flux(cnd_ctx *c, const double *cur)
 {
     if (seg_on(c, CND_KIND_GRAD, 0)) return run_grad_flux(c, cur);
     if (int r = run_grad(c, 0, cur)) return r;
-    hipLaunchKernelGGL(k_visc_flux, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dinst, c->dpt, cur, c->grad, c->met,
+    LAUNCH(c, k_visc_flux, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dinst, c->dpt, cur, c->grad, c->met,
                        c->fl, c->NT);
     return check_launch(c);
 }
@@ -1093,7 +1094,7 @@ int enqueue_stage(cnd_ctx *c, int nk, bool whole)
 {
     const double *cur = nk == 1 ? c->qo : c->qa;
     const unsigned ib = unsigned((c->ninst + 63) / 64);
-    if (c->any_frame) hipLaunchKernelGGL(k_stage_begin, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst, nk);
+    if (c->any_frame) LAUNCH(c, k_stage_begin, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst, nk);
     int r;
     // the time step of stage 1 runs beside the gradient sweeps of viscous
     // stages, which read neither dt nor the maxima (its time then counts in
@@ -1102,21 +1103,20 @@ int enqueue_stage(cnd_ctx *c, int nk, bool whole)
     if (nk == 1) {
         auto tstep = [&] {
             const int npt = int(c->hpt.size());
-            hipLaunchKernelGGL(k_tstep, dim3(std::min(unsigned(npt), kTstepBlocks)), dim3(kPts), 0, c->st, c->dblk,
+            LAUNCH(c, k_tstep, dim3(std::min(unsigned(npt), kTstepBlocks)), dim3(kPts), 0, c->st, c->dblk,
                                c->dinst, c->dtab, c->ninst, c->dpt, npt, cur, c->met, c->tstep_done, c->NT);
             return check_launch(c);
         };
-        Section sec(c, CND_SEC_TSTEP, 1);
+        Section sec(c, CND_SEC_TSTEP);
         if ((r = tstep_side ? on_side(c, tstep) : tstep())) return r;
     }
     if (c->any_visc) {
         // the primitives, then eta and zeta in one launch, or the eta sweep
         // beside the zeta sweep when it is a segmented one
         const bool joint = eta_zeta_joint(c, CND_KIND_GRAD);
-        const bool xi_tiled = !seg_on(c, CND_KIND_GRAD, 0);
         {
             const bool have = whole && nk > 1 && c->avg_self;   // primitives from the previous stage's end
-            Section sec(c, CND_SEC_GRAD, (joint ? 1 : 2) + (have ? 0 : 1));
+            Section sec(c, CND_SEC_GRAD);
             if (!have && (r = run_prims(c, cur))) return r;
             if (joint) {
                 if ((r = run_grad(c, 1, cur, true))) return r;
@@ -1133,11 +1133,11 @@ int enqueue_stage(cnd_ctx *c, int nk, bool whole)
                 }
             }
         }
-        Section sec(c, CND_SEC_STRESS, xi_tiled ? 2 : 1);
+        Section sec(c, CND_SEC_STRESS);
         if ((r = run_xi_grad_flux(c, cur))) return r;
     } else if (const unsigned dirs = inv_flux_dirs(c)) {
-        Section sec(c, CND_SEC_STRESS, 1);
-        hipLaunchKernelGGL(dirs == 7u ? k_inv_flux<true> : k_inv_flux<false>, pts_grid(c), dim3(kPts), 0, c->st,
+        Section sec(c, CND_SEC_STRESS);
+        LAUNCH(c, dirs == 7u ? k_inv_flux<true> : k_inv_flux<false>, pts_grid(c), dim3(kPts), 0, c->st,
                            c->dblk, c->dinst, c->dpt, cur, c->met, c->fl, c->NT, dirs);
     }
     const bool fused = fuse_possible(c) && seg_on(c, CND_KIND_FLUX, c->fuse_dir);
@@ -1145,7 +1145,7 @@ int enqueue_stage(cnd_ctx *c, int nk, bool whole)
     // the flux sweeps the update does not take in: eta and zeta in one launch,
     // or the eta one beside the others when it is a segmented one
     const bool joint = !(fused && c->fuse_dir == 2) && eta_zeta_joint(c, CND_KIND_FLUX);
-    Section sec(c, CND_SEC_FLUX, (fused ? 2 : 3) - (joint ? 1 : 0));
+    Section sec(c, CND_SEC_FLUX);
     const int other = fused && c->fuse_dir == 0 ? 2 : 0;
     if (joint) {
         if (fused) {
@@ -1169,44 +1169,44 @@ int enqueue_stage(cnd_ctx *c, int nk, bool whole)
     if (c->any_gcbc) {
         const FaceSet fs = face_set(c, c->drva);
         const Faces3 cmf3{{c->cmf[0], c->cmf[1], c->cmf[2]}};
-        Section sec(c, CND_SEC_GCBC, 2);
-        hipLaunchKernelGGL(k_gcbc_setup, faces_grid(c), dim3(kLine), 0, c->st, c->dblk, c->dinst, fs,
+        Section sec(c, CND_SEC_GCBC);
+        LAUNCH(c, k_gcbc_setup, faces_grid(c), dim3(kLine), 0, c->st, c->dblk, c->dinst, fs,
                            cmf3, cur, c->de, c->met, c->NT);
-        hipLaunchKernelGGL(k_gcbc_update, faces_grid(c), dim3(kLine, kGcbcBand), 0, c->st, c->dblk, c->dinst, c->dtab,
+        LAUNCH(c, k_gcbc_update, faces_grid(c), dim3(kLine, kGcbcBand), 0, c->st, c->dblk, c->dinst, c->dtab,
                            fs, cmf3, cur, c->de, c->met, c->NT);
     }
     // The update half's frame velocity is read only by the wall condition
     // (and, after the step, by the output); without walls the next stage's
     // frame velocity replaces it unread, and stage 4's is set at the end of
     // the step.
-    if (c->any_wall && c->any_frame) hipLaunchKernelGGL(k_stage_mid, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst, nk);
+    if (c->any_wall && c->any_frame) LAUNCH(c, k_stage_mid, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst, nk);
     if (fused) {   // (walls are characteristic faces: never with walls)
-        Section sec(c, CND_SEC_UPDATE, 1);
+        Section sec(c, CND_SEC_UPDATE);
         if ((r = run_flux_update(c, nk, c->qa))) return r;
     } else {
-        Section sec(c, CND_SEC_UPDATE, 1);
-        hipLaunchKernelGGL(c->any_wall ? k_update<true> : k_update<false>, pts_grid(c), dim3(kPts), 0, c->st, c->dblk,
+        Section sec(c, CND_SEC_UPDATE);
+        LAUNCH(c, c->any_wall ? k_update<true> : k_update<false>, pts_grid(c), dim3(kPts), 0, c->st, c->dblk,
                            c->dinst, c->dpt, cur, c->qo, c->de, c->met, c->sponge, c->qa, c->NT, nk);
     }
-    Section avg(c, CND_SEC_AVG, 1);
+    Section avg(c, CND_SEC_AVG);
     if (c->jn.n > 0) {
         const unsigned nb = unsigned((c->jn.n + 127) / 128);
-        hipLaunchKernelGGL(k_junc_gather, dim3(nb, 5), dim3(128), 0, c->st, c->jn, c->qa, c->NT);
-        hipLaunchKernelGGL(k_junc_scatter, dim3(nb, 5), dim3(128), 0, c->st, c->jn, c->qa, c->NT);
+        LAUNCH(c, k_junc_gather, dim3(nb, 5), dim3(128), 0, c->st, c->jn, c->qa, c->NT);
+        LAUNCH(c, k_junc_scatter, dim3(nb, 5), dim3(128), 0, c->st, c->jn, c->qa, c->NT);
     }
     if (c->avg_self) {
         const FaceSet fs = face_set(c, c->surf);
         const int nfb = 2 * (fs.n01 + ntiles(c, 2));
         const bool prims = whole && nk < 4 && prims_wanted(c);
         c->ended = whole && nk == 4 && !c->any_frame;
-        hipLaunchKernelGGL(k_self_avg, dim3(unsigned(nfb + (prims ? int(c->hpt.size()) : 0))), dim3(kPts), 0, c->st,
+        LAUNCH(c, k_self_avg, dim3(unsigned(nfb + (prims ? int(c->hpt.size()) : 0))), dim3(kPts), 0, c->st,
                            c->dblk, c->dinst, c->ninst, fs, nfb, c->dpt, c->qa, prims ? c->fl : nullptr, c->NT,
                            c->ended ? 1 : 0);
     } else if (c->any_avg) {
         const FaceSet fs = face_set(c, c->surf);
         const dim3 grid(unsigned(fs.n01 + ntiles(c, 2)), 2);
-        hipLaunchKernelGGL(k_surf_snap, grid, dim3(kLine), 0, c->st, c->dblk, fs, c->qa, c->NT);
-        hipLaunchKernelGGL(k_surf_avg, grid, dim3(kLine), 0, c->st, c->dblk, fs, c->qa, c->NT);
+        LAUNCH(c, k_surf_snap, grid, dim3(kLine), 0, c->st, c->dblk, fs, c->qa, c->NT);
+        LAUNCH(c, k_surf_avg, grid, dim3(kLine), 0, c->st, c->dblk, fs, c->qa, c->NT);
     }
     return check_launch(c);
 }
@@ -1215,13 +1215,13 @@ int enqueue_end(cnd_ctx *c)
 {
     const unsigned ib = unsigned((c->ninst + 63) / 64);
     if (!c->ended)
-        hipLaunchKernelGGL(k_end_step, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst,
+        LAUNCH(c, k_end_step, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst,
                            c->any_frame && !c->any_wall ? 1 : 0);
     c->ended = false;
     if (c->recording) {
-        hipLaunchKernelGGL(k_record, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dinst, c->dpt, c->qo, c->qa,
+        LAUNCH(c, k_record, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dinst, c->dpt, c->qo, c->qa,
                            c->qb, c->NT);
-        hipLaunchKernelGGL(k_record_clock, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst, 0);
+        LAUNCH(c, k_record_clock, dim3(ib), dim3(64), 0, c->st, c->dinst, c->ninst, 0);
     }
     return check_launch(c);
 }

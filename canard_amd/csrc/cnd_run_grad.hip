@@ -32,7 +32,7 @@ __global__ __launch_bounds__(kPts) void k_prims(const BlkDev *__restrict__ blks,
 int run_prims(cnd_ctx *c, const double *cur)
 {
     if (prims_wanted(c))
-        hipLaunchKernelGGL(k_prims, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dpt, cur, c->fl, c->NT);
+        LAUNCH(c, k_prims, pts_grid(c), dim3(kPts), 0, c->st, c->dblk, c->dpt, cur, c->fl, c->NT);
     return check_launch(c);
 }
 
