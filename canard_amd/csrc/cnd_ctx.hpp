@@ -195,8 +195,8 @@ struct SegLaunch {
 };
 
 // Eta and zeta sweeps of a kind go in one launch where both have the same
-// shape and the lanes the direction with fewer segments leaves idle are at
-// most a quarter: a launch of a small block is a chain of latencies (10-15 us
+// shape, its LDS serves both, and the lanes the direction with fewer segments
+// leaves idle are at most a quarter: a launch of a small block is a chain of latencies (10-15 us
 // from 17^3 to 65^3 points), so one launch takes half the time of two, and
 // on large blocks it fills the GPU as two streams did.
 inline bool eta_zeta_joint(const cnd_ctx *c, int kind)
@@ -206,6 +206,10 @@ inline bool eta_zeta_joint(const cnd_ctx *c, int kind)
     const int pi = p_index(kShapes[sh].P), li = l_index(kShapes[sh].L);
     if (c->classes[li][pi][1].size() > 1 || c->classes[li][pi][2].size() > 1) return false;
     const int a = c->segs[li][1], b = c->segs[li][2], m = std::max(a, b);
+    // the launch takes the more segments of the one and the partner points of either
+    if (seg_lds_bytes(kShapes[sh], 1, std::max(c->seg_sp[kind][1], c->seg_sp[kind][2]), std::max(c->nmax[1], c->nmax[2]),
+                      c->part_other[1] || c->part_other[2]) > size_t(c->lds_max))
+        return false;
     const int64_t na = int64_t(c->hstiles[pi][1].size()), nb = int64_t(c->hstiles[pi][2].size());
     return 4 * ((m - a) * na + (m - b) * nb) <= m * (na + nb);
 }
