@@ -94,7 +94,7 @@ struct cnd_ctx {
     bool part_other[3] = {};   // some block has another block as interface partner along d
     int64_t ys_len = 0;        // doubles in the forward-value scratch
     double *drva[3] = {}, *cmf[3] = {}, *surf[3] = {};
-    float *gradf = nullptr;   // mixed precision: the gradients in FP32
+    float *gradf = nullptr;   // mixed precision: the eta and zeta gradients (fields 4 .. 11) in FP32
     JuncDev jn;
     std::vector<char> grid_set;
     bool metrics_ready = false, state_in_qo = false;
@@ -196,9 +196,9 @@ struct SegLaunch {
 
 // Eta and zeta sweeps of a kind go in one launch where both have the same
 // shape, its LDS serves both, and the lanes the direction with fewer segments
-// leaves idle are at most a quarter: a launch of a small block is a chain of latencies (10-15 us
-// from 17^3 to 65^3 points), so one launch takes half the time of two, and
-// on large blocks it fills the GPU as two streams did.
+// leaves idle are at most a quarter: a launch of a small block is a chain of
+// latencies (10-15 us from 17^3 to 65^3 points), so one launch takes half the
+// time of two, and on large blocks it fills the GPU as two streams did.
 inline bool eta_zeta_joint(const cnd_ctx *c, int kind)
 {
     const int sh = c->shape[kind][1];

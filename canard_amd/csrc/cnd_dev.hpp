@@ -26,7 +26,6 @@ struct BlkDev {
     int part[3][2];     // partner block per face (-1: none)
     int qd[3][2];       // 1: quasi-disjoint closure rows at this face
     int inst;           // ensemble instance
-    int gcbc_any;       // any characteristic face in this block
     int64_t off;        // first global point index
     int64_t foff[3];    // first pencil of this block in per-direction face buffers
     int lu[2][3];       // first LU row (scheme, direction) in the LU table

@@ -1310,7 +1310,7 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
                 B.qd[d][e] = (cd == kInterStraight || cd == kInterSub || cd == kPeriodic) ? 1 : 0;
                 if (B.qd[d][e] && B.part[d][e] != b) c->part_other[d] = true;
                 if (cd == kNonReflective || cd == kWallInviscid || cd == kWallViscous || cd == kInterCurv) {
-                    c->any_gcbc = true; B.gcbc_any = 1;
+                    c->any_gcbc = true;
                 }
                 if (cd == kWallInviscid || cd == kWallViscous) c->any_wall = true;
                 if (cd == kInterCurv || cd == kInterStraight || cd == kPeriodic) {
@@ -1430,7 +1430,7 @@ int cnd_create(const cnd_params *params, int ninst, const cnd_block *blocks, int
                 ok(dalloc(c, &c->sp_par, 5 * ninst)) && ok(dalloc(c, &c->tstep_done, 1));
     for (int li = 0; good && li < kNumL; ++li) good = ok(dalloc(c, &c->dpk[li], segtab[li].size()));
     if (good && c->any_sponge) good = ok(dalloc(c, &c->sponge, 2 * NT));
-    if (good && precision == CND_MIXED) good = ok(dalloc(c, &c->gradf, 12 * NT));
+    if (good && precision == CND_MIXED && c->any_visc) good = ok(dalloc(c, &c->gradf, 12 * NT));
     for (int d = 0; good && d < 3; ++d)
         good = ok(dalloc(c, &c->dtiles[d], c->htiles[d].size())) && ok(dalloc(c, &c->drva[d], 10 * c->FT[d])) &&
                ok(dalloc(c, &c->cmf[d], 6 * c->FT[d])) && ok(dalloc(c, &c->surf[d], 10 * c->FT[d]));
@@ -1687,8 +1687,8 @@ static int tune(cnd_ctx *c)
         c->seg_sp[kind][d] = sh == kTiled ? 0 : shape_sp(c, sh, d, kind_nv(kind, d));
     };
     // a compiled shape worth timing: it fits, no shape with the same segments
-    // and pencils but fewer segments per pencil does, and, for sweeps that
-    // stage nothing in runs, none that differs in the run length only
+    // and pencils but fewer segments per pencil does, and none before it that
+    // differs in the run length only
     auto worth = [&](int kind, int d, int sh) {
         const int nv = kind_nv(kind, d);
         if (shape_sp(c, sh, d, nv) == 0) return false;
@@ -1697,7 +1697,7 @@ static int tune(cnd_ctx *c)
             const ShapeInfo &B = kShapes[o];
             if (o == sh || B.L != A.L || B.P != A.P || B.XI != A.XI || shape_sp(c, o, d, nv) == 0) continue;
             if (B.SPMAX < A.SPMAX) return false;
-            if (B.SPMAX == A.SPMAX && (A.XI || nv == 1) && o < sh) return false;
+            if (B.SPMAX == A.SPMAX && o < sh) return false;
         }
         return true;
     };

@@ -58,9 +58,10 @@ constexpr int kLuBatch = 12;
 // Points whose sources a thread reads back together at a xi store.
 constexpr int kOutBatch = 8;
 
-// Segments of an n-point pencil for lanes of at most L points: 0 when no
-// partition fits (a segment holding a pencil end must contain the 12 points
-// its closure rows use).  Segments are as even as possible.
+// Segments of an n-point pencil for lanes of at most L points: 0 when one of
+// them would have fewer than seg_min_rows(L) rows.  The closure rows of an end
+// lie inside one segment that way; the source values they are formed from may
+// come from several lanes.  Segments are as even as possible.
 __host__ __device__ inline int seg_count(int n, int L)
 {
     const int S = (n + L - 1) / L;
@@ -106,11 +107,12 @@ struct SegShape {
 // same order (pencils n | 1 points apart), so staging and stores address
 // both by e.
 
-// One lane's view of its segment: rows a .. a + len - 1 of the line, held
-// right-aligned in Y[kb .. L - 1] (kb = L - len); Y[0 .. kb - 1] are
-// pass-through registers.
+// One lane's segment s of the S of its line, held right-aligned in
+// Y[kb .. L - 1]; Y[0 .. kb - 1] are pass-through registers.  exi: the lane's
+// place in the exchange buffer, segments P apart, the second value of a pair
+// exs further on; ok: the lane has a segment.
 struct SegLane {
-    int a, len, kb, s, S, n, L, ok, exi, exs, v, p, P, SP;
+    int kb, s, S, ok, exi, exs, P;
 };
 
 // LU row of a pass-through register: the forward step y = (Y - l0 ya) - l1 yb
@@ -244,11 +246,13 @@ template <class S> struct sink_pre<S, std::void_t<typename S::Pre>> : std::true_
 
 // One tile of P pencils of block tile.b along d.
 //  Src: load(g, b, Raw&), finish(Raw, b, double (&)[NV])
-//  Sink: store(g, b, const double (&)[NV]), put(g, b, v, x), ends(side, pencil, v, x);
+//  Sink: ends(side, pencil, v, x) and, by sweep and kind,
+//        store(g, b, const double (&)[NV]): xi sweeps, all variables of a point;
 //        fold(f, x): the value to write given the source f and the result x,
-//        put_raw: write such a value (eta/zeta sweeps, which still hold the
-//        source in registers, use these instead of put);
-//        optionally Pre, pre and put_pre (sink_pre)
+//        put_raw(g, b, v, y): write such a value (eta/zeta sweeps, which still
+//        hold the source in registers, and xi ones with kReadBack, which read
+//        it back with src(g, v));
+//        Pre, pre and put_pre (sink_pre) instead of these
 template <int NV, int SCH, int L, int P, bool XI, class Src, class Sink>
 __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const TabDev *__restrict__ tabs,
                                          const SegTabs &tb, Tile tile, int d, int n45, int SP, const Src &src,
@@ -604,7 +608,7 @@ __device__ __forceinline__ void seg_tile(const BlkDev *__restrict__ blks, const 
     }
 
     // ---- 4. solve ---------------------------------------------------------------
-    const SegLane ln{a, len, kb, s, S, n, L, lane_ok, (v * SP + s) * P + p, NV * SP * P, v, p, P, SP};
+    const SegLane ln{kb, s, S, lane_ok, (v * SP + s) * P + p, NV * SP * P, P};
     seg_solve<L>(Y, ln, LUs, SM, ex);
     if (lane_ok && s == 0) {
         double x0 = 0.0;
