@@ -11,7 +11,7 @@ state resident in HBM.
 
 Prints one JSON line.  value = nominal cells x 4 RK stages x K / seconds.
 With --compare-mixed 1 (the default for an FP64 run) the same workload is
-then run in mixed precision (FP32 gradients) for the same W + K steps; the
+then run in mixed precision (FP32 eta and zeta gradients) for the same W + K steps; the
 line's "mixed" object gives its rate, its speed-up over FP64 and the max-norm relative error of
 each conserved variable against the FP64 state after W + K steps.
 """
@@ -150,7 +150,7 @@ def ensemble_compare(steps, warmup, count=32, sizes=(32, 48, 64, 96, 128)):
     replayed as a hipGraph.  Batched: every instance in one context, one
     launch per kernel over all of them.  Separate: one context (and stream)
     per instance, all queued before any is waited for.  Batched mixed: the
-    batched context in mixed precision (FP32 gradients).  All are autotuned and warmed up before the timed steps."""
+    batched context in mixed precision (FP32 eta and zeta gradients).  All are autotuned and warmed up before the timed steps."""
     from canard_amd import cases
     from canard_amd.solver import CND_FP64, CND_MIXED, Case
     blocks, grids, states, params, draws = cases.config4(count=count, sizes=sizes)
@@ -283,7 +283,7 @@ def main():
                  "speedup_vs_fp64": dt / dtm, "steps_compared": a.warmup + a.steps,
                  "max_rel_err_per_variable": err, "error_target": 1e-6,
                  "sections_ms_per_step": {k: v[0] / a.steps for k, v in msec.items()},
-                 "note": "FP32 velocity and temperature gradients; line solves, state, metrics, fluxes, right-hand "
+                 "note": "FP32 velocity and temperature gradients along eta and zeta; line solves, state, metrics, fluxes, right-hand "
                          "sides, RK update and GCBC in FP64. Error: max-norm over the field after warmup + steps steps against the FP64 run, "
                          "momentum components against the largest momentum component."}
         del qm

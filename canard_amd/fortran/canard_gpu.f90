@@ -10,7 +10,7 @@
 ! nml_physics, nml_gridgen, nml_sponge as in the reference (README.md:44-99),
 ! plus nml_gpu for the switches of the GPU library:
 !   viscous   (1)  Navier-Stokes (the reference's -DVISCOUS build) or Euler (0)
-!   precision (0)  0 FP64, 1 mixed (FP32 gradients)
+!   precision (0)  0 FP64, 1 mixed (FP32 eta and zeta gradients)
 !   maxsteps  (-1) stop after this many steps as well (-1: no cap)
 !   icase  ('vortex') initial condition for nts=0: 'vortex' (initialo,
 !          mo_physics.f90:117-140) or 'tgv' (Taylor-Green vortex)

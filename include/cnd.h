@@ -39,11 +39,13 @@ enum {
     CND_ENOMEM = -4
 };
 
-/* Precision of the step: CND_FP64; CND_MIXED, the stage's velocity and
- * temperature gradients stored in FP32 (line solves, state, metrics, fluxes,
- * right-hand sides, RK update and characteristic boundaries are FP64: an FP32
- * line solve needs an FP64 refinement to stay within 1e-6 of FP64 over a
- * run, and the two together cost more than the FP64 solve).                */
+/* Precision of the step: CND_FP64; CND_MIXED, a viscous stage's velocity and
+ * temperature gradients along eta and zeta stored in FP32 (xi gradients, line
+ * solves, state, metrics, fluxes, right-hand sides, RK update and
+ * characteristic boundaries are FP64: an FP32 line solve needs an FP64
+ * refinement to stay within 1e-6 of FP64 over a run, and the two together
+ * cost more than the FP64 solve).  Steps without viscous terms are those of
+ * CND_FP64.                                                                */
 enum { CND_FP64 = 0, CND_MIXED = 1 };
 
 typedef struct cnd_ctx cnd_ctx;
@@ -150,11 +152,14 @@ int cnd_filter_sweep(cnd_ctx *ctx, int dir, double *const *f);
  * (mo_timer.f90:84-98): HIP events on the context stream bracket every
  * kernel group while profiling is on (not inside graph replays).
  * Sections: CND_SEC_FILTER (filter sweeps), CND_SEC_TSTEP (time step),
- * CND_SEC_GRAD (velocity/temperature gradient sweeps), CND_SEC_STRESS
- * (stress assembly), CND_SEC_FLUX (flux sweeps), CND_SEC_GCBC,
- * CND_SEC_UPDATE (sponge + RK update), CND_SEC_AVG (wall, junction and
- * surface averaging).  cnd_profile_read synchronizes and returns the summed
- * milliseconds and kernel launches of one section since the last enable.   */
+ * CND_SEC_GRAD (primitives, eta and zeta gradient sweeps), CND_SEC_STRESS
+ * (xi gradients, stresses and stored fluxes), CND_SEC_FLUX (flux sweeps the
+ * update is not part of), CND_SEC_GCBC, CND_SEC_UPDATE (sponge, RK update and
+ * wall condition, with the last flux sweep where that carries the update),
+ * CND_SEC_AVG (junction and surface averaging, with the next stage's
+ * primitives and the end of the step where one launch does all).
+ * cnd_profile_read synchronizes and returns the summed milliseconds and
+ * kernel launches of one section since the last enable.                    */
 enum { CND_SEC_FILTER = 0, CND_SEC_TSTEP, CND_SEC_GRAD, CND_SEC_STRESS, CND_SEC_FLUX,
        CND_SEC_GCBC, CND_SEC_UPDATE, CND_SEC_AVG, CND_NSEC };
 int cnd_profile(cnd_ctx *ctx, int enable);
@@ -217,10 +222,10 @@ int cnd_write_plt(const char *path, const char *title, int file_type, int nvar,
  * (gradient sweeps), CND_KIND_FLUX (flux sweeps), CND_KIND_FIELD (single
  * field sweeps: metrics, cnd_deriv_sweep).  Before the first step (or on
  * cnd_tune) every compiled shape that fits the blocks -- segments of L
- * points (lanes per pencil), pencils per workgroup, staging run length --
- * and, in FP64, the tiled one-lane-per-pencil sweep are timed on the
- * context's arrays per kind and direction, and the fastest is kept; all of
- * them give the same values up to rounding.  CANARD_TUNE=0 in the
+ * points (lanes per pencil), pencils per workgroup -- and, in FP64, the tiled
+ * one-lane-per-pencil sweep are timed on the context's arrays per kind and
+ * direction (eta and zeta together where they can share a launch), and the
+ * fastest is kept; all of them give the same values up to rounding.  CANARD_TUNE=0 in the
  * environment keeps the defaults.  cnd_tuning reports the choice: shape
  * index (-1: tiled), segment length L (0: tiled), pencils per workgroup,
  * segments per pencil in the launch, and the measured milliseconds (0 if
@@ -231,8 +236,8 @@ int cnd_tune(cnd_ctx *ctx);
  * the automatic tuning off for this context.                               */
 int cnd_set_shape(cnd_ctx *ctx, int kind, int dir, int shape);
 /* Compiled shape number shape (0, 1, ...): segment length, pencils per
- * workgroup, staging run length, and whether it is a xi (1) or eta/zeta (0)
- * shape; CND_EINVAL past the last one.                                     */
+ * workgroup, a run length that no sweep uses any more, and whether it is a xi
+ * (1) or eta/zeta (0) shape; CND_EINVAL past the last one.                 */
 int cnd_shape_info(int shape, int *seg_len, int *pencils, int *run, int *xi);
 int cnd_tuning(const cnd_ctx *ctx, int kind, int dir, int *shape, int *seg_len,
                int *pencils, int *segments, double *ms);
