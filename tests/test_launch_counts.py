@@ -68,7 +68,8 @@ def stub(tmp_path_factory):
 @pytest.mark.parametrize("name", CASES)
 def test_sections_count_every_launch(stub, name):
     code = CHILD.format(root=ROOT, stub=stub, case=CASES[name])
-    r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, LD_PRELOAD=stub, CANARD_TUNE="0"),
+    preload = " ".join([stub] + os.environ.get("LD_PRELOAD", "").split())   # in front of what is there
+    r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, LD_PRELOAD=preload, CANARD_TUNE="0"),
                        capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr
     word = r.stdout.split()

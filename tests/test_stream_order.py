@@ -43,7 +43,8 @@ def stub(tmp_path_factory):
 @pytest.mark.parametrize("case", [SELF, FREE, PAIR], ids=["self", "free", "pair"])
 def test_first_work_of_a_context_is_ordered(stub, case):
     code = CHILD.format(root=ROOT, stub=stub, mcd=case[0], nbc=case[1])
-    r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, LD_PRELOAD=stub, CANARD_TUNE="0"),
+    preload = " ".join([stub] + os.environ.get("LD_PRELOAD", "").split())   # in front of what is there
+    r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, LD_PRELOAD=preload, CANARD_TUNE="0"),
                        capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr
     word = r.stdout.split()
